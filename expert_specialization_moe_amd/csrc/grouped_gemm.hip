@@ -1105,73 +1105,82 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   if (num_experts < kXcds && e >= num_experts && e < kXcds) ws[ws_xcd_counter(e)] = 0;
 }
 
+// Sum of `v` over this lane and the lanes below it, on the vector ALU alone (DPP row shifts and row broadcasts; a
+// ds_bpermute shuffle costs a trip to LDS per step).
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, :2, :4, :8 (rows of 16 lanes)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 // The schedule built by the GEMM kernel itself (one launch per call; schedule.h, kSelfScheduleMaxExperts): every
-// workgroup does what schedule_kernel does, one thread per expert, with block-wide scans instead of that kernel's
-// per-thread loops (this runs in front of every workgroup's first tile), and writes the records into `ws`, where
-// the hand-out loop finds them with scalar loads.  All workgroups write the same values.  The launch constants are
-// returned instead of stored.  `lds` is the ring, free before the first tile.
+// workgroup does what schedule_kernel does and writes the records into `ws`, where the hand-out loop finds them with
+// scalar loads.  All workgroups write the same values.  The launch constants are returned instead of stored.  `lds` is
+// the ring, free before the first tile.
+//
+// This runs in front of every workgroup's first tile, so it is latency from end to end.  The ranking compares every pair
+// of experts: all 512 threads share that work (512 / E threads per expert, each over its slice of the other experts,
+// four keys to an LDS read), and the prefix sums stay on the vector ALU.  One thread per expert walking all others took
+// 2.6 / 4.4 / 7.9 / 13.7 us at 8 / 32 / 128 / 256 experts; whole calls this way: 8 experts x 32 rows x 256 x 512
+// 10.5 -> 9.4 us, 256 x 32 x 7168 x 256 173.9 -> 163.9 us, 128 x 8 x 768 x 4096 82.9 -> 77.2 us, 32 x 8 x 7168 x 2048
+// 79.1 -> 77.5 us.
 __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, int& hblocks, int& ltotal, int& lsplit, int& lshare) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
-  int* s_m = (int*)lds;                         // rows by expert
-  int* s_blocks = s_m + kThreads;               // heavy blocks by schedule position
-  int* s_items = s_blocks + kThreads;           // light items by schedule position
-  int* s_wave = s_items + kThreads;             // per wavefront: blocks, items
-  long* s_cost = (long*)(s_wave + 2 * kWaves);  // per wavefront: heavy cost, light cost
-  const int E = g.num_experts, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int* s_key = (int*)lds;                       // order keys by expert, the list padded with keys that come last
+  int* s_rank = s_key + kThreads;               // schedule position by expert
+  v4i* s_rec = (v4i*)(s_rank + kThreads);       // by schedule position: heavy blocks, light items, expert, rows
+  int* s_wave = (int*)(s_rec + kThreads);       // per wavefront: blocks, items
+  long* s_cost = (long*)(s_wave + 2 * kWaves);  // per expert: heavy cost, light cost
+  const int E = g.num_experts, t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const SchedPolicy policy = g.policy;
   int* ws = g.ws;
   int m = 0;
   if (t < E) m = g.problem_sizes[t * 3];
   if (m < 0) m = 0;
-  s_m[t] = m;
-  s_blocks[t] = 0;
-  s_items[t] = 0;
+  const int key = sched_order_key(m, policy);
+  s_key[t] = t < E ? key : 0x7fffffff;
+  s_rank[t] = 0;
+  const int epad = E > 1 ? 1 << (32 - __builtin_clz(E - 1)) : 1;   // experts, rounded up to a power of two (at most 512)
+  const int logp = 31 - __builtin_clz(epad), parts = kThreads >> logp;
   __syncthreads();
-  long hc = 0, lc = 0;
-  if (t < E) {
-    int pos = t;
-    if (policy.order != 1) {
-      pos = 0;
-      const int key = sched_order_key(m, policy);
-      for (int j = 0; j < E; j++) {
-        const int kj = sched_order_key(s_m[j], policy);
-        pos += (kj < key) || (kj == key && j < t);
-      }
+  if (policy.order != 1) {
+    // slice `part` of the other experts, in fours; an expert comes in front of another of the same key if its index is lower
+    const int e = t & (epad - 1), part = t >> logp;
+    const int quads = (epad + 3) >> 2, per = (quads + parts - 1) / parts;
+    const int ke = s_key[e];
+    int rank = 0;
+    for (int q = part * per; q < (part + 1) * per && q < quads; q++) {
+      const v4i k = *(const v4i*)(s_key + q * 4);
+#pragma unroll
+      for (int i = 0; i < 4; i++) rank += k[i] < ke + (q * 4 + i < e ? 1 : 0);
     }
-    ws[ws_rec(pos) + kRecExpert] = t;
-    ws[ws_rec(pos) + kRecRows] = m;
-    s_blocks[pos] = sched_heavy_blocks(m, g.n, policy);
-    s_items[pos] = sched_light_items(m, g.n, policy);
-    hc = sched_heavy_cost(m, g.n, policy);
-    lc = sched_light_cost(m, g.n, policy);
+    if (e < E && rank) atomicAdd(&s_rank[e], rank);
   }
+  s_rec[t] = v4i{0, 0, 0, 0};
+  int hb = 0, li = 0;
+  if (t < E) {
+    hb = sched_heavy_blocks(m, g.n, policy);
+    li = sched_light_items(m, g.n, policy);
+    s_cost[2 * t] = sched_heavy_cost(m, g.n, policy);
+    s_cost[2 * t + 1] = sched_light_cost(m, g.n, policy);
+  }
+  __syncthreads();
+  if (t < E) s_rec[policy.order != 1 ? s_rank[t] : t] = v4i{hb, li, t, m};
   __syncthreads();
   // exclusive prefix sums over the schedule positions (thread = position): inclusive scan inside the wavefront, then
   // the totals of the wavefronts in front
-  const int b = s_blocks[t], it = s_items[t];
-  int sb = b, si = it;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int ub = __shfl_up(sb, d), ui = __shfl_up(si, d);
-    if (lane >= d) {
-      sb += ub;
-      si += ui;
-    }
-  }
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    hc += __shfl_xor(hc, d);
-    lc += __shfl_xor(lc, d);
-  }
+  const v4i rec = s_rec[t];
+  const int sb = wave_inclusive_sum(rec[0]), si = wave_inclusive_sum(rec[1]);
   if (lane == 63) {
     s_wave[2 * wave] = sb;
     s_wave[2 * wave + 1] = si;
-    s_cost[2 * wave] = hc;
-    s_cost[2 * wave + 1] = lc;
   }
   __syncthreads();
   int blocks_before = 0, items_before = 0, blocks = 0, items = 0;
-  long heavy_cost = 0, light_cost = 0;
 #pragma unroll
   for (int w = 0; w < kWaves; w++) {
     const int wb = s_wave[2 * w], wi = s_wave[2 * w + 1];
@@ -1181,23 +1190,31 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, i
     }
     blocks += wb;
     items += wi;
-    heavy_cost += s_cost[2 * w];
-    light_cost += s_cost[2 * w + 1];
   }
-  if (t < E) {
-    ws[ws_rec(t) + kRecBlock] = blocks_before + sb - b;
-    ws[ws_rec(t) + kRecItem] = items_before + si - it;
-  }
-  if (t == 0) {
-    ws[ws_rec(E) + kRecBlock] = blocks;
-    ws[ws_rec(E) + kRecItem] = items;
-    ws[ws_rec(E) + kRecExpert] = -1;
-    ws[ws_rec(E) + kRecRows] = 0;
-  }
+  // record t; record E closes the prefix sums
+  if (t < E) *(v4i*)(ws + ws_rec(t)) = v4i{blocks_before + sb - rec[0], items_before + si - rec[1], rec[2], rec[3]};
+  if (t == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
+  static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
   hblocks = __builtin_amdgcn_readfirstlane(blocks);
+  items = __builtin_amdgcn_readfirstlane(items);
   lsplit = __builtin_amdgcn_readfirstlane(sched_light_split(items, policy));
-  ltotal = __builtin_amdgcn_readfirstlane(lsplit + 2 * (items - lsplit));
-  lshare = __builtin_amdgcn_readfirstlane(sched_light_share(heavy_cost, light_cost, policy));
+  ltotal = lsplit + 2 * (items - lsplit);
+  // The cost totals decide how many workgroups start on which kind: needed only where a launch has both.
+  lshare = 0;
+  if (hblocks > 0 && items > 0) {
+    long hc = 0, lc = 0;
+    for (int e = lane; e < E; e += 64) {   // every wavefront sums all experts: no further barrier
+      hc += s_cost[2 * e];
+      lc += s_cost[2 * e + 1];
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      hc += __shfl_xor(hc, d);
+      lc += __shfl_xor(lc, d);
+    }
+    lshare = sched_light_share(hc, lc, policy);
+  }
+  lshare = __builtin_amdgcn_readfirstlane(lshare);
   // the records are read back with scalar loads: every store of this workgroup has to be in L2 first.  (Also a
   // compiler-visible full wait in front of the copy-pipelined K loops, which count their own copies.)
   __builtin_amdgcn_s_waitcnt(0);
