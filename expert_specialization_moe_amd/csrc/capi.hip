@@ -39,7 +39,7 @@ extern "C" int esmoe_launch_swiglu_quant(const void* in, int in_dtype, void* q, 
 
 namespace {
 
-constexpr long kRouteChunk = 1024;   // pairs per wavefront in routing.hip
+constexpr long kRouteChunk = 1024;   // fewest pairs of a chunk in routing.hip
 
 thread_local char g_err[512] = "";
 

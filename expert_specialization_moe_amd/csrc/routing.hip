@@ -5,7 +5,7 @@
 // (counts -> expert_offsets prefix sum: benchmark/benchmark_es_fp8_blockwise_moe.py:44-56,72-88;
 // blockscale_offsets = prefix sum of the counts rounded up to 128:
 // test/test_es_sm100_mxfp8_blockscaled_grouped_quant.py:42-60).  Here the same integers come out of
-// three small kernels, so a caller never synchronises with the host between routing and the GEMMs.
+// one or two small kernels, so a caller never synchronises with the host between routing and the GEMMs.
 //
 //   pair p = (token p / topk, choice p % topk), id = topk_ids[p] - first_expert; local if 0 <= id < E
 //   counts[e]             = number of local pairs with id == e
@@ -15,16 +15,22 @@
 //   dst_row[p]            = expert_offsets[id] + (number of local pairs q < p with the same id), or -1
 // The rank is by pair index, so the permutation is stable and the result is deterministic.
 //
-// Pairs are cut into chunks of kChunk; one wavefront owns a chunk.  Pass 1 counts ids per chunk, pass 2
-// (one workgroup, thread = expert) scans the chunk counts of each expert and then the experts, pass 3
-// ranks the pairs of a chunk 64 at a time with running per-expert counters in LDS.
+// Pairs are cut into chunks, one workgroup of 16 wavefronts each, a pair per thread (of a chunk longer than 1024 pairs:
+// of each 1024 in turn).  A workgroup needs, beside its own pairs, every expert's count over all pairs and over the
+// pairs in front of its chunk.  It forms both itself, from the ids (up to kDirectPairs pairs: ONE launch) or from the
+// chunks' counts that a first launch wrote: nothing waits for another workgroup, and every workgroup knows the offsets.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace esmoe {
 
-constexpr int kChunk = 1024;       // pairs per wavefront
-constexpr int kMaxRouteExperts = 1024;
+constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / 64;
+constexpr int kMaxRouteExperts = 1024;   // a thread per expert
+constexpr int kMaxChunks = 256;
+// Pairs up to which every workgroup counts all ids itself: a pass of LDS atomics over all of them, 1.3 us per 8192 pairs,
+// where the counts cost a launch and a pass over [chunks, experts] words.  128 experts, direct against counts: 8192 pairs
+// 5.2 / 6.0 us, 16384 pairs 7.1 / 6.1 us, 32768 pairs 11.4 / 6.3 us.
+constexpr long kDirectPairs = 8192;
 
 // Lanes of the wavefront that hold the same id as this lane: one ballot per bit of the id instead of one round per
 // distinct id (64 pairs over 32 experts are ~25 distinct ids, and a round costs as much as all the ballots together).
@@ -40,170 +46,158 @@ __device__ __forceinline__ unsigned long long lanes_with_same_id(int id, int bit
 }
 __device__ __forceinline__ int id_bits(int num_experts) { return num_experts > 1 ? 32 - __builtin_clz(num_experts - 1) : 0; }
 
-__global__ void __launch_bounds__(64) route_count_kernel(const int* __restrict__ ids, long num_pairs, int first_expert,
-                                                         int num_experts, int* __restrict__ chunk_counts) {
-  __shared__ int s_cnt[kMaxRouteExperts];
-  const int lane = threadIdx.x;
-  for (int e = lane; e < num_experts; e += 64) s_cnt[e] = 0;
-  __syncthreads();
-  const long base = (long)blockIdx.x * kChunk;
-  for (int i = lane; i < kChunk; i += 64) {
-    const long p = base + i;
-    if (p < num_pairs) {
-      const int id = ids[p] - first_expert;
-      if (id >= 0 && id < num_experts) atomicAdd(&s_cnt[id], 1);
-    }
-  }
-  __syncthreads();
-  for (int e = lane; e < num_experts; e += 64) chunk_counts[(long)blockIdx.x * num_experts + e] = s_cnt[e];
+// Local expert of pair p, or -1 (another rank's expert, or past the last pair).
+__device__ __forceinline__ int local_id(int raw, long p, long num_pairs, int first_expert, int num_experts) {
+  const unsigned id = (unsigned)raw - (unsigned)first_expert;
+  return p < num_pairs && id < (unsigned)num_experts ? (int)id : -1;
 }
 
-__global__ void __launch_bounds__(1024) route_scan_kernel(int* __restrict__ chunk_counts, int num_chunks, int num_experts,
-                                                          int n, int k, int* __restrict__ problem_sizes,
-                                                          int* __restrict__ expert_offsets,
-                                                          int* __restrict__ blockscale_offsets) {
+// Pairs per chunk: 1024, or as many times 1024 as keep the chunks at most kMaxChunks.
+__host__ __device__ inline long route_chunk_pairs(long num_pairs) {
+  const long per = (num_pairs + kMaxChunks - 1) / kMaxChunks;
+  return per <= kRouteThreads ? kRouteThreads : (per + kRouteThreads - 1) / kRouteThreads * kRouteThreads;
+}
+
+__global__ void __launch_bounds__(kRouteThreads) route_count_kernel(const int* __restrict__ ids, long num_pairs, int first_expert,
+                                                                    int num_experts, long chunk, int* __restrict__ chunk_counts) {
   __shared__ int s_cnt[kMaxRouteExperts];
-  const int e = threadIdx.x;
-  int total = 0;
-  if (e < num_experts) {
-    // exclusive scan over the chunks, in place: chunk_counts[c][e] becomes the rank base of chunk c.  Sixteen chunks
-    // are read before any is written back, so that a thread waits for memory once per sixteen chunks, not per chunk.
-    constexpr int kBatch = 16;
-    for (int c0 = 0; c0 < num_chunks; c0 += kBatch) {
+  const int tid = threadIdx.x;
+  s_cnt[tid] = 0;
+  __syncthreads();
+  const long base = (long)blockIdx.x * chunk;
+  for (long off = 0; off < chunk; off += kRouteThreads) {
+    const long p = base + off + tid;
+    const int id = local_id(p < num_pairs ? ids[p] : 0, p, num_pairs, first_expert, num_experts);
+    if (id >= 0) atomicAdd(&s_cnt[id], 1);
+  }
+  __syncthreads();
+  if (tid < num_experts) chunk_counts[(long)blockIdx.x * num_experts + tid] = s_cnt[tid];
+}
+
+// Sum of `v` over this lane and the lanes below it, on the vector ALU (DPP row shifts and row broadcasts).
+__device__ __forceinline__ int route_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, :2, :4, :8 (rows of 16 lanes)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// One workgroup per chunk.  DIRECT: counts from the ids; otherwise from chunk_counts [gridDim.x, num_experts].
+//
+// Latency from end to end (one workgroup per CU, a few thousand pairs): every id is read once per use with eight loads
+// in flight, a wavefront's 64 pairs are ranked by ballots once, and the prefix sums run on the vector ALU.  As one
+// workgroup that took up to 16384 pairs in dependent rounds, and as three launches past that, 128 experts took 10.5 us at
+// 512 pairs (now 3.5), 22.3 at 16384 (6.1), 20.2 at 32768 (6.3), 24.6 at 131072 (8.0).
+template <bool DIRECT>
+__global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* __restrict__ ids, long num_pairs, int first_expert,
+                                                              int num_experts, long chunk, const int* __restrict__ chunk_counts,
+                                                              int n, int k, int* __restrict__ problem_sizes,
+                                                              int* __restrict__ expert_offsets, int* __restrict__ blockscale_offsets,
+                                                              int* __restrict__ dst_row) {
+  __shared__ int s_wave[kRouteWaves][kMaxRouteExperts];   // a wavefront's pairs of every expert, then their first row
+  __shared__ int s_before[kMaxRouteExperts];              // pairs of every expert in the chunks in front
+  __shared__ int s_rest[kMaxRouteExperts];                // and in this chunk and the ones behind
+  __shared__ int s_sum[kRouteWaves][2];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int E = num_experts, me = blockIdx.x;
+  const long base = (long)me * chunk;
+  int raw = base + tid < num_pairs ? ids[base + tid] : 0;   // this thread's pair of the chunk's first 1024
+  s_before[tid] = 0;
+  s_rest[tid] = 0;
+  for (int e = lane; e < E; e += 64) s_wave[w][e] = 0;
+  __syncthreads();
+  constexpr int kBatch = 8;   // loads in flight
+  if constexpr (DIRECT) {
+    for (long p0 = 0; p0 < num_pairs; p0 += kBatch * kRouteThreads) {
       int v[kBatch];
 #pragma unroll
-      for (int u = 0; u < kBatch; u++) v[u] = c0 + u < num_chunks ? chunk_counts[(long)(c0 + u) * num_experts + e] : 0;
+      for (int u = 0; u < kBatch; u++) {
+        const long p = p0 + u * kRouteThreads + tid;
+        v[u] = p < num_pairs ? ids[p] : 0;
+      }
 #pragma unroll
       for (int u = 0; u < kBatch; u++) {
-        if (c0 + u < num_chunks) chunk_counts[(long)(c0 + u) * num_experts + e] = total;
-        total += v[u];
+        const long first = p0 + u * kRouteThreads;
+        if (first >= num_pairs) break;
+        const int id = local_id(v[u], first + tid, num_pairs, first_expert, E);
+        if (id >= 0) atomicAdd(first < base ? &s_before[id] : &s_rest[id], 1);   // (base is a multiple of 1024)
       }
     }
-    s_cnt[e] = total;
-  }
-  __syncthreads();
-  if (e < num_experts) {
-    int off = 0, boff = 0;
-    for (int j = 0; j < e; j++) {
-      const int c = s_cnt[j];
-      off += c;
-      boff += (c + 127) & ~127;
-    }
-    expert_offsets[e] = off;
-    blockscale_offsets[e] = boff;
-    problem_sizes[e * 3 + 0] = total;
-    problem_sizes[e * 3 + 1] = n;
-    problem_sizes[e * 3 + 2] = k;
-    if (e == num_experts - 1) {
-      expert_offsets[num_experts] = off + total;
-      blockscale_offsets[num_experts] = boff + ((total + 127) & ~127);
+  } else {
+    // the counts as one flat array: thread t takes the words t, t + 1024, ...
+    const int words = (int)gridDim.x * E, mine = me * E;
+    for (int i0 = 0; i0 < words; i0 += kBatch * kRouteThreads) {
+      int v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        const int i = i0 + u * kRouteThreads + tid;
+        v[u] = i < words ? chunk_counts[i] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        const int i = i0 + u * kRouteThreads + tid;
+        if (v[u] != 0) atomicAdd(i < mine ? &s_before[i % E] : &s_rest[i % E], v[u]);
+      }
     }
   }
-}
-
-__global__ void __launch_bounds__(64) route_rank_kernel(const int* __restrict__ ids, long num_pairs, int first_expert,
-                                                        int num_experts, const int* __restrict__ chunk_base,
-                                                        const int* __restrict__ expert_offsets,
-                                                        int* __restrict__ dst_row) {
-  __shared__ int s_run[kMaxRouteExperts];   // next free row of every expert for this chunk
-  const int lane = threadIdx.x;
-  for (int e = lane; e < num_experts; e += 64) s_run[e] = expert_offsets[e] + chunk_base[(long)blockIdx.x * num_experts + e];
-  __syncthreads();
-  const long base = (long)blockIdx.x * kChunk;
-  const int bits = id_bits(num_experts);
-  for (int step = 0; step < kChunk / 64; step++) {
-    const long p = base + step * 64 + lane;
-    if (base + step * 64 >= num_pairs) break;   // wave-uniform
-    int id = -1;
-    if (p < num_pairs) {
-      id = ids[p] - first_expert;
-      if (id < 0 || id >= num_experts) id = -1;
-    }
-    // lanes with the same id take consecutive rows in lane order; the first of them moves the expert's counter on
-    int row = -1;
+  const int bits = id_bits(E);
+  int run = 0;   // thread e: next free row of expert e
+  for (long off = 0;;) {
+    const long p = base + off + tid;
+    const int id = local_id(raw, p, num_pairs, first_expert, E);
+    // lanes with the same id take consecutive rows in lane order
     const unsigned long long same = lanes_with_same_id(id, bits);
-    const int before = __builtin_popcountll(same & ((1ull << lane) - 1ull));
-    if (id >= 0) row = s_run[id] + before;
-    __builtin_amdgcn_wave_barrier();
-    if (id >= 0 && before == 0) s_run[id] += __builtin_popcountll(same);
-    __builtin_amdgcn_wave_barrier();
-    if (p < num_pairs) dst_row[p] = row;
-  }
-}
-
-// Small inputs (at most kSmallChunks chunks, at most kSmallExperts experts): the three passes in one workgroup of
-// kSmallChunks wavefronts, wavefront w owning chunk w, with the per-chunk counters in LDS instead of the workspace.
-// Same integers as the three-kernel route; saves two launches, which is most of the time at decode sizes.
-constexpr int kSmallChunks = 16;
-constexpr int kSmallExperts = 256;
-
-__global__ void __launch_bounds__(kSmallChunks * 64) route_small_kernel(const int* __restrict__ ids, long num_pairs,
-                                                                       int first_expert, int num_experts, int n, int k,
-                                                                       int* __restrict__ problem_sizes,
-                                                                       int* __restrict__ expert_offsets,
-                                                                       int* __restrict__ blockscale_offsets,
-                                                                       int* __restrict__ dst_row) {
-  __shared__ int s_cnt[kSmallChunks][kSmallExperts];   // per-chunk counts, then each chunk's next free row per expert
-  __shared__ int s_tot[kSmallExperts];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  for (int i = tid; i < kSmallChunks * kSmallExperts; i += kSmallChunks * 64) (&s_cnt[0][0])[i] = 0;
-  __syncthreads();
-  const long base = (long)w * kChunk;
-  for (int i = lane; i < kChunk; i += 64) {
-    const long p = base + i;
-    if (p < num_pairs) {
-      const int id = ids[p] - first_expert;
-      if (id >= 0 && id < num_experts) atomicAdd(&s_cnt[w][id], 1);
+    const int rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+    if (id >= 0 && rank == 0) s_wave[w][id] = __builtin_popcountll(same);
+    __syncthreads();
+    if (off == 0) {
+      // the offsets: prefix sums over the experts, thread = expert
+      const int before = s_before[tid], total = before + s_rest[tid], padded = (total + 127) & ~127;
+      const int so = route_inclusive_sum(total), sp = route_inclusive_sum(padded);
+      if (lane == 63) {
+        s_sum[w][0] = so;
+        s_sum[w][1] = sp;
+      }
+      __syncthreads();
+      int o = so - total, bo = sp - padded;
+#pragma unroll
+      for (int i = 0; i < kRouteWaves; i++) {
+        o += i < w ? s_sum[i][0] : 0;
+        bo += i < w ? s_sum[i][1] : 0;
+      }
+      run = o + before;
+      if (me == 0 && tid < E) {
+        expert_offsets[tid] = o;
+        blockscale_offsets[tid] = bo;
+        problem_sizes[tid * 3 + 0] = total;
+        problem_sizes[tid * 3 + 1] = n;
+        problem_sizes[tid * 3 + 2] = k;
+        if (tid == E - 1) {
+          expert_offsets[E] = o + total;
+          blockscale_offsets[E] = bo + padded;
+        }
+      }
     }
-  }
-  __syncthreads();
-  if (tid < num_experts) {
-    int total = 0;
-    for (int c = 0; c < kSmallChunks; c++) {
-      const int v = s_cnt[c][tid];
-      s_cnt[c][tid] = total;
-      total += v;
+    if (tid < E) {   // every wavefront's first row of expert tid
+      int c[kRouteWaves];
+#pragma unroll
+      for (int i = 0; i < kRouteWaves; i++) c[i] = s_wave[i][tid];
+#pragma unroll
+      for (int i = 0; i < kRouteWaves; i++) {
+        s_wave[i][tid] = run;
+        run += c[i];
+      }
     }
-    s_tot[tid] = total;
-  }
-  __syncthreads();
-  if (tid < num_experts) {
-    int off = 0, boff = 0;
-    for (int j = 0; j < tid; j++) {
-      const int c = s_tot[j];
-      off += c;
-      boff += (c + 127) & ~127;
-    }
-    const int total = s_tot[tid];
-    expert_offsets[tid] = off;
-    blockscale_offsets[tid] = boff;
-    problem_sizes[tid * 3 + 0] = total;
-    problem_sizes[tid * 3 + 1] = n;
-    problem_sizes[tid * 3 + 2] = k;
-    if (tid == num_experts - 1) {
-      expert_offsets[num_experts] = off + total;
-      blockscale_offsets[num_experts] = boff + ((total + 127) & ~127);
-    }
-    for (int c = 0; c < kSmallChunks; c++) s_cnt[c][tid] += off;
-  }
-  __syncthreads();
-  const int bits = id_bits(num_experts);
-  for (int step = 0; step < kChunk / 64; step++) {
-    const long p = base + step * 64 + lane;
-    if (base + step * 64 >= num_pairs) break;   // wave-uniform
-    int id = -1;
-    if (p < num_pairs) {
-      id = ids[p] - first_expert;
-      if (id < 0 || id >= num_experts) id = -1;
-    }
-    int row = -1;
-    const unsigned long long same = lanes_with_same_id(id, bits);
-    const int before = __builtin_popcountll(same & ((1ull << lane) - 1ull));
-    if (id >= 0) row = s_cnt[w][id] + before;
-    __builtin_amdgcn_wave_barrier();
-    if (id >= 0 && before == 0) s_cnt[w][id] += __builtin_popcountll(same);
-    __builtin_amdgcn_wave_barrier();
-    if (p < num_pairs) dst_row[p] = row;
+    __syncthreads();
+    if (p < num_pairs) dst_row[p] = id >= 0 ? s_wave[w][id] + rank : -1;
+    off += kRouteThreads;
+    if (off >= chunk || base + off >= num_pairs) break;   // the same for the whole workgroup
+    raw = base + off + tid < num_pairs ? ids[base + off + tid] : 0;
+    __syncthreads();
+    for (int e = lane; e < E; e += 64) s_wave[w][e] = 0;   // (rewritten by this wavefront only)
   }
 }
 
@@ -264,20 +258,17 @@ extern "C" int esmoe_launch_route_metadata(const int* ids, long num_pairs, int f
                                            int* problem_sizes, int* expert_offsets, int* blockscale_offsets, int* dst_row,
                                            int* chunk_counts, hipStream_t stream) {
   using namespace esmoe;
-  const int chunks = (int)((num_pairs + kChunk - 1) / kChunk);
-  if (chunks <= kSmallChunks && num_experts <= kSmallExperts) {
-    hipLaunchKernelGGL(route_small_kernel, dim3(1), dim3(kSmallChunks * 64), 0, stream, ids, num_pairs, first_expert,
-                       num_experts, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
+  const long chunk = route_chunk_pairs(num_pairs);
+  const int chunks = num_pairs > 0 ? (int)((num_pairs + chunk - 1) / chunk) : 1;
+  if (num_pairs <= kDirectPairs) {
+    hipLaunchKernelGGL(route_kernel<true>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
+                       chunk, (const int*)nullptr, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
     return (int)hipGetLastError();
   }
-  if (chunks > 0)
-    hipLaunchKernelGGL(route_count_kernel, dim3(chunks), dim3(64), 0, stream, ids, num_pairs, first_expert, num_experts,
-                       chunk_counts);
-  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3((num_experts + 63) & ~63), 0, stream, chunk_counts, chunks,
-                     num_experts, n, k, problem_sizes, expert_offsets, blockscale_offsets);
-  if (chunks > 0)
-    hipLaunchKernelGGL(route_rank_kernel, dim3(chunks), dim3(64), 0, stream, ids, num_pairs, first_expert, num_experts,
-                       chunk_counts, expert_offsets, dst_row);
+  hipLaunchKernelGGL(route_count_kernel, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
+                     chunk, chunk_counts);
+  hipLaunchKernelGGL(route_kernel<false>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
+                     chunk, chunk_counts, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
   return (int)hipGetLastError();
 }
 

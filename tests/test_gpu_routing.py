@@ -48,6 +48,28 @@ def test_route_metadata_bit_exact(esmoe, seed, pairs, experts, first, span):
         assert np.array_equal(g, r), name
 
 
+@pytest.mark.parametrize("pairs,experts,first,span", [(63, 2, 0, 2), (1023, 1023, 0, 1024), (2048, 64, 1, 64), (8192, 1024, 7, 2000),
+                                                       (8193, 1024, 0, 1024), (16385, 1, 0, 3), (262144, 60, 0, 64),
+                                                       (262145, 256, 0, 256), (600001, 100, 3, 128)])
+def test_route_metadata_edges(esmoe, pairs, experts, first, span):
+    """Edges of the chunks: a pair per thread, counts taken from the ids up to 8192 pairs and from a launch in front
+    past that, more than one round of 1024 pairs per chunk past 262144; skewed ids, some of them -1."""
+    from expert_specialization_moe_amd import _native
+
+    rng = np.random.default_rng(pairs)
+    ids = (first + np.minimum(rng.geometric(min(0.9, 4.0 / span), size=pairs) - 1, span - 1)).astype(np.int32)
+    ids[rng.random(pairs) < 0.05] = -1
+    got = _capi_route(_native, ids, first, experts, 256, 128)
+    local = (ids >= first) & (ids < first + experts)
+    counts = np.bincount(ids[local] - first, minlength=experts)
+    offsets, padded = np.concatenate([[0], np.cumsum(counts)]), np.concatenate([[0], np.cumsum((counts + 127) // 128 * 128)])
+    dst = np.full(pairs, -1, np.int64)
+    order = np.argsort(ids[local], kind="stable")   # local pairs by expert, then by pair index
+    dst[np.flatnonzero(local)[order]] = np.arange(order.size)
+    assert np.array_equal(got[0], np.stack([counts, np.full(experts, 256), np.full(experts, 128)], axis=1))
+    assert np.array_equal(got[1], offsets) and np.array_equal(got[2], padded) and np.array_equal(got[3], dst)
+
+
 def test_route_rejects(esmoe):
     from expert_specialization_moe_amd import _native
 
