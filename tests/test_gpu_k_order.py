@@ -1,0 +1,71 @@
+"""Rows a multiple of 4096 bytes apart: every expert starts its K blocks at a place of its own and wraps around.
+
+The order is one per expert whatever tile computes an element, so every forced tile height must give the bytes of the
+device schedule and the fused epilogues those of projection -> stand-alone quantiser.  FP8-blockwise is also checked against
+a product of the dequantised operands in fp64: one rounding to bfloat16 (2^-8 of the value) plus K roundings of fp32 sums
+(K * 2^-24 of the sum of the products' magnitudes).  MXFP8 against the same with the oracle's dequantisation, the
+magnitudes' sum taken as 60 times the largest output (K random products of one size sum to about their number's root).
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import mxfp8 as omx
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [4096, 8192, 12288])
+@pytest.mark.parametrize("kind", ["fp8", "mx"])
+def test_wrapped_k_order_is_the_same_for_every_tile(esmoe, kind, k):
+    from expert_specialization_moe_amd import _native, workloads as W
+
+    n, rows = 512, [1, 200, 0, 33, 16, 130, 64, 65, 400, 7, 17]   # eleven starts; every tile height and its edges
+    dt = torch.bfloat16
+    prob = W.Problem("wrap", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
+    if kind == "mx":
+        ops = W.make_mxfp8_operands(prob, "cuda", seed=k, out_dtype=dt, weight_std=0.05)
+        mm = H.capi_mx_mm
+    else:
+        ops = W.make_fp8_blockwise_operands(prob, "cuda", seed=k, out_dtype=dt, weight_std=0.05)
+        mm = H.capi_fp8_mm
+    base = mm(_native, ops, 0, out=torch.full_like(ops["output"], 3.0)).clone()
+    for bm in (16, 32, 64, 128, 192):
+        forced = mm(_native, ops, bm, out=torch.full_like(ops["output"], 3.0))
+        assert torch.equal(base.view(torch.int16), forced.view(torch.int16)), f"tile height {bm}"
+    if kind == "fp8":
+        a = ops["a"].double() * ops["scales_a"].double().repeat_interleave(128, dim=1)
+        sb = ops["scales_b_phys"].double().repeat_interleave(128, dim=1).repeat_interleave(128, dim=2)
+        off = 0
+        for i, m in enumerate(rows):
+            w = ops["b_phys"][i].double() * sb[i]
+            ref, mag = a[off:off + m] @ w.t(), a[off:off + m].abs() @ w.abs().t()
+            bound = ref.abs() * 2.0 ** -8 + mag * (k * 2.0 ** -24)
+            assert ((base[off:off + m].double() - ref).abs() <= bound).all(), f"expert {i}"
+            off += m
+        q = torch.zeros((off, n // 2), dtype=torch.uint8, device="cuda")
+        sc = torch.zeros((off, n // 256), dtype=torch.float32, device="cuda")
+        esmoe.es_fp8_blockwise_scaled_grouped_mm_swiglu_quant(q, sc, ops["a"], ops["b"], ops["scales_a"], ops["scales_b"],
+                                                              ops["problem_sizes"], ops["expert_offsets"], ops["workspace"], dt)
+        q2, sc2 = esmoe.es_swiglu_quant_1x128(base)
+        assert torch.equal(q, q2.view(torch.uint8)) and torch.equal(sc, sc2)
+    else:
+        codes, scales = H.codes(ops["a"]), omx.unswizzle_scales
+        off = 0
+        for i, m in enumerate(rows):
+            if m:
+                sa = scales(ops["sfa"].cpu().numpy().reshape(-1), m, k, base=int(ops["blockscale_offsets"][i]) * (k // 32))
+                sw = scales(ops["sfb_phys"].cpu().numpy().reshape(-1), n, k, base=i * n * (k // 32))
+                ref = omx.dequant_rows(codes[off:off + m], sa).astype(np.float64) @ omx.dequant_rows(H.codes(ops["b_phys"][i]), sw).astype(np.float64).T
+                y = H.f32(base[off:off + m]).astype(np.float64)
+                bound = np.abs(ref) * 2.0 ** -8 + k * 2.0 ** -24 * np.abs(ref).max() * 60
+                assert (np.abs(y - ref) <= bound).all(), f"expert {i}"
+            off += m
+        q = torch.zeros((sum(rows), n // 2), dtype=torch.uint8, device="cuda")
+        sf = torch.zeros((ops["sfa"].shape[0], n // 64), dtype=torch.uint8, device="cuda")
+        esmoe.es_mxfp8_blockscaled_grouped_mm_swiglu_quant(q, sf, ops["a"], ops["b"], ops["sfa"], ops["sfb"], ops["problem_sizes"],
+                                                           ops["expert_offsets"], ops["blockscale_offsets"], dt)
+        q2, sf2 = torch.zeros_like(q), torch.zeros_like(sf)
+        esmoe.es_swiglu_mxfp8_grouped_quant(base, ops["problem_sizes"], ops["expert_offsets"], ops["blockscale_offsets"], q2, sf2)
+        assert torch.equal(q, q2) and torch.equal(sf, sf2)
