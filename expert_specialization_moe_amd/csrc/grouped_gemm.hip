@@ -47,6 +47,7 @@ namespace esmoe {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -394,8 +395,17 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
 // rows and the matching 128 up rows, interleaved so that every wavefront holds gate and up of the same columns; the
 // epilogue forms silu(gate) * up and quantises it for the down projection (fp8-blockwise: 1x128 blocks with fp32
 // scales, tile_epilogue; mxfp8: 1x32 blocks with E8M0 scales, tile_epilogue_mxq) instead of writing the projection.
+//
+// `cols` (plain 256-column tiles only; 1 otherwise): a strip of so many neighbouring whole tiles of one expert, walked as one
+// stream of cols * K/128 stages.  The copies of the next tile's first stages are on their way while a tile ends, and its
+// output leaves as buffer stores that the counted waits leave in flight: a tile alone pays the ticket, the look-up and
+// the first stages' trip from memory, about 5 us, which at K = 256 is nine tenths of its time (256 experts x 32 rows,
+// 7168 x 256: 164 us one by one, 128 us as strips).  A strip has at most 32 stages (sched_light_draw; its weight block
+// scales share one tile's table of 256).
 template <int MT, bool MX, bool FUSE, int BN = kBN>
-__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, uint8_t* lds) {
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, int cols, uint8_t* lds) {
+  constexpr bool kStrip = !FUSE && BN == kBN;
+  static_assert(kStripBlocks <= kMaxKB, "the weight block scales of a strip share the table of one tile");
   static_assert(!(FUSE && BN != kBN), "the fused epilogues need gate and up columns of a whole quantisation block in one tile");
   static_assert(MT == 1 || MT == 2 || MT == 4, "short tiles; 128- and 192-row tiles are gemm_tile_pp / gemm_tile_pp_mx");
   using G = TileGeom<MT, MX, BN>;
@@ -457,8 +467,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     sclds = G::kABytes + G::kWBytes + (wave & 1) * 1024;
   }
 
-  // scales of positions 4c .. 4c+3 into chunk buffer c & 1 (`rot` is a multiple of 4)
-  auto issue_sa_chunk = [&](int c) { dma16(sc_base + (long)kb_at(4 * c) * 4, scoff, lds0 + sclds + (c & 1) * 4096); };
+  // scales of positions p .. p+3 (p and `rot` are multiples of 4) into chunk buffer c & 1
+  auto issue_sa_chunk = [&](int c, int p) { dma16(sc_base + (long)kb_at(p) * 4, scoff, lds0 + sclds + (c & 1) * 4096); };
   // copies of position p's K block into ring slot buf: this wavefront's token blocks (consecutive 8-row blocks
   // wave*kACopies + i; short tiles are copied by several wavefronts), its 4 weight blocks, its share
   // of the scales.  Each copy has a per-lane byte offset from the operand's pointer for the K block: source row
@@ -506,7 +516,22 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     if (w_once) dma16xn<true>(lw, w_ptr + (long)kb * 128, vw);
     else dma16xn<false>(lw, w_ptr + (long)kb * 128, vw);
   };
-  auto issue = [&](int p, int buf) { const int kb = kb_at(p); issue_a(kb, buf); issue_w(kb, buf); };
+  // next stage of the tile or strip: position ip of its current column tile
+  const int stages = kStrip ? cols * KB : KB;
+  int ip = 0;
+  auto issue_next = [&](int buf) {
+    const int kb = kb_at(ip);
+    issue_a(kb, buf);
+    issue_w(kb, buf);
+    ip++;
+    if constexpr (kStrip) {
+      if (ip == KB) {   // on to the next column tile
+        ip = 0;
+        w_ptr += (long)kBN * K;
+        if constexpr (MX) sc_base += (wave & 1) == 0 ? (long)KB * 1024 : 0;
+      }
+    }
+  };
 
   // ---- fragment read plan ----------------------------------------------------------------
   // token fragment of row tile mt: LDS row ra = mw + mt*16 + r, chunks gq and gq+4
@@ -515,7 +540,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   const int afrag_lo = (mw + r) * 128 + swz(r, gq) * 16;
   const int wfrag_lo = G::kABytes + (nw + r) * 128 + swz(r, gq) * 16;
   constexpr int kScaleOff = G::kABytes + G::kWBytes;
-  const float* sb_tab = s_sb + (FUSE ? 0 : (nw >> 7)) * kMaxKB;   // FUSE: table 0 = gate block, table 1 = up block
+  // weight block scales: strips keep [2 * cols column blocks][K/128], by K block; the others [2][kMaxKB], by position (FUSE:
+  // table 0 = gate block, table 1 = up block)
+  const float* sb_tab = kStrip ? s_sb + (nw >> 7) * KB : s_sb + (FUSE ? 0 : (nw >> 7)) * kMaxKB;
   // mxfp8: per-lane bases of the scale dwords (weight rows nw + r, token rows mw + r of a tall tile)
   // (FUSE: n-tile 0 = gate rows n0/2 + wn*16 + r in the first tile, n-tile 1 the up rows at the same place in the second)
   const int sfw_lane = FUSE ? kScaleOff + ((wn & 1) * 16 + r) * 16 + (wn >> 1) * 4
@@ -543,9 +570,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     float sb_up;   // FUSE: scale of the up rows' weight block (sb is the gate rows')
   };
 
+  int pos = 0;   // position of the stage at hand inside its column tile
   auto read_scales_fp8 = [&](int kb, int buf, Frags& f) {
     const uint8_t* lb = lds + buf * G::kStageBytes;
-    f.sb = sb_tab[kb];
+    f.sb = sb_tab[kStrip ? kb_at(pos) : kb];
     if constexpr (FUSE) f.sb_up = sb_tab[kMaxKB + kb];
 #pragma unroll
     for (int mt = 0; mt < MTW; mt++) {
@@ -640,7 +668,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   // wavefront w copies positions 64*(w & 3) .. +63 of column block w >> 2, lanes past KB repeat the last
   // one), then NBUF-1 K blocks in flight.  The scale copy is asynchronous like the others and older than
   // all of them, so the first wait below covers it and nothing here waits for a whole stage.
-  if constexpr (!MX) {
+  if constexpr (!MX && kStrip) {
+    // one run of memory: 2 * cols * KB <= 512 floats, 64 to a wavefront (lanes past the end repeat the last)
+    int n = 2 * cols * KB;
+    if (n0 + kBN > N) n = KB;   // a last column tile of 128 columns
+    if (wave * 64 < n) {
+      const int i = wave * 64 + lane < n ? wave * 64 + lane : n - 1;
+      dma4(g.sb + ((long)e * (N >> 7) + (n0 >> 7)) * KB, (uint32_t)i * 4, lds0 + kRingBytes + wave * 256);
+    }
+  } else if constexpr (!MX) {
     const int blk = wave >> 2, kb0 = (wave & 3) * 64;
     if (kb0 < KB) {
       int nb = (n0 >> 7) + blk;
@@ -650,14 +686,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
       dma4(g.sb + ((long)e * (N >> 7) + nb) * KB, (uint32_t)kbi * 4, lds0 + kRingBytes + (blk * kMaxKB + kb0) * 4);
     }
   }
-  if (sa4 && wave * 64 < G::BM) issue_sa_chunk(0);
+  if (sa4 && wave * 64 < G::BM) issue_sa_chunk(0, 0);
 #pragma unroll
   for (int s = 0; s < NBUF - 1; s++) {
-    if (s < KB) issue(s, s);
+    if (s < stages) issue_next(s);
   }
   // copies outstanding per in-flight stage (the chunked scale copies are older than any stage that
   // may still be in flight when their data is needed, see the loop)
-  if (KB < NBUF - 1) wait_vmcnt<0>();
+  if (stages < NBUF - 1) wait_vmcnt<0>();
   else if (sa4) wait_vmcnt<(NBUF - 2) * (G::kCopiesPerStage - 1)>();
   else wait_vmcnt<(NBUF - 2) * G::kCopiesPerStage>();
   block_barrier();
@@ -666,38 +702,82 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   // top of iteration kb into the slot that iteration kb - 1 read (kb counts positions of the expert's K order).  (Two groups of wavefronts half an iteration apart, as in
   // the tall tiles, were measured for every short height and both kernels: 0.2-14 % slower; a short tile is bound by its
   // weight stream, not by the overlap of reads and MFMAs.)
-  auto wait_stage = [&](bool more, int chunk_young) {
+  // Strips: a finished column tile's kStores output stores stay in flight as well while they are younger than the stage
+  // waited for (vmcnt counts loads and stores in one order); two tiles' worth (K = 128) is waited for as one, the safe side.
+  constexpr int kStores = MTW * NTW;
+  auto wait_stage = [&](bool more, bool chunk_young, bool stores_young) {
     // all of this wavefront's copies except those of the newest NBUF-2 K blocks have landed
-    if (!more) wait_vmcnt<0>();
-    else if (!sa4) wait_vmcnt<(NBUF - 2) * G::kCopiesPerStage>();
-    else if (chunk_young) wait_vmcnt<(NBUF - 2) * (G::kCopiesPerStage - 1) + 1>();
-    else wait_vmcnt<(NBUF - 2) * (G::kCopiesPerStage - 1)>();
+    if (!more) {
+      wait_vmcnt<0>();
+    } else if (kStrip && stores_young) {
+      if (!sa4) wait_vmcnt<(NBUF - 2) * G::kCopiesPerStage + kStores>();
+      else wait_vmcnt<(NBUF - 2) * (G::kCopiesPerStage - 1) + kStores>();   // (a young chunk is waited for with the stage)
+    } else {
+      if (!sa4) wait_vmcnt<(NBUF - 2) * G::kCopiesPerStage>();
+      else if (chunk_young) wait_vmcnt<(NBUF - 2) * (G::kCopiesPerStage - 1) + 1>();
+      else wait_vmcnt<(NBUF - 2) * (G::kCopiesPerStage - 1)>();
+    }
   };
-  int buf = 0, nbuf = NBUF - 1;  // ring slots of K block kb and of K block kb + NBUF - 1
+  // Output of a strip: the tile's rows as a buffer, so that every lane of every wavefront stores without a branch (a fixed
+  // number of stores to count) and the hardware drops rows at or past M; column `n` of a last tile's absent half likewise.
+  [[maybe_unused]] uint32_t voff = 0;
+  [[maybe_unused]] __amdgpu_buffer_rsrc_t out_buf;
+  if constexpr (kStrip) {
+    const int rows = M - m0 < G::BM ? M - m0 : G::BM;
+    out_buf = __builtin_amdgcn_make_buffer_rsrc((uint8_t*)g.out + (row_base + m0) * (long)N * 2, 0, rows * N * 2, 0x00027000);
+    voff = wave_active ? (uint32_t)((mw + r) * N + n0 + nw + gq * 4) * 2 : 0x40000000u;
+  }
+  int buf = 0, nbuf = NBUF - 1;  // ring slots of stage kb and of stage kb + NBUF - 1
   int chunk_age = NBUF;          // iterations since this wavefront issued a scale-chunk copy
+  int store_age = NBUF;          // iterations since a column tile's output was stored
+  int cpos = 0;                  // first position of the scale chunk being read
   Frags f;
-  for (int kb = 0; kb < KB; kb++) {
-    const bool more = kb + NBUF - 1 < KB;
+  for (int kb = 0; kb < stages; kb++) {
+    const bool more = kb + NBUF - 1 < stages;
     // next chunk of activation scales, 4 K blocks before its first use (only the wavefronts whose
     // 64 rows exist in the tile fetch); `chunk_age` counts the iterations since, so that the wait
     // below can leave it in flight with the newest stages
-    if (sa4 && (kb & 3) == 0 && kb + 4 < KB && wave * 64 < G::BM) {
-      issue_sa_chunk((kb >> 2) + 1);
-      chunk_age = 0;
+    if (sa4 && (kb & 3) == 0 && kb + 4 < stages) {
+      cpos = cpos + 4 == KB ? 0 : cpos + 4;
+      if (wave * 64 < G::BM) {
+        issue_sa_chunk((kb >> 2) + 1, cpos);
+        chunk_age = 0;
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (more) issue(kb + NBUF - 1, nbuf);
+    if (more) issue_next(nbuf);
     __builtin_amdgcn_sched_barrier(0);
     read_phase(kb, buf, f);
     __builtin_amdgcn_sched_barrier(0);
     mfma_phase(f);
     __builtin_amdgcn_sched_barrier(0);
-    wait_stage(more, chunk_age < NBUF - 2);
+    wait_stage(more, chunk_age < NBUF - 2, store_age < NBUF - 2);
     chunk_age++;
+    store_age++;
     block_barrier();
     buf = buf + 1 == NBUF ? 0 : buf + 1;
     nbuf = nbuf + 1 == NBUF ? 0 : nbuf + 1;
+    if constexpr (kStrip) {
+      if (++pos == KB) {   // the column tile is done
+        pos = 0;
+        sb_tab += 2 * KB;
+        store_age = 0;
+#pragma unroll
+        for (int mt = 0; mt < MTW; mt++) {
+#pragma unroll
+          for (int nt = 0; nt < NTW; nt++) {
+            const v4f v = {acc[nt][mt][0], acc[nt][mt][1], acc[nt][mt][2], acc[nt][mt][3]};
+            const v2i w = g.out_dtype == 0 ? __builtin_bit_cast(v2i, __builtin_convertvector(v, bf16x4))
+                                           : __builtin_bit_cast(v2i, __builtin_convertvector(v, f16x4));
+            __builtin_amdgcn_raw_buffer_store_b64(w, out_buf, voff + (uint32_t)(mt * 16 * N + nt * 16) * 2, 0, 0);
+            acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
+          }
+        }
+        voff += kBN * 2;
+      }
+    }
   }
+  if constexpr (kStrip) return;
 
   if constexpr (MX && FUSE) tile_epilogue_mxq<G::BM, MTW, NTW, G::kWavesN>(g, acc, ebso, M, m0, n0, row_base, mw, wn, lane, lds);
   else tile_epilogue<G::BM, MTW, NTW, G::kWavesN, FUSE>(g, acc, M, m0, n0, row_base, mw, nw, wn, lane, wave_active, lds);
@@ -1286,39 +1366,51 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
 #pragma unroll
   for (int x = 0; x < kXcds; x++)
     if (x >= hblocks) dead |= 1 << x;
+  // Light tickets in hand, [have, have_end), of one draw (sched_light_draw).
+  int have = 0, have_end = 0, seen = 0;
   for (;;) {
     const bool light = (phase == 0) == light_first;
     const int xq = (xcd + q) & (kXcds - 1);
-    if ((dead >> (light ? 8 : xq)) & 1) {   // nothing (left) in this queue: the next XCD's, then the other kind
-      if (light || ++q == kXcds) {
-        q = 0;
-        if (++phase == 2) break;
+    int v = have;   // the light ticket or the heavy block at hand
+    int ticket = 0;
+    if (!light || have == have_end) {
+      if ((dead >> (light ? 8 : xq)) & 1) {   // nothing (left) in this queue: the next XCD's, then the other kind
+        if (light || ++q == kXcds) {
+          q = 0;
+          if (++phase == 2) break;
+        }
+        continue;
       }
-      continue;
-    }
-    if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], 1);
-    __syncthreads();
-    const int ticket = __builtin_amdgcn_readfirstlane(s_item);
-    const int kind = light ? kRecItem : kRecBlock;
-    const int v = light ? ticket : sched_ticket_block(xq, ticket);
-    if (v >= (light ? ltotal : hblocks)) {   // this queue is exhausted: see which others are
-      dead |= 1 << (light ? 8 : xq);
-      __syncthreads();                        // s_item and s_counters are rewritten next
-      // (worth its round trip only when every XCD has a queue to try: the look itself reads the hot counter line)
-      if (hblocks <= kXcds) continue;
-      if (threadIdx.x < kXcds + 1)
-        s_counters[threadIdx.x] = __hip_atomic_load(threadIdx.x < kXcds ? &ws[ws_xcd_counter(threadIdx.x)] : &ws[kWsLightCounter],
-                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int draw = light ? sched_light_draw(ltotal, seen, (int)gridDim.x, g.k >> 7) : 1;
+      if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
       __syncthreads();
+      ticket = __builtin_amdgcn_readfirstlane(s_item);
+      v = light ? ticket : sched_ticket_block(xq, ticket);
+      if (v >= (light ? ltotal : hblocks)) {   // this queue is exhausted: see which others are
+        dead |= 1 << (light ? 8 : xq);
+        __syncthreads();                        // s_item and s_counters are rewritten next
+        // (worth its round trip only when every XCD has a queue to try: the look itself reads the hot counter line)
+        if (hblocks <= kXcds) continue;
+        if (threadIdx.x < kXcds + 1)
+          s_counters[threadIdx.x] = __hip_atomic_load(threadIdx.x < kXcds ? &ws[ws_xcd_counter(threadIdx.x)] : &ws[kWsLightCounter],
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
 #pragma unroll
-      for (int x = 0; x < kXcds; x++) {
-        // queue x holds the blocks x, x + 8, ...: 32 tickets each
-        const int tickets = x < hblocks ? ((hblocks - x + kXcds - 1) / kXcds) * kBlkTiles : 0;
-        if (__builtin_amdgcn_readfirstlane(s_counters[x]) >= tickets) dead |= 1 << x;
+        for (int x = 0; x < kXcds; x++) {
+          // queue x holds the blocks x, x + 8, ...: 32 tickets each
+          const int tickets = x < hblocks ? ((hblocks - x + kXcds - 1) / kXcds) * kBlkTiles : 0;
+          if (__builtin_amdgcn_readfirstlane(s_counters[x]) >= tickets) dead |= 1 << x;
+        }
+        if (__builtin_amdgcn_readfirstlane(s_counters[kXcds]) >= ltotal) dead |= 256;
+        continue;
       }
-      if (__builtin_amdgcn_readfirstlane(s_counters[kXcds]) >= ltotal) dead |= 256;
-      continue;
+      if (light) {
+        seen = v;
+        have = v;
+        have_end = v + draw < ltotal ? v + draw : ltotal;
+      }
     }
+    const int kind = light ? kRecItem : kRecBlock;
     // schedule position of v: the last one whose first block (item) is <= v, found by bisection over the prefix
     // sums with scalar loads.  The records are written by the schedule kernel and only read here, so they stay in
     // the scalar cache, where a step costs a fraction of what a trip to L2 costs while the chip streams weights.
@@ -1339,8 +1431,21 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
     const int ebso = MX ? sload(g.blockscale_offsets, e * 4) : 0;
     const int local = idx - first;
     TileCoord t;
-    if (light) t = sched_decode_light(local, M, g.policy, half);
-    else if (!sched_decode_heavy(local, ticket % kBlkTiles, M, g.n, g.policy, &t)) {
+    int cols = 1;
+    if (light) {
+      t = sched_decode_light(local, M, g.policy, half);
+      if constexpr (!FUSE) {
+        // the tickets in hand that are whole 256-column items of the same expert, or both halves of such, go as one strip
+        int whole = half < 0 ? (have_end < lsplit ? have_end : lsplit) - v : half == 0 ? (have_end - v) >> 1 : 0;
+        if (whole > (g.n >> 8) - local) whole = (g.n >> 8) - local;
+        if (whole > 1) cols = whole;
+        if (half == 0 && whole > 0) {
+          t.nt = 4;
+          half = -2;
+        }
+      }
+      have = v + (half == -2 ? 2 * cols : cols);
+    } else if (!sched_decode_heavy(local, ticket % kBlkTiles, M, g.n, g.policy, &t)) {
       __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
       continue;
     }
@@ -1364,14 +1469,14 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
       else gemm_tile_pp<8, FUSE>(g, e, erow, M, t.m0, t.n0, lds);
     } else if (!FUSE && t.nt == 2) {
       if constexpr (!FUSE) {
-        if (t.mt == 1) gemm_tile<1, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, lds);
-        else if (t.mt == 2) gemm_tile<2, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, lds);
-        else gemm_tile<4, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, lds);
+        if (t.mt == 1) gemm_tile<1, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, 1, lds);
+        else if (t.mt == 2) gemm_tile<2, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, 1, lds);
+        else gemm_tile<4, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, 1, lds);
       }
     } else {
-      if (t.mt == 1) gemm_tile<1, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, lds);
-      else if (t.mt == 2) gemm_tile<2, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, lds);
-      else gemm_tile<4, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, lds);
+      if (t.mt == 1) gemm_tile<1, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, cols, lds);
+      else if (t.mt == 2) gemm_tile<2, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, cols, lds);
+      else gemm_tile<4, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, cols, lds);
     }
   }
   // The last workgroup to leave zeroes the hand-out counters (nobody draws any more: every workgroup counts itself

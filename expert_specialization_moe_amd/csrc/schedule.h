@@ -169,6 +169,28 @@ ESMOE_HD int sched_light_item_of_ticket(int ticket, int split, int* half) {
   return split + ((ticket - split) >> 1);
 }
 
+// Light tickets that a workgroup takes with one draw, when the last light ticket it saw was `seen` (0 at first): half its
+// share of what was left then, within bounds that go by the item's length in K blocks.  Neighbouring tickets of one expert run
+// as one strip (grouped_gemm.hip, gemm_tile), so the upper bound is also a strip's: 32 K blocks, 1 MB of weights.  Longer
+// strips put the workgroups' streams further apart in memory and run slower: 64 experts x 8 rows, upper bound 16 / 32 / 64 /
+// 256 blocks: K = 256 209 / 206 / 219 / 220 us, K = 1024 187 / 181 / 189 / 189 us (single tickets: 282 and 190 us).  The lower
+// bound is 16 K blocks, for launches that give every workgroup two such draws: below it the draw and the first stages'
+// trip from memory, about 5 us, outweigh the even end of the launch.  The whole share instead of half: up to 15 % slower.
+// All quotients are by the next power of two: a division is a chain of some forty instructions, and this stands in front of
+// a workgroup's first tile.
+constexpr int kStripBlocks = 32;
+ESMOE_HD int sched_log2_ceil(int v) { return v > 1 ? 32 - __builtin_clz((unsigned)v - 1) : 0; }
+ESMOE_HD int sched_light_draw(int total, int seen, int workgroups, int kblocks) {
+  const int lk = sched_log2_ceil(kblocks), lw = sched_log2_ceil(workgroups) + 1;
+  const int most = kStripBlocks >> lk;
+  int least = (kStripBlocks / 2) >> lk;
+  if (least > total >> lw) least = total >> lw;
+  int draw = (total - seen) >> lw;
+  if (draw < least) draw = least;
+  if (draw > most) draw = most;
+  return draw > 1 ? draw : 1;
+}
+
 // Item `item` of a light expert; half = -1: the whole 256-column item, 0 / 1: its first / second 128 columns.
 ESMOE_HD TileCoord sched_decode_light(int item, int m, const SchedPolicy& p, int half = -1) {
   TileCoord t;
