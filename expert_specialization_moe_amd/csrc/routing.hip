@@ -224,30 +224,44 @@ __global__ void __launch_bounds__(256) permute_rows_kernel(const uint8_t* __rest
   }
 }
 
-// The same packing for topk > 1 (at most 64): one wavefront per token reads the row once and writes it to every
-// local destination of the token's pairs, where one wavefront per pair would read it topk times.
+constexpr int kPermutePiece = 4096;           // four 16-byte loads in flight per lane
+// Workgroups of a launch: 2^28 threads (a grid holds fewer than 2^32); past that a wavefront takes several pieces.
+constexpr long kMaxPermuteGroups = 1 << 20;
+
+// The same packing for topk > 1 (at most 64): one wavefront per piece of 4096 bytes of a token's row reads it once and
+// writes it to every local destination of the token's pairs, where one wavefront per pair would read it topk times.
+//
+// Bound by the output's bytes.  A wavefront per token walked the pieces one after the other: at 1003 tokens four wavefronts
+// per CU, each waiting for memory four times.  Pieces of 1024 bytes are slower (1003 tokens x 14336 bytes: 14.6 against
+// 12.7 us, 2048 x 8192: 27.4 / 24.7).  Plain stores: the packed rows are what the caller quantises next, and what the
+// 256 MB cache keeps of them is not fetched from HBM; non-temporal ones cost 28.0 - 29.0 us here and another 3 us there.
+//   2048 tokens x 8 KB x top-8, packing + 1x128 quantisation:      32.0 + 34.3 -> 25.4 + 31.3 us
+//   1003 tokens x 14 KB x top-4, packing + MXFP8 quantisation:     16.5 + 18.1 -> 12.6 + 16.2 us
+//   16384 tokens x 8 KB x top-8 (1.07 GB out, past that cache):     262 +  258 ->  194 +  274 us
 __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_t* __restrict__ in,
-                                                                    const int* __restrict__ dst_row, long num_tokens,
-                                                                    int topk, long row_bytes, uint8_t* __restrict__ out) {
+                                                                    const int* __restrict__ dst_row, long num_pieces,
+                                                                    int pieces, int topk, long row_bytes,
+                                                                    uint8_t* __restrict__ out) {
   typedef int v4i __attribute__((ext_vector_type(4)));
-  const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= num_tokens) return;
   const int lane = threadIdx.x & 63;
-  const int mine = lane < topk ? dst_row[t * topk + lane] : -1;   // lane j: destination of the token's pair j
-  if (__ballot(mine >= 0) == 0) return;                           // no local pair
-  const uint8_t* src = in + t * row_bytes;
-  for (long off = lane * 16; off < row_bytes; off += 4096) {
+  for (long piece = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); piece < num_pieces;
+       piece += (long)gridDim.x * 4) {
+    const long t = piece / pieces;
+    const int mine = lane < topk ? dst_row[t * topk + lane] : -1;   // lane j: destination of the token's pair j
+    if (__ballot(mine >= 0) == 0) continue;                         // no local pair: the row is not read
+    const long off = (piece - t * pieces) * kPermutePiece + lane * 16;
+    const uint8_t* src = in + t * row_bytes + off;
     v4i v[4];
 #pragma unroll
     for (int u = 0; u < 4; u++)
-      if (off + u * 1024 < row_bytes) v[u] = __builtin_nontemporal_load((const v4i*)(src + off + u * 1024));
+      if (off + u * 1024 < row_bytes) v[u] = __builtin_nontemporal_load((const v4i*)(src + u * 1024));
     for (int j = 0; j < topk; j++) {
       const int dst = __builtin_amdgcn_readlane(mine, j);
       if (dst < 0) continue;
-      uint8_t* d = out + (long)dst * row_bytes;
+      uint8_t* d = out + (long)dst * row_bytes + off;
 #pragma unroll
       for (int u = 0; u < 4; u++)
-        if (off + u * 1024 < row_bytes) __builtin_nontemporal_store(v[u], (v4i*)(d + off + u * 1024));
+        if (off + u * 1024 < row_bytes) *(v4i*)(d + u * 1024) = v[u];
     }
   }
 }
@@ -278,8 +292,11 @@ extern "C" int esmoe_launch_permute_rows(const void* in, const int* dst_row, lon
   if (num_pairs == 0) return 0;
   if (topk > 1 && topk <= 64 && num_pairs % topk == 0) {
     const long tokens = num_pairs / topk;
-    hipLaunchKernelGGL(permute_rows_by_token_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, stream,
-                       (const uint8_t*)in, dst_row, tokens, topk, row_bytes, (uint8_t*)out);
+    const int pieces = (int)((row_bytes + kPermutePiece - 1) / kPermutePiece);
+    const long groups = (tokens * pieces + 3) / 4;
+    const dim3 grid((unsigned)(groups < kMaxPermuteGroups ? groups : kMaxPermuteGroups));
+    hipLaunchKernelGGL(permute_rows_by_token_kernel, grid, dim3(256), 0, stream, (const uint8_t*)in, dst_row,
+                       tokens * pieces, pieces, topk, row_bytes, (uint8_t*)out);
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(permute_rows_kernel, dim3((unsigned)((num_pairs + 3) / 4)), dim3(256), 0, stream, (const uint8_t*)in,

@@ -98,6 +98,27 @@ def test_permute_rows_of_topk_pairs(esmoe, topk, row_elems):
     assert np.array_equal(H.hp_to_f32(packed.cpu()), oroute.permute_rows(H.hp_to_f32(x), dst_r, topk, total))
 
 
+@pytest.mark.parametrize("tokens,topk,row_elems", [
+    (1, 2, 8), (3, 5, 2048 - 8), (5, 3, 2048), (6, 2, 2048 + 8), (7, 4, 4096), (9, 2, 3 * 2048 + 520),   # around 4096 bytes
+    (4 * (1 << 20) + 5, 2, 8),   # more pieces than a full grid has wavefronts
+])
+def test_permute_rows_pieces(esmoe, tokens, topk, row_elems):
+    """Rows of one piece, a part of one and several, and a launch whose wavefronts take more than one piece: a copy, so
+    every byte is the source's; rows without a local pair in between, output rows that no pair names untouched."""
+    gen = torch.Generator(device="cuda").manual_seed(row_elems + topk)
+    x = torch.randint(-30000, 30000, (tokens, row_elems), generator=gen, device="cuda", dtype=torch.int16)
+    pairs = tokens * topk
+    dst = torch.randperm(pairs, generator=gen, device="cuda").to(torch.int32)
+    dst[torch.rand(pairs, generator=gen, device="cuda") < 0.3] = -1
+    dst.view(tokens, topk)[tokens // 2] = -1
+    out = torch.full((pairs, row_elems), 31000, dtype=torch.int16, device="cuda")
+    want = out.clone()
+    local = dst >= 0
+    want[dst[local].long()] = x[torch.nonzero(local).flatten() // topk]
+    esmoe.es_permute_rows(x.view(torch.bfloat16), dst, topk, out.view(torch.bfloat16))
+    assert torch.equal(out, want)
+
+
 def test_routed_fp8_layer_on_device(esmoe):
     """ids -> metadata -> packed rows -> 1x128 quant -> grouped GEMM, all on the device, against the oracle chain."""
     from expert_specialization_moe_amd import workloads as W
