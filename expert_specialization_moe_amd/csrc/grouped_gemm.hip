@@ -400,7 +400,7 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
 // stream of cols * K/128 stages.  The copies of the next tile's first stages are on their way while a tile ends, and its
 // output leaves as buffer stores that the counted waits leave in flight: a tile alone pays the ticket, the look-up and
 // the first stages' trip from memory, about 5 us, which at K = 256 is nine tenths of its time (256 experts x 32 rows,
-// 7168 x 256: 164 us one by one, 128 us as strips).  A strip has at most 32 stages (sched_light_draw; its weight block
+// 7168 x 256: 164 us one by one, 136 us as strips).  A strip has at most 32 stages (sched_light_draw; its weight block
 // scales share one tile's table of 256).
 template <int MT, bool MX, bool FUSE, int BN = kBN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, int cols, uint8_t* lds) {
@@ -720,6 +720,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   };
   // Output of a strip: the tile's rows as a buffer, so that every lane of every wavefront stores without a branch (a fixed
   // number of stores to count) and the hardware drops rows at or past M; column `n` of a last tile's absent half likewise.
+  // Plain stores: the 32-byte pieces of a row have to merge in L2 (with the non-temporal hint 206 us instead of 136 at 256
+  // experts x 32 rows, 7168 x 256).
   [[maybe_unused]] uint32_t voff = 0;
   [[maybe_unused]] __amdgpu_buffer_rsrc_t out_buf;
   if constexpr (kStrip) {
