@@ -227,17 +227,23 @@ __global__ void __launch_bounds__(256) permute_rows_kernel(const uint8_t* __rest
 constexpr int kPermutePiece = 4096;           // four 16-byte loads in flight per lane
 // Workgroups of a launch: 2^28 threads (a grid holds fewer than 2^32); past that a wavefront takes several pieces.
 constexpr long kMaxPermuteGroups = 1 << 20;
+constexpr long kPlainPermuteBytes = 32L << 20;   // outputs above this are stored plainly (below)
 
 // The same packing for topk > 1 (at most 64): one wavefront per piece of 4096 bytes of a token's row reads it once and
 // writes it to every local destination of the token's pairs, where one wavefront per pair would read it topk times.
 //
 // Bound by the output's bytes.  A wavefront per token walked the pieces one after the other: at 1003 tokens four wavefronts
 // per CU, each waiting for memory four times.  Pieces of 1024 bytes are slower (1003 tokens x 14336 bytes: 14.6 against
-// 12.7 us, 2048 x 8192: 27.4 / 24.7).  Plain stores: the packed rows are what the caller quantises next, and what the
-// 256 MB cache keeps of them is not fetched from HBM; non-temporal ones cost 28.0 - 29.0 us here and another 3 us there.
+// 12.7 us, 2048 x 8192: 27.4 / 24.7).
+// PLAIN, for outputs above 32 MB: the packed rows are what the caller quantises next, and what the 256 MB cache keeps of them
+// is not fetched from HBM; non-temporal stores cost 28.0 - 29.0 us here and another 3 us there.  An output that the eight
+// 4 MB L2s hold is written with the hint: plain stores leave it there dirty, and the launch's end waits until it is
+// written back (packing + 1x128 quantisation, plain / hint: 1024 tokens x 4 KB x top-8 23.7 / 19.1 us, 2048 x 8 KB x top-2
+// 23.5 / 21.1, 64 x 8 KB x top-8 10.0 / 8.6).
 //   2048 tokens x 8 KB x top-8, packing + 1x128 quantisation:      32.0 + 34.3 -> 25.4 + 31.3 us
 //   1003 tokens x 14 KB x top-4, packing + MXFP8 quantisation:     16.5 + 18.1 -> 12.6 + 16.2 us
 //   16384 tokens x 8 KB x top-8 (1.07 GB out, past that cache):     262 +  258 ->  194 +  274 us
+template <bool PLAIN>
 __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_t* __restrict__ in,
                                                                     const int* __restrict__ dst_row, long num_pieces,
                                                                     int pieces, int topk, long row_bytes,
@@ -261,7 +267,10 @@ __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_
       uint8_t* d = out + (long)dst * row_bytes + off;
 #pragma unroll
       for (int u = 0; u < 4; u++)
-        if (off + u * 1024 < row_bytes) *(v4i*)(d + u * 1024) = v[u];
+        if (off + u * 1024 < row_bytes) {
+          if constexpr (PLAIN) *(v4i*)(d + u * 1024) = v[u];
+          else __builtin_nontemporal_store(v[u], (v4i*)(d + u * 1024));
+        }
     }
   }
 }
@@ -295,8 +304,12 @@ extern "C" int esmoe_launch_permute_rows(const void* in, const int* dst_row, lon
     const int pieces = (int)((row_bytes + kPermutePiece - 1) / kPermutePiece);
     const long groups = (tokens * pieces + 3) / 4;
     const dim3 grid((unsigned)(groups < kMaxPermuteGroups ? groups : kMaxPermuteGroups));
-    hipLaunchKernelGGL(permute_rows_by_token_kernel, grid, dim3(256), 0, stream, (const uint8_t*)in, dst_row,
-                       tokens * pieces, pieces, topk, row_bytes, (uint8_t*)out);
+    if (num_pairs > kPlainPermuteBytes / row_bytes)
+      hipLaunchKernelGGL(permute_rows_by_token_kernel<true>, grid, dim3(256), 0, stream, (const uint8_t*)in, dst_row,
+                         tokens * pieces, pieces, topk, row_bytes, (uint8_t*)out);
+    else
+      hipLaunchKernelGGL(permute_rows_by_token_kernel<false>, grid, dim3(256), 0, stream, (const uint8_t*)in, dst_row,
+                         tokens * pieces, pieces, topk, row_bytes, (uint8_t*)out);
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(permute_rows_kernel, dim3((unsigned)((num_pairs + 3) / 4)), dim3(256), 0, stream, (const uint8_t*)in,

@@ -100,6 +100,7 @@ def test_permute_rows_of_topk_pairs(esmoe, topk, row_elems):
 
 @pytest.mark.parametrize("tokens,topk,row_elems", [
     (1, 2, 8), (3, 5, 2048 - 8), (5, 3, 2048), (6, 2, 2048 + 8), (7, 4, 4096), (9, 2, 3 * 2048 + 520),   # around 4096 bytes
+    (2100, 2, 4104),             # the same past 32 MB of output, where the stores are plain
     (4 * (1 << 20) + 5, 2, 8),   # more pieces than a full grid has wavefronts
 ])
 def test_permute_rows_pieces(esmoe, tokens, topk, row_elems):
