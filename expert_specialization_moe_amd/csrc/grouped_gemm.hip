@@ -410,7 +410,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   static_assert(MT == 1 || MT == 2 || MT == 4, "short tiles; 128- and 192-row tiles are gemm_tile_pp / gemm_tile_pp_mx");
   using G = TileGeom<MT, MX, BN>;
   constexpr int MTW = G::MTW, NTW = G::NTW, NBUF = G::kNBuf;
-  const int tid = threadIdx.x;
+  int tid = threadIdx.x;
+  // (hidden from the compiler, which otherwise forms this tile's addresses once in front of the hand-out loop and keeps them
+  // in vector registers that the tall tiles do not have: four were spilled to scratch)
+  asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / G::kWavesN, wn = wave % G::kWavesN;
@@ -422,8 +425,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   const int mw = wm * (MTW * 16);          // first token row of this wavefront inside the tile
   const bool wave_active = n0 + nw < N;
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
-  const int rot = sched_first_kb(e, K);
-  auto kb_at = [&](int p) { return p + rot < KB ? p + rot : p + rot - KB; };   // K block of position p
   float* s_sb = (float*)(lds + kRingBytes);  // [2][kMaxKB] weight block scales of the tile's two 128-column blocks
   constexpr int kSaChunkOff = kRingBytes + 2 * kMaxKB * 4;
 
@@ -467,9 +468,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     sclds = G::kABytes + G::kWBytes + (wave & 1) * 1024;
   }
 
-  // scales of positions p .. p+3 (p and `rot` are multiples of 4) into chunk buffer c & 1
-  auto issue_sa_chunk = [&](int c, int p) { dma16(sc_base + (long)kb_at(p) * 4, scoff, lds0 + sclds + (c & 1) * 4096); };
-  // copies of position p's K block into ring slot buf: this wavefront's token blocks (consecutive 8-row blocks
+  // scales of K blocks kb .. kb+3 (kb a multiple of 4) into chunk buffer c & 1
+  auto issue_sa_chunk = [&](int c, int kb) { dma16(sc_base + (long)kb * 4, scoff, lds0 + sclds + (c & 1) * 4096); };
+  // copies of K block kb into ring slot buf: this wavefront's token blocks (consecutive 8-row blocks
   // wave*kACopies + i; short tiles are copied by several wavefronts), its 4 weight blocks, its share
   // of the scales.  Each copy has a per-lane byte offset from the operand's pointer for the K block: source row
   // (token rows past the expert's last are replaced by the last, weight blocks past the last weight row by valid
@@ -516,13 +517,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     if (w_once) dma16xn<true>(lw, w_ptr + (long)kb * 128, vw);
     else dma16xn<false>(lw, w_ptr + (long)kb * 128, vw);
   };
-  // next stage of the tile or strip: position ip of its current column tile
+  // next stage of the tile or strip: K block ip of its current column tile
   const int stages = kStrip ? cols * KB : KB;
   int ip = 0;
   auto issue_next = [&](int buf) {
-    const int kb = kb_at(ip);
-    issue_a(kb, buf);
-    issue_w(kb, buf);
+    issue_a(ip, buf);
+    issue_w(ip, buf);
     ip++;
     if constexpr (kStrip) {
       if (ip == KB) {   // on to the next column tile
@@ -540,8 +540,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   const int afrag_lo = (mw + r) * 128 + swz(r, gq) * 16;
   const int wfrag_lo = G::kABytes + (nw + r) * 128 + swz(r, gq) * 16;
   constexpr int kScaleOff = G::kABytes + G::kWBytes;
-  // weight block scales: strips keep [2 * cols column blocks][K/128], by K block; the others [2][kMaxKB], by position (FUSE:
-  // table 0 = gate block, table 1 = up block)
+  // weight block scales: strips keep [2 * cols column blocks][K/128], the others [2][kMaxKB] (FUSE: table 0 = gate block,
+  // table 1 = up block)
   const float* sb_tab = kStrip ? s_sb + (nw >> 7) * KB : s_sb + (FUSE ? 0 : (nw >> 7)) * kMaxKB;
   // mxfp8: per-lane bases of the scale dwords (weight rows nw + r, token rows mw + r of a tall tile)
   // (FUSE: n-tile 0 = gate rows n0/2 + wn*16 + r in the first tile, n-tile 1 the up rows at the same place in the second)
@@ -570,10 +570,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     float sb_up;   // FUSE: scale of the up rows' weight block (sb is the gate rows')
   };
 
-  int pos = 0;   // position of the stage at hand inside its column tile
+  int pos = 0;   // K block of the stage at hand inside its column tile
   auto read_scales_fp8 = [&](int kb, int buf, Frags& f) {
     const uint8_t* lb = lds + buf * G::kStageBytes;
-    f.sb = sb_tab[kStrip ? kb_at(pos) : kb];
+    f.sb = sb_tab[kStrip ? pos : kb];
     if constexpr (FUSE) f.sb_up = sb_tab[kMaxKB + kb];
 #pragma unroll
     for (int mt = 0; mt < MTW; mt++) {
@@ -664,8 +664,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   };
 
   // ---- pipeline --------------------------------------------------------------------------
-  // prologue: the weight block scales of the whole tile ([2 column blocks][KB] floats behind the ring, by position:
-  // wavefront w copies positions 64*(w & 3) .. +63 of column block w >> 2, lanes past KB repeat the last
+  // prologue: the weight block scales of the whole tile ([2 column blocks][KB] floats behind the ring:
+  // wavefront w copies K blocks 64*(w & 3) .. +63 of column block w >> 2, lanes past KB repeat the last
   // one), then NBUF-1 K blocks in flight.  The scale copy is asynchronous like the others and older than
   // all of them, so the first wait below covers it and nothing here waits for a whole stage.
   if constexpr (!MX && kStrip) {
@@ -682,7 +682,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
       int nb = (n0 >> 7) + blk;
       if (nb * 128 >= N) nb = n0 >> 7;
       if constexpr (FUSE) nb = (n0 >> 8) + blk * (N >> 8);   // gate block of these columns, up block I/128 further
-      const int kbi = kb_at(kb0 + lane < KB ? kb0 + lane : KB - 1);
+      const int kbi = kb0 + lane < KB ? kb0 + lane : KB - 1;
       dma4(g.sb + ((long)e * (N >> 7) + nb) * KB, (uint32_t)kbi * 4, lds0 + kRingBytes + (blk * kMaxKB + kb0) * 4);
     }
   }
@@ -699,7 +699,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   block_barrier();
 
   // All eight wavefronts run in step, one barrier per K block: the stage of K block kb + NBUF - 1 is requested at the
-  // top of iteration kb into the slot that iteration kb - 1 read (kb counts positions of the expert's K order).  (Two groups of wavefronts half an iteration apart, as in
+  // top of iteration kb into the slot that iteration kb - 1 read.  (Two groups of wavefronts half an iteration apart, as in
   // the tall tiles, were measured for every short height and both kernels: 0.2-14 % slower; a short tile is bound by its
   // weight stream, not by the overlap of reads and MFMAs.)
   // Strips: a finished column tile's kStores output stores stay in flight as well while they are younger than the stage
@@ -732,7 +732,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   int buf = 0, nbuf = NBUF - 1;  // ring slots of stage kb and of stage kb + NBUF - 1
   int chunk_age = NBUF;          // iterations since this wavefront issued a scale-chunk copy
   int store_age = NBUF;          // iterations since a column tile's output was stored
-  int cpos = 0;                  // first position of the scale chunk being read
+  int cpos = 0;                  // first K block of the scale chunk being read
   Frags f;
   for (int kb = 0; kb < stages; kb++) {
     const bool more = kb + NBUF - 1 < stages;
@@ -817,8 +817,6 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
   // a K that is no multiple of 512 overlaps the one before instead of reaching past the row.
   const int K = g.k, N = g.n, KB = K >> 7, NCH = (KB + 3) >> 2;
   auto chunk_first_kb = [&](int c) { const int f = 4 * c < KB - 4 ? 4 * c : KB - 4; return f > 0 ? f : 0; };
-  const int rot = sched_first_kb(e, K);
-  auto kb_at = [&](int p) { return p + rot < KB ? p + rot : p + rot - KB; };   // K block of position p (see k_loop)
   const long row_base = erow;
   const int nw = wj * 64, mw = grp * GR;
   const bool wave_active = n0 + nw < N;
@@ -857,9 +855,8 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
     const int grow = trow > a_last ? a_last : trow;
     vs[q] = (uint32_t)grow * (uint32_t)KB * 4 + ((lane & 3) < KB ? (lane & 3) : KB - 1) * 4;
   }
-  // (position 0 of the expert's K order; k_loop takes a row off where the order wraps)
-  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K + rot * 128 - kBias;
-  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K + rot * 128 - kBias;
+  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K - kBias;
+  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K - kBias;
   const uint8_t* sa_ptr = (const uint8_t*)(g.sa + (row_base + m0) * KB);
   const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + wj * kTCopies * 1024;   // + slot * kTSlot
   const uint32_t w_dst = lds0 + wave * 4096;                                        // + slot * kWSlot
@@ -888,7 +885,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
       int nb = (n0 >> 7) + blk;
       if (nb * 128 >= N) nb = n0 >> 7;
       if constexpr (FUSE) nb = (n0 >> 8) + blk * (N >> 8);
-      const int kbi = kb_at(kb0 + lane < KB ? kb0 + lane : KB - 1);
+      const int kbi = kb0 + lane < KB ? kb0 + lane : KB - 1;
       dma4(g.sb + ((long)e * (N >> 7) + nb) * KB, (uint32_t)kbi * 4, lds0 + kSbBase + (blk * kMaxKB + kb0) * 4);
     }
   }
@@ -896,7 +893,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
     // scale chunks 0 and 1 in the pieces the loop uses: wavefront wj the four 16-row pieces of rows (wj & 1)*64 .. +64
     // of chunk wj >> 1
     const int ch = (wj >> 1) < NCH ? (wj >> 1) : NCH - 1;
-    const uint8_t* src = sa_ptr + (long)kb_at(chunk_first_kb(ch)) * 4;
+    const uint8_t* src = sa_ptr + (long)chunk_first_kb(ch) * 4;
 #pragma unroll
     for (int q = 0; q < 4; q++) dma4(src, vs[q], s_dst + (wj >> 1) * kSaBuf + q * 256);
   }
@@ -927,36 +924,16 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
     for (int i = 0; i < 4; i++) vw[i] += kbw0 * 128;
   }
   uint32_t wl = wfrag, wh = wfrag ^ 64, al = afrag, ah = afrag ^ 64;
-  // kb counts positions of the expert's K order (sched_first_kb).  Between two statements stands only what moves with every
-  // K block; the rest is an event every four K blocks (scale chunks: c = kb / 4 is read from buffer c % 3, chunk c + 2
-  // fetched into the buffer of chunk c - 1) or once per tile: iteration kb fetches the weights of position kb + 2 and the
-  // tokens of position kb + 1, so their pointers step back to the row's start in front of iterations wrap - 2 and wrap - 1.
-  // (This code delays the next copies: with the chunk arithmetic in every iteration 39 instructions stood here.)
-  const int wrap = rot ? KB - rot : KB + 8;
-  auto chunk_src = [&](int c) { return sa_ptr + (long)kb_at(chunk_first_kb(c < NCH ? c : NCH - 1)) * 4; };
   auto k_loop = [&](auto nt_hint) {
     constexpr bool kNt = decltype(nt_hint)::value;
-    uint32_t sab = 0;                                  // buffer of the chunk being read, in bytes
-    uint32_t sar = 0, ls = s_dst + 2 * kSaBuf;         // scales read from sa_rd + sar; piece fetched to ls
-    const uint8_t* sp = chunk_src(2);
-    int next = 4;
-    for (int kb = 0; kb < KB; kb++, sar += 4, ls += 256) {
-      if (kb == next) {
-        next = (kb & ~3) + 4;
-        if ((kb & 3) == 0) {
-          ls = s_dst + sab;
-          sab = sab == 2 * kSaBuf ? 0 : sab + kSaBuf;
-          sar = sab + (kb - chunk_first_kb(kb >> 2)) * 4;
-          sp = chunk_src((kb >> 2) + 2);
-          if (kb == wrap - 4) next = wrap - 2;
-        } else if (kb == wrap - 2) {
-          w_ptr -= K;
-          next = wrap - 1;
-        } else {
-          a_ptr -= K;
-        }
-      }
-      const uint32_t sal = sa_rd + sar;
+    int sabuf = 0;   // buffer of the scale chunk of K block kb: (kb / 4) % 3
+    for (int kb = 0; kb < KB; kb++) {
+      const int q = kb & 3;
+      const int chw = (kb >> 2) + 2 < NCH ? (kb >> 2) + 2 : NCH - 1;
+      const int sanext = sabuf >= 1 ? sabuf - 1 : 2;         // (kb / 4 + 2) % 3
+      const uint32_t ls = s_dst + sanext * kSaBuf + q * 256;
+      const uint8_t* sp = sa_ptr + (long)chunk_first_kb(chw) * 4;
+      const uint32_t sal = sa_rd + sabuf * kSaBuf + (kb - chunk_first_kb(kb >> 2)) * 4;
       const uint32_t sbl = sb_rd + kb * 4;
       const uint32_t vsq = vs[0];
 #define ESMOE_PP_STMT(NAME)                                                                                      \
@@ -968,8 +945,9 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
       else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PP12);
       else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PP8F);
       else ESMOE_PP_STMT(ESMOE_PP8);
-      // the offsets of the chunk's four pieces take turns
+      // the piece offsets rotate with q; the chunk buffer advances every fourth K block
       { const uint32_t t = vs[0]; vs[0] = vs[1]; vs[1] = vs[2]; vs[2] = vs[3]; vs[3] = t; }
+      if (q == 3) sabuf = sabuf == 2 ? 0 : sabuf + 1;
     }
   };
   if (w_once) k_loop(std::true_type{}); else k_loop(std::false_type{});
@@ -1002,7 +980,6 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
   const int grp = wave >> 2, wj = wave & 3;
   const int r = lane & 15, gq = lane >> 4;
   const int K = g.k, N = g.n, KB = K >> 7, kc = K >> 5;
-  const int rot = sched_first_kb(e, K);
   const long row_base = erow;
   const int nw = wj * 64, mw = grp * GR;
   const bool wave_active = n0 + nw < N;
@@ -1033,9 +1010,8 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
     }
     vw[i] = (uint32_t)(row + crow) * (uint32_t)K + (swz(blk * 8 + crow, cslot) << 4) + kBias - i * 1024;
   }
-  // (position 0 of the expert's K order, see k_loop of gemm_tile_pp)
-  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K + rot * 128 - kBias;
-  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K + rot * 128 - kBias;
+  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K - kBias;
+  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K - kBias;
   const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + wj * kTCopies * 1024;   // + slot * kTSlot
   const uint32_t w_dst = lds0 + wave * 4096;                                        // + slot * kWSlot
   // scale copies, one per wavefront and K block: wavefront 0 the weight scale tiles (with the weight stage),
@@ -1062,7 +1038,6 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
     vs = 0;
     s_dst = lds0 + kSpare;
   }
-  s_ptr += rot * 512;
   // (wave-uniform by construction; said again so that they live in scalar registers)
   s_dst = __builtin_amdgcn_readfirstlane(s_dst);
   s_ptr = (const uint8_t*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)s_ptr >> 32)) << 32) |
@@ -1129,17 +1104,9 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
   uint32_t sfal[MTW];
 #pragma unroll
   for (int mt = 0; mt < MTW; mt++) sfal[mt] = sfa_rd[mt];
-  // (positions and the places where the pointers step back as in gemm_tile_pp; the scale tiles go with their operand)
-  const int wrap = rot ? KB - rot : KB + 8;
   auto k_loop = [&](auto nt_hint) {
     constexpr bool kNt = decltype(nt_hint)::value;
-    int next = wrap - 2;
     for (int kb = 0; kb < KB; kb++) {
-      if (kb == next) {
-        if (kb == wrap - 2) w_ptr -= K; else a_ptr -= K;
-        if ((kb == wrap - 2) == (s_role == 0)) s_ptr -= (long)KB * 512;
-        next = wrap - 1;
-      }
       if constexpr (MT == 12 && FUSE) ESMOE_PP_STMT(ESMOE_PPX12F);
       else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PPX12);
       else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PPX8F);

@@ -58,21 +58,6 @@ ESMOE_HD int sched_nt_for(int, const SchedPolicy&) { return 4; }
 
 ESMOE_HD int sched_ntiles(int n, int nt) { return (n + nt * 64 - 1) / (nt * 64); }
 
-// K order.  Every output element is accumulated K block by K block (128 columns) in one order whatever tile computes it:
-// from this block to the last one, then from block 0 on.  The start is 0 unless rows are a multiple of 4096 bytes apart.
-// Then all rows of a weight panel share their address bits 7-11, a K block of a tile goes through one of the sixteen
-// channels of its L2 (and as few of the memory's), and tiles that all start with block 0 stay in step and queue for one
-// channel after the other: 64 experts x 8 rows x 4096 x 4096 took 211 us (5.1 TB/s) where K = 3968 and 4224 ran at
-// 6.2-6.3 TB/s.  With the experts' starts spread over the row the same call takes 170 us.  (Rows 2048 bytes apart reach two
-// channels per K block and lose nothing: 6.3 TB/s.)  The start depends on the expert alone, not on the column or the tile
-// height, so that tall, short, half and gate-up tiles give the same bits; it is a multiple of 4 blocks (activation
-// scales come in chunks of 4) and at least 8 blocks before the row's end (what a tall tile's prologue fetches).
-ESMOE_HD int sched_first_kb(int e, int k) {
-  if (k & 4095) return 0;
-  const uint32_t slots = (uint32_t)k / 512 - 1;                    // starts 0, 4, ..., k/128 - 8
-  return (int)((((uint32_t)e * 0x9E3779B1u) >> 16) * slots >> 16) * 4;   // multiplicative hashing: neighbours far apart
-}
-
 // ---- XCD-aware hand-out ------------------------------------------------------------------
 // The 256 CUs sit in 8 XCDs with one L2 each, and workgroup i of a launch runs on XCD i % 8.  Tiles
 // of one expert that share token rows or weight rows should therefore run at the same time on the

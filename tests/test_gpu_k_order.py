@@ -1,7 +1,9 @@
-"""Rows a multiple of 4096 bytes apart: every expert starts its K blocks at a place of its own and wraps around.
+"""One K order for every tile and every place in the list, also where rows are a multiple of 4096 bytes apart.
 
-The order is one per expert whatever tile computes an element, so every forced tile height must give the bytes of the
-device schedule and the fused epilogues those of projection -> stand-alone quantiser.  FP8-blockwise is also checked against
+Every output element is accumulated K block by K block from the first to the last, whatever tile computes it and wherever its
+expert stands in the call: every forced tile height must give the bytes of the device schedule, the fused epilogues those of
+projection -> stand-alone quantiser, and an expert listed elsewhere, or in a call of its own, its own bytes again (another
+rank's share of the same experts is such a call).  FP8-blockwise is also checked against
 a product of the dequantised operands in fp64: one rounding to bfloat16 (2^-8 of the value) plus K roundings of fp32 sums
 (K * 2^-24 of the sum of the products' magnitudes).  MXFP8 against the same with the oracle's dequantisation, the
 magnitudes' sum taken as 60 times the largest output (K random products of one size sum to about their number's root).
@@ -69,3 +71,26 @@ def test_wrapped_k_order_is_the_same_for_every_tile(esmoe, kind, k):
         q2, sf2 = torch.zeros_like(q), torch.zeros_like(sf)
         esmoe.es_swiglu_mxfp8_grouped_quant(base, ops["problem_sizes"], ops["expert_offsets"], ops["blockscale_offsets"], q2, sf2)
         assert torch.equal(q, q2) and torch.equal(sf, sf2)
+
+
+@pytest.mark.parametrize("k", [4096, 8192, 12288, 7168])
+@pytest.mark.parametrize("kind", ["fp8", "mx"])
+def test_an_experts_bytes_do_not_depend_on_its_place_in_the_list(esmoe, kind, k):
+    from expert_specialization_moe_amd import _native, workloads as W
+
+    n, rows = 512, [1, 200, 0, 33, 16, 130, 64, 400, 7]
+    prob = W.Problem("place", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
+    make, mm = (W.make_mxfp8_operands, H.capi_mx_mm) if kind == "mx" else (W.make_fp8_blockwise_operands, H.capi_fp8_mm)
+    ops = make(prob, "cuda", seed=k, out_dtype=torch.bfloat16, weight_std=0.05)
+    base = mm(_native, ops, 0).clone()
+    offs = W.offsets_of(rows)
+    weights = ("b_phys", "sfb_phys") if kind == "mx" else ("b_phys", "scales_b_phys")
+    lists = [[8, 7, 6, 5, 4, 3, 2, 1, 0], [3, 0, 8, 1, 7, 2, 6, 4, 5]] + [[e] for e in range(len(rows))]
+    for order in lists:
+        moved = dict(ops, output=torch.full_like(ops["output"], float("nan")))
+        for name in weights + ("problem_sizes", "expert_offsets") + (("blockscale_offsets",) if kind == "mx" else ()):
+            moved[name] = (ops[name].view(len(rows), n, k // 32) if name == "sfb_phys" else ops[name])[order].contiguous()
+        got = mm(_native, moved, 0)
+        for e in order:
+            sl = slice(int(offs[e]), int(offs[e]) + rows[e])
+            assert torch.equal(got[sl].view(torch.int16), base[sl].view(torch.int16)), f"expert {e} of {order}"
