@@ -719,15 +719,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     }
   };
   // Output of a strip: the tile's rows as a buffer, so that every lane of every wavefront stores without a branch (a fixed
-  // number of stores to count) and the hardware drops rows at or past M; column `n` of a last tile's absent half likewise.
+  // number of stores to count) and the hardware drops rows at or past M and the columns of a last tile's absent half
+  // (strip_buffer_bytes).  Outputs too wide for 32-bit offsets leave through tile_epilogue behind the loop.
   // Plain stores: the 32-byte pieces of a row have to merge in L2 (with the non-temporal hint 206 us instead of 136 at 256
   // experts x 32 rows, 7168 x 256).
   [[maybe_unused]] uint32_t voff = 0;
   [[maybe_unused]] __amdgpu_buffer_rsrc_t out_buf;
+  const bool by_buffer = kStrip && strip_by_buffer(N);
   if constexpr (kStrip) {
     const int rows = M - m0 < G::BM ? M - m0 : G::BM;
-    out_buf = __builtin_amdgcn_make_buffer_rsrc((uint8_t*)g.out + (row_base + m0) * (long)N * 2, 0, rows * N * 2, 0x00027000);
-    voff = wave_active ? (uint32_t)((mw + r) * N + n0 + nw + gq * 4) * 2 : 0x40000000u;
+    out_buf = __builtin_amdgcn_make_buffer_rsrc((uint8_t*)g.out + (row_base + m0) * (long)N * 2, 0,
+                                                (int)strip_buffer_bytes(rows, N, wave_active), 0x00027000);
+    voff = strip_buffer_offset(mw + r, N, n0 + nw + gq * 4);
   }
   int buf = 0, nbuf = NBUF - 1;  // ring slots of stage kb and of stage kb + NBUF - 1
   int chunk_age = NBUF;          // iterations since this wavefront issued a scale-chunk copy
@@ -760,7 +763,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     buf = buf + 1 == NBUF ? 0 : buf + 1;
     nbuf = nbuf + 1 == NBUF ? 0 : nbuf + 1;
     if constexpr (kStrip) {
-      if (++pos == KB) {   // the column tile is done
+      if (++pos == KB && by_buffer) {   // the column tile is done
         pos = 0;
         sb_tab += 2 * KB;
         store_age = 0;
@@ -771,7 +774,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
             const v4f v = {acc[nt][mt][0], acc[nt][mt][1], acc[nt][mt][2], acc[nt][mt][3]};
             const v2i w = g.out_dtype == 0 ? __builtin_bit_cast(v2i, __builtin_convertvector(v, bf16x4))
                                            : __builtin_bit_cast(v2i, __builtin_convertvector(v, f16x4));
-            __builtin_amdgcn_raw_buffer_store_b64(w, out_buf, voff + (uint32_t)(mt * 16 * N + nt * 16) * 2, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b64(w, out_buf, voff + strip_buffer_offset(mt * 16, N, nt * 16), 0, 0);
             acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
           }
         }
@@ -779,7 +782,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
       }
     }
   }
-  if constexpr (kStrip) return;
+  if (by_buffer) return;
 
   if constexpr (MX && FUSE) tile_epilogue_mxq<G::BM, MTW, NTW, G::kWavesN>(g, acc, ebso, M, m0, n0, row_base, mw, wn, lane, lds);
   else tile_epilogue<G::BM, MTW, NTW, G::kWavesN, FUSE>(g, acc, M, m0, n0, row_base, mw, nw, wn, lane, wave_active, lds);
@@ -1407,7 +1410,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
         // the tickets in hand that are whole 256-column items of the same expert, or both halves of such, go as one strip
         int whole = half < 0 ? (have_end < lsplit ? have_end : lsplit) - v : half == 0 ? (have_end - v) >> 1 : 0;
         if (whole > (g.n >> 8) - local) whole = (g.n >> 8) - local;
-        if (whole > 1) cols = whole;
+        if (whole > 1 && strip_by_buffer(g.n)) cols = whole;
         if (half == 0 && whole > 0) {
           t.nt = 4;
           half = -2;
