@@ -21,6 +21,9 @@
 // chunks' counts that a first launch wrote: nothing waits for another workgroup, and every workgroup knows the offsets.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
+
+#include "permute_rule.h"
 
 namespace esmoe {
 
@@ -225,9 +228,7 @@ __global__ void __launch_bounds__(256) permute_rows_kernel(const uint8_t* __rest
 }
 
 constexpr int kPermutePiece = 4096;           // four 16-byte loads in flight per lane
-// Workgroups of a launch: 2^28 threads (a grid holds fewer than 2^32); past that a wavefront takes several pieces.
-constexpr long kMaxPermuteGroups = 1 << 20;
-constexpr long kPlainPermuteBytes = 32L << 20;   // outputs above this are stored plainly (below)
+constexpr long kMaxPermutePieces = 1L << 22;     // of a launch (2^28 threads; a grid holds fewer than 2^32): larger inputs take several
 
 // The same packing for topk > 1 (at most 64): one wavefront per piece of 4096 bytes of a token's row reads it once and
 // writes it to every local destination of the token's pairs, where one wavefront per pair would read it topk times.
@@ -235,32 +236,43 @@ constexpr long kPlainPermuteBytes = 32L << 20;   // outputs above this are store
 // Bound by the output's bytes.  A wavefront per token walked the pieces one after the other: at 1003 tokens four wavefronts
 // per CU, each waiting for memory four times.  Pieces of 1024 bytes are slower (1003 tokens x 14336 bytes: 14.6 against
 // 12.7 us, 2048 x 8192: 27.4 / 24.7).
-// PLAIN, for outputs above 32 MB: the packed rows are what the caller quantises next, and what the 256 MB cache keeps of them
-// is not fetched from HBM; non-temporal stores cost 28.0 - 29.0 us here and another 3 us there.  An output that the eight
-// 4 MB L2s hold is written with the hint: plain stores leave it there dirty, and the launch's end waits until it is
-// written back (packing + 1x128 quantisation, plain / hint: 1024 tokens x 4 KB x top-8 23.7 / 19.1 us, 2048 x 8 KB x top-2
-// 23.5 / 21.1, 64 x 8 KB x top-8 10.0 / 8.6).
-//   2048 tokens x 8 KB x top-8, packing + 1x128 quantisation:      32.0 + 34.3 -> 25.4 + 31.3 us
-//   1003 tokens x 14 KB x top-4, packing + MXFP8 quantisation:     16.5 + 18.1 -> 12.6 + 16.2 us
-//   16384 tokens x 8 KB x top-8 (1.07 GB out, past that cache):     262 +  258 ->  194 +  274 us
-template <bool PLAIN>
+// Plain stores, where the launch moves more than 60 MB: the packed rows are what the caller quantises next, and what the
+// 256 MB cache keeps of them is not fetched from HBM.  Below that they are slower than the non-temporal ones: they leave the
+// rows dirty in the eight 4 MB L2s, and the launch's end waits until they are written back.  How many pairs have a local
+// destination (under expert parallelism an eighth or so) stands in dst_row alone: every wavefront looks at the same 128
+// pairs, in runs of eight spread over the call.  Packing + 1x128 quantisation, plain / hint / as chosen:
+//   512 tokens x 14 KB x top-4, 28 MB packed:     21.8 /  17.7 /  17.8 us   2048 x 8 KB x top-8, 1/8 local, 16 MB:  16.4 / 13.3 / 13.2
+//   700 x 14 KB x top-4, 38 MB:                   24.6 /  21.1 /  21.1      4096 x 4 KB x top-8, 1/8 local, 16 MB:  16.2 / 11.9 / 12.3
+//   1003 x 14 KB x top-8, 110 MB:                 48.5 /  53.8 /  48.5      4096 x 14 KB x top-8, 1/8 local, 56 MB: 36.0 / 37.3 / 36.1
+//   4096 x 8 KB x top-8, 256 MB:                 104.8 / 123.3 / 104.8      8192 x 14 KB x top-8, 1/64 local, 14 MB: 17.0 / 14.6 / 14.7
 __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_t* __restrict__ in,
-                                                                    const int* __restrict__ dst_row, long num_pieces,
-                                                                    int pieces, int topk, long row_bytes,
-                                                                    uint8_t* __restrict__ out) {
+                                                                    const int* __restrict__ dst_row, uint32_t num_pieces,
+                                                                    uint32_t pieces, int topk, long row_bytes, int plain_from,
+                                                                    long sample_step, uint8_t* __restrict__ out) {
   typedef int v4i __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63;
-  for (long piece = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); piece < num_pieces;
-       piece += (long)gridDim.x * 4) {
-    const long t = piece / pieces;
-    const int mine = lane < topk ? dst_row[t * topk + lane] : -1;   // lane j: destination of the token's pair j
-    if (__ballot(mine >= 0) == 0) continue;                         // no local pair: the row is not read
-    const long off = (piece - t * pieces) * kPermutePiece + lane * 16;
-    const uint8_t* src = in + t * row_bytes + off;
-    v4i v[4];
+  const uint32_t piece = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (piece >= num_pieces) return;
+  const uint32_t t = pieces == 1 ? piece : piece / pieces;
+  const int mine = lane < topk ? dst_row[(long)t * topk + lane] : -1;   // lane j: destination of the token's pair j
+  if (__ballot(mine >= 0) == 0) return;                               // no local pair: the row is not read
+  const long off = (long)(piece - t * pieces) * kPermutePiece + lane * 16;
+  const uint8_t* src = in + (long)t * row_bytes + off;
+  v4i v[4];
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-      if (off + u * 1024 < row_bytes) v[u] = __builtin_nontemporal_load((const v4i*)(src + u * 1024));
+  for (int u = 0; u < 4; u++)
+    if (off + u * 1024 < row_bytes) v[u] = __builtin_nontemporal_load((const v4i*)(src + u * 1024));
+  // (behind the row's loads: the samples come from a cache and are there first)
+  bool plain = false;
+  if (plain_from <= kPermuteSamples) {
+    int sample[kPermuteSamples / 64], local = 0;
+#pragma unroll
+    for (int u = 0; u < kPermuteSamples / 64; u++) sample[u] = dst_row[(u * 8 + lane / kPermuteRun) * sample_step + lane % kPermuteRun];
+#pragma unroll
+    for (int u = 0; u < kPermuteSamples / 64; u++) local += __builtin_popcountll(__ballot(sample[u] >= 0));
+    plain = local >= plain_from;
+  }
+  auto store = [&](auto hint) {   // (a loop per form: stores of both kinds in one would be merged into plain ones)
     for (int j = 0; j < topk; j++) {
       const int dst = __builtin_amdgcn_readlane(mine, j);
       if (dst < 0) continue;
@@ -268,11 +280,12 @@ __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_
 #pragma unroll
       for (int u = 0; u < 4; u++)
         if (off + u * 1024 < row_bytes) {
-          if constexpr (PLAIN) *(v4i*)(d + u * 1024) = v[u];
-          else __builtin_nontemporal_store(v[u], (v4i*)(d + u * 1024));
+          if constexpr (decltype(hint)::value) __builtin_nontemporal_store(v[u], (v4i*)(d + u * 1024));
+          else *(v4i*)(d + u * 1024) = v[u];
         }
     }
-  }
+  };
+  if (plain) store(std::false_type{}); else store(std::true_type{});
 }
 
 }  // namespace esmoe
@@ -300,16 +313,15 @@ extern "C" int esmoe_launch_permute_rows(const void* in, const int* dst_row, lon
   using namespace esmoe;
   if (num_pairs == 0) return 0;
   if (topk > 1 && topk <= 64 && num_pairs % topk == 0) {
-    const long tokens = num_pairs / topk;
-    const int pieces = (int)((row_bytes + kPermutePiece - 1) / kPermutePiece);
-    const long groups = (tokens * pieces + 3) / 4;
-    const dim3 grid((unsigned)(groups < kMaxPermuteGroups ? groups : kMaxPermuteGroups));
-    if (num_pairs > kPlainPermuteBytes / row_bytes)
-      hipLaunchKernelGGL(permute_rows_by_token_kernel<true>, grid, dim3(256), 0, stream, (const uint8_t*)in, dst_row,
-                         tokens * pieces, pieces, topk, row_bytes, (uint8_t*)out);
-    else
-      hipLaunchKernelGGL(permute_rows_by_token_kernel<false>, grid, dim3(256), 0, stream, (const uint8_t*)in, dst_row,
-                         tokens * pieces, pieces, topk, row_bytes, (uint8_t*)out);
+    const long tokens = num_pairs / topk, pieces = (row_bytes + kPermutePiece - 1) / kPermutePiece;
+    const int plain_from = permute_plain_from(tokens, topk, row_bytes);
+    const long step = pieces < kMaxPermutePieces ? kMaxPermutePieces / pieces : 1;   // tokens of a launch
+    for (long t = 0; t < tokens; t += step) {
+      const long n = tokens - t < step ? tokens - t : step;
+      hipLaunchKernelGGL(permute_rows_by_token_kernel, dim3((unsigned)((n * pieces + 3) / 4)), dim3(256), 0, stream,
+                         (const uint8_t*)in + t * row_bytes, dst_row + t * topk, (uint32_t)(n * pieces), (uint32_t)pieces, topk, row_bytes,
+                         n * topk >= kPermuteSamples ? plain_from : kPermuteSamples + 1, permute_sample_step(n * topk), (uint8_t*)out);
+    }
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(permute_rows_kernel, dim3((unsigned)((num_pairs + 3) / 4)), dim3(256), 0, stream, (const uint8_t*)in,

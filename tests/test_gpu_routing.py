@@ -120,6 +120,28 @@ def test_permute_rows_pieces(esmoe, tokens, topk, row_elems):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("tokens,topk,row_elems,share", [
+    (16, 8, 262152, 1.0),        # as many pairs as are looked at, 67 MB packed
+    (15, 8, 262152, 1.0),        # fewer
+    (4200, 2, 4104, 1.0), (4200, 8, 4104, 0.06), (4200, 8, 4104, 0.5), (4200, 8, 4104, 0.0),
+    (2100, 64, 520, 1.0),
+])
+def test_permute_rows_plain_and_hinted_stores(esmoe, tokens, topk, row_elems, share):
+    """Both kinds of stores, chosen by a look at dst_row: the same copy either way."""
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randint(-30000, 30000, (tokens, row_elems), generator=gen, device="cuda", dtype=torch.int16)
+    pairs = tokens * topk
+    local = torch.rand(pairs, generator=gen, device="cuda") < share
+    rows = int(local.sum())
+    dst = torch.full((pairs,), -1, dtype=torch.int32, device="cuda")
+    dst[local] = torch.randperm(rows, generator=gen, device="cuda").to(torch.int32)
+    out = torch.full((rows + 2, row_elems), 31000, dtype=torch.int16, device="cuda")
+    want = out.clone()
+    want[dst[local].long()] = x[torch.nonzero(local).flatten() // topk]
+    esmoe.es_permute_rows(x.view(torch.bfloat16), dst, topk, out.view(torch.bfloat16))
+    assert torch.equal(out, want)
+
+
 def test_routed_fp8_layer_on_device(esmoe):
     """ids -> metadata -> packed rows -> 1x128 quant -> grouped GEMM, all on the device, against the oracle chain."""
     from expert_specialization_moe_amd import workloads as W
