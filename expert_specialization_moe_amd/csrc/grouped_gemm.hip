@@ -1353,7 +1353,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
         }
         continue;
       }
-      const int draw = light ? sched_light_draw(ltotal, seen, (int)gridDim.x, g.k >> 7) : 1;
+      const int draw = light ? sched_light_draw(ltotal, seen, (int)gridDim.x, g.k >> 7, !FUSE) : 1;
       if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
       __syncthreads();
       ticket = __builtin_amdgcn_readfirstlane(s_item);

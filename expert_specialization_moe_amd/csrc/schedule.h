@@ -161,11 +161,15 @@ ESMOE_HD int sched_light_item_of_ticket(int ticket, int split, int* half) {
 // 256 blocks: K = 256 209 / 206 / 219 / 220 us, K = 1024 187 / 181 / 189 / 189 us (single tickets: 282 and 190 us).  The lower
 // bound is 16 K blocks, for launches that give every workgroup two such draws: below it the draw and the first stages'
 // trip from memory, about 5 us, outweigh the even end of the launch.  The whole share instead of half: up to 15 % slower.
+// `strips`: false in the kernels with a fused epilogue, which walk every tile by itself: several tickets at once only make the
+// end of their launch uneven (SwiGLU + 1x128 quantisation, 64 experts x 48 rows, 7168 x 512: 73 us with single tickets, 82
+// with up to eight).
 // All quotients are by the next power of two: a division is a chain of some forty instructions, and this stands in front of
 // a workgroup's first tile.
 constexpr int kStripBlocks = 32;
 ESMOE_HD int sched_log2_ceil(int v) { return v > 1 ? 32 - __builtin_clz((unsigned)v - 1) : 0; }
-ESMOE_HD int sched_light_draw(int total, int seen, int workgroups, int kblocks) {
+ESMOE_HD int sched_light_draw(int total, int seen, int workgroups, int kblocks, bool strips) {
+  if (!strips) return 1;
   const int lk = sched_log2_ceil(kblocks), lw = sched_log2_ceil(workgroups) + 1;
   const int most = kStripBlocks >> lk;
   int least = (kStripBlocks / 2) >> lk;

@@ -18,6 +18,7 @@ using namespace esmoe;
 extern "C" {
 int by_buffer(int n) { return strip_by_buffer(n); }
 unsigned buffer_bytes(int rows, int n, int active) { return strip_buffer_bytes(rows, n, active != 0); }
+int draw(int total, int seen, int workgroups, int kblocks, int strips) { return sched_light_draw(total, seen, workgroups, kblocks, strips != 0); }
 unsigned buffer_offset(int row, int n, int col) { return strip_buffer_offset(row, n, col); }
 }
 """
@@ -57,3 +58,23 @@ def test_stores_through_a_buffer_reach_their_element_or_are_dropped(host, n):
 @pytest.mark.parametrize("n", [(1 << 24) + 128, 1 << 25, (1 << 31) - 128])
 def test_wider_outputs_do_not_use_a_buffer(host, n):
     assert not host.by_buffer(n)
+
+
+@pytest.mark.parametrize("kblocks", [1, 2, 3, 4, 5, 8, 11, 12, 16, 17, 31, 32, 33, 56, 256])
+@pytest.mark.parametrize("workgroups", [1, 8, 255, 256, 304])
+def test_a_draw_is_at_most_a_strip(host, kblocks, workgroups):
+    for total in (1, 2, 15, 16, 255, 257, 1000, 7168, 1 << 20):
+        for seen in sorted({0, 1, total // 3, total // 2, total - 1}):
+            draw = host.draw(total, seen, workgroups, kblocks, 1)
+            assert draw >= 1 and (draw == 1 or draw * kblocks <= 32)
+            # no more than half a workgroup's share of what was left, but in a launch that has two such draws for everyone
+            # tickets of up to 16 K blocks
+            assert draw <= max(1, (total - seen) // (2 * workgroups), min(16 // kblocks, total // (2 * workgroups)))
+            assert host.draw(total, seen, workgroups, kblocks, 0) == 1   # kernels without strips
+
+
+def test_draws_at_benchmark_sizes(host):
+    """256 workgroups; 256 experts x 7168 columns at K = 256, 70 x 8192 at K = 512, 32 x 7168 at K = 2048."""
+    assert [host.draw(256 * 28, seen, 256, 2, 1) for seen in (0, 4000, 7000)] == [14, 8, 8]
+    assert host.draw(70 * 32, 0, 256, 4, 1) == 4
+    assert host.draw(32 * 28, 0, 256, 16, 1) == 1
