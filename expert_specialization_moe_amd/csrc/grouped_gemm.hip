@@ -412,8 +412,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   constexpr int MTW = G::MTW, NTW = G::NTW, NBUF = G::kNBuf;
   int tid = threadIdx.x;
   // (hidden from the compiler, which otherwise forms this tile's addresses once in front of the hand-out loop and keeps them
-  // in vector registers that the tall tiles do not have: four were spilled to scratch)
-  asm volatile("" : "+v"(tid));
+  // in vector registers that the tall tiles do not have: four were spilled to scratch.  The fused kernels have enough, and
+  // forming the addresses for every tile costs them 0.2 us a tile.)
+  if constexpr (!FUSE) asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / G::kWavesN, wn = wave % G::kWavesN;
@@ -1309,14 +1310,14 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, i
 }
 
 template <bool MX, bool FUSE>
-__global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
+__global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   __shared__ int s_item;
   __shared__ int s_counters[kXcds + 1];
-  int* ws = g.ws;
+  int* ws = args.ws;
   int hblocks, ltotal, lsplit, lshare;
-  if (g.self_schedule) {
-    self_schedule(g, lds, hblocks, ltotal, lsplit, lshare);
+  if (args.self_schedule) {
+    self_schedule(args, lds, hblocks, ltotal, lsplit, lshare);
   } else {
     hblocks = ws[kWsHeavyBlocks];
     ltotal = ws[kWsLightTotal];
@@ -1340,7 +1341,15 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs g) {
     if (x >= hblocks) dead |= 1 << x;
   // Light tickets in hand, [have, have_end), of one draw (sched_light_draw).
   int have = 0, have_end = 0, seen = 0;
+  typedef const __attribute__((address_space(4))) GemmArgs* KernArgs;
+  KernArgs kernargs = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
   for (;;) {
+    // The arguments are read anew for every tile (scalar loads that hit): kept across tiles, what the many tile functions
+    // need of them were up to 80 scalar registers spilled to lanes of vector registers, with reloads in front of every tile
+    // and inside the strips' K loops.  Read anew 0 to 15 are spilled: 8 experts x 48 rows, 768 x 512 10.8 -> 10.0 us, fused
+    // 13.1 -> 12.1; 256 experts x 32 rows, 7168 x 256 fused 182 -> 167 us.
+    asm volatile("" : "+s"(kernargs));
+    const GemmArgs& g = *(const GemmArgs*)kernargs;
     const bool light = (phase == 0) == light_first;
     const int xq = (xcd + q) & (kXcds - 1);
     int v = have;   // the light ticket or the heavy block at hand

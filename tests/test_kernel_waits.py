@@ -10,6 +10,8 @@ costs 30-40 % of the loop's speed with no wrong result to give it away.  The tes
 (no GPU needed) and checks every loop that contains MFMAs.
 
 2. The kernels must not spill a vector register (test_grouped_gemm_kernels_spill_no_vector_register).
+
+3. No K loop may reload a spilled register of either kind (test_no_reload_in_k_loops).
 """
 import importlib.util
 import os
@@ -87,3 +89,12 @@ def test_no_compiler_inserted_vmcnt_wait_in_k_loops(kernel_asm):
     assert not stray, stray
     # and the explicit ones are there
     assert all(any("explicit" in t for _, t in b) for b in loops.values())
+
+
+def test_no_reload_in_k_loops(kernel_asm):
+    """A spilled scalar register lives in a lane of a vector register (v_writelane / v_readlane), a spilled vector register in
+    scratch memory; the kernels use neither instruction otherwise inside the loops."""
+    loops = _mfma_loops(kernel_asm)
+    assert len(loops) >= 12, sorted(loops)
+    reloads = [(k, n, t) for k, b in loops.items() for n, t in b if re.match(r"(v_readlane|v_writelane|scratch_)", t)]
+    assert not reloads, reloads
