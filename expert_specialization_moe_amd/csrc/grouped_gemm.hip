@@ -1416,11 +1416,9 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     if (light) {
       t = sched_decode_light(local, M, g.policy, half);
       if constexpr (!FUSE) {
-        // the tickets in hand that are whole 256-column items of the same expert, or both halves of such, go as one strip
-        int whole = half < 0 ? (have_end < lsplit ? have_end : lsplit) - v : half == 0 ? (have_end - v) >> 1 : 0;
-        if (whole > (g.n >> 8) - local) whole = (g.n >> 8) - local;
-        if (whole > 1 && strip_by_buffer(g.n)) cols = whole;
-        if (half == 0 && whole > 0) {
+        const int tiles = sched_strip_tiles(v, have_end, lsplit, local, g.n, half);
+        if (tiles > 1) cols = tiles;
+        if (half == 0 && tiles > 0) {   // both halves: one whole tile
           t.nt = 4;
           half = -2;
         }

@@ -190,6 +190,16 @@ ESMOE_HD bool strip_by_buffer(int n) { return n <= kMaxStripN; }
 ESMOE_HD uint32_t strip_buffer_bytes(int rows, int n, bool wave_active) { return wave_active ? (uint32_t)rows * (uint32_t)n * 2 : 0; }
 ESMOE_HD uint32_t strip_buffer_offset(int row, int n, int col) { return ((uint32_t)row * (uint32_t)n + (uint32_t)col) * 2; }
 
+// Whole column tiles that run as one strip from light ticket `v` on (half `half` of column tile `local` of its expert): the
+// tickets in hand, up to `end`, that are whole items of the expert, or both halves of such.  0: the ticket is a half by itself;
+// a 128-column last tile is never part of a strip.
+ESMOE_HD int sched_strip_tiles(int v, int end, int split, int local, int n, int half) {
+  int tiles = half < 0 ? (end < split ? end : split) - v : half == 0 ? (end - v) >> 1 : 0;
+  if (tiles > (n >> 8) - local) tiles = (n >> 8) - local;
+  if (tiles > 1 && !strip_by_buffer(n)) tiles = 1;
+  return tiles > 0 ? tiles : 0;
+}
+
 // Item `item` of a light expert; half = -1: the whole 256-column item, 0 / 1: its first / second 128 columns.
 ESMOE_HD TileCoord sched_decode_light(int item, int m, const SchedPolicy& p, int half = -1) {
   TileCoord t;

@@ -1,13 +1,16 @@
-"""Index functions of schedule.h that the short tiles use, compiled for the host.
+"""Index functions of schedule.h that the short tiles and their strips use, compiled for the host.
 
 The output of a short tile leaves through a buffer descriptor with 32-bit offsets: every element of the tile's rows must be
 stored where 64-bit arithmetic puts it, and everything else (rows past the expert's last, the absent half of a last column
-tile of 128 columns) must be dropped.
+tile of 128 columns) must be dropped.  A draw of light tickets is at most a strip long, and however the workgroups' draws
+fall, the strips and single tiles cut from them cover every column of every expert once.
 """
 import ctypes
 import os
+import random
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -19,20 +22,25 @@ extern "C" {
 int by_buffer(int n) { return strip_by_buffer(n); }
 unsigned buffer_bytes(int rows, int n, int active) { return strip_buffer_bytes(rows, n, active != 0); }
 int draw(int total, int seen, int workgroups, int kblocks, int strips) { return sched_light_draw(total, seen, workgroups, kblocks, strips != 0); }
+int strip_tiles(int v, int end, int split, int local, int n, int half) { return sched_strip_tiles(v, end, split, local, n, half); }
+int item_of_ticket(int ticket, int split, int* half) { return sched_light_item_of_ticket(ticket, split, half); }
 unsigned buffer_offset(int row, int n, int col) { return strip_buffer_offset(row, n, col); }
 }
 """
 
 
-@pytest.fixture(scope="module")
-def host(tmp_path_factory):
-    d = tmp_path_factory.mktemp("host")
-    (d / "host.cpp").write_text(SOURCE)
+def schedule_functions(folder):
+    (folder / "host.cpp").write_text(SOURCE)
     csrc = os.path.join(ROOT, "expert_specialization_moe_amd", "csrc")
-    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{csrc}", str(d / "host.cpp"), "-o", str(d / "host.so")], check=True)
-    lib = ctypes.CDLL(str(d / "host.so"))
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{csrc}", str(folder / "host.cpp"), "-o", str(folder / "host.so")], check=True)
+    lib = ctypes.CDLL(str(folder / "host.so"))
     lib.buffer_bytes.restype = lib.buffer_offset.restype = ctypes.c_uint
     return lib
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    return schedule_functions(tmp_path_factory.mktemp("host"))
 
 
 # 8388736: the first width with a last tile of 128 columns whose 64 rows end past 2^30 bytes
@@ -78,3 +86,70 @@ def test_draws_at_benchmark_sizes(host):
     assert [host.draw(256 * 28, seen, 256, 2, 1) for seen in (0, 4000, 7000)] == [14, 8, 8]
     assert host.draw(70 * 32, 0, 256, 4, 1) == 4
     assert host.draw(32 * 28, 0, 256, 16, 1) == 1
+
+
+def light_tickets(native, rows, n, kind=0):
+    """(light tickets of a launch, the first that is a half item, records [experts + 1, 4]) from the host mirror."""
+    e = len(rows)
+    ps = np.array([[m, n, 512] for m in rows], dtype=np.int32)
+    ws = np.zeros(native.lib.esmoe_gemm_workspace_bytes(e) // 4, dtype=np.int32)
+    rc = native.lib.esmoe_host_schedule(ps.ctypes.data_as(ctypes.c_void_p), e, n, 0, kind, ws.ctypes.data_as(ctypes.c_void_p))
+    assert rc == 0, native.last_error()
+    first = 64 + 32 * 8
+    return int(ws[1]), int(ws[4]), ws[first:first + 4 * (e + 1)].reshape(e + 1, 4)
+
+
+@pytest.mark.parametrize("n,k,experts", [(128, 128, 9), (256, 128, 300), (384, 128, 900), (640, 256, 256), (3200, 128, 200), (4224, 128, 512),
+                                         (7168, 256, 256), (7168, 2048, 32), (2176, 384, 160), (16384, 128, 130)])
+@pytest.mark.parametrize("workgroups", [3, 256])
+def test_strips_cover_every_column_once(host, n, k, experts, workgroups):
+    """The hand-out loop's light side with the workgroups' draws in random order."""
+    from expert_specialization_moe_amd import _native
+
+    rng = random.Random(n + k + experts)
+    rows = [rng.choice((0, 1, 16, 33, 64, 300)) for _ in range(experts)]
+    total, split, rec = light_tickets(_native, rows, n)
+    firsts = rec[:, 1]
+    cover = np.zeros((experts, n // 128), dtype=np.int32)
+    half = ctypes.c_int()
+    counter, active, longest, crossing = 0, [[0, w] for w in range(workgroups)], 1, 0
+    while active:
+        i = rng.randrange(len(active))
+        draw = host.draw(total, active[i][0], workgroups, k // 128, 1)
+        v, counter = counter, counter + draw
+        if v >= total:
+            active.pop(i)
+            continue
+        active[i][0] = v
+        end, experts_of_draw = min(v + draw, total), set()
+        while v < end:
+            idx = host.item_of_ticket(v, split, ctypes.byref(half))
+            pos = int(np.searchsorted(firsts[:experts], idx, side="right")) - 1
+            e, local, m = int(rec[pos, 2]), idx - int(firsts[pos]), int(rec[pos, 3])
+            assert 0 < m <= 64 and 0 <= local < (n + 255) // 256
+            experts_of_draw.add(e)
+            h = half.value
+            tiles = host.strip_tiles(v, end, split, local, n, h)
+            if tiles > 1 or (h >= 0 and tiles):
+                assert (local + tiles) * 256 <= n and (tiles == 1 or tiles * k <= 32 * 128)
+            if h < 0:
+                cols, used, first, width = max(tiles, 1), max(tiles, 1), local * 2, 2 * max(tiles, 1)
+            elif tiles:
+                cols, used, first, width = tiles, 2 * tiles, local * 2, 2 * tiles
+            else:
+                cols, used, first, width = 1, 1, local * 2 + h, 1
+            cover[e, first:min(first + width, n // 128)] += 1
+            longest = max(longest, cols)
+            v += used
+        assert v == end
+        crossing += len(experts_of_draw) > 1
+    for e, m in enumerate(rows):
+        assert (cover[e] == (1 if 0 < m <= 64 else 0)).all(), e
+    if workgroups == 3 and k < 2048 and n >= 512:
+        assert longest > 1 and (crossing > 0 or n * k >= 4096 * 1024)
+
+
+def test_tiles_of_very_wide_outputs_are_no_strips(host):
+    n = (1 << 24) + 256
+    assert host.strip_tiles(0, 8, 100, 0, n, -1) == 1 and host.strip_tiles(100, 108, 100, 0, n, 0) == 1
+    assert host.strip_tiles(0, 8, 100, 0, 1 << 24, -1) == 8
