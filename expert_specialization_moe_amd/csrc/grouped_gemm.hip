@@ -42,6 +42,7 @@
 #include "pp_phase.h"
 #include "schedule.h"
 #include "swiglu.h"
+#include "wave_scan.h"
 
 namespace esmoe {
 
@@ -399,8 +400,7 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
 // `cols` (plain 256-column tiles only; 1 otherwise): a strip of so many neighbouring whole tiles of one expert, walked as one
 // stream of cols * K/128 stages.  The copies of the next tile's first stages are on their way while a tile ends, and its
 // output leaves as buffer stores that the counted waits leave in flight: a tile alone pays the ticket, the look-up and
-// the first stages' trip from memory, about 5 us, which at K = 256 is nine tenths of its time (256 experts x 32 rows,
-// 7168 x 256: 164 us one by one, 136 us as strips).  A strip has at most 32 stages (sched_light_draw; its weight block
+// the first stages' trip from memory, about 5 us (256 experts x 32 rows, 7168 x 256: 164 us one by one, 136 us as strips).  A strip has at most 32 stages (sched_light_draw; its weight block
 // scales share one tile's table of 256).
 template <int MT, bool MX, bool FUSE, int BN = kBN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, int cols, uint8_t* lds) {
@@ -1193,18 +1193,6 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   if (num_experts < kXcds && e >= num_experts && e < kXcds) ws[ws_xcd_counter(e)] = 0;
 }
 
-// Sum of `v` over this lane and the lanes below it, on the vector ALU alone (DPP row shifts and row broadcasts; a
-// ds_bpermute shuffle costs a trip to LDS per step).
-__device__ __forceinline__ int wave_inclusive_sum(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, :2, :4, :8 (rows of 16 lanes)
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 // The schedule built by the GEMM kernel itself (one launch per call; schedule.h, kSelfScheduleMaxExperts): every
 // workgroup does what schedule_kernel does and writes the records into `ws`, where the hand-out loop finds them with
 // scalar loads.  All workgroups write the same values.  The launch constants are returned instead of stored.  `lds` is
@@ -1213,9 +1201,9 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
 // This runs in front of every workgroup's first tile, so it is latency from end to end.  The ranking compares every pair
 // of experts: all 512 threads share that work (512 / E threads per expert, each over its slice of the other experts,
 // four keys to an LDS read), and the prefix sums stay on the vector ALU.  One thread per expert walking all others took
-// 2.6 / 4.4 / 7.9 / 13.7 us at 8 / 32 / 128 / 256 experts; whole calls this way: 8 experts x 32 rows x 256 x 512
-// 10.5 -> 9.4 us, 256 x 32 x 7168 x 256 173.9 -> 163.9 us, 128 x 8 x 768 x 4096 82.9 -> 77.2 us, 32 x 8 x 7168 x 2048
-// 79.1 -> 77.5 us.
+// 2.6 / 4.4 / 7.9 / 13.7 us at 8 / 32 / 128 / 256 experts; whole calls with this alone: 8 experts x 32 rows x 256 x 512
+// 10.5 -> 9.4 us (9.3 now), 256 x 32 x 7168 x 256 173.9 -> 163.9 us (137 now, as strips), 32 x 8 x 7168 x 2048
+// 79.1 -> 77.5 us (77.4 now).
 __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, int& hblocks, int& ltotal, int& lsplit, int& lshare) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
   int* s_key = (int*)lds;                       // order keys by expert, the list padded with keys that come last

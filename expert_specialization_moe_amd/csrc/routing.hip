@@ -24,14 +24,15 @@
 #include <type_traits>
 
 #include "permute_rule.h"
+#include "wave_scan.h"
 
 namespace esmoe {
 
 constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / 64;
 constexpr int kMaxRouteExperts = 1024;   // a thread per expert
 constexpr int kMaxChunks = 256;
-// Pairs up to which every workgroup counts all ids itself: a pass of LDS atomics over all of them, 1.3 us per 8192 pairs,
-// where the counts cost a launch and a pass over [chunks, experts] words.  128 experts, direct against counts: 8192 pairs
+// Pairs up to which every workgroup counts all ids itself, a pass of LDS atomics over all of them, where the counts cost a
+// launch and a pass over [chunks, experts] words.  128 experts, direct against counts: 8192 pairs
 // 5.2 / 6.0 us, 16384 pairs 7.1 / 6.1 us, 32768 pairs 11.4 / 6.3 us.
 constexpr long kDirectPairs = 8192;
 
@@ -75,17 +76,6 @@ __global__ void __launch_bounds__(kRouteThreads) route_count_kernel(const int* _
   }
   __syncthreads();
   if (tid < num_experts) chunk_counts[(long)blockIdx.x * num_experts + tid] = s_cnt[tid];
-}
-
-// Sum of `v` over this lane and the lanes below it, on the vector ALU (DPP row shifts and row broadcasts).
-__device__ __forceinline__ int route_inclusive_sum(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, :2, :4, :8 (rows of 16 lanes)
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-  return v;
 }
 
 // One workgroup per chunk.  DIRECT: counts from the ids; otherwise from chunk_counts [gridDim.x, num_experts].
@@ -159,7 +149,7 @@ __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* __restr
     if (off == 0) {
       // the offsets: prefix sums over the experts, thread = expert
       const int before = s_before[tid], total = before + s_rest[tid], padded = (total + 127) & ~127;
-      const int so = route_inclusive_sum(total), sp = route_inclusive_sum(padded);
+      const int so = wave_inclusive_sum(total), sp = wave_inclusive_sum(padded);
       if (lane == 63) {
         s_sum[w][0] = so;
         s_sum[w][1] = sp;

@@ -140,6 +140,9 @@ ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolic
 // 128-column halves each: a launch ends on light items (they are the last of the light-first workgroups' queue, and
 // what the others turn to when the heavy tickets are gone), fewer of them are left than there are workgroups, and an
 // item holds a CU for as long as a tall tile, so halves spread the end of the launch over twice the CUs.
+// Where a draw takes several tickets (sched_light_draw, K of up to 1024 in launches of many items) most halves of the tail
+// come out of one draw together and run as the whole tile again (sched_strip_tiles); only what a draw begins or ends with
+// stays a half.
 // Tickets [0, split) are the whole items 0 .. split-1, tickets split + 2j and split + 2j + 1 the halves of item split + j.
 ESMOE_HD int sched_light_split(int items, const SchedPolicy& p) {
   const int narrow = p.narrow_tail < items ? p.narrow_tail : items;
@@ -253,8 +256,8 @@ ESMOE_HD int ws_words(int num_experts) { return kWsHeader + (num_experts + 1) * 
 
 // One launch per call: when the counters of a workspace are known to be zero (a workspace the library owns: it is
 // zeroed when it is allocated, and the last workgroup to leave a launch zeroes the counters again), the GEMM kernel
-// needs no schedule kernel in front of it: every workgroup ranks the experts and builds the records itself, one
-// thread per expert, and writes them (the same values from every workgroup) for its own scalar loads.
+// needs no schedule kernel in front of it: every workgroup ranks the experts with all of its 512 threads (so no more experts
+// than that), builds the records itself and writes them (the same values from every workgroup) for its own scalar loads.
 constexpr int kSelfScheduleMaxExperts = 512;
 
 }  // namespace esmoe

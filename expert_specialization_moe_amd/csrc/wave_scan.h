@@ -1,0 +1,19 @@
+// Prefix sum over a wavefront, on the vector ALU alone.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace esmoe {
+
+// Sum of `v` over this lane and the lanes below it (DPP row shifts and row broadcasts; a ds_bpermute shuffle costs a trip to
+// LDS per step).
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, :2, :4, :8 (rows of 16 lanes)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+}  // namespace esmoe
