@@ -19,6 +19,7 @@
 // of each 1024 in turn).  A workgroup needs, beside its own pairs, every expert's count over all pairs and over the
 // pairs in front of its chunk.  It forms both itself, from the ids (up to kDirectPairs pairs: ONE launch) or from the
 // chunks' counts that a first launch wrote: nothing waits for another workgroup, and every workgroup knows the offsets.
+// dst_row may be the ids' own buffer.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <type_traits>
@@ -85,11 +86,11 @@ __global__ void __launch_bounds__(kRouteThreads) route_count_kernel(const int* _
 // workgroup that took up to 16384 pairs in dependent rounds, and as three launches past that, 128 experts took 10.5 us at
 // 512 pairs (now 3.5), 22.3 at 16384 (6.1), 20.2 at 32768 (6.3), 24.6 at 131072 (8.0).
 template <bool DIRECT>
-__global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* __restrict__ ids, long num_pairs, int first_expert,
+__global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, long num_pairs, int first_expert,
                                                               int num_experts, long chunk, const int* __restrict__ chunk_counts,
                                                               int n, int k, int* __restrict__ problem_sizes,
                                                               int* __restrict__ expert_offsets, int* __restrict__ blockscale_offsets,
-                                                              int* __restrict__ dst_row) {
+                                                              int* dst_row) {
   __shared__ int s_wave[kRouteWaves][kMaxRouteExperts];   // a wavefront's pairs of every expert, then their first row
   __shared__ int s_before[kMaxRouteExperts];              // pairs of every expert in the chunks in front
   __shared__ int s_rest[kMaxRouteExperts];                // and in this chunk and the ones behind
@@ -286,7 +287,9 @@ extern "C" int esmoe_launch_route_metadata(const int* ids, long num_pairs, int f
   using namespace esmoe;
   const long chunk = route_chunk_pairs(num_pairs);
   const int chunks = num_pairs > 0 ? (int)((num_pairs + chunk - 1) / chunk) : 1;
-  if (num_pairs <= kDirectPairs) {
+  // (ids that are overwritten by their rows, dst_row == ids: with several workgroups none may still count from the ids when
+  // another writes rows; route_kernel<false> reads a pair's id only in the thread that writes its row)
+  if (num_pairs <= kDirectPairs && (chunks == 1 || dst_row != ids)) {
     hipLaunchKernelGGL(route_kernel<true>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
                        chunk, (const int*)nullptr, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
     return (int)hipGetLastError();

@@ -251,7 +251,8 @@ int esmoe_swiglu_quant_1x128(const void* in, int in_dtype, void* q, float* scale
  *   problem_sizes [E,3] = (count_e, n, k);  expert_offsets [E+1], blockscale_offsets [E+1]: exclusive prefix
  *            sums of the counts and of the counts rounded up to 128, last entry = total
  *   dst_row [num_pairs]: row of pair p in the packed [sum count, .] tensors (pairs of one expert keep
- *            their order, so the result is deterministic), -1 for skipped pairs
+ *            their order, so the result is deterministic), -1 for skipped pairs; may be topk_ids itself, the other
+ *            outputs and the workspace may not overlap it
  *   workspace: esmoe_route_workspace_bytes(num_pairs, num_experts) bytes of device scratch
  */
 size_t esmoe_route_workspace_bytes(long num_pairs, int num_experts);

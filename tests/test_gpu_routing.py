@@ -13,14 +13,14 @@ from tests import helpers as H
 pytestmark = pytest.mark.gpu
 
 
-def _capi_route(native, ids, first, experts, n, k):
+def _capi_route(native, ids, first, experts, n, k, in_place=False):
     lib = native.lib
     pairs = ids.size
     d_ids = torch.from_numpy(ids.reshape(-1)).cuda()
     ps = torch.full((experts, 3), -7, dtype=torch.int32, device="cuda")
     eo = torch.full((experts + 1,), -7, dtype=torch.int32, device="cuda")
     bso = torch.full((experts + 1,), -7, dtype=torch.int32, device="cuda")
-    dst = torch.full((max(pairs, 1),), -7, dtype=torch.int32, device="cuda")
+    dst = d_ids if in_place else torch.full((max(pairs, 1),), -7, dtype=torch.int32, device="cuda")
     wsb = lib.esmoe_route_workspace_bytes(pairs, experts)
     ws = torch.empty((wsb,), dtype=torch.uint8, device="cuda")
     rc = lib.esmoe_route_metadata(H.ptr(d_ids) if pairs else None, pairs, first, experts, n, k, H.ptr(ps), H.ptr(eo), H.ptr(bso),
@@ -68,6 +68,18 @@ def test_route_metadata_edges(esmoe, pairs, experts, first, span):
     dst[np.flatnonzero(local)[order]] = np.arange(order.size)
     assert np.array_equal(got[0], np.stack([counts, np.full(experts, 256), np.full(experts, 128)], axis=1))
     assert np.array_equal(got[1], offsets) and np.array_equal(got[2], padded) and np.array_equal(got[3], dst)
+
+
+@pytest.mark.parametrize("pairs,experts", [(1000, 32), (1025, 200), (8192, 128), (8193, 128), (300000, 64)])
+def test_route_metadata_over_the_ids(esmoe, pairs, experts):
+    """Rows written over the ids (one buffer for topk_ids and dst_row): one workgroup, several, several rounds per chunk."""
+    from expert_specialization_moe_amd import _native
+
+    ids = np.random.default_rng(pairs).integers(0, experts + 5, size=pairs).astype(np.int32)
+    got = _capi_route(_native, ids.copy(), 0, experts, 256, 128, in_place=True)
+    ref = oroute.route_metadata(ids, 0, experts, 256, 128)
+    for name, g, r in zip(("problem_sizes", "expert_offsets", "blockscale_offsets", "dst_row"), got, ref):
+        assert np.array_equal(g, r), name
 
 
 def test_route_rejects(esmoe):
