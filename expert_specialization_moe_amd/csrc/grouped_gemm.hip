@@ -400,8 +400,8 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
 // `cols` (plain 256-column tiles only; 1 otherwise): a strip of so many neighbouring whole tiles of one expert, walked as one
 // stream of cols * K/128 stages.  The copies of the next tile's first stages are on their way while a tile ends, and its
 // output leaves as buffer stores that the counted waits leave in flight: a tile alone pays the ticket, the look-up and
-// the first stages' trip from memory, about 5 us (256 experts x 32 rows, 7168 x 256: 164 us one by one, 136 us as strips).  A strip has at most 32 stages (sched_light_draw; its weight block
-// scales share one tile's table of 256).
+// the first stages' trip from memory, about 5 us (256 experts x 32 rows, 7168 x 256: 164 us one by one, 135 us as strips).
+// A strip has at most 32 stages (sched_light_draw; its weight block scales share one tile's table of 256).
 template <int MT, bool MX, bool FUSE, int BN = kBN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, int cols, uint8_t* lds) {
   constexpr bool kStrip = !FUSE && BN == kBN;
@@ -1202,7 +1202,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
 // of experts: all 512 threads share that work (512 / E threads per expert, each over its slice of the other experts,
 // four keys to an LDS read), and the prefix sums stay on the vector ALU.  One thread per expert walking all others took
 // 2.6 / 4.4 / 7.9 / 13.7 us at 8 / 32 / 128 / 256 experts; whole calls with this alone: 8 experts x 32 rows x 256 x 512
-// 10.5 -> 9.4 us (9.3 now), 256 x 32 x 7168 x 256 173.9 -> 163.9 us (137 now, as strips), 32 x 8 x 7168 x 2048
+// 10.5 -> 9.4 us (9.3 now), 256 x 32 x 7168 x 256 173.9 -> 163.9 us (135 now, as strips), 32 x 8 x 7168 x 2048
 // 79.1 -> 77.5 us (77.4 now).
 __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, int& hblocks, int& ltotal, int& lsplit, int& lshare) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");

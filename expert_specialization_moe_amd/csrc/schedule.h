@@ -187,7 +187,7 @@ ESMOE_HD int sched_light_draw(int total, int seen, int workgroups, int kblocks, 
 // offsets from row m0, and whatever lies at or past the descriptor's size is dropped.  So the size has to be exact, every
 // offset of a row past the last must stay past it, and a wavefront whose columns do not exist (the absent half of a last
 // tile of 128 columns, which would land in the next row) gets a descriptor of size 0.  64 rows fit 32 bits up to
-// n = 2^25; wider outputs, from 2^24 on, take 64-bit addresses and one tile at a time.
+// n = 2^25; wider outputs, beyond 2^24, take 64-bit addresses and one tile at a time.
 constexpr int kMaxStripN = 1 << 24;
 ESMOE_HD bool strip_by_buffer(int n) { return n <= kMaxStripN; }
 ESMOE_HD uint32_t strip_buffer_bytes(int rows, int n, bool wave_active) { return wave_active ? (uint32_t)rows * (uint32_t)n * 2 : 0; }

@@ -5,8 +5,9 @@ expert stands in the call: every forced tile height must give the bytes of the d
 projection -> stand-alone quantiser, and an expert listed elsewhere, or in a call of its own, its own bytes again (another
 rank's share of the same experts is such a call).  FP8-blockwise is also checked against
 a product of the dequantised operands in fp64: one rounding to bfloat16 (2^-8 of the value) plus K roundings of fp32 sums
-(K * 2^-24 of the sum of the products' magnitudes).  MXFP8 against the same with the oracle's dequantisation, the
-magnitudes' sum taken as 60 times the largest output (K random products of one size sum to about their number's root).
+(K * 2^-24 of the sum of the products' magnitudes).  MXFP8 against the same with the oracle's dequantisation and a tighter
+count: a sum passes one MFMA of 128 products and one addition per K block, K / 128 + 128 steps that lose at most 2^-23 of
+the magnitudes' sum each (whether they round or cut off).
 """
 import numpy as np
 import pytest
@@ -23,7 +24,7 @@ pytestmark = pytest.mark.gpu
 def test_wrapped_k_order_is_the_same_for_every_tile(esmoe, kind, k):
     from expert_specialization_moe_amd import _native, workloads as W
 
-    n, rows = 512, [1, 200, 0, 33, 16, 130, 64, 65, 400, 7, 17]   # eleven starts; every tile height and its edges
+    n, rows = 512, [1, 200, 0, 33, 16, 130, 64, 65, 400, 7, 17]   # every tile height and its edges
     dt = torch.bfloat16
     prob = W.Problem("wrap", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
     if kind == "mx":
@@ -59,9 +60,10 @@ def test_wrapped_k_order_is_the_same_for_every_tile(esmoe, kind, k):
             if m:
                 sa = scales(ops["sfa"].cpu().numpy().reshape(-1), m, k, base=int(ops["blockscale_offsets"][i]) * (k // 32))
                 sw = scales(ops["sfb_phys"].cpu().numpy().reshape(-1), n, k, base=i * n * (k // 32))
-                ref = omx.dequant_rows(codes[off:off + m], sa).astype(np.float64) @ omx.dequant_rows(H.codes(ops["b_phys"][i]), sw).astype(np.float64).T
+                a, w = omx.dequant_rows(codes[off:off + m], sa).astype(np.float64), omx.dequant_rows(H.codes(ops["b_phys"][i]), sw).astype(np.float64)
+                ref, mag = a @ w.T, np.abs(a) @ np.abs(w).T
                 y = H.f32(base[off:off + m]).astype(np.float64)
-                bound = np.abs(ref) * 2.0 ** -8 + k * 2.0 ** -24 * np.abs(ref).max() * 60
+                bound = np.abs(ref) * 2.0 ** -8 + mag * ((k / 128 + 128) * 2.0 ** -23)
                 assert (np.abs(y - ref) <= bound).all(), f"expert {i}"
             off += m
         q = torch.zeros((sum(rows), n // 2), dtype=torch.uint8, device="cuda")

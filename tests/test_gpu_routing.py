@@ -112,11 +112,11 @@ def test_permute_rows_of_topk_pairs(esmoe, topk, row_elems):
 
 @pytest.mark.parametrize("tokens,topk,row_elems", [
     (1, 2, 8), (3, 5, 2048 - 8), (5, 3, 2048), (6, 2, 2048 + 8), (7, 4, 4096), (9, 2, 3 * 2048 + 520),   # around 4096 bytes
-    (2100, 2, 4104),             # the same past 32 MB of output, where the stores are plain
-    (4 * (1 << 20) + 5, 2, 8),   # more pieces than a full grid has wavefronts
+    (2100, 2, 4104),             # the same with 3 x 2100 pieces, 52 MB moved
+    (4 * (1 << 20) + 5, 2, 8),   # more pieces than one launch takes
 ])
 def test_permute_rows_pieces(esmoe, tokens, topk, row_elems):
-    """Rows of one piece, a part of one and several, and a launch whose wavefronts take more than one piece: a copy, so
+    """Rows of one piece, a part of one and several, and a call of more than one launch: a copy, so
     every byte is the source's; rows without a local pair in between, output rows that no pair names untouched."""
     gen = torch.Generator(device="cuda").manual_seed(row_elems + topk)
     x = torch.randint(-30000, 30000, (tokens, row_elems), generator=gen, device="cuda", dtype=torch.int16)
