@@ -1193,29 +1193,50 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   if (num_experts < kXcds && e >= num_experts && e < kXcds) ws[ws_xcd_counter(e)] = 0;
 }
 
+template <bool FUSE>
+__device__ __forceinline__ SchedFirst first_tickets(const GemmArgs& g, int hblocks, int ltotal, int lshare) {
+  return sched_first_tickets((int)gridDim.x, hblocks, ltotal, lshare, sched_light_draw(ltotal, 0, (int)gridDim.x, g.k >> 7, !FUSE));
+}
+
+// What a workgroup has to know of its first ticket (self_schedule).
+struct FirstRecord {
+  int first;   // first light item, or heavy block, of the expert
+  int expert, rows;
+  int row, scale_row;   // expert_offsets[expert], blockscale_offsets[expert]
+};
+
 // The schedule built by the GEMM kernel itself (one launch per call; schedule.h, kSelfScheduleMaxExperts): every
 // workgroup does what schedule_kernel does and writes the records into `ws`, where the hand-out loop finds them with
 // scalar loads.  All workgroups write the same values.  The launch constants are returned instead of stored.  `lds` is
-// the ring, free before the first tile.
+// the ring, free before the first tile.  The record of the workgroup's first ticket goes into `s_first` as well, so that
+// nothing in front of the first tile waits for the records' way to memory and back: the hand-out loop does before it reads one.
 //
 // This runs in front of every workgroup's first tile, so it is latency from end to end.  The ranking compares every pair
 // of experts: all 512 threads share that work (512 / E threads per expert, each over its slice of the other experts,
 // four keys to an LDS read), and the prefix sums stay on the vector ALU.  One thread per expert walking all others took
 // 2.6 / 4.4 / 7.9 / 13.7 us at 8 / 32 / 128 / 256 experts; whole calls with this alone: 8 experts x 32 rows x 256 x 512
-// 10.5 -> 9.4 us (9.3 now), 256 x 32 x 7168 x 256 173.9 -> 163.9 us (135 now, as strips), 32 x 8 x 7168 x 2048
-// 79.1 -> 77.5 us (77.4 now).
-__device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, int& hblocks, int& ltotal, int& lsplit, int& lshare) {
+// 10.5 -> 9.4 us, 256 x 32 x 7168 x 256 173.9 -> 163.9 us, 32 x 8 x 7168 x 2048 79.1 -> 77.5 us.  First tickets without a
+// draw, with their record from LDS (schedule.h, sched_first_tickets): 9.2 -> 6.9, 129.0 -> 125.8 (as strips) and 77.0 -> 75.6.
+template <bool MX, bool FUSE>
+__device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, FirstRecord* s_first, int& hblocks, int& ltotal, int& lsplit,
+                                              SchedFirst& f) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
   int* s_key = (int*)lds;                       // order keys by expert, the list padded with keys that come last
   int* s_rank = s_key + kThreads;               // schedule position by expert
   v4i* s_rec = (v4i*)(s_rank + kThreads);       // by schedule position: heavy blocks, light items, expert, rows
   int* s_wave = (int*)(s_rec + kThreads);       // per wavefront: blocks, items
   long* s_cost = (long*)(s_wave + 2 * kWaves);  // per expert: heavy cost, light cost
+  v2i* s_row = (v2i*)(s_cost + 2 * kThreads);   // per expert: first row, first scale row
   const int E = g.num_experts, t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const SchedPolicy policy = g.policy;
   int* ws = g.ws;
   int m = 0;
-  if (t < E) m = g.problem_sizes[t * 3];
+  v2i row = {0, 0};
+  if (t < E) {
+    m = g.problem_sizes[t * 3];
+    row[0] = g.expert_offsets[t];
+    if constexpr (MX) row[1] = g.blockscale_offsets[t];
+  }
   if (m < 0) m = 0;
   const int key = sched_order_key(m, policy);
   s_key[t] = t < E ? key : 0x7fffffff;
@@ -1237,6 +1258,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, i
     if (e < E && rank) atomicAdd(&s_rank[e], rank);
   }
   s_rec[t] = v4i{0, 0, 0, 0};
+  s_row[t] = row;
   int hb = 0, li = 0;
   if (t < E) {
     hb = sched_heavy_blocks(m, g.n, policy);
@@ -1276,7 +1298,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, i
   lsplit = __builtin_amdgcn_readfirstlane(sched_light_split(items, policy));
   ltotal = lsplit + 2 * (items - lsplit);
   // The cost totals decide how many workgroups start on which kind: needed only where a launch has both.
-  lshare = 0;
+  int lshare = 0;
   if (hblocks > 0 && items > 0) {
     long hc = 0, lc = 0;
     for (int e = lane; e < E; e += 64) {   // every wavefront sums all experts: no further barrier
@@ -1291,9 +1313,17 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, i
     lshare = sched_light_share(hc, lc, policy);
   }
   lshare = __builtin_amdgcn_readfirstlane(lshare);
-  // the records are read back with scalar loads: every store of this workgroup has to be in L2 first.  (Also a
-  // compiler-visible full wait in front of the copy-pipelined K loops, which count their own copies.)
-  __builtin_amdgcn_s_waitcnt(0);
+  // the thread whose schedule position the first ticket belongs to says so
+  f = first_tickets<FUSE>(g, hblocks, ltotal, lshare);
+  const int wg = (int)blockIdx.x, ticket = sched_first_ticket(wg, f);
+  int half = -1;
+  const bool light = sched_first_is_light(wg, f);
+  const int idx = light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(wg % kXcds, ticket);
+  const int before = light ? items_before + si - rec[1] : blocks_before + sb - rec[0];
+  if (idx >= before && idx < before + (light ? rec[1] : rec[0])) {
+    const v2i rows = s_row[rec[2]];
+    *s_first = FirstRecord{before, rec[2], rec[3], rows[0], rows[1]};
+  }
   __syncthreads();
 }
 
@@ -1302,33 +1332,43 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   __shared__ int s_item;
   __shared__ int s_counters[kXcds + 1];
+  __shared__ FirstRecord s_first;
   int* ws = args.ws;
-  int hblocks, ltotal, lsplit, lshare;
+  // (the line of the arguments that holds the operands' addresses: asked for with the others, not in front of the first tile)
+  asm volatile("" ::"s"(args.a));
+  int hblocks, ltotal, lsplit;
+  SchedFirst first;
   if (args.self_schedule) {
-    self_schedule(args, lds, hblocks, ltotal, lsplit, lshare);
+    self_schedule<MX, FUSE>(args, lds, &s_first, hblocks, ltotal, lsplit, first);
   } else {
     hblocks = ws[kWsHeavyBlocks];
     ltotal = ws[kWsLightTotal];
     lsplit = ws[kWsLightSplit];
-    lshare = ws[kWsLightShare];
+    first = first_tickets<FUSE>(args, hblocks, ltotal, ws[kWsLightShare]);
   }
   // Workgroup i runs on XCD i % 8 (HW_REG_XCC_ID = 20, bits [3:0], says so directly).  Of every 32 workgroups
   // of an XCD the last `light_share` start on the light items, the others on the heavy tickets; either kind
   // moves on to the other when its own is exhausted.
   const int xcd = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & (kXcds - 1);
-  const int per_xcd = (int)gridDim.x / kXcds > 0 ? (int)gridDim.x / kXcds : 1;
-  const bool light_first = (int)(blockIdx.x / kXcds) * 32 / per_xcd >= 32 - lshare;
+  const bool light_first = sched_first_is_light((int)blockIdx.x, first);
   int phase = 0, q = 0;
   // Queues known to be exhausted (bits 0-7: the XCDs' heavy queues, bit 8: the light items).  When a draw comes back
   // past the end of its queue and the launch has heavy blocks on every XCD, one look at all nine counters marks every
   // queue that has run dry, so that a workgroup leaving its own queue does not spend an atomic round trip (about a
   // microsecond under load) on each empty one.
-  int dead = ltotal == 0 ? 256 : 0;
-#pragma unroll
-  for (int x = 0; x < kXcds; x++)
-    if (x >= hblocks) dead |= 1 << x;
-  // Light tickets in hand, [have, have_end), of one draw (sched_light_draw).
-  int have = 0, have_end = 0, seen = 0;
+  const int undrawn = sched_undrawn_queues(hblocks, ltotal, first);
+  int dead = undrawn;
+  // Tickets in hand, [have, have_end): at first those that go by the workgroup's index (sched_first_tickets), then what a
+  // draw gave (light ones: sched_light_draw).  `xq`: their queue.
+  int have = sched_first_ticket((int)blockIdx.x, first), xq = (int)blockIdx.x % kXcds;
+  int have_end = have + (light_first ? first.light_draw : 1), seen = have;
+  {
+    const int total = light_first ? ltotal : sched_queue_tickets(xq, hblocks);
+    if (have_end > total) have_end = total;
+    if (have > have_end) have = have_end;
+  }
+  bool from_lds = args.self_schedule != 0;   // the next record is the first ticket's
+  bool records_pending = from_lds;           // this workgroup's records may still be on their way to memory
   typedef const __attribute__((address_space(4))) GemmArgs* KernArgs;
   KernArgs kernargs = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
   for (;;) {
@@ -1339,10 +1379,10 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     asm volatile("" : "+s"(kernargs));
     const GemmArgs& g = *(const GemmArgs*)kernargs;
     const bool light = (phase == 0) == light_first;
-    const int xq = (xcd + q) & (kXcds - 1);
-    int v = have;   // the light ticket or the heavy block at hand
-    int ticket = 0;
-    if (!light || have == have_end) {
+    if (have == have_end) {
+      if (dead == kAllQueues) break;
+      from_lds = false;
+      xq = (xcd + q) & (kXcds - 1);
       if ((dead >> (light ? 8 : xq)) & 1) {   // nothing (left) in this queue: the next XCD's, then the other kind
         if (light || ++q == kXcds) {
           q = 0;
@@ -1351,11 +1391,11 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
         continue;
       }
       const int draw = light ? sched_light_draw(ltotal, seen, (int)gridDim.x, g.k >> 7, !FUSE) : 1;
+      const int total = light ? ltotal : sched_queue_tickets(xq, hblocks);
       if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
       __syncthreads();
-      ticket = __builtin_amdgcn_readfirstlane(s_item);
-      v = light ? ticket : sched_ticket_block(xq, ticket);
-      if (v >= (light ? ltotal : hblocks)) {   // this queue is exhausted: see which others are
+      const int ticket = (light ? first.light_base : first.heavy_ranks) + __builtin_amdgcn_readfirstlane(s_item);
+      if (ticket >= total) {   // this queue is exhausted: see which others are
         dead |= 1 << (light ? 8 : xq);
         __syncthreads();                        // s_item and s_counters are rewritten next
         // (worth its round trip only when every XCD has a queue to try: the look itself reads the hot counter line)
@@ -1366,53 +1406,65 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
         __syncthreads();
 #pragma unroll
         for (int x = 0; x < kXcds; x++) {
-          // queue x holds the blocks x, x + 8, ...: 32 tickets each
-          const int tickets = x < hblocks ? ((hblocks - x + kXcds - 1) / kXcds) * kBlkTiles : 0;
-          if (__builtin_amdgcn_readfirstlane(s_counters[x]) >= tickets) dead |= 1 << x;
+          if (first.heavy_ranks + __builtin_amdgcn_readfirstlane(s_counters[x]) >= sched_queue_tickets(x, hblocks)) dead |= 1 << x;
         }
-        if (__builtin_amdgcn_readfirstlane(s_counters[kXcds]) >= ltotal) dead |= 256;
+        if (first.light_base + __builtin_amdgcn_readfirstlane(s_counters[kXcds]) >= ltotal) dead |= 256;
         continue;
       }
-      if (light) {
-        seen = v;
-        have = v;
-        have_end = v + draw < ltotal ? v + draw : ltotal;
-      }
+      have = ticket;
+      have_end = ticket + draw < total ? ticket + draw : total;
+      if (light) seen = ticket;
     }
     const int kind = light ? kRecItem : kRecBlock;
-    // schedule position of v: the last one whose first block (item) is <= v, found by bisection over the prefix
-    // sums with scalar loads.  The records are written by the schedule kernel and only read here, so they stay in
-    // the scalar cache, where a step costs a fraction of what a trip to L2 costs while the chip streams weights.
     // (a light ticket past `lsplit` is one half of an item of the narrow tail)
     int half = -1;
-    const int idx = light ? sched_light_item_of_ticket(v, lsplit, &half) : v;
-    int lo = 0, hi = g.num_experts;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (sload(ws, (ws_rec(mid) + kind) * 4) <= idx) lo = mid; else hi = mid;
+    const int idx = light ? sched_light_item_of_ticket(have, lsplit, &half) : sched_ticket_block(xq, have);
+    int rec_first, e, M, erow, ebso = 0;
+    if (from_lds) {
+      rec_first = __builtin_amdgcn_readfirstlane(s_first.first);
+      e = __builtin_amdgcn_readfirstlane(s_first.expert);
+      M = __builtin_amdgcn_readfirstlane(s_first.rows);
+      erow = __builtin_amdgcn_readfirstlane(s_first.row);
+      if constexpr (MX) ebso = __builtin_amdgcn_readfirstlane(s_first.scale_row);
+      from_lds = false;
+    } else {
+      if (records_pending) {   // every store of this workgroup has to be in L2 before a record is read
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        records_pending = false;
+      }
+      // schedule position of idx: the last one whose first block (item) is <= idx, found by bisection over the prefix
+      // sums with scalar loads.  The records are only read from here on, so they stay in
+      // the scalar cache, where a step costs a fraction of what a trip to L2 costs while the chip streams weights.
+      int lo = 0, hi = g.num_experts;
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (sload(ws, (ws_rec(mid) + kind) * 4) <= idx) lo = mid; else hi = mid;
+      }
+      // the whole record in one load, then the expert's first row (and first scale row) through the scalar cache as
+      // well: a vector load here waits its turn behind the weight streams of the whole chip
+      const v4i rec = sload4(ws, ws_rec(lo) * 4);
+      rec_first = __builtin_amdgcn_readfirstlane(light ? rec[kRecItem] : rec[kRecBlock]);
+      e = __builtin_amdgcn_readfirstlane(rec[kRecExpert]);
+      M = __builtin_amdgcn_readfirstlane(rec[kRecRows]);
+      erow = sload(g.expert_offsets, e * 4);
+      if constexpr (MX) ebso = sload(g.blockscale_offsets, e * 4);
     }
-    // the whole record in one load, then the expert's first row (and first scale row) through the scalar cache as
-    // well: a vector load here waits its turn behind the weight streams of the whole chip
-    const v4i rec = sload4(ws, ws_rec(lo) * 4);
-    const int first = __builtin_amdgcn_readfirstlane(light ? rec[kRecItem] : rec[kRecBlock]);
-    const int e = __builtin_amdgcn_readfirstlane(rec[kRecExpert]), M = __builtin_amdgcn_readfirstlane(rec[kRecRows]);
-    const int erow = sload(g.expert_offsets, e * 4);
-    const int ebso = MX ? sload(g.blockscale_offsets, e * 4) : 0;
-    const int local = idx - first;
+    const int local = idx - rec_first;
     TileCoord t;
     int cols = 1;
     if (light) {
       t = sched_decode_light(local, M, g.policy, half);
       if constexpr (!FUSE) {
-        const int tiles = sched_strip_tiles(v, have_end, lsplit, local, g.n, half);
+        const int tiles = sched_strip_tiles(have, have_end, lsplit, local, g.n, half);
         if (tiles > 1) cols = tiles;
         if (half == 0 && tiles > 0) {   // both halves: one whole tile
           t.nt = 4;
           half = -2;
         }
       }
-      have = v + (half == -2 ? 2 * cols : cols);
-    } else if (!sched_decode_heavy(local, ticket % kBlkTiles, M, g.n, g.policy, &t)) {
+      have += half == -2 ? 2 * cols : cols;
+    } else if (!sched_decode_heavy(local, have++ % kBlkTiles, M, g.n, g.policy, &t)) {
       __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
       continue;
     }
@@ -1447,8 +1499,9 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     }
   }
   // The last workgroup to leave zeroes the hand-out counters (nobody draws any more: every workgroup counts itself
-  // out after its last draw), so a workspace that held zero counters before the launch holds them again after it.
-  if (threadIdx.x == 0) {
+  // out after its last draw), so a workspace that held zero counters before the launch holds them again after it.  A launch
+  // of first tickets only has drawn from none.
+  if (undrawn != kAllQueues && threadIdx.x == 0) {
     const int left = atomicAdd(&ws[kWsExitCounter], 1);
     if (left == (int)gridDim.x - 1) {
 #pragma unroll

@@ -237,6 +237,44 @@ ESMOE_HD int sched_light_share(long heavy_cost, long light_cost, const SchedPoli
 // Heavy ticket `ticket` of XCD `xcd` -> launch-wide block index (the caller compares it with the block total).
 ESMOE_HD int sched_ticket_block(int xcd, int ticket) { return (ticket / kBlkTiles) * kXcds + xcd; }
 
+// Tickets of XCD `xcd`'s queue when the launch has `hblocks` heavy blocks: queue x holds the blocks x, x + 8, ..., 32 tickets each.
+ESMOE_HD int sched_queue_tickets(int xcd, int hblocks) { return xcd < hblocks ? (hblocks - xcd + kXcds - 1) / kXcds * kBlkTiles : 0; }
+
+// First tickets: a workgroup's first ticket goes by its index, and the counters hand out what lies behind these.  Atomic adds to
+// one address are served one every 12 ns, so 256 workgroups that all begin with a draw wait 3 us for the last of them, and as
+// long again to count themselves out; a launch whose tickets are all first ones needs neither.
+// `heavy_ranks`: the workgroups 8 r + x with r below it start on queue x with ticket r, the others on the light tickets, `light_draw`
+// neighbouring ones each.
+struct SchedFirst {
+  int heavy_ranks;
+  int light_draw;
+  int light_base;   // first light ticket that is drawn from the counter (a queue's: heavy_ranks)
+};
+ESMOE_HD SchedFirst sched_first_tickets(int workgroups, int hblocks, int ltotal, int light_share, int light_draw) {
+  SchedFirst f;
+  const int per_xcd = workgroups / kXcds;
+  if (hblocks == 0) f.heavy_ranks = 0;
+  else if (ltotal == 0) f.heavy_ranks = per_xcd;   // (the workgroups past a multiple of eight begin with a draw)
+  else f.heavy_ranks = ((kBlkTiles - light_share) * per_xcd + kBlkTiles - 1) / kBlkTiles;
+  f.light_draw = light_draw;
+  const int light_first = workgroups - f.heavy_ranks * kXcds;
+  f.light_base = light_first > 0 ? light_first * light_draw : 0;
+  return f;
+}
+ESMOE_HD bool sched_first_is_light(int workgroup, const SchedFirst& f) { return workgroup >= f.heavy_ranks * kXcds; }
+// First ticket of `workgroup`, of the light ones or of queue workgroup % 8; may lie past the last ticket there is.
+ESMOE_HD int sched_first_ticket(int workgroup, const SchedFirst& f) {
+  return sched_first_is_light(workgroup, f) ? (workgroup - f.heavy_ranks * kXcds) * f.light_draw : workgroup / kXcds;
+}
+// Queues that hold nothing but first tickets: bits 0-7 the XCDs' queues, bit 8 the light tickets (all nine: no counter is used).
+constexpr int kAllQueues = (1 << (kXcds + 1)) - 1;
+ESMOE_HD int sched_undrawn_queues(int hblocks, int ltotal, const SchedFirst& f) {
+  // a queue of b blocks has 32 b tickets: the queues with no more than `rounds` blocks, and they come last
+  const int rounds = f.heavy_ranks / kBlkTiles, more = hblocks - rounds * kXcds;   // blocks past that many rounds of all queues
+  const int drawn = more <= 0 ? 0 : more < kXcds ? more : kXcds;
+  return (f.light_base >= ltotal ? 1 << kXcds : 0) | (((1 << kXcds) - 1) & ~((1 << drawn) - 1));
+}
+
 // Workspace layout (int32 words).
 constexpr int kWsLightCounter = 32;  // next light ticket to hand out (every counter has a 128-byte line of its own)
 constexpr int kWsLightTotal = 1;     // number of light tickets: whole items, then two per item of the narrow tail

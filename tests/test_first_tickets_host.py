@@ -1,0 +1,70 @@
+"""First tickets (schedule.h, sched_first_tickets), compiled for the host.
+
+A workgroup's first ticket goes by its index and the counters hand out what lies behind: together they give every light ticket
+and every ticket of every XCD's queue once, whatever the kinds, the share and the number of workgroups, and a queue is named
+undrawn exactly where nothing lies behind.
+"""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include "schedule.h"
+using namespace esmoe;
+extern "C" {
+int queue_tickets(int xcd, int hblocks) { return sched_queue_tickets(xcd, hblocks); }
+int first(int wgs, int hblocks, int ltotal, int share, int draw, int wg, int* light, int* heavy_base, int* light_base, int* undrawn) {
+  const SchedFirst f = sched_first_tickets(wgs, hblocks, ltotal, share, draw);
+  *light = sched_first_is_light(wg, f);
+  *heavy_base = f.heavy_ranks;
+  *light_base = f.light_base;
+  *undrawn = sched_undrawn_queues(hblocks, ltotal, f);
+  return sched_first_ticket(wg, f);
+}
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("first")
+    (folder / "host.cpp").write_text(SOURCE)
+    csrc = os.path.join(ROOT, "expert_specialization_moe_amd", "csrc")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{csrc}", str(folder / "host.cpp"), "-o", str(folder / "host.so")], check=True)
+    return ctypes.CDLL(str(folder / "host.so"))
+
+
+@pytest.mark.parametrize("workgroups", [1, 7, 8, 9, 255, 256, 304])
+def test_first_and_drawn_tickets_cover_every_ticket_once(host, workgroups):
+    rng = random.Random(workgroups)
+    out = [ctypes.c_int() for _ in range(4)]
+    refs = [ctypes.byref(o) for o in out]
+    cases = [(0, 0), (0, 1), (1, 0), (0, workgroups), (0, workgroups + 1), (8, 0), (9, 0), (16, 0), (17, 0), (7, 5), (8, 400), (40, 2000)]
+    cases += [(rng.randrange(80), rng.randrange(1500)) for _ in range(40)]
+    for hblocks, ltotal in cases:
+        share, draw = rng.randrange(33) if hblocks and ltotal else 0, rng.choice((1, 1, 2, 5, 14, 32))
+        queues = [host.queue_tickets(x, hblocks) for x in range(8)]
+        assert sum(queues) == 32 * hblocks
+        light, heavy = [0] * ltotal, [[0] * q for q in queues]
+        for wg in range(workgroups):
+            t = host.first(workgroups, hblocks, ltotal, share, draw, wg, *refs)
+            assert t >= 0
+            if out[0].value:
+                for v in range(t, min(t + draw, ltotal)):
+                    light[v] += 1
+            elif t < queues[wg % 8]:
+                heavy[wg % 8][t] += 1
+        heavy_base, light_base, undrawn = (o.value for o in out[1:])
+        for v in range(light_base, ltotal):
+            light[v] += 1
+        for q in heavy:
+            for v in range(heavy_base, len(q)):
+                q[v] += 1
+        assert all(c == 1 for c in light) and all(c == 1 for q in heavy for c in q), (hblocks, ltotal, share, draw)
+        want = (256 if light_base >= ltotal else 0) | sum(1 << x for x in range(8) if heavy_base >= queues[x])
+        assert undrawn == want
