@@ -1134,7 +1134,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   __shared__ int s_m[1024];
   __shared__ int s_blocks[1024];
   __shared__ int s_items[1024];
-  __shared__ long s_cost[1024][2];
+  __shared__ long s_cost[1024][2];   // heavy, light
   const int e = threadIdx.x;
   int m = 0;
   if (e < num_experts) m = problem_sizes[e * 3];
@@ -1186,7 +1186,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
         heavy_cost += s_cost[j][0];
         light_cost += s_cost[j][1];
       }
-      ws[kWsLightShare] = sched_light_share(heavy_cost, light_cost, policy);
+      ws[kWsLightShare] = sched_light_share((float)heavy_cost, (float)light_cost, policy);
     }
     if (pos < kXcds) ws[ws_xcd_counter(pos)] = 0;
   }
@@ -1211,119 +1211,144 @@ struct FirstRecord {
 // the ring, free before the first tile.  The record of the workgroup's first ticket goes into `s_first` as well, so that
 // nothing in front of the first tile waits for the records' way to memory and back: the hand-out loop does before it reads one.
 //
-// This runs in front of every workgroup's first tile, so it is latency from end to end.  The ranking compares every pair
-// of experts: all 512 threads share that work (512 / E threads per expert, each over its slice of the other experts,
-// four keys to an LDS read), and the prefix sums stay on the vector ALU.  One thread per expert walking all others took
-// 2.6 / 4.4 / 7.9 / 13.7 us at 8 / 32 / 128 / 256 experts; whole calls with this alone: 8 experts x 32 rows x 256 x 512
-// 10.5 -> 9.4 us, 256 x 32 x 7168 x 256 173.9 -> 163.9 us, 32 x 8 x 7168 x 2048 79.1 -> 77.5 us.  First tickets without a
-// draw, with their record from LDS (schedule.h, sched_first_tickets): 9.2 -> 6.9, 129.0 -> 125.8 (as strips) and 77.0 -> 75.6.
+// This runs in front of every workgroup's first tile, so it is latency from end to end: trips to LDS, barriers and, at some five
+// clocks each, instructions.  Light experts (and empty ones) have at most 64 rows and the same number of items each, so a count
+// per row number puts them in order, and an expert's first item is its rank times that number.  Experts of one wavefront find
+// those of their row number with a ballot per bit.  Only heavy experts are compared with each other, packed into a list (all 512 threads
+// share the comparisons), and only they need a prefix sum.  Comparing all experts took 0.5 / 1.1 / 3.7 us at 8 / 32 / 256 experts and
+// the cost totals of a launch with both kinds 0.8 us.  Whole calls, first tickets without a draw (schedule.h, sched_first_tickets): 8 experts
+// x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us.
 template <bool MX, bool FUSE>
 __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, FirstRecord* s_first, int& hblocks, int& ltotal, int& lsplit,
                                               SchedFirst& f) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
-  int* s_key = (int*)lds;                       // order keys by expert, the list padded with keys that come last
-  int* s_rank = s_key + kThreads;               // schedule position by expert
-  v4i* s_rec = (v4i*)(s_rank + kThreads);       // by schedule position: heavy blocks, light items, expert, rows
-  int* s_wave = (int*)(s_rec + kThreads);       // per wavefront: blocks, items
-  long* s_cost = (long*)(s_wave + 2 * kWaves);  // per expert: heavy cost, light cost
-  v2i* s_row = (v2i*)(s_cost + 2 * kThreads);   // per expert: first row, first scale row
+  constexpr int kLightRows = 64, kHistStride = kLightRows + 4;
+  int* s_hist = (int*)lds;                              // [kWaves][kHistStride]: experts of a wavefront by rows (0 .. 64)
+  int* s_heavy = s_hist + kWaves * kHistStride;         // [kWaves]: heavy experts of a wavefront
+  v4f* s_sums = (v4f*)(s_heavy + kWaves);               // [kWaves]: blocks, heavy cost, light cost
+  int* s_key = (int*)(s_sums + kWaves);                 // heavy experts' keys, in index order
+  int* s_rank = s_key + kThreads;                       // their ranks
+  int* s_blocks = s_rank + kThreads;                    // by rank: blocks of the expert, then blocks in front inside the wavefront
   const int E = g.num_experts, t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const SchedPolicy policy = g.policy;
   int* ws = g.ws;
-  int m = 0;
-  v2i row = {0, 0};
+  int m = 0, row = 0, scale_row = 0;
   if (t < E) {
     m = g.problem_sizes[t * 3];
-    row[0] = g.expert_offsets[t];
-    if constexpr (MX) row[1] = g.blockscale_offsets[t];
+    row = g.expert_offsets[t];
+    if constexpr (MX) scale_row = g.blockscale_offsets[t];
   }
-  if (m < 0) m = 0;
-  const int key = sched_order_key(m, policy);
-  s_key[t] = t < E ? key : 0x7fffffff;
+  s_hist[wave * kHistStride + lane] = 0;   // (a wavefront's LDS accesses stay in order)
+  if (lane == 0) s_hist[wave * kHistStride + kLightRows] = 0;
   s_rank[t] = 0;
-  const int epad = E > 1 ? 1 << (32 - __builtin_clz(E - 1)) : 1;   // experts, rounded up to a power of two (at most 512)
-  const int logp = 31 - __builtin_clz(epad), parts = kThreads >> logp;
+  // (waited for here: a load that the compiler holds for outstanding puts a wait of its own into the K loops)
+  asm volatile("" : "+v"(row), "+v"(scale_row));
+  if (m < 0) m = 0;
+  const bool heavy = t < E && sched_is_heavy(m, policy), light = t < E && !heavy;
+  uint64_t same = __ballot(light);   // light experts of this wavefront with as many rows
+#pragma unroll
+  for (int i = 0; i < 7; i++) {
+    const bool bit = (m >> i) & 1;
+    const uint64_t set = __ballot(bit);
+    same &= bit ? set : ~set;
+  }
+  const uint64_t heavies = __ballot(heavy);
+  const int same_before = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0));
+  if (light && same_before == 0) s_hist[wave * kHistStride + m] = __builtin_popcountll(same);
+  if (lane == 0) s_heavy[wave] = __builtin_popcountll(heavies);
   __syncthreads();
-  if (policy.order != 1) {
-    // slice `part` of the other experts, in fours; an expert comes in front of another of the same key if its index is lower
-    const int e = t & (epad - 1), part = t >> logp;
-    const int quads = (epad + 3) >> 2, per = (quads + parts - 1) / parts;
-    const int ke = s_key[e];
-    int rank = 0;
+  const int waves = (E + 63) >> 6;   // that hold experts
+  int by_rows = 0, rank = same_before, heavy_before = 0, num_heavy = 0;
+  for (int w = 0; w < waves; w++) {
+    by_rows += s_hist[w * kHistStride + 1 + lane];   // lane: experts with lane + 1 rows
+    if (light && w < wave) rank += s_hist[w * kHistStride + m];
+    const int h = s_heavy[w];
+    num_heavy += h;
+    if (w < wave) heavy_before += h;
+  }
+  num_heavy = __builtin_amdgcn_readfirstlane(num_heavy);
+  const int fewer = wave_inclusive_sum(by_rows);   // experts with 1 .. lane + 1 rows
+  const int num_light = __builtin_amdgcn_readlane(fewer, 63);
+  const int up_to = __shfl(fewer, m - 1);
+  rank += num_light - (m > 0 ? up_to : 0);   // those with more rows come first
+  const int ntl = sched_ntiles(g.n, 4);
+  const int items = num_light * ntl;
+  int pos = num_heavy + rank, before = 0, mine = 0;   // schedule position; first item or block, and number of them
+  if (light) {
+    before = (rank < num_light ? rank : num_light) * ntl;
+    mine = m > 0 ? ntl : 0;
+  }
+  int blocks = 0, lshare = 0;
+  if (num_heavy > 0) {
+    const int h = heavy_before + __builtin_amdgcn_mbcnt_hi((uint32_t)(heavies >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)heavies, 0));
+    if (heavy) s_key[h] = sched_order_key(m, policy);
+    if (t >= num_heavy && t < ((num_heavy + 3) & ~3)) s_key[t] = 0x7fffffff;
+    int hb = 0;
+    float heavy_cost = 0.f, light_cost = 0.f;
+    if (heavy) {
+      hb = sched_heavy_blocks(m, g.n, policy);
+      heavy_cost = (float)sched_heavy_cost(m, g.n, policy);
+    } else if (light) {
+      light_cost = (float)sched_light_cost(m, g.n, policy);
+    }
+    __syncthreads();
+    // slice `part` of the list, in fours; an expert comes in front of another of the same key if its index is lower
+    const int logp = sched_log2_ceil(num_heavy), logparts = 9 - logp;
+    static_assert(kThreads == 1 << 9, "threads");
+    const int i = t & ((1 << logp) - 1), part = t >> logp;
+    const int quads = (num_heavy + 3) >> 2, per = (quads + (1 << logparts) - 1) >> logparts;
+    const int ki = s_key[i];
+    int r = 0;
+#pragma unroll 4
     for (int q = part * per; q < (part + 1) * per && q < quads; q++) {
       const v4i k = *(const v4i*)(s_key + q * 4);
 #pragma unroll
-      for (int i = 0; i < 4; i++) rank += k[i] < ke + (q * 4 + i < e ? 1 : 0);
+      for (int c = 0; c < 4; c++) r += k[c] < ki + (q * 4 + c < i ? 1 : 0);
     }
-    if (e < E && rank) atomicAdd(&s_rank[e], rank);
-  }
-  s_rec[t] = v4i{0, 0, 0, 0};
-  s_row[t] = row;
-  int hb = 0, li = 0;
-  if (t < E) {
-    hb = sched_heavy_blocks(m, g.n, policy);
-    li = sched_light_items(m, g.n, policy);
-    s_cost[2 * t] = sched_heavy_cost(m, g.n, policy);
-    s_cost[2 * t + 1] = sched_light_cost(m, g.n, policy);
-  }
-  __syncthreads();
-  if (t < E) s_rec[policy.order != 1 ? s_rank[t] : t] = v4i{hb, li, t, m};
-  __syncthreads();
-  // exclusive prefix sums over the schedule positions (thread = position): inclusive scan inside the wavefront, then
-  // the totals of the wavefronts in front
-  const v4i rec = s_rec[t];
-  const int sb = wave_inclusive_sum(rec[0]), si = wave_inclusive_sum(rec[1]);
-  if (lane == 63) {
-    s_wave[2 * wave] = sb;
-    s_wave[2 * wave + 1] = si;
-  }
-  __syncthreads();
-  int blocks_before = 0, items_before = 0, blocks = 0, items = 0;
+    if (i < num_heavy && r) atomicAdd(&s_rank[i], r);
+    __syncthreads();
+    if (heavy) {
+      pos = s_rank[h];
+      s_blocks[pos] = hb;
+      mine = hb;
+    }
+    __syncthreads();
+    const int b = t < num_heavy ? s_blocks[t] : 0;
+    const int sb = wave_inclusive_sum(b);
+    heavy_cost = wave_sum_last(heavy_cost);
+    light_cost = wave_sum_last(light_cost);
+    if (lane == 63) s_sums[wave] = v4f{__builtin_bit_cast(float, sb), heavy_cost, light_cost, 0.f};
+    s_blocks[t] = sb - b;
+    __syncthreads();
+    float hc = 0.f, lc = 0.f;
+    if (heavy) before = s_blocks[pos];
 #pragma unroll
-  for (int w = 0; w < kWaves; w++) {
-    const int wb = s_wave[2 * w], wi = s_wave[2 * w + 1];
-    if (w < wave) {
-      blocks_before += wb;
-      items_before += wi;
+    for (int w = 0; w < kWaves; w++) {
+      const v4f v = s_sums[w];
+      const int wb = __builtin_bit_cast(int, v[0]);
+      blocks += wb;
+      if (heavy && w < pos >> 6) before += wb;
+      hc += v[1];
+      lc += v[2];
     }
-    blocks += wb;
-    items += wi;
+    blocks = __builtin_amdgcn_readfirstlane(blocks);
+    // how many workgroups start on which kind, where a launch has both
+    if (items > 0) lshare = __builtin_amdgcn_readfirstlane(sched_light_share(hc, lc, policy));
   }
-  // record t; record E closes the prefix sums
-  if (t < E) *(v4i*)(ws + ws_rec(t)) = v4i{blocks_before + sb - rec[0], items_before + si - rec[1], rec[2], rec[3]};
+  // the expert's record, at its schedule position; record E closes the prefix sums
+  if (t < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, t, m} : v4i{blocks, before, t, m};
   if (t == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
-  hblocks = __builtin_amdgcn_readfirstlane(blocks);
-  items = __builtin_amdgcn_readfirstlane(items);
-  lsplit = __builtin_amdgcn_readfirstlane(sched_light_split(items, policy));
+  hblocks = blocks;
+  lsplit = sched_light_split(items, policy);
   ltotal = lsplit + 2 * (items - lsplit);
-  // The cost totals decide how many workgroups start on which kind: needed only where a launch has both.
-  int lshare = 0;
-  if (hblocks > 0 && items > 0) {
-    long hc = 0, lc = 0;
-    for (int e = lane; e < E; e += 64) {   // every wavefront sums all experts: no further barrier
-      hc += s_cost[2 * e];
-      lc += s_cost[2 * e + 1];
-    }
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      hc += __shfl_xor(hc, d);
-      lc += __shfl_xor(lc, d);
-    }
-    lshare = sched_light_share(hc, lc, policy);
-  }
-  lshare = __builtin_amdgcn_readfirstlane(lshare);
-  // the thread whose schedule position the first ticket belongs to says so
+  // the thread of the expert that the first ticket belongs to says so
   f = first_tickets<FUSE>(g, hblocks, ltotal, lshare);
   const int wg = (int)blockIdx.x, ticket = sched_first_ticket(wg, f);
   int half = -1;
-  const bool light = sched_first_is_light(wg, f);
-  const int idx = light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(wg % kXcds, ticket);
-  const int before = light ? items_before + si - rec[1] : blocks_before + sb - rec[0];
-  if (idx >= before && idx < before + (light ? rec[1] : rec[0])) {
-    const v2i rows = s_row[rec[2]];
-    *s_first = FirstRecord{before, rec[2], rec[3], rows[0], rows[1]};
-  }
+  const bool first_light = sched_first_is_light(wg, f);
+  const int idx = first_light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(wg % kXcds, ticket);
+  if ((first_light ? light : heavy) && idx >= before && idx < before + mine) *s_first = FirstRecord{before, t, m, row, scale_row};
   __syncthreads();
 }
 

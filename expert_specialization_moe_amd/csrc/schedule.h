@@ -39,6 +39,21 @@ struct TileCoord {
   int n0;  // first column
 };
 
+// a / b for a >= 0, b > 0.  On the device an integer division by a variable is a chain of some forty instructions, and the
+// schedule of an expert with more than 64 rows takes seven of them in front of the first tile, as does every heavy ticket; for
+// a < 2^22 the float quotient is off by less than one, and the remainder says which way.
+ESMOE_HD int sched_div(int a, int b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (a < (1 << 22)) {
+    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+    const int r = a - q * b;
+    q += r >= b ? 1 : 0;
+    return r < 0 ? q - 1 : q;
+  }
+#endif
+  return a / b;
+}
+
 // The tile heights the kernels are compiled for.
 ESMOE_HD bool sched_valid_mt(int mt) { return mt == 1 || mt == 2 || mt == 4 || mt == 8 || mt == 12; }
 
@@ -92,7 +107,7 @@ ESMOE_HD int sched_order_key(int m, const SchedPolicy& p) {
 // Row tiles of an expert: full big tiles plus one remainder tile.
 ESMOE_HD int sched_mtiles(int m, const SchedPolicy& p) {
   const int rows = (p.force_mt ? p.force_mt : p.big_mt) * 16;
-  return (m + rows - 1) / rows;
+  return sched_div(m + rows - 1, rows);
 }
 
 // Block shape for an expert with mtl x ntl tiles: at most kBlkM tiles high and kBlkTiles tiles in all, with
@@ -100,10 +115,10 @@ ESMOE_HD int sched_mtiles(int m, const SchedPolicy& p) {
 // 6 x 16 -> 6 x 4; 1 x 16 -> 1 x 16).  Near-square blocks (in bytes) fetch the least per tile.
 ESMOE_HD void sched_block_shape(int mtl, int ntl, int* bm, int* bn) {
   const int rb = (mtl + kBlkM - 1) / kBlkM;
-  *bm = (mtl + rb - 1) / rb;
-  const int w = kBlkTiles / *bm;
-  const int cb = (ntl + w - 1) / w;
-  *bn = (ntl + cb - 1) / cb;
+  *bm = sched_div(mtl + rb - 1, rb);
+  const int w = sched_div(kBlkTiles, *bm);
+  const int cb = sched_div(ntl + w - 1, w);
+  *bn = sched_div(ntl + cb - 1, cb);
 }
 
 ESMOE_HD int sched_heavy_blocks(int m, int n, const SchedPolicy& p) {
@@ -111,7 +126,7 @@ ESMOE_HD int sched_heavy_blocks(int m, int n, const SchedPolicy& p) {
   const int mtl = sched_mtiles(m, p), ntl = sched_ntiles(n, 4);
   int bm, bn;
   sched_block_shape(mtl, ntl, &bm, &bn);
-  return ((mtl + bm - 1) / bm) * ((ntl + bn - 1) / bn);
+  return sched_div(mtl + bm - 1, bm) * sched_div(ntl + bn - 1, bn);
 }
 
 ESMOE_HD int sched_light_items(int m, int n, const SchedPolicy& p) {
@@ -123,9 +138,10 @@ ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolic
   const int mtl = sched_mtiles(m, p), ntl = sched_ntiles(n, 4);
   int bm, bn;
   sched_block_shape(mtl, ntl, &bm, &bn);
-  const int nbc = (ntl + bn - 1) / bn;
+  const int nbc = sched_div(ntl + bn - 1, bn);
   if (idx >= bm * bn) return false;
-  const int mi = (lb / nbc) * bm + idx / bn, ni = (lb % nbc) * bn + idx % bn;
+  const int rb = sched_div(lb, nbc), r = sched_div(idx, bn);
+  const int mi = rb * bm + r, ni = (lb - rb * nbc) * bn + idx - r * bn;
   if (mi >= mtl || ni >= ntl) return false;
   const int big = p.force_mt ? p.force_mt : p.big_mt;
   const int m0 = mi * big * 16;
@@ -219,19 +235,19 @@ ESMOE_HD TileCoord sched_decode_light(int item, int m, const SchedPolicy& p, int
 ESMOE_HD long sched_heavy_cost(int m, int n, const SchedPolicy& p) {
   if (!sched_is_heavy(m, p)) return 0;
   const int big = (p.force_mt ? p.force_mt : p.big_mt) * 16;
-  const int full = m / big, rem = m - full * big;
+  const int full = sched_div(m, big), rem = m - full * big;
   const int rows = full * big + (rem ? (p.force_mt ? big : sched_cover_mt(rem, p.big_mt) * 16) : 0);
   return (long)(rows + 16 * sched_mtiles(m, p)) * sched_ntiles(n, 4);
 }
 ESMOE_HD long sched_light_cost(int m, int n, const SchedPolicy& p) {
   return (long)sched_light_items(m, n, p) * (75 + m / 3);
 }
-// Workgroups of every 32 that start on the light items.
-ESMOE_HD int sched_light_share(long heavy_cost, long light_cost, const SchedPolicy& p) {
+// Workgroups of every 32 that start on the light items.  (Floats: it is an estimate, and a 64-bit division and sum of both costs
+// stood 0.8 us in front of the first tile.)
+ESMOE_HD int sched_light_share(float heavy_cost, float light_cost, const SchedPolicy& p) {
   if (p.light_share >= 0) return p.light_share > 32 ? 32 : p.light_share;
   if (heavy_cost <= 0 || light_cost <= 0) return 0;
-  const long total = heavy_cost + light_cost;
-  return (int)((32 * light_cost + total / 2) / total);
+  return (int)(32 * light_cost / (heavy_cost + light_cost) + 0.5f);
 }
 
 // Heavy ticket `ticket` of XCD `xcd` -> launch-wide block index (the caller compares it with the block total).
