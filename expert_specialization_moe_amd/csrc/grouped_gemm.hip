@@ -177,6 +177,31 @@ __device__ __forceinline__ void store_staged_rows(const uint8_t* stage, int stri
   }
 }
 
+// Four accumulators as the output's 16-bit type (0 bf16, 1 fp16).
+__device__ __forceinline__ v2i out_half4(v4f v, int out_dtype) {
+  return out_dtype == 0 ? __builtin_bit_cast(v2i, __builtin_convertvector(v, bf16x4)) : __builtin_bit_cast(v2i, __builtin_convertvector(v, f16x4));
+}
+// A lane of group gq = lane / 16 holds columns 4*gq .. +4 of one row in each of two 16-column tiles, `x` and `y`.  Odd groups give
+// their part of x for the even neighbour's part of y: groups 0 and 2 end with columns 0 .. 8 and 8 .. 16 of the first tile,
+// groups 1 and 3 with those of the second, 16 contiguous bytes a lane.
+__device__ __forceinline__ v4i pair_halves(v2i x, v2i y) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+  return v4i{(int)lo[0], (int)hi[0], (int)lo[1], (int)hi[1]};
+}
+__device__ __forceinline__ int pair_column(int gq) { return (gq & 1) * 16 + (gq >> 1) * 8; }   // of the two tiles' 32
+
+// Whether a short tile's output leaves with the non-temporal hint.  Without it the pieces of a row merge in L2 first, and the
+// eight L2s keep the lines dirty and write them back in front of later weights and at the launch's end; with it every 64-byte
+// piece goes out by itself.  Tiles of many rows and more K blocks are better off with it, tiles that are little more than their
+// stores without (128 experts, 4096 columns, plain / hinted, us): 32 rows each K = 1536 160.4 / 147.4, K = 512 61.6 / 61.6,
+// K = 640 75.0 / 72.3; 256 x 32 rows x 7168, K = 256 115.5 / 123.3; 16 rows each K = 1536 149.1 / 139.9; 8 rows each K = 1024
+// 91.0 / 92.2, K = 1536 137.0 / 135.2; 2 rows each K = 1536 114.4 / 116.1.
+template <int MT>
+__device__ __forceinline__ bool short_out_nt(int kblocks, int rows) {
+  return MT >= 2 ? kblocks >= 4 : kblocks >= 12 && rows > 8;
+}
+
 // Epilogue of a tile: `acc[nt][mt][i]` holds, for this lane, columns n0 + nw + nt*16 + 4*gq + i of token row
 // m0 + mw + mt*16 + r (gq = lane / 16, r = lane % 16).  Plain form: convert and store.  FUSE: SwiGLU and the 1x128
 // quantisation (the wavefront's first NTW/2 column tiles are gate columns, the rest the matching up columns).
@@ -282,22 +307,21 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, Acc& acc, int M
     }
     return;
   }
-  if (wave_active) {
+  // short tiles: 16 contiguous bytes a lane where there are two tiles to trade halves, next to each other in columns (whole
+  // tiles) or in rows (halves of 128 columns, whose wavefronts have one column tile)
+  if constexpr (!FUSE && kWavesN == kWaves) {
+    if (!wave_active) return;
+    if constexpr (NTW == 1 && MTW == 1) {
+      const int m = m0 + mw + r;
+      if (m < M) *(v2i*)((uint8_t*)g.out + ((row_base + m) * (long)N + n0 + nw + gq * 4) * 2) = out_half4(acc[0][0], g.out_dtype);
+    } else {
 #pragma unroll
-    for (int mt = 0; mt < MTW; mt++) {
-      int m = m0 + mw + mt * 16 + r;
-      if (m < M) {
-        long orow = (row_base + m) * (long)N;
-#pragma unroll
-        for (int nt = 0; nt < NTW; nt++) {
-          int n = n0 + nw + nt * 16 + gq * 4;
-          const v4f v = {acc[nt][mt][0], acc[nt][mt][1], acc[nt][mt][2], acc[nt][mt][3]};
-          if (g.out_dtype == 0) {
-            *(bf16x4*)((__bf16*)g.out + orow + n) = __builtin_convertvector(v, bf16x4);
-          } else {
-            *(f16x4*)((_Float16*)g.out + orow + n) = __builtin_convertvector(v, f16x4);
-          }
-        }
+      for (int i = 0; i < MTW * NTW / 2; i++) {
+        const v4i line = NTW == 2 ? pair_halves(out_half4(acc[0][i], g.out_dtype), out_half4(acc[NTW - 1][i], g.out_dtype))
+                                  : pair_halves(out_half4(acc[0][2 * i], g.out_dtype), out_half4(acc[0][2 * i + 1], g.out_dtype));
+        const int m = m0 + mw + r + (NTW == 2 ? i * 16 : (2 * i + (gq & 1)) * 16);
+        const int n = n0 + nw + (NTW == 2 ? pair_column(gq) : (gq >> 1) * 8);
+        if (m < M) *(v4i*)((uint8_t*)g.out + ((row_base + m) * (long)N + n) * 2) = line;
       }
     }
   }
@@ -705,7 +729,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   // weight stream, not by the overlap of reads and MFMAs.)
   // Strips: a finished column tile's kStores output stores stay in flight as well while they are younger than the stage
   // waited for (vmcnt counts loads and stores in one order); two tiles' worth (K = 128) is waited for as one, the safe side.
-  constexpr int kStores = MTW * NTW;
+  constexpr int kStores = MTW * NTW / 2;
   auto wait_stage = [&](bool more, bool chunk_young, bool stores_young) {
     // all of this wavefront's copies except those of the newest NBUF-2 K blocks have landed
     if (!more) {
@@ -722,16 +746,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   // Output of a strip: the tile's rows as a buffer, so that every lane of every wavefront stores without a branch (a fixed
   // number of stores to count) and the hardware drops rows at or past M and the columns of a last tile's absent half
   // (strip_buffer_bytes).  Outputs too wide for 32-bit offsets leave through tile_epilogue behind the loop.
-  // Plain stores: the 32-byte pieces of a row have to merge in L2 (with the non-temporal hint 206 us instead of 136 at 256
-  // experts x 32 rows, 7168 x 256).
+  // The two column tiles of a wavefront trade halves between neighbouring lane groups (pair_halves), so that a lane holds 16
+  // contiguous bytes and a store writes 64-byte pieces of sixteen rows in half as many instructions as 32-byte ones straight from
+  // the MFMA layout (256 experts x 32 rows, 7168 x 256: 122.4 -> 115.5 us).
   [[maybe_unused]] uint32_t voff = 0;
   [[maybe_unused]] __amdgpu_buffer_rsrc_t out_buf;
   const bool by_buffer = kStrip && strip_by_buffer(N);
+  const bool out_nt = short_out_nt<MT>(KB, M);
   if constexpr (kStrip) {
     const int rows = M - m0 < G::BM ? M - m0 : G::BM;
     out_buf = __builtin_amdgcn_make_buffer_rsrc((uint8_t*)g.out + (row_base + m0) * (long)N * 2, 0,
                                                 (int)strip_buffer_bytes(rows, N, wave_active), 0x00027000);
-    voff = strip_buffer_offset(mw + r, N, n0 + nw + gq * 4);
+    voff = strip_buffer_offset(mw + r, N, n0 + nw + pair_column(gq));
   }
   int buf = 0, nbuf = NBUF - 1;  // ring slots of stage kb and of stage kb + NBUF - 1
   int chunk_age = NBUF;          // iterations since this wavefront issued a scale-chunk copy
@@ -770,14 +796,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
         store_age = 0;
 #pragma unroll
         for (int mt = 0; mt < MTW; mt++) {
+          static_assert(NTW == 2 || !kStrip, "a wavefront of a strip has one pair of column tiles");
+          const v4i line = pair_halves(out_half4(acc[0][mt], g.out_dtype), out_half4(acc[NTW - 1][mt], g.out_dtype));
+          const uint32_t off = voff + strip_buffer_offset(mt * 16, N, 0);
+          if (out_nt) __builtin_amdgcn_raw_buffer_store_b128(line, out_buf, off, 0, 2);
+          else __builtin_amdgcn_raw_buffer_store_b128(line, out_buf, off, 0, 0);
 #pragma unroll
-          for (int nt = 0; nt < NTW; nt++) {
-            const v4f v = {acc[nt][mt][0], acc[nt][mt][1], acc[nt][mt][2], acc[nt][mt][3]};
-            const v2i w = g.out_dtype == 0 ? __builtin_bit_cast(v2i, __builtin_convertvector(v, bf16x4))
-                                           : __builtin_bit_cast(v2i, __builtin_convertvector(v, f16x4));
-            __builtin_amdgcn_raw_buffer_store_b64(w, out_buf, voff + strip_buffer_offset(mt * 16, N, nt * 16), 0, 0);
-            acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-          }
+          for (int nt = 0; nt < NTW; nt++) acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
         }
         voff += kBN * 2;
       }
