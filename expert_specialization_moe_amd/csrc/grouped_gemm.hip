@@ -427,7 +427,8 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
 // the first stages' trip from memory, about 5 us (256 experts x 32 rows, 7168 x 256: 164 us one by one, 135 us as strips).
 // A strip has at most 32 stages (sched_light_draw; its weight block scales share one tile's table of 256).
 template <int MT, bool MX, bool FUSE, int BN = kBN>
-__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, int cols, uint8_t* lds) {
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb, int erow, int ebso, int M, int m0, int n0, int cols,
+                                          uint8_t* lds) {
   constexpr bool kStrip = !FUSE && BN == kBN;
   static_assert(kStripBlocks <= kMaxKB, "the weight block scales of a strip share the table of one tile");
   static_assert(!(FUSE && BN != kBN), "the fused epilogues need gate and up columns of a whole quantisation block in one tile");
@@ -542,16 +543,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     if (w_once) dma16xn<true>(lw, w_ptr + (long)kb * 128, vw);
     else dma16xn<false>(lw, w_ptr + (long)kb * 128, vw);
   };
-  // next stage of the tile or strip: K block ip of its current column tile
+  // next stage of the tile or strip: K block ip of its current column tile, from the first of the expert's K order round to it
   const int stages = kStrip ? cols * KB : KB;
-  int ip = 0;
+  int ip = first_kb;
   auto issue_next = [&](int buf) {
     issue_a(ip, buf);
     issue_w(ip, buf);
-    ip++;
+    ip = ip + 1 == KB ? 0 : ip + 1;
     if constexpr (kStrip) {
-      if (ip == KB) {   // on to the next column tile
-        ip = 0;
+      if (ip == first_kb) {   // on to the next column tile
         w_ptr += (long)kBN * K;
         if constexpr (MX) sc_base += (wave & 1) == 0 ? (long)KB * 1024 : 0;
       }
@@ -595,11 +595,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     float sb_up;   // FUSE: scale of the up rows' weight block (sb is the gate rows')
   };
 
-  int pos = 0;   // K block of the stage at hand inside its column tile
+  int pos = first_kb;   // K block of the stage at hand inside its column tile
   auto read_scales_fp8 = [&](int kb, int buf, Frags& f) {
     const uint8_t* lb = lds + buf * G::kStageBytes;
-    f.sb = sb_tab[kStrip ? pos : kb];
-    if constexpr (FUSE) f.sb_up = sb_tab[kMaxKB + kb];
+    f.sb = sb_tab[pos];
+    if constexpr (FUSE) f.sb_up = sb_tab[kMaxKB + pos];
 #pragma unroll
     for (int mt = 0; mt < MTW; mt++) {
       f.sc[mt] = sa4 ? *(const float*)(lds + sa4_lane + ((kb >> 2) & 1) * 4096 + (kb & 3) * 4 + mt * 256)
@@ -711,7 +711,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
       dma4(g.sb + ((long)e * (N >> 7) + nb) * KB, (uint32_t)kbi * 4, lds0 + kRingBytes + (blk * kMaxKB + kb0) * 4);
     }
   }
-  if (sa4 && wave * 64 < G::BM) issue_sa_chunk(0, 0);
+  if (sa4 && wave * 64 < G::BM) issue_sa_chunk(0, first_kb);
 #pragma unroll
   for (int s = 0; s < NBUF - 1; s++) {
     if (s < stages) issue_next(s);
@@ -762,7 +762,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
   int buf = 0, nbuf = NBUF - 1;  // ring slots of stage kb and of stage kb + NBUF - 1
   int chunk_age = NBUF;          // iterations since this wavefront issued a scale-chunk copy
   int store_age = NBUF;          // iterations since a column tile's output was stored
-  int cpos = 0;                  // first K block of the scale chunk being read
+  int cpos = first_kb;           // first K block of the scale chunk being read
   Frags f;
   for (int kb = 0; kb < stages; kb++) {
     const bool more = kb + NBUF - 1 < stages;
@@ -789,9 +789,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
     block_barrier();
     buf = buf + 1 == NBUF ? 0 : buf + 1;
     nbuf = nbuf + 1 == NBUF ? 0 : nbuf + 1;
+    pos = pos + 1 == KB ? 0 : pos + 1;
     if constexpr (kStrip) {
-      if (++pos == KB && by_buffer) {   // the column tile is done
-        pos = 0;
+      if (pos == first_kb && by_buffer) {   // the column tile is done
         sb_tab += 2 * KB;
         store_age = 0;
 #pragma unroll
@@ -830,7 +830,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int erow, in
 // slot is refilled with stage kb + 3 from 2kb + 2 on, three or more intervals before 2kb + 6; a group's token stage
 // kb is read in its memory and matrix phase of kb and refilled in its memory phase of kb + 1 with stage kb + 2.
 template <int MT, bool FUSE>
-__device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow, int M, int m0, int n0, uint8_t* lds) {
+__device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first_kb, int erow, int M, int m0, int n0, uint8_t* lds) {
   static_assert(MT == 8 || MT == 12, "hand-scheduled K block: 128- and 192-row tiles");
   constexpr int MTW = MT / 2, NTW = 4, BM = MT * 16, GR = MTW * 16;
   constexpr int kTCopies = MTW / 2;                 // token copies per wavefront and K block (8 rows each)
@@ -846,6 +846,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
   // a K that is no multiple of 512 overlaps the one before instead of reaching past the row.
   const int K = g.k, N = g.n, KB = K >> 7, NCH = (KB + 3) >> 2;
   auto chunk_first_kb = [&](int c) { const int f = 4 * c < KB - 4 ? 4 * c : KB - 4; return f > 0 ? f : 0; };
+  auto kb_at = [&](int p) { return p + first_kb < KB ? p + first_kb : p + first_kb - KB; };   // K block of position p (see k_loop)
   const long row_base = erow;
   const int nw = wj * 64, mw = grp * GR;
   const bool wave_active = n0 + nw < N;
@@ -884,8 +885,9 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
     const int grow = trow > a_last ? a_last : trow;
     vs[q] = (uint32_t)grow * (uint32_t)KB * 4 + ((lane & 3) < KB ? (lane & 3) : KB - 1) * 4;
   }
-  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K - kBias;
-  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K - kBias;
+  // (position 0 of the expert's K order; k_loop takes a row off where the order wraps)
+  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K + first_kb * 128 - kBias;
+  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K + first_kb * 128 - kBias;
   const uint8_t* sa_ptr = (const uint8_t*)(g.sa + (row_base + m0) * KB);
   const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + wj * kTCopies * 1024;   // + slot * kTSlot
   const uint32_t w_dst = lds0 + wave * 4096;                                        // + slot * kWSlot
@@ -914,7 +916,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
       int nb = (n0 >> 7) + blk;
       if (nb * 128 >= N) nb = n0 >> 7;
       if constexpr (FUSE) nb = (n0 >> 8) + blk * (N >> 8);
-      const int kbi = kb0 + lane < KB ? kb0 + lane : KB - 1;
+      const int kbi = kb_at(kb0 + lane < KB ? kb0 + lane : KB - 1);
       dma4(g.sb + ((long)e * (N >> 7) + nb) * KB, (uint32_t)kbi * 4, lds0 + kSbBase + (blk * kMaxKB + kb0) * 4);
     }
   }
@@ -922,7 +924,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
     // scale chunks 0 and 1 in the pieces the loop uses: wavefront wj the four 16-row pieces of rows (wj & 1)*64 .. +64
     // of chunk wj >> 1
     const int ch = (wj >> 1) < NCH ? (wj >> 1) : NCH - 1;
-    const uint8_t* src = sa_ptr + (long)chunk_first_kb(ch) * 4;
+    const uint8_t* src = sa_ptr + (long)kb_at(chunk_first_kb(ch)) * 4;
 #pragma unroll
     for (int q = 0; q < 4; q++) dma4(src, vs[q], s_dst + (wj >> 1) * kSaBuf + q * 256);
   }
@@ -970,16 +972,58 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
     if constexpr (kNt) asm volatile(NAME##_BODY_NT : NAME##_OUTS : NAME##_INS : NAME##_CLOBBERS);                 \
     else asm volatile(NAME##_BODY : NAME##_OUTS : NAME##_INS : NAME##_CLOBBERS);                                  \
   } while (0)
-      if constexpr (MT == 12 && FUSE) ESMOE_PP_STMT(ESMOE_PP12F);
-      else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PP12);
-      else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PP8F);
-      else ESMOE_PP_STMT(ESMOE_PP8);
+#define ESMOE_PP_K_BLOCK()                                                                                       \
+  do {                                                                                                           \
+    if constexpr (MT == 12 && FUSE) ESMOE_PP_STMT(ESMOE_PP12F);                                                  \
+    else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PP12);                                                      \
+    else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PP8F);                                                          \
+    else ESMOE_PP_STMT(ESMOE_PP8);                                                                               \
+  } while (0)
+      ESMOE_PP_K_BLOCK();
       // the piece offsets rotate with q; the chunk buffer advances every fourth K block
       { const uint32_t t = vs[0]; vs[0] = vs[1]; vs[1] = vs[2]; vs[2] = vs[3]; vs[3] = t; }
       if (q == 3) sabuf = sabuf == 2 ? 0 : sabuf + 1;
     }
   };
-  if (w_once) k_loop(std::true_type{}); else k_loop(std::false_type{});
+  // The same for a K order that starts at block first_kb (K a multiple of 4096, so every chunk is whole) and wraps; kb counts
+  // its positions.  Iteration kb fetches the weights of position kb + 2, the tokens of position kb + 1 and a piece of the scale
+  // chunk two ahead, so the pointers step back to the row's start at different times; past the last chunk the first ones are
+  // fetched again.  (A loop of its own: the few instructions more between two statements cost tiles of five K blocks 3 %.)
+  auto k_loop_from = [&](auto nt_hint) {
+    constexpr bool kNt = decltype(nt_hint)::value;
+    const int wrap = KB - first_kb;
+    uint32_t sab = 0, sal = sa_rd, sbl = sb_rd, ls = s_dst + 2 * kSaBuf;
+    const uint8_t* sp = sa_ptr + kb_at(8) * 4;
+    const uint8_t* const sp_end = sa_ptr + KB * 4;
+    int kb = 0;
+    do {
+      const bool weights = kb == wrap - 2, tokens = kb == wrap - 1;
+      if (weights) w_ptr -= K;
+      if (tokens) a_ptr -= K;
+      const int end = weights ? wrap - 1 : tokens || kb > wrap ? KB : wrap - 2;
+      do {
+      const uint32_t vsq = vs[0];
+      ESMOE_PP_K_BLOCK();
+      { const uint32_t t = vs[0]; vs[0] = vs[1]; vs[1] = vs[2]; vs[2] = vs[3]; vs[3] = t; }
+      kb++;
+      sal += 4;
+      sbl += 4;
+      ls += 256;
+      if ((kb & 3) == 0) {
+        ls = s_dst + sab;
+        sab = sab == 2 * kSaBuf ? 0 : sab + kSaBuf;
+        sal = sa_rd + sab;
+        sp += 16;
+        if (sp == sp_end) sp = sa_ptr;
+      }
+      } while (kb < end);
+    } while (kb < KB);
+  };
+  if (first_kb == 0) {
+    if (w_once) k_loop(std::true_type{}); else k_loop(std::false_type{});
+  } else {
+    if (w_once) k_loop_from(std::true_type{}); else k_loop_from(std::false_type{});
+  }
   // the copies past the last K block (they fetched it again) must have landed before anything reuses the ring
   wait_vmcnt<0>();
   if (grp == 0) block_barrier();
@@ -996,7 +1040,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int erow,
 // A tile may start in the middle of a 128-row scale tile (full tiles are 192 rows): a lane finds the scale dword of
 // its row from the row's position inside the two tiles that were fetched for its group.
 template <int MT, bool FUSE>
-__device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int erow, int ebso, int M, int m0, int n0, uint8_t* lds) {
+__device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int first_kb, int erow, int ebso, int M, int m0, int n0, uint8_t* lds) {
   static_assert(MT == 8 || MT == 12, "hand-scheduled K block: 128- and 192-row tiles");
   constexpr int MTW = MT / 2, NTW = 4, BM = MT * 16, GR = MTW * 16;
   constexpr int kTCopies = MTW / 2;
@@ -1039,8 +1083,9 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
     }
     vw[i] = (uint32_t)(row + crow) * (uint32_t)K + (swz(blk * 8 + crow, cslot) << 4) + kBias - i * 1024;
   }
-  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K - kBias;
-  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K - kBias;
+  // (position 0 of the expert's K order, see k_loop of gemm_tile_pp)
+  const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K + first_kb * 128 - kBias;
+  const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K + first_kb * 128 - kBias;
   const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + wj * kTCopies * 1024;   // + slot * kTSlot
   const uint32_t w_dst = lds0 + wave * 4096;                                        // + slot * kWSlot
   // scale copies, one per wavefront and K block: wavefront 0 the weight scale tiles (with the weight stage),
@@ -1067,6 +1112,7 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
     vs = 0;
     s_dst = lds0 + kSpare;
   }
+  s_ptr += first_kb * 512;
   // (wave-uniform by construction; said again so that they live in scalar registers)
   s_dst = __builtin_amdgcn_readfirstlane(s_dst);
   s_ptr = (const uint8_t*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)s_ptr >> 32)) << 32) |
@@ -1133,14 +1179,24 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
   uint32_t sfal[MTW];
 #pragma unroll
   for (int mt = 0; mt < MTW; mt++) sfal[mt] = sfa_rd[mt];
+  // (positions, and the places where the pointers step back, as in gemm_tile_pp; the scale tiles go with their operand)
+  const int wrap = first_kb ? KB - first_kb : KB + 8;
   auto k_loop = [&](auto nt_hint) {
     constexpr bool kNt = decltype(nt_hint)::value;
-    for (int kb = 0; kb < KB; kb++) {
+    int kb = 0;
+    do {
+      const bool weights = kb == wrap - 2, tokens = kb == wrap - 1;
+      if (weights) w_ptr -= K;
+      if (tokens) a_ptr -= K;
+      if (s_role == 0 ? weights : tokens) s_ptr -= (long)KB * 512;
+      const int end = weights ? wrap - 1 : kb < wrap - 2 && wrap - 2 < KB ? wrap - 2 : KB;
+      do {
       if constexpr (MT == 12 && FUSE) ESMOE_PP_STMT(ESMOE_PPX12F);
       else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PPX12);
       else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PPX8F);
       else ESMOE_PP_STMT(ESMOE_PPX8);
-    }
+      } while (++kb < end);
+    } while (kb < KB);
   };
   if (w_once) k_loop(std::true_type{}); else k_loop(std::false_type{});
   wait_vmcnt<0>();
@@ -1151,10 +1207,19 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int er
 }
 
 // ---------------------------------------------------------------------------------------------
+// First K block of expert e's K order, in units of kStartUnit (schedule.h, sched_k_start): 16 bytes of its weight scales.
+__device__ __forceinline__ int expert_k_start(const float* sb, const uint8_t* sfb, int e, int n, int k) {
+  if (!sched_spread_k(k)) return 0;
+  const long first = sfb ? (long)e * n * (k >> 5) : (long)e * (n >> 7) * (k >> 7) * 4;
+  const v4i s = *(const v4i*)((sfb ? sfb : (const uint8_t*)sb) + first);
+  return sched_k_start((uint32_t)s[0], (uint32_t)s[1], (uint32_t)s[2], (uint32_t)s[3]);
+}
+
 // Schedule kernel: one workgroup, thread = expert (E <= 1024, as the reference's pre-compute kernel,
 // es_fp8_blockwise_launcher.cuh:53,74).  Ranks the experts by rows (most first), prefix-sums the heavy
 // experts' tile blocks and the light experts' items over that order, and zeroes the hand-out counters.
-__global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ problem_sizes, int num_experts, int n,
+__global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ problem_sizes, const float* __restrict__ sb,
+                                                        const uint8_t* __restrict__ sfb, int num_experts, int n, int k,
                                                         SchedPolicy policy, int* __restrict__ ws) {
   __shared__ int s_m[1024];
   __shared__ int s_blocks[1024];
@@ -1176,7 +1241,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
         pos += (kj < key) || (kj == key && j < e);
       }
     }
-    ws[ws_rec(pos) + kRecExpert] = e;
+    ws[ws_rec(pos) + kRecExpert] = rec_expert_word(e, expert_k_start(sb, sfb, e, n, k));
     ws[ws_rec(pos) + kRecRows] = m;
     s_blocks[pos] = sched_heavy_blocks(m, n, policy);
     s_items[pos] = sched_light_items(m, n, policy);
@@ -1226,7 +1291,7 @@ __device__ __forceinline__ SchedFirst first_tickets(const GemmArgs& g, int hbloc
 // What a workgroup has to know of its first ticket (self_schedule).
 struct FirstRecord {
   int first;   // first light item, or heavy block, of the expert
-  int expert, rows;
+  int expert, rows;   // (the expert's word: rec_expert, rec_first_kb)
   int row, scale_row;   // expert_offsets[expert], blockscale_offsets[expert]
 };
 
@@ -1257,17 +1322,18 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   const int E = g.num_experts, t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const SchedPolicy policy = g.policy;
   int* ws = g.ws;
-  int m = 0, row = 0, scale_row = 0;
+  int m = 0, row = 0, scale_row = 0, word = t;
   if (t < E) {
     m = g.problem_sizes[t * 3];
     row = g.expert_offsets[t];
     if constexpr (MX) scale_row = g.blockscale_offsets[t];
+    word = rec_expert_word(t, expert_k_start(g.sb, MX ? g.sfb : nullptr, t, g.n, g.k));
   }
   s_hist[wave * kHistStride + lane] = 0;   // (a wavefront's LDS accesses stay in order)
   if (lane == 0) s_hist[wave * kHistStride + kLightRows] = 0;
   s_rank[t] = 0;
   // (waited for here: a load that the compiler holds for outstanding puts a wait of its own into the K loops)
-  asm volatile("" : "+v"(row), "+v"(scale_row));
+  asm volatile("" : "+v"(row), "+v"(scale_row), "+v"(word));
   if (m < 0) m = 0;
   const bool heavy = t < E && sched_is_heavy(m, policy), light = t < E && !heavy;
   uint64_t same = __ballot(light);   // light experts of this wavefront with as many rows
@@ -1361,7 +1427,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
     if (items > 0) lshare = __builtin_amdgcn_readfirstlane(sched_light_share(hc, lc, policy));
   }
   // the expert's record, at its schedule position; record E closes the prefix sums
-  if (t < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, t, m} : v4i{blocks, before, t, m};
+  if (t < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
   if (t == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
   hblocks = blocks;
@@ -1373,7 +1439,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   int half = -1;
   const bool first_light = sched_first_is_light(wg, f);
   const int idx = first_light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(wg % kXcds, ticket);
-  if ((first_light ? light : heavy) && idx >= before && idx < before + mine) *s_first = FirstRecord{before, t, m, row, scale_row};
+  if ((first_light ? light : heavy) && idx >= before && idx < before + mine) *s_first = FirstRecord{before, word, m, row, scale_row};
   __syncthreads();
 }
 
@@ -1469,10 +1535,10 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     // (a light ticket past `lsplit` is one half of an item of the narrow tail)
     int half = -1;
     const int idx = light ? sched_light_item_of_ticket(have, lsplit, &half) : sched_ticket_block(xq, have);
-    int rec_first, e, M, erow, ebso = 0;
+    int rec_first, word, M, erow, ebso = 0;
     if (from_lds) {
       rec_first = __builtin_amdgcn_readfirstlane(s_first.first);
-      e = __builtin_amdgcn_readfirstlane(s_first.expert);
+      word = __builtin_amdgcn_readfirstlane(s_first.expert);
       M = __builtin_amdgcn_readfirstlane(s_first.rows);
       erow = __builtin_amdgcn_readfirstlane(s_first.row);
       if constexpr (MX) ebso = __builtin_amdgcn_readfirstlane(s_first.scale_row);
@@ -1495,11 +1561,12 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       // well: a vector load here waits its turn behind the weight streams of the whole chip
       const v4i rec = sload4(ws, ws_rec(lo) * 4);
       rec_first = __builtin_amdgcn_readfirstlane(light ? rec[kRecItem] : rec[kRecBlock]);
-      e = __builtin_amdgcn_readfirstlane(rec[kRecExpert]);
+      word = __builtin_amdgcn_readfirstlane(rec[kRecExpert]);
       M = __builtin_amdgcn_readfirstlane(rec[kRecRows]);
-      erow = sload(g.expert_offsets, e * 4);
-      if constexpr (MX) ebso = sload(g.blockscale_offsets, e * 4);
+      erow = sload(g.expert_offsets, rec_expert(word) * 4);
+      if constexpr (MX) ebso = sload(g.blockscale_offsets, rec_expert(word) * 4);
     }
+    const int e = rec_expert(word), first_kb = rec_first_kb(word);
     const int local = idx - rec_first;
     TileCoord t;
     int cols = 1;
@@ -1531,21 +1598,21 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     // ones, also as 128-column halves.  The host refuses a policy that asks for any other height (launch_gemm), so
     // every ticket finds its tile function here.
     if (t.mt == 12) {
-      if constexpr (MX) gemm_tile_pp_mx<12, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, lds);
-      else gemm_tile_pp<12, FUSE>(g, e, erow, M, t.m0, t.n0, lds);
+      if constexpr (MX) gemm_tile_pp_mx<12, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
+      else gemm_tile_pp<12, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
     } else if (t.mt == 8) {
-      if constexpr (MX) gemm_tile_pp_mx<8, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, lds);
-      else gemm_tile_pp<8, FUSE>(g, e, erow, M, t.m0, t.n0, lds);
+      if constexpr (MX) gemm_tile_pp_mx<8, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
+      else gemm_tile_pp<8, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
     } else if (!FUSE && t.nt == 2) {
       if constexpr (!FUSE) {
-        if (t.mt == 1) gemm_tile<1, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, 1, lds);
-        else if (t.mt == 2) gemm_tile<2, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, 1, lds);
-        else gemm_tile<4, MX, false, 128>(g, e, erow, ebso, M, t.m0, t.n0, 1, lds);
+        if (t.mt == 1) gemm_tile<1, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
+        else if (t.mt == 2) gemm_tile<2, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
+        else gemm_tile<4, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
       }
     } else {
-      if (t.mt == 1) gemm_tile<1, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, cols, lds);
-      else if (t.mt == 2) gemm_tile<2, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, cols, lds);
-      else gemm_tile<4, MX, FUSE>(g, e, erow, ebso, M, t.m0, t.n0, cols, lds);
+      if (t.mt == 1) gemm_tile<1, MX, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, cols, lds);
+      else if (t.mt == 2) gemm_tile<2, MX, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, cols, lds);
+      else gemm_tile<4, MX, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, cols, lds);
     }
   }
   // The last workgroup to leave zeroes the hand-out counters (nobody draws any more: every workgroup counts itself
@@ -1599,8 +1666,8 @@ extern "C" int esmoe_launch_grouped_gemm(const esmoe::GemmArgs* args, int mx, in
   using namespace esmoe;
   if (args->self_schedule && args->num_experts > kSelfScheduleMaxExperts) return (int)hipErrorInvalidValue;
   if (!args->self_schedule) {
-    hipLaunchKernelGGL(schedule_kernel, dim3(1), dim3((args->num_experts + 63) & ~63), 0, stream, args->problem_sizes, args->num_experts,
-                       args->n, args->policy, args->ws);
+    hipLaunchKernelGGL(schedule_kernel, dim3(1), dim3((args->num_experts + 63) & ~63), 0, stream, args->problem_sizes, args->sb, args->sfb,
+                       args->num_experts, args->n, args->k, args->policy, args->ws);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return (int)err;
   }

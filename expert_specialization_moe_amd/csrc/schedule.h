@@ -291,6 +291,23 @@ ESMOE_HD int sched_undrawn_queues(int hblocks, int ltotal, const SchedFirst& f) 
   return (f.light_base >= ltotal ? 1 << kXcds : 0) | (((1 << kXcds) - 1) & ~((1 << drawn) - 1));
 }
 
+// First K block of an expert's K order.  With K a multiple of 4096 all rows of a weight panel share address bits 7-11: a K block of a
+// tile goes through one L2 channel of sixteen, and tiles that all begin with block 0 stay in step and queue for one channel
+// after the other (128 experts x 8 rows: 768 x 4096 88.3 us in step, 68.6 apart; 4096 x 4096 337 and 325; the projection of a 64-token
+// expert MLP with hidden size 4096 19 us less).  So every expert begins at a place of its own, a multiple of four K blocks in the first
+// 32, and wraps; large launches, bound by the matrix cores, take as long either way.  The place goes by the expert's weight scales, so that its bytes depend on its rows and weights
+// alone, not on where or among which others it is listed: a hash of the differences between its first scales (four fp32 block
+// scales, or sixteen E8M0 bytes as four words), which a common power of two in all scales does not change.  Equal scales: block 0.
+ESMOE_HD bool sched_spread_k(int k) { return (k & 4095) == 0; }
+constexpr int kStartUnit = 4;
+ESMOE_HD int sched_k_start(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3) {   // in units of kStartUnit K blocks
+  uint32_t h = (s1 - s0) * 0x9e3779b1u;
+  h = ((h << 13 | h >> 19) ^ (s2 - s0)) * 0x85ebca6bu;
+  h = ((h << 13 | h >> 19) ^ (s3 - s0)) * 0xc2b2ae35u;
+  h = (h ^ h >> 16) * 0x7feb352du;
+  return (int)(h >> 29);
+}
+
 // Workspace layout (int32 words).
 constexpr int kWsLightCounter = 32;  // next light ticket to hand out (every counter has a 128-byte line of its own)
 constexpr int kWsLightTotal = 1;     // number of light tickets: whole items, then two per item of the narrow tail
@@ -304,6 +321,10 @@ constexpr int kWsHeader = 64 + 32 * kXcds;   // then one record of kRecWords per
 // Record E closes the prefix sums: {heavy blocks, light items, -1, 0}.
 constexpr int kRecWords = 4;
 constexpr int kRecBlock = 0, kRecItem = 1, kRecExpert = 2, kRecRows = 3;
+// The expert's word also holds where its K order starts (sched_k_start).
+ESMOE_HD int rec_expert_word(int expert, int k_start) { return expert | k_start << 16; }
+ESMOE_HD int rec_expert(int word) { return word & 0xffff; }
+ESMOE_HD int rec_first_kb(int word) { return (word >> 16) * kStartUnit; }
 ESMOE_HD int ws_xcd_counter(int xcd) { return kWsXcdCounter + 32 * xcd; }
 ESMOE_HD int ws_rec(int pos) { return kWsHeader + pos * kRecWords; }
 ESMOE_HD int ws_words(int num_experts) { return kWsHeader + (num_experts + 1) * kRecWords; }
