@@ -560,7 +560,7 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
     ws_host[esmoe::ws_rec(pos) + esmoe::kRecRows] = rows_of(e);
   }
   int blocks = 0, items = 0;
-  long heavy_cost = 0, light_cost = 0;
+  float heavy_cost = 0, light_cost = 0;
   for (int pos = 0; pos < num_experts; pos++) {
     const int m = ws_host[esmoe::ws_rec(pos) + esmoe::kRecRows];
     ws_host[esmoe::ws_rec(pos) + esmoe::kRecBlock] = blocks;

@@ -122,6 +122,11 @@ __device__ __forceinline__ int sload(const int* base, int byte_offset) {
   asm volatile("s_load_dword %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(base), "s"(__builtin_amdgcn_readfirstlane(byte_offset)) : "memory");
   return __builtin_amdgcn_readfirstlane(v);
 }
+__device__ __forceinline__ void sload3(const int* base, int o0, int o1, int o2, int& v0, int& v1, int& v2) {
+  asm volatile("s_load_dword %0, %3, %4\n\ts_load_dword %1, %3, %5\n\ts_load_dword %2, %3, %6\n\ts_waitcnt lgkmcnt(0)"
+               : "=&s"(v0), "=&s"(v1), "=&s"(v2) : "s"(base), "s"(__builtin_amdgcn_readfirstlane(o0)),
+                 "s"(__builtin_amdgcn_readfirstlane(o1)), "s"(__builtin_amdgcn_readfirstlane(o2)) : "memory");
+}
 __device__ __forceinline__ v4i sload4(const int* base, int byte_offset) {   // 16 bytes, 16-byte aligned
   v4i v;
   asm volatile("s_load_dwordx4 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(base), "s"(__builtin_amdgcn_readfirstlane(byte_offset)) : "memory");
@@ -1224,7 +1229,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   __shared__ int s_m[1024];
   __shared__ int s_blocks[1024];
   __shared__ int s_items[1024];
-  __shared__ long s_cost[1024][2];   // heavy, light
+  __shared__ float s_cost[1024][2];   // heavy, light
   const int e = threadIdx.x;
   int m = 0;
   if (e < num_experts) m = problem_sizes[e * 3];
@@ -1271,12 +1276,12 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
       ws[kWsLightTotal] = split + 2 * (items - split);
       ws[kWsLightCounter] = 0;
       ws[kWsExitCounter] = 0;
-      long heavy_cost = 0, light_cost = 0;
+      float heavy_cost = 0, light_cost = 0;
       for (int j = 0; j < num_experts; j++) {
         heavy_cost += s_cost[j][0];
         light_cost += s_cost[j][1];
       }
-      ws[kWsLightShare] = sched_light_share((float)heavy_cost, (float)light_cost, policy);
+      ws[kWsLightShare] = sched_light_share(heavy_cost, light_cost, policy);
     }
     if (pos < kXcds) ws[ws_xcd_counter(pos)] = 0;
   }
@@ -1307,7 +1312,9 @@ struct FirstRecord {
 // those of their row number with a ballot per bit.  Only heavy experts are compared with each other, packed into a list (all 512 threads
 // share the comparisons), and only they need a prefix sum.  Comparing all experts took 0.5 / 1.1 / 3.7 us at 8 / 32 / 256 experts and
 // the cost totals of a launch with both kinds 0.8 us.  Whole calls, first tickets without a draw (schedule.h, sched_first_tickets): 8 experts
-// x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us.
+// x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting
+// instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us; half as many divisions and a four-way search of the records:
+// 75.2 -> 74.7 (with both kinds of experts), an expert MLP of 1003 tokens in MXFP8 377.5 -> 376.1.
 template <bool MX, bool FUSE>
 __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, FirstRecord* s_first, int& hblocks, int& ltotal, int& lsplit,
                                               SchedFirst& f) {
@@ -1378,9 +1385,9 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
     float heavy_cost = 0.f, light_cost = 0.f;
     if (heavy) {
       hb = sched_heavy_blocks(m, g.n, policy);
-      heavy_cost = (float)sched_heavy_cost(m, g.n, policy);
+      heavy_cost = sched_heavy_cost(m, g.n, policy);
     } else if (light) {
-      light_cost = (float)sched_light_cost(m, g.n, policy);
+      light_cost = sched_light_cost(m, g.n, policy);
     }
     __syncthreads();
     // slice `part` of the list, in fours; an expert comes in front of another of the same key if its index is lower
@@ -1549,13 +1556,17 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
         __syncthreads();
         records_pending = false;
       }
-      // schedule position of idx: the last one whose first block (item) is <= idx, found by bisection over the prefix
-      // sums with scalar loads.  The records are only read from here on, so they stay in
-      // the scalar cache, where a step costs a fraction of what a trip to L2 costs while the chip streams weights.
+      // schedule position of idx: the last one whose first block (item) is <= idx, found by halving the prefix sums twice a
+      // step, with scalar loads.  The records are only read from here on, so they stay in the scalar cache, where a step costs
+      // a fraction of what a trip to L2 costs while the chip streams weights, and three loads as much as one.
       int lo = 0, hi = g.num_experts;
       while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (sload(ws, (ws_rec(mid) + kind) * 4) <= idx) lo = mid; else hi = mid;
+        const int d = (hi - lo + 3) >> 2;
+        auto at = [&](int pos) { return (ws_rec(pos < g.num_experts ? pos : g.num_experts) + kind) * 4; };
+        int v0, v1, v2;
+        sload3(ws, at(lo + d), at(lo + 2 * d), at(lo + 3 * d), v0, v1, v2);   // (past `hi`: more than idx as well)
+        lo += ((v0 <= idx ? 1 : 0) + (v1 <= idx ? 1 : 0) + (v2 <= idx ? 1 : 0)) * d;
+        if (hi > lo + d) hi = lo + d;
       }
       // the whole record in one load, then the expert's first row (and first scale row) through the scalar cache as
       // well: a vector load here waits its turn behind the weight streams of the whole chip

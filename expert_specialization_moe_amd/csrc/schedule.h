@@ -40,18 +40,17 @@ struct TileCoord {
 };
 
 // a / b for a >= 0, b > 0.  On the device an integer division by a variable is a chain of some forty instructions, and the
-// schedule of an expert with more than 64 rows takes seven of them in front of the first tile, as does every heavy ticket; for
-// a < 2^22 the float quotient is off by less than one, and the remainder says which way.
+// schedule of an expert with more than 64 rows takes four of them in front of the first tile, as does every heavy ticket.  The float
+// quotient of a number below 2^31 is off by less than 2^9, that of what it leaves by less than one, and the last remainder says which way.
 ESMOE_HD int sched_div(int a, int b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (a < (1 << 22)) {
-    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
-    const int r = a - q * b;
-    q += r >= b ? 1 : 0;
-    return r < 0 ? q - 1 : q;
-  }
-#endif
+  const float inverse = __builtin_amdgcn_rcpf((float)b);
+  const int q = (int)((float)a * inverse), left = (int)((uint32_t)a - (uint32_t)q * (uint32_t)b);
+  const int more = (int)((float)left * inverse), r = left - more * b;
+  return q + more + (r >= b ? 1 : 0) - (r < 0 ? 1 : 0);
+#else
   return a / b;
+#endif
 }
 
 // The tile heights the kernels are compiled for.
@@ -113,20 +112,27 @@ ESMOE_HD int sched_mtiles(int m, const SchedPolicy& p) {
 // Block shape for an expert with mtl x ntl tiles: at most kBlkM tiles high and kBlkTiles tiles in all, with
 // the rows and the columns of the grid split evenly over the blocks (21 x 16 tiles -> blocks of 7 x 4;
 // 6 x 16 -> 6 x 4; 1 x 16 -> 1 x 16).  Near-square blocks (in bytes) fetch the least per tile.
-ESMOE_HD void sched_block_shape(int mtl, int ntl, int* bm, int* bn) {
-  const int rb = (mtl + kBlkM - 1) / kBlkM;
-  *bm = sched_div(mtl + rb - 1, rb);
-  const int w = sched_div(kBlkTiles, *bm);
-  const int cb = sched_div(ntl + w - 1, w);
-  *bn = sched_div(ntl + cb - 1, cb);
+// rb = ceil(mtl / 8) rows of blocks are bm = ceil(mtl / rb) <= 8 tiles high, and since mtl > 8 (rb - 1) >= bm (rb - 1) it takes all
+// rb of them; the same for the columns.
+struct SchedBlocks {
+  int bm, rb;      // tiles of a block's column, rows of blocks
+  int width, cb;   // most tiles of a block's row, columns of blocks (a block's row: sched_block_cols)
+};
+ESMOE_HD SchedBlocks sched_block_shape(int mtl, int ntl) {
+  static_assert(kBlkM == 8 && kBlkTiles == 32, "the table of widths");
+  SchedBlocks b;
+  b.rb = (mtl + kBlkM - 1) / kBlkM;
+  b.bm = sched_div(mtl + b.rb - 1, b.rb);
+  b.width = (int)(0x04040506080a1020ull >> ((b.bm - 1) * 8)) & 0xff;   // kBlkTiles / bm for bm = 1 .. 8
+  b.cb = sched_div(ntl + b.width - 1, b.width);
+  return b;
 }
+ESMOE_HD int sched_block_cols(const SchedBlocks& b, int ntl) { return sched_div(ntl + b.cb - 1, b.cb); }
 
 ESMOE_HD int sched_heavy_blocks(int m, int n, const SchedPolicy& p) {
   if (!sched_is_heavy(m, p)) return 0;
-  const int mtl = sched_mtiles(m, p), ntl = sched_ntiles(n, 4);
-  int bm, bn;
-  sched_block_shape(mtl, ntl, &bm, &bn);
-  return sched_div(mtl + bm - 1, bm) * sched_div(ntl + bn - 1, bn);
+  const SchedBlocks b = sched_block_shape(sched_mtiles(m, p), sched_ntiles(n, 4));
+  return b.rb * b.cb;
 }
 
 ESMOE_HD int sched_light_items(int m, int n, const SchedPolicy& p) {
@@ -136,12 +142,11 @@ ESMOE_HD int sched_light_items(int m, int n, const SchedPolicy& p) {
 // Tile `idx` (0..31) of block `lb` of a heavy expert; false if it falls outside the expert's grid.
 ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolicy& p, TileCoord* t) {
   const int mtl = sched_mtiles(m, p), ntl = sched_ntiles(n, 4);
-  int bm, bn;
-  sched_block_shape(mtl, ntl, &bm, &bn);
-  const int nbc = sched_div(ntl + bn - 1, bn);
+  const SchedBlocks b = sched_block_shape(mtl, ntl);
+  const int bm = b.bm, bn = sched_block_cols(b, ntl);
   if (idx >= bm * bn) return false;
-  const int rb = sched_div(lb, nbc), r = sched_div(idx, bn);
-  const int mi = rb * bm + r, ni = (lb - rb * nbc) * bn + idx - r * bn;
+  const int rb = sched_div(lb, b.cb), r = sched_div(idx, bn);
+  const int mi = rb * bm + r, ni = (lb - rb * b.cb) * bn + idx - r * bn;
   if (mi >= mtl || ni >= ntl) return false;
   const int big = p.force_mt ? p.force_mt : p.big_mt;
   const int m0 = mi * big * 16;
@@ -232,15 +237,14 @@ ESMOE_HD TileCoord sched_decode_light(int item, int m, const SchedPolicy& p, int
 // Cost estimates in units of one tile row streamed through a CU: a heavy tile costs its padded rows; a light
 // item is bound by streaming its 256 weight rows (and its few token rows) from HBM at one CU's rate, which
 // takes as long as about 75 rows of a heavy tile.
-ESMOE_HD long sched_heavy_cost(int m, int n, const SchedPolicy& p) {
+ESMOE_HD float sched_heavy_cost(int m, int n, const SchedPolicy& p) {
   if (!sched_is_heavy(m, p)) return 0;
-  const int big = (p.force_mt ? p.force_mt : p.big_mt) * 16;
-  const int full = sched_div(m, big), rem = m - full * big;
-  const int rows = full * big + (rem ? (p.force_mt ? big : sched_cover_mt(rem, p.big_mt) * 16) : 0);
-  return (long)(rows + 16 * sched_mtiles(m, p)) * sched_ntiles(n, 4);
+  const int big = (p.force_mt ? p.force_mt : p.big_mt) * 16, tiles = sched_mtiles(m, p), above = (tiles - 1) * big;
+  const int rows = above + (p.force_mt ? big : sched_cover_mt(m - above, p.big_mt) * 16);
+  return (float)(rows + 16 * tiles) * (float)sched_ntiles(n, 4);
 }
-ESMOE_HD long sched_light_cost(int m, int n, const SchedPolicy& p) {
-  return (long)sched_light_items(m, n, p) * (75 + m / 3);
+ESMOE_HD float sched_light_cost(int m, int n, const SchedPolicy& p) {
+  return (float)sched_light_items(m, n, p) * (float)(75 + m / 3);
 }
 // Workgroups of every 32 that start on the light items.  (Floats: it is an estimate, and a 64-bit division and sum of both costs
 // stood 0.8 us in front of the first tile.)
