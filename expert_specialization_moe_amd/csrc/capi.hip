@@ -609,7 +609,8 @@ int esmoe_host_decode_heavy(const int32_t* problem_sizes_host, const int32_t* ws
   if (pos < 0) return fail(ESMOE_ERR_INVALID_ARGUMENT, "workspace does not hold a schedule");
   const int32_t* rec = ws_host + esmoe::ws_rec(pos);
   esmoe::TileCoord t;
-  if (!esmoe::sched_decode_heavy(blk - rec[esmoe::kRecBlock], ticket % esmoe::kBlkTiles, rec[esmoe::kRecRows], n, p, &t))
+  bool past = false;
+  if (!esmoe::sched_decode_heavy(blk - rec[esmoe::kRecBlock], ticket % esmoe::kBlkTiles, rec[esmoe::kRecRows], n, p, &t, &past))
     return 1;   // ticket outside the expert's tile grid: skipped
   fill_out5(out5, rec[esmoe::kRecExpert], t);
   return 0;

@@ -139,15 +139,18 @@ ESMOE_HD int sched_light_items(int m, int n, const SchedPolicy& p) {
   return (m > 0 && !sched_is_heavy(m, p)) ? sched_ntiles(n, 4) : 0;
 }
 
-// Tile `idx` (0..31) of block `lb` of a heavy expert; false if it falls outside the expert's grid.
-ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolicy& p, TileCoord* t) {
+// Tile `idx` (0..31) of block `lb` of a heavy expert; false if it falls outside the expert's grid (`past`: and so do the block's
+// tickets behind it).
+ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolicy& p, TileCoord* t, bool* past) {
   const int mtl = sched_mtiles(m, p), ntl = sched_ntiles(n, 4);
   const SchedBlocks b = sched_block_shape(mtl, ntl);
   const int bm = b.bm, bn = sched_block_cols(b, ntl);
-  if (idx >= bm * bn) return false;
-  const int rb = sched_div(lb, b.cb), r = sched_div(idx, bn);
+  const int rb = sched_div(lb, b.cb), rows = mtl - rb * bm < bm ? mtl - rb * bm : bm;   // (the last row of blocks may be lower)
+  *past = idx >= rows * bn;
+  if (*past) return false;
+  const int r = sched_div(idx, bn);
   const int mi = rb * bm + r, ni = (lb - rb * b.cb) * bn + idx - r * bn;
-  if (mi >= mtl || ni >= ntl) return false;
+  if (ni >= ntl) return false;
   const int big = p.force_mt ? p.force_mt : p.big_mt;
   const int m0 = mi * big * 16;
   t->mt = p.force_mt ? p.force_mt : (m - m0 >= big * 16 ? big : sched_cover_mt(m - m0, big));
