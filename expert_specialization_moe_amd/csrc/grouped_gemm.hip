@@ -1282,6 +1282,13 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
         light_cost += s_cost[j][1];
       }
       ws[kWsLightShare] = sched_light_share(heavy_cost, light_cost, policy);
+      int block_tiles = 0;
+      for (int j = 0; j < num_experts; j++)
+        if (sched_is_heavy(s_m[j], policy)) {
+          const int tiles = sched_block_tiles(s_m[j], n, policy);
+          block_tiles = tiles > block_tiles ? tiles : block_tiles;
+        }
+      ws[kWsBlockLog] = sched_log2_ceil(block_tiles);
     }
     if (pos < kXcds) ws[ws_xcd_counter(pos)] = 0;
   }
@@ -1289,8 +1296,8 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
 }
 
 template <bool FUSE>
-__device__ __forceinline__ SchedFirst first_tickets(const GemmArgs& g, int hblocks, int ltotal, int lshare) {
-  return sched_first_tickets((int)gridDim.x, hblocks, ltotal, lshare, sched_light_draw(ltotal, 0, (int)gridDim.x, g.k >> 7, !FUSE));
+__device__ __forceinline__ SchedFirst first_tickets(const GemmArgs& g, int hblocks, int block_log, int ltotal, int lshare) {
+  return sched_first_tickets((int)gridDim.x, hblocks, block_log, ltotal, lshare, sched_light_draw(ltotal, 0, (int)gridDim.x, g.k >> 7, !FUSE));
 }
 
 // What a workgroup has to know of its first ticket (self_schedule).
@@ -1322,7 +1329,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   constexpr int kLightRows = 64, kHistStride = kLightRows + 4;
   int* s_hist = (int*)lds;                              // [kWaves][kHistStride]: experts of a wavefront by rows (0 .. 64)
   int* s_heavy = s_hist + kWaves * kHistStride;         // [kWaves]: heavy experts of a wavefront
-  v4f* s_sums = (v4f*)(s_heavy + kWaves);               // [kWaves]: blocks, heavy cost, light cost
+  v4f* s_sums = (v4f*)(s_heavy + kWaves);               // [kWaves]: blocks, heavy cost, light cost, block_log
   int* s_key = (int*)(s_sums + kWaves);                 // heavy experts' keys, in index order
   int* s_rank = s_key + kThreads;                       // their ranks
   int* s_blocks = s_rank + kThreads;                    // by rank: blocks of the expert, then blocks in front inside the wavefront
@@ -1376,15 +1383,16 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
     before = (rank < num_light ? rank : num_light) * ntl;
     mine = m > 0 ? ntl : 0;
   }
-  int blocks = 0, lshare = 0;
+  int blocks = 0, block_log = 0, lshare = 0;   // block_log: of the most tiles of a block, rounded up
   if (num_heavy > 0) {
     const int h = heavy_before + __builtin_amdgcn_mbcnt_hi((uint32_t)(heavies >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)heavies, 0));
     if (heavy) s_key[h] = sched_order_key(m, policy);
     if (t >= num_heavy && t < ((num_heavy + 3) & ~3)) s_key[t] = 0x7fffffff;
-    int hb = 0;
+    int hb = 0, tiles = 0;
     float heavy_cost = 0.f, light_cost = 0.f;
     if (heavy) {
       hb = sched_heavy_blocks(m, g.n, policy);
+      tiles = sched_block_tiles(m, g.n, policy);
       heavy_cost = sched_heavy_cost(m, g.n, policy);
     } else if (light) {
       light_cost = sched_light_cost(m, g.n, policy);
@@ -1415,7 +1423,9 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
     const int sb = wave_inclusive_sum(b);
     heavy_cost = wave_sum_last(heavy_cost);
     light_cost = wave_sum_last(light_cost);
-    if (lane == 63) s_sums[wave] = v4f{__builtin_bit_cast(float, sb), heavy_cost, light_cost, 0.f};
+#pragma unroll
+    for (int i = 0; i < kBlkLog; i++) block_log += __ballot(tiles > 1 << i) != 0;
+    if (lane == 63) s_sums[wave] = v4f{__builtin_bit_cast(float, sb), heavy_cost, light_cost, __builtin_bit_cast(float, block_log)};
     s_blocks[t] = sb - b;
     __syncthreads();
     float hc = 0.f, lc = 0.f;
@@ -1426,10 +1436,14 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
       const int wb = __builtin_bit_cast(int, v[0]);
       blocks += wb;
       if (heavy && w < pos >> 6) before += wb;
+      const float packed = v[3];   // (the cast of a vector's element itself reads element 0)
+      const int log = __builtin_bit_cast(int, packed);
+      block_log = log > block_log ? log : block_log;
       hc += v[1];
       lc += v[2];
     }
     blocks = __builtin_amdgcn_readfirstlane(blocks);
+    block_log = __builtin_amdgcn_readfirstlane(block_log);
     // how many workgroups start on which kind, where a launch has both
     if (items > 0) lshare = __builtin_amdgcn_readfirstlane(sched_light_share(hc, lc, policy));
   }
@@ -1441,7 +1455,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   lsplit = sched_light_split(items, policy);
   ltotal = lsplit + 2 * (items - lsplit);
   // the thread of the expert that the first ticket belongs to says so
-  f = first_tickets<FUSE>(g, hblocks, ltotal, lshare);
+  f = first_tickets<FUSE>(g, hblocks, block_log, ltotal, lshare);
   const int wg = (int)blockIdx.x, ticket = sched_first_ticket(wg, f);
   int half = -1;
   const bool first_light = sched_first_is_light(wg, f);
@@ -1467,7 +1481,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     hblocks = ws[kWsHeavyBlocks];
     ltotal = ws[kWsLightTotal];
     lsplit = ws[kWsLightSplit];
-    first = first_tickets<FUSE>(args, hblocks, ltotal, ws[kWsLightShare]);
+    first = first_tickets<FUSE>(args, hblocks, ws[kWsBlockLog], ltotal, ws[kWsLightShare]);
   }
   // Workgroup i runs on XCD i % 8 (HW_REG_XCC_ID = 20, bits [3:0], says so directly).  Of every 32 workgroups
   // of an XCD the last `light_share` start on the light items, the others on the heavy tickets; either kind
@@ -1517,7 +1531,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       const int total = light ? ltotal : sched_queue_tickets(xq, hblocks);
       if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
       __syncthreads();
-      const int ticket = (light ? first.light_base : first.heavy_ranks) + __builtin_amdgcn_readfirstlane(s_item);
+      const int ticket = (light ? first.light_base : first.heavy_base) + __builtin_amdgcn_readfirstlane(s_item);
       if (ticket >= total) {   // this queue is exhausted: see which others are
         dead |= 1 << (light ? 8 : xq);
         __syncthreads();                        // s_item and s_counters are rewritten next
@@ -1529,7 +1543,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
         __syncthreads();
 #pragma unroll
         for (int x = 0; x < kXcds; x++) {
-          if (first.heavy_ranks + __builtin_amdgcn_readfirstlane(s_counters[x]) >= sched_queue_tickets(x, hblocks)) dead |= 1 << x;
+          if (first.heavy_base + __builtin_amdgcn_readfirstlane(s_counters[x]) >= sched_queue_tickets(x, hblocks)) dead |= 1 << x;
         }
         if (first.light_base + __builtin_amdgcn_readfirstlane(s_counters[kXcds]) >= ltotal) dead |= 256;
         continue;
@@ -1598,7 +1612,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       // one by one (a block of 6 x 4 tiles has eight of them, one of 1 x 5 twenty-seven, and each costs a draw and a look-up, 2 to
       // 3 us): 31 experts x 81 rows, 1280 x 768 24.1 -> 22.0 us, 45 experts, 3062 rows, 1024 x 2304 37.4 -> 35.3, MXFP8 MLP of 819
       // tokens, 64 experts 196.7 -> 187; 131072 rows, 3072 x 4096 1643 -> 1635.
-      const int next = (have + kBlkTiles - 1) / kBlkTiles * kBlkTiles - first.heavy_ranks;   // (`have` is one on)
+      const int next = (have + kBlkTiles - 1) / kBlkTiles * kBlkTiles - first.heavy_base;   // (`have` is one on)
       if (past && next > 0 && threadIdx.x == 0) atomicMax(&ws[ws_xcd_counter(xq)], next);
       __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
       continue;

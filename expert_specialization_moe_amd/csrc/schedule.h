@@ -87,7 +87,7 @@ ESMOE_HD int sched_ntiles(int n, int nt) { return (n + nt * 64 - 1) / (nt * 64);
 // estimates below) starts on the light items while the rest start on the heavy tickets, and each
 // side moves on to the other kind when its own runs out.
 constexpr int kBlkM = 8;
-constexpr int kBlkTiles = 32;
+constexpr int kBlkLog = 5, kBlkTiles = 1 << kBlkLog;
 constexpr int kXcds = 8;
 
 ESMOE_HD bool sched_is_heavy(int m, const SchedPolicy& p) { return p.force_mt ? m > 0 : m > 64; }
@@ -133,6 +133,13 @@ ESMOE_HD int sched_heavy_blocks(int m, int n, const SchedPolicy& p) {
   if (!sched_is_heavy(m, p)) return 0;
   const SchedBlocks b = sched_block_shape(sched_mtiles(m, p), sched_ntiles(n, 4));
   return b.rb * b.cb;
+}
+
+// No block of a heavy expert has more tiles.  (Exact with one column of blocks; with several a block has at least half as many.)
+ESMOE_HD int sched_block_tiles(int m, int n, const SchedPolicy& p) {
+  const int ntl = sched_ntiles(n, 4);
+  const SchedBlocks b = sched_block_shape(sched_mtiles(m, p), ntl);
+  return b.bm * (ntl < b.width ? ntl : b.width);
 }
 
 ESMOE_HD int sched_light_items(int m, int n, const SchedPolicy& p) {
@@ -266,19 +273,34 @@ ESMOE_HD int sched_queue_tickets(int xcd, int hblocks) { return xcd < hblocks ? 
 // First tickets: a workgroup's first ticket goes by its index, and the counters hand out what lies behind these.  Atomic adds to
 // one address are served one every 12 ns, so 256 workgroups that all begin with a draw wait 3 us for the last of them, and as
 // long again to count themselves out; a launch whose tickets are all first ones needs neither.
-// `heavy_ranks`: the workgroups 8 r + x with r below it start on queue x with ticket r, the others on the light tickets, `light_draw`
-// neighbouring ones each.
+// `heavy_ranks`: the workgroups 8 r + x with r below it start on queue x, the others on the light tickets, `light_draw` neighbouring
+// ones each.  Where no block of the launch has more than 16 tiles (`block_log`: sched_log2_ceil of the most), a queue's first workgroups
+// take the tiles of its first `blocks` blocks, a power of two of tickets of each, and nobody draws the rest of those blocks' tickets,
+// which are no tiles; otherwise they take the tickets of its first block.  When the later blocks had to be drawn a queue's 32
+// workgroups stood in line for them, and many found no tile: 14 experts, 1717 rows, 2944 x 1536 27.3 -> 23.6 us, 10 experts,
+// 1602 rows, 768 x 3072 44.7 -> 40.1, 18 experts, 9341 rows, 768 x 4864 49.7 -> 46.9; launches of larger blocks pay some 0.1 us
+// for the look.
 struct SchedFirst {
   int heavy_ranks;
+  int blocks, share_log;   // a first workgroup r of a queue: ticket r % 2^share_log of block r >> share_log, if below `blocks`
+  int heavy_base;          // first ticket of a queue that is drawn from its counter
   int light_draw;
-  int light_base;   // first light ticket that is drawn from the counter (a queue's: heavy_ranks)
+  int light_base;          // first light ticket that is
 };
-ESMOE_HD SchedFirst sched_first_tickets(int workgroups, int hblocks, int ltotal, int light_share, int light_draw) {
+ESMOE_HD SchedFirst sched_first_tickets(int workgroups, int hblocks, int block_log, int ltotal, int light_share, int light_draw) {
   SchedFirst f;
   const int per_xcd = workgroups / kXcds;
   if (hblocks == 0) f.heavy_ranks = 0;
   else if (ltotal == 0) f.heavy_ranks = per_xcd;   // (the workgroups past a multiple of eight begin with a draw)
   else f.heavy_ranks = ((kBlkTiles - light_share) * per_xcd + kBlkTiles - 1) / kBlkTiles;
+  f.share_log = block_log;
+  f.blocks = f.heavy_ranks >> f.share_log;
+  f.heavy_base = f.blocks * kBlkTiles;
+  if (block_log >= kBlkLog || f.blocks == 0) {
+    f.share_log = 31;   // one block, as many tickets of it as there are workgroups
+    f.blocks = 1;
+    f.heavy_base = f.heavy_ranks;
+  }
   f.light_draw = light_draw;
   const int light_first = workgroups - f.heavy_ranks * kXcds;
   f.light_base = light_first > 0 ? light_first * light_draw : 0;
@@ -287,13 +309,15 @@ ESMOE_HD SchedFirst sched_first_tickets(int workgroups, int hblocks, int ltotal,
 ESMOE_HD bool sched_first_is_light(int workgroup, const SchedFirst& f) { return workgroup >= f.heavy_ranks * kXcds; }
 // First ticket of `workgroup`, of the light ones or of queue workgroup % 8; may lie past the last ticket there is.
 ESMOE_HD int sched_first_ticket(int workgroup, const SchedFirst& f) {
-  return sched_first_is_light(workgroup, f) ? (workgroup - f.heavy_ranks * kXcds) * f.light_draw : workgroup / kXcds;
+  if (sched_first_is_light(workgroup, f)) return (workgroup - f.heavy_ranks * kXcds) * f.light_draw;
+  const int r = workgroup / kXcds, block = r >> f.share_log;
+  return block < f.blocks ? block * kBlkTiles + (r - (block << f.share_log)) : 0x7fffffff - kBlkTiles;
 }
 // Queues that hold nothing but first tickets: bits 0-7 the XCDs' queues, bit 8 the light tickets (all nine: no counter is used).
 constexpr int kAllQueues = (1 << (kXcds + 1)) - 1;
 ESMOE_HD int sched_undrawn_queues(int hblocks, int ltotal, const SchedFirst& f) {
   // a queue of b blocks has 32 b tickets: the queues with no more than `rounds` blocks, and they come last
-  const int rounds = f.heavy_ranks / kBlkTiles, more = hblocks - rounds * kXcds;   // blocks past that many rounds of all queues
+  const int rounds = f.heavy_base / kBlkTiles, more = hblocks - rounds * kXcds;   // blocks past that many rounds of all queues
   const int drawn = more <= 0 ? 0 : more < kXcds ? more : kXcds;
   return (f.light_base >= ltotal ? 1 << kXcds : 0) | (((1 << kXcds) - 1) & ~((1 << drawn) - 1));
 }
@@ -321,6 +345,7 @@ constexpr int kWsLightTotal = 1;     // number of light tickets: whole items, th
 constexpr int kWsHeavyBlocks = 2;    // number of heavy blocks
 constexpr int kWsLightShare = 3;     // workgroups of every 32 that start on the light items
 constexpr int kWsLightSplit = 4;     // first light ticket that is a half item (sched_light_split)
+constexpr int kWsBlockLog = 5;       // sched_log2_ceil of the most tiles of a heavy block (sched_block_tiles)
 constexpr int kWsExitCounter = 16;   // workgroups of the launch that have left the hand-out loop: the last one zeroes every counter
 constexpr int kWsXcdCounter = 64;    // next heavy ticket of XCD x at word kWsXcdCounter + 32 * x (ws_xcd_counter)
 constexpr int kWsHeader = 64 + 32 * kXcds;   // then one record of kRecWords per schedule position, E + 1 of them

@@ -1,8 +1,8 @@
 """First tickets (schedule.h, sched_first_tickets), compiled for the host.
 
 A workgroup's first ticket goes by its index and the counters hand out what lies behind: together they give every light ticket
-and every ticket of every XCD's queue once, whatever the kinds, the share and the number of workgroups, and a queue is named
-undrawn exactly where nothing lies behind.
+and every ticket of every XCD's queue that may be a tile once, whatever the kinds, the share, the tiles of a block and the number
+of workgroups, and a queue is named undrawn exactly where nothing lies behind.
 """
 import ctypes
 import os
@@ -18,10 +18,10 @@ SOURCE = r"""
 using namespace esmoe;
 extern "C" {
 int queue_tickets(int xcd, int hblocks) { return sched_queue_tickets(xcd, hblocks); }
-int first(int wgs, int hblocks, int ltotal, int share, int draw, int wg, int* light, int* heavy_base, int* light_base, int* undrawn) {
-  const SchedFirst f = sched_first_tickets(wgs, hblocks, ltotal, share, draw);
+int first(int wgs, int hblocks, int block_tiles, int ltotal, int share, int draw, int wg, int* light, int* heavy_base, int* light_base, int* undrawn) {
+  const SchedFirst f = sched_first_tickets(wgs, hblocks, sched_log2_ceil(block_tiles), ltotal, share, draw);
   *light = sched_first_is_light(wg, f);
-  *heavy_base = f.heavy_ranks;
+  *heavy_base = f.heavy_base;
   *light_base = f.light_base;
   *undrawn = sched_undrawn_queues(hblocks, ltotal, f);
   return sched_first_ticket(wg, f);
@@ -48,11 +48,12 @@ def test_first_and_drawn_tickets_cover_every_ticket_once(host, workgroups):
     cases += [(rng.randrange(80), rng.randrange(1500)) for _ in range(40)]
     for hblocks, ltotal in cases:
         share, draw = rng.randrange(33) if hblocks and ltotal else 0, rng.choice((1, 1, 2, 5, 14, 32))
+        tiles = rng.choice((1, 2, 3, 5, 8, 9, 16, 17, 24, 32))   # of a block: its first tickets, the others are no tiles
         queues = [host.queue_tickets(x, hblocks) for x in range(8)]
         assert sum(queues) == 32 * hblocks
         light, heavy = [0] * ltotal, [[0] * q for q in queues]
         for wg in range(workgroups):
-            t = host.first(workgroups, hblocks, ltotal, share, draw, wg, *refs)
+            t = host.first(workgroups, hblocks, tiles, ltotal, share, draw, wg, *refs)
             assert t >= 0
             if out[0].value:
                 for v in range(t, min(t + draw, ltotal)):
@@ -65,6 +66,7 @@ def test_first_and_drawn_tickets_cover_every_ticket_once(host, workgroups):
         for q in heavy:
             for v in range(heavy_base, len(q)):
                 q[v] += 1
-        assert all(c == 1 for c in light) and all(c == 1 for q in heavy for c in q), (hblocks, ltotal, share, draw)
+        assert all(c == 1 for c in light), (hblocks, ltotal, share, draw)
+        assert all(c == 1 or (c == 0 and t % 32 >= tiles) for q in heavy for t, c in enumerate(q)), (hblocks, tiles, ltotal, share)
         want = (256 if light_base >= ltotal else 0) | sum(1 << x for x in range(8) if heavy_base >= queues[x])
         assert undrawn == want

@@ -25,6 +25,11 @@ CASES = {
     "nine_blocks": ([100] * 9, 512, 256),
     "both": ([100] * 5 + [7] * 30, 768, 512),
     "many_of_both": ([70] * 20 + [16] * 300 + [400], 384, 256),
+    "blocks_of_three": ([150] * 70, 768, 256),       # 9 a queue; four tickets of each of the first eight are first ones
+    "blocks_of_one": ([65] * 300, 256, 128),
+    "blocks_of_sixteen": ([1500] * 17, 512, 128),
+    "blocks_of_eighteen": ([1100] * 9, 640, 128),     # handed out as blocks of 32
+    "small_blocks_and_light": ([100] * 40 + [3] * 60, 512, 256),
 }
 
 
