@@ -1,7 +1,8 @@
 // Persistent grouped GEMM for gfx950 (MI355X): FP8-blockwise and MXFP8 variants.
 //
-// One launch serves every expert.  A one-workgroup schedule kernel turns problem_sizes into a list of workgroup
-// tiles (schedule.h); persistent workgroups of 8 wavefronts then pull tiles from atomic counters.  A tile is
+// One launch serves every expert.  Every workgroup (self_schedule), or a one-workgroup schedule kernel in front, turns
+// problem_sizes into a list of workgroup tiles (schedule.h); persistent workgroups of 8 wavefronts start on the tile that
+// their index gives and then pull tiles from atomic counters.  A tile is
 // (MT*16) token rows x 256 weight rows, MT in {1, 2, 4} (short tiles, gemm_tile) or {8, 12} (tall tiles,
 // gemm_tile_pp / gemm_tile_pp_mx); the short items that end a launch are handed out as two 128-column halves.
 //
@@ -22,7 +23,7 @@
 //
 // MFMA mapping (v_mfma[_scale]_f32_16x16x128_f8f6f4, both operands e4m3):
 //   * the weight rows ride on the instruction's "A" side and the token rows on its "B" side, so a lane ends up with
-//     4 consecutive output columns of one token row (one packed 8-byte store);
+//     4 consecutive output columns of one token row (8 bytes; two lanes' worth make one 16-byte store);
 //   * lane l feeds row (l % 16); its 8 operand registers hold K bytes [16*(l/16), +16) and [64 + 16*(l/16), +16)
 //     of the 128-wide K block;
 //   * for the scaled form lane l supplies the E8M0 scale of row (l % 16), K sub-block (l / 16) in byte 0 of the
@@ -288,7 +289,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, Acc& acc, int M
     // wavefront reads back only what it wrote itself, so no barrier) it writes whole 128-byte lines of eight rows, in half
     // as many instructions.  Rows are 144 bytes apart in LDS to spread the banks.  Whole lines of output are stored with the
     // non-temporal hint: nothing in this launch reads them, and they should not push operand panels out of L2 (C4 -3 %,
-    // C1 -1.8 %; the short tiles' 8-byte pieces are better off merging in L2: C2 +0.6 % with the hint).
+    // C1 -1.8 %; the short tiles' stores have a rule of their own: short_out_nt).
     constexpr int kRows = MTW * 16, kStride = 144;
     uint8_t* const region = lds + ((mw / kRows) * kWavesN + wn) * (kRows * kStride);
 #pragma unroll
@@ -429,7 +430,8 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
 // `cols` (plain 256-column tiles only; 1 otherwise): a strip of so many neighbouring whole tiles of one expert, walked as one
 // stream of cols * K/128 stages.  The copies of the next tile's first stages are on their way while a tile ends, and its
 // output leaves as buffer stores that the counted waits leave in flight: a tile alone pays the ticket, the look-up and
-// the first stages' trip from memory, about 5 us (256 experts x 32 rows, 7168 x 256: 164 us one by one, 135 us as strips).
+// the first stages' trip from memory, about 5 us (256 experts x 32 rows, 7168 x 256: 164 us one by one, 135 us as
+// strips, 116 with the schedule and the stores as they are now).
 // A strip has at most 32 stages (sched_light_draw; its weight block scales share one tile's table of 256).
 template <int MT, bool MX, bool FUSE, int BN = kBN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb, int erow, int ebso, int M, int m0, int n0, int cols,
@@ -1230,13 +1232,15 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   __shared__ int s_blocks[1024];
   __shared__ int s_items[1024];
   __shared__ float s_cost[1024][2];   // heavy, light
+  __shared__ int s_block_log;         // kWsBlockLog
   const int e = threadIdx.x;
   int m = 0;
   if (e < num_experts) m = problem_sizes[e * 3];
   if (m < 0) m = 0;
   s_m[e] = m;
+  if (e == 0) s_block_log = 0;
   __syncthreads();
-  int pos = e;
+  int pos = e, tiles = 0;
   if (e < num_experts) {
     if (policy.order != 1) {
       pos = 0;
@@ -1252,7 +1256,12 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
     s_items[pos] = sched_light_items(m, n, policy);
     s_cost[pos][0] = sched_heavy_cost(m, n, policy);
     s_cost[pos][1] = sched_light_cost(m, n, policy);
+    if (sched_is_heavy(m, policy)) tiles = sched_block_tiles(m, n, policy);
   }
+  int block_log = 0;   // (over the wavefront)
+#pragma unroll
+  for (int i = 0; i < kBlkLog; i++) block_log += __ballot(tiles > 1 << i) != 0;
+  if (block_log > 0 && (e & 63) == 0) atomicMax(&s_block_log, block_log);
   __syncthreads();
   if (e < num_experts) {
     // exclusive prefix sums over schedule positions, one position per thread
@@ -1282,13 +1291,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
         light_cost += s_cost[j][1];
       }
       ws[kWsLightShare] = sched_light_share(heavy_cost, light_cost, policy);
-      int block_tiles = 0;
-      for (int j = 0; j < num_experts; j++)
-        if (sched_is_heavy(s_m[j], policy)) {
-          const int tiles = sched_block_tiles(s_m[j], n, policy);
-          block_tiles = tiles > block_tiles ? tiles : block_tiles;
-        }
-      ws[kWsBlockLog] = sched_log2_ceil(block_tiles);
+      ws[kWsBlockLog] = s_block_log;
     }
     if (pos < kXcds) ws[ws_xcd_counter(pos)] = 0;
   }
