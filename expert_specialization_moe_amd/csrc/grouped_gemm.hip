@@ -1501,7 +1501,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   // Tickets in hand, [have, have_end): at first those that go by the workgroup's index (sched_first_tickets), then what a
   // draw gave (light ones: sched_light_draw).  `xq`: their queue.
   int have = sched_first_ticket((int)blockIdx.x, first), xq = (int)blockIdx.x % kXcds;
-  int have_end = have + (light_first ? first.light_draw : 1), seen = have;
+  int have_end = have + (light_first ? first.light_draw : 1), seen = sched_first_seen((int)blockIdx.x, first);
   {
     const int total = light_first ? ltotal : sched_queue_tickets(xq, hblocks);
     if (have_end > total) have_end = total;

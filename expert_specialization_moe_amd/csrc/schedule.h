@@ -313,6 +313,9 @@ ESMOE_HD int sched_first_ticket(int workgroup, const SchedFirst& f) {
   const int r = workgroup / kXcds, block = r >> f.share_log;
   return block < f.blocks ? block * kBlkTiles + (r - (block << f.share_log)) : 0x7fffffff - kBlkTiles;
 }
+// Last light ticket that `workgroup` knows of before its first draw (`seen` of sched_light_draw): its own first one if that is a
+// light one; a heavy ticket says nothing about the light queue.
+ESMOE_HD int sched_first_seen(int workgroup, const SchedFirst& f) { return sched_first_is_light(workgroup, f) ? sched_first_ticket(workgroup, f) : 0; }
 // Queues that hold nothing but first tickets: bits 0-7 the XCDs' queues, bit 8 the light tickets (all nine: no counter is used).
 constexpr int kAllQueues = (1 << (kXcds + 1)) - 1;
 ESMOE_HD int sched_undrawn_queues(int hblocks, int ltotal, const SchedFirst& f) {

@@ -26,6 +26,10 @@ int first(int wgs, int hblocks, int block_tiles, int ltotal, int share, int draw
   *undrawn = sched_undrawn_queues(hblocks, ltotal, f);
   return sched_first_ticket(wg, f);
 }
+int seen(int wgs, int hblocks, int block_tiles, int ltotal, int share, int draw, int wg) {
+  return sched_first_seen(wg, sched_first_tickets(wgs, hblocks, sched_log2_ceil(block_tiles), ltotal, share, draw));
+}
+int light_draw(int total, int seen, int workgroups, int kblocks) { return sched_light_draw(total, seen, workgroups, kblocks, true); }
 }
 """
 
@@ -70,3 +74,21 @@ def test_first_and_drawn_tickets_cover_every_ticket_once(host, workgroups):
         assert all(c == 1 or (c == 0 and t % 32 >= tiles) for q in heavy for t, c in enumerate(q)), (hblocks, tiles, ltotal, share)
         want = (256 if light_base >= ltotal else 0) | sum(1 << x for x in range(8) if heavy_base >= queues[x])
         assert undrawn == want
+
+
+def test_a_heavy_first_ticket_says_nothing_about_the_light_queue(host):
+    """A workgroup that starts on a heavy ticket has seen no light one, whatever the ticket's number (also where it gets none: of a
+    queue's 24 workgroups the last eight, behind one block of 16 tiles), and its first light draw is that of a workgroup that has seen nothing;
+    one that starts on light tickets has seen its own."""
+    out = [ctypes.c_int() for _ in range(4)]
+    refs = [ctypes.byref(o) for o in out]
+    for hblocks, tiles, ltotal, share, draw in ((90, 16, 4000, 8, 4), (16, 32, 4000, 8, 4), (300, 4, 2000, 20, 1), (1, 1, 500, 16, 2)):
+        none = 0
+        for wg in range(256):
+            ticket = host.first(256, hblocks, tiles, ltotal, share, draw, wg, *refs)
+            seen = host.seen(256, hblocks, tiles, ltotal, share, draw, wg)
+            none += ticket > 1 << 30
+            assert seen == (ticket if out[0].value else 0), (wg, ticket, seen)
+            if not out[0].value:
+                assert host.light_draw(ltotal, seen, 256, 1) == min(max(ltotal >> 9, 1), 32)
+        assert none == (64 if tiles == 16 else 0)
