@@ -1214,11 +1214,14 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int fi
 }
 
 // ---------------------------------------------------------------------------------------------
-// First K block of expert e's K order, in units of kStartUnit (schedule.h, sched_k_start): 16 bytes of its weight scales.
+// First K block of expert e's K order, in units of kStartUnit (schedule.h, sched_k_start): 16 bytes of its weight scales, which
+// the entry points let begin at any multiple of four bytes (still one load: global memory takes dword alignment).
+typedef v4i __attribute__((aligned(4))) v4i_dwords;
+static_assert(alignof(v4i_dwords) == 4, "promises the compiler no more than the entry points ask for");
 __device__ __forceinline__ int expert_k_start(const float* sb, const uint8_t* sfb, int e, int n, int k) {
   if (!sched_spread_k(k)) return 0;
   const long first = sfb ? (long)e * n * (k >> 5) : (long)e * (n >> 7) * (k >> 7) * 4;
-  const v4i s = *(const v4i*)((sfb ? sfb : (const uint8_t*)sb) + first);
+  const v4i s = *(const v4i_dwords*)((sfb ? sfb : (const uint8_t*)sb) + first);
   return sched_k_start((uint32_t)s[0], (uint32_t)s[1], (uint32_t)s[2], (uint32_t)s[3]);
 }
 

@@ -61,3 +61,25 @@ def test_more_experts_than_the_kernel_schedules_itself(esmoe):
                     expert_offsets=(ops["expert_offsets"][sl] - i * half * m).contiguous())
         got = _mm(_native, part, "fp8", None, torch.full_like(ops["output"][rl], 3.0))
         assert torch.equal(got.view(torch.int16), whole[rl].view(torch.int16)), i
+
+
+@pytest.mark.parametrize("kind", ["fp8", "mx"])
+def test_scales_that_begin_four_bytes_behind_a_16_byte_boundary(esmoe, kind):
+    """The entry points ask for four bytes: the same bytes as with aligned scales, in both schedules, short and tall tiles."""
+    from expert_specialization_moe_amd import _native, workloads as W
+
+    n, k, rows = 384, 4096, [5, 64, 0, 200, 33]
+    prob = W.Problem("under", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
+    make = W.make_mxfp8_operands if kind == "mx" else W.make_fp8_blockwise_operands
+    ops = make(prob, "cuda", seed=4, out_dtype=torch.bfloat16, weight_std=0.05)
+    base = _mm(_native, ops, kind, None, torch.full_like(ops["output"], 3.0)).clone()
+    moved = dict(ops)
+    for name in ("sfa", "sfb_phys") if kind == "mx" else ("scales_a", "scales_b_phys"):
+        buffer = torch.empty((4 + ops[name].numel() * ops[name].element_size(),), dtype=torch.uint8, device="cuda")
+        moved[name] = buffer[4:].view(ops[name].dtype).view(ops[name].shape)
+        moved[name].copy_(ops[name])
+        assert moved[name].data_ptr() % 16 == 4
+    ws = torch.zeros((_native.lib.esmoe_gemm_workspace_bytes(len(rows)),), dtype=torch.uint8, device="cuda")
+    for workspace in (None, ws):
+        got = _mm(_native, moved, kind, workspace, torch.full_like(base, 3.0))
+        assert torch.equal(got.view(torch.int16), base.view(torch.int16))
