@@ -50,6 +50,10 @@ namespace esmoe {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+// 16 bytes of a caller's scales or output, which the entry points let begin at any multiple of four (scales) or eight bytes
+// (output): still one instruction, global memory takes dword alignment, but the compiler is promised no more than that.
+typedef v4i __attribute__((aligned(4))) v4i_dwords;
+static_assert(alignof(v4i_dwords) == 4, "the type's own alignment would be 16");
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -179,7 +183,7 @@ __device__ __forceinline__ void store_staged_rows(const uint8_t* stage, int stri
 #pragma unroll
   for (int row = tid >> 3; row < BM; row += kThreads / 8) {
     const int m = m0 + row;
-    if (m < M) __builtin_nontemporal_store(*(const v4i*)(stage + row * stride + (tid & 7) * 16), (v4i*)(dst + (long)m * pitch + (tid & 7) * 16));
+    if (m < M) __builtin_nontemporal_store(*(const v4i*)(stage + row * stride + (tid & 7) * 16), (v4i_dwords*)(dst + (long)m * pitch + (tid & 7) * 16));
   }
 }
 
@@ -309,7 +313,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, Acc& acc, int M
       const int row = i * 8 + rr;
       const int m = m0 + mw + row;
       const v4i line = *(const v4i*)(region + row * kStride + ch * 16);
-      if (wave_active && m < M) __builtin_nontemporal_store(line, (v4i*)((uint8_t*)g.out + ((row_base + m) * (long)N + n0 + nw) * 2 + ch * 16));
+      if (wave_active && m < M) __builtin_nontemporal_store(line, (v4i_dwords*)((uint8_t*)g.out + ((row_base + m) * (long)N + n0 + nw) * 2 + ch * 16));
     }
     return;
   }
@@ -327,7 +331,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, Acc& acc, int M
                                   : pair_halves(out_half4(acc[0][2 * i], g.out_dtype), out_half4(acc[0][2 * i + 1], g.out_dtype));
         const int m = m0 + mw + r + (NTW == 2 ? i * 16 : (2 * i + (gq & 1)) * 16);
         const int n = n0 + nw + (NTW == 2 ? pair_column(gq) : (gq >> 1) * 8);
-        if (m < M) *(v4i*)((uint8_t*)g.out + ((row_base + m) * (long)N + n) * 2) = line;
+        if (m < M) *(v4i_dwords*)((uint8_t*)g.out + ((row_base + m) * (long)N + n) * 2) = line;
       }
     }
   }
@@ -1214,10 +1218,7 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int fi
 }
 
 // ---------------------------------------------------------------------------------------------
-// First K block of expert e's K order, in units of kStartUnit (schedule.h, sched_k_start): 16 bytes of its weight scales, which
-// the entry points let begin at any multiple of four bytes (still one load: global memory takes dword alignment).
-typedef v4i __attribute__((aligned(4))) v4i_dwords;
-static_assert(alignof(v4i_dwords) == 4, "promises the compiler no more than the entry points ask for");
+// First K block of expert e's K order, in units of kStartUnit (schedule.h, sched_k_start): 16 bytes of its weight scales.
 __device__ __forceinline__ int expert_k_start(const float* sb, const uint8_t* sfb, int e, int n, int k) {
   if (!sched_spread_k(k)) return 0;
   const long first = sfb ? (long)e * n * (k >> 5) : (long)e * (n >> 7) * (k >> 7) * 4;
