@@ -559,7 +559,7 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
     ws_host[esmoe::ws_rec(pos) + esmoe::kRecExpert] = e;
     ws_host[esmoe::ws_rec(pos) + esmoe::kRecRows] = rows_of(e);
   }
-  int blocks = 0, items = 0;
+  int blocks = 0, items = 0, block_log = 0;
   float heavy_cost = 0, light_cost = 0;
   for (int pos = 0; pos < num_experts; pos++) {
     const int m = ws_host[esmoe::ws_rec(pos) + esmoe::kRecRows];
@@ -569,6 +569,8 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
     items += esmoe::sched_light_items(m, n, p);
     heavy_cost += esmoe::sched_heavy_cost(m, n, p);
     light_cost += esmoe::sched_light_cost(m, n, p);
+    const int log = esmoe::sched_is_heavy(m, p) ? esmoe::sched_log2_ceil(esmoe::sched_block_tiles(m, n, p)) : 0;
+    if (log > block_log) block_log = log;
   }
   int32_t* last = ws_host + esmoe::ws_rec(num_experts);
   last[esmoe::kRecBlock] = blocks;
@@ -577,10 +579,12 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
   last[esmoe::kRecRows] = 0;
   ws_host[esmoe::kWsLightShare] = esmoe::sched_light_share(heavy_cost, light_cost, p);
   ws_host[esmoe::kWsHeavyBlocks] = blocks;
+  ws_host[esmoe::kWsBlockLog] = block_log;
   const int split = esmoe::sched_light_split(items, p);
   ws_host[esmoe::kWsLightSplit] = split;
   ws_host[esmoe::kWsLightTotal] = split + 2 * (items - split);
   ws_host[esmoe::kWsLightCounter] = 0;
+  ws_host[esmoe::kWsExitCounter] = 0;
   for (int x = 0; x < esmoe::kXcds; x++) ws_host[esmoe::ws_xcd_counter(x)] = 0;
   return 0;
 }
@@ -612,7 +616,7 @@ int esmoe_host_decode_heavy(const int32_t* problem_sizes_host, const int32_t* ws
   bool past = false;
   if (!esmoe::sched_decode_heavy(blk - rec[esmoe::kRecBlock], ticket % esmoe::kBlkTiles, rec[esmoe::kRecRows], n, p, &t, &past))
     return 1;   // ticket outside the expert's tile grid: skipped
-  fill_out5(out5, rec[esmoe::kRecExpert], t);
+  fill_out5(out5, esmoe::rec_expert(rec[esmoe::kRecExpert]), t);
   return 0;
 }
 
@@ -629,7 +633,7 @@ int esmoe_host_decode_light(const int32_t* problem_sizes_host, const int32_t* ws
   const int32_t* rec = ws_host + esmoe::ws_rec(pos);
   const esmoe::TileCoord t = esmoe::sched_decode_light(idx - rec[esmoe::kRecItem], rec[esmoe::kRecRows], p, half);
   if (t.n0 >= n) return 1;   // second half of a last column tile that is 128 columns wide: skipped
-  fill_out5(out5, rec[esmoe::kRecExpert], t);
+  fill_out5(out5, esmoe::rec_expert(rec[esmoe::kRecExpert]), t);
   return 0;
 }
 

@@ -78,6 +78,10 @@ int esmoe_stream_workspace(void* stream, void** workspace, size_t* bytes);
  * force_bm: 0 lets the device-side schedule pick an M-tile shape per expert;
  *           16/32/64/128/192 forces that single shape for every tile (benchmarking).
  * Rows of `out` that belong to no expert (M_e == 0) are not written.
+ *
+ * An element's K blocks are summed in one order per expert, whatever else the call holds: 0, 1, 2, ... or, for K a multiple of
+ * 4096, from a block that a hash of the first 16 bytes of the expert's weight scales gives, and round.  This holds for all grouped
+ * GEMM entry points.
  */
 int esmoe_fp8_blockwise_grouped_mm(void* out, int out_dtype, const void* a, const void* b, const float* sa,
                                    const float* sb, const int32_t* problem_sizes, const int32_t* expert_offsets,
@@ -269,8 +273,11 @@ int esmoe_permute_rows(const void* in, const int32_t* dst_row, long num_pairs, i
  * Host mirrors of the device-side tile schedule, for inspection and CPU tests; they touch no GPU.
  * No counterpart in the reference (its schedule lives inside CUTLASS's grouped tile scheduler).
  * esmoe_host_schedule fills `ws_host` (esmoe_gemm_workspace_bytes(E) bytes of host memory) from host
- * copies of problem_sizes exactly as the schedule kernel fills the device workspace: words 1 and 2 are
- * the number of light items and of heavy blocks.
+ * copies of problem_sizes as the schedule kernel fills the device workspace: words 1 and 2 are
+ * the number of light items and of heavy blocks, word 5 the size class of the blocks.  One thing the mirror does not see: for K a
+ * multiple of 4096 the device notes in bits 16 and up of a record's expert word where the expert's K order starts, in units of
+ * four K blocks, which depends on the weight scales (see esmoe_fp8_blockwise_grouped_mm); the mirror leaves these bits 0, and
+ * the decode functions take records of either kind.
  * Experts with more than 64 rows are "heavy": their tiles are handed out in blocks of 8 x 4 tiles, block b
  * to XCD b % 8, through one ticket counter per XCD; esmoe_host_decode_heavy maps ticket `ticket` of XCD `xcd`
  * to out5 = {expert, tile rows, tile cols, m0, n0} and returns 0, or 1 if the ticket falls outside the

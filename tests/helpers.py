@@ -104,6 +104,18 @@ def capi_mx_mm(native, ops, force_bm=0, out=None):
     return out
 
 
+def k_start_blocks(scale_bytes):
+    """First K block of an expert's K order for K a multiple of 4096, from the first 16 bytes of its weight scales: the arithmetic
+    of schedule.h (sched_k_start), written out here on plain integers."""
+    s, mask = [int(v) for v in np.frombuffer(bytes(scale_bytes), dtype="<u4", count=4)], 0xffffffff
+    rot = lambda h: (h << 13 | h >> 19) & mask
+    h = (s[1] - s[0]) * 0x9e3779b1 & mask
+    h = ((rot(h) ^ (s[2] - s[0] & mask)) * 0x85ebca6b) & mask
+    h = ((rot(h) ^ (s[3] - s[0] & mask)) * 0xc2b2ae35) & mask
+    h = ((h ^ h >> 16) * 0x7feb352d) & mask
+    return 4 * (h >> 29)
+
+
 def hp_to_f32(t: torch.Tensor) -> np.ndarray:
     """bf16/fp16 tensor -> float32 numpy (exact)."""
     return t.detach().float().cpu().numpy()

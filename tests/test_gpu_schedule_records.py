@@ -1,4 +1,4 @@
-"""Records that the GEMM kernel's own schedule writes (self_schedule), against the host mirror's.
+"""Records that the GEMM kernel's own schedule (self_schedule) and the schedule kernel write, against the host mirror's.
 
 Light experts are placed by a count per row number, heavy ones by comparisons among themselves: the lists have ties, every row
 number around the border of the two kinds, empty experts, one kind only, full wavefronts of experts and one expert more, and heavy lists
@@ -48,3 +48,45 @@ def test_records_equal_the_host_mirror(esmoe, name, force_bm):
     first = 64 + 32 * 8
     got, want = (v[first:first + 4 * (experts + 1)].reshape(-1, 4) for v in (dev, host))
     assert np.array_equal(got, want), np.flatnonzero((got != want).any(axis=1))
+
+
+@pytest.mark.parametrize("kind", ["fp8", "mx"])
+def test_both_schedules_note_where_an_experts_k_order_starts(esmoe, kind):
+    """K = 4096: above an expert's index stands its start as the hash of its own first scales gives it, every place among them; under
+    it, and everywhere else, both schedules write what the host mirror writes (the schedule kernel the launch constants too), and
+    the mirror's decode functions read the device's records."""
+    from expert_specialization_moe_amd import _native, workloads as W
+
+    lib, n, k = _native.lib, 640, 4096
+    rows = [(5, 64, 0, 70, 33, 200, 1, 16)[i % 8] for i in range(96)]
+    experts, bits = len(rows), 1 if kind == "mx" else 0
+    prob = W.Problem("starts", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
+    ops = (W.make_mxfp8_operands if kind == "mx" else W.make_fp8_blockwise_operands)(prob, "cuda", seed=9, out_dtype=torch.bfloat16, weight_std=0.05)
+    scales = ops["sfb_phys" if kind == "mx" else "scales_b_phys"].reshape(experts, -1).contiguous().view(torch.uint8).cpu().numpy()
+    starts = [H.k_start_blocks(scales[e].tobytes()) for e in range(experts)]
+    assert set(starts) == {0, 4, 8, 12, 16, 20, 24, 28}
+    words = lib.esmoe_gemm_workspace_bytes(experts) // 4
+    ptr = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    ps, host = np.array([[m, n, k] for m in rows], dtype=np.int32), np.zeros(words, dtype=np.int32)
+    assert lib.esmoe_host_schedule(ptr(ps), experts, n, 0, bits, ptr(host)) == 0, _native.last_error()
+    ws = torch.full((words,), -1, dtype=torch.int32, device="cuda").view(torch.uint8)
+    out = torch.full_like(ops["output"], 3.0)
+    _mm(_native, ops, kind, ws, out)
+    own = _mm(_native, ops, kind, None, torch.full_like(out, 3.0))
+    assert torch.equal(own.view(torch.int16), out.view(torch.int16))
+    kernel, first = ws.view(torch.int32).cpu().numpy(), 64 + 32 * 8
+    want = host[first:first + 4 * (experts + 1)].reshape(-1, 4).copy()
+    want[:-1, 2] |= np.array([starts[e] // 4 for e in want[:-1, 2]], dtype=np.int32) << 16
+    for dev in (kernel, _read_stream_workspace(_native, words)):
+        got = dev[first:first + 4 * (experts + 1)].reshape(-1, 4)
+        assert np.array_equal(got, want), np.flatnonzero((got != want).any(axis=1))
+    header = [1, 2, 3, 4, 5, 16, 32] + [64 + 32 * x for x in range(8)]
+    assert kernel[header].tolist() == host[header].tolist()
+    tile, mirror = np.zeros(5, dtype=np.int32), np.zeros(5, dtype=np.int32)
+    for item in range(int(host[1])):
+        rc = [lib.esmoe_host_decode_light(ptr(ps), ptr(w), experts, n, 0, bits, item, ptr(t)) for w, t in ((kernel, tile), (host, mirror))]
+        assert rc[0] == rc[1] and (rc[0] or np.array_equal(tile, mirror)), item
+    for xcd in range(8):
+        for ticket in range(64):
+            rc = [lib.esmoe_host_decode_heavy(ptr(ps), ptr(w), experts, n, 0, bits, xcd, ticket, ptr(t)) for w, t in ((kernel, tile), (host, mirror))]
+            assert rc[0] == rc[1] and (rc[0] or np.array_equal(tile, mirror)), (xcd, ticket)

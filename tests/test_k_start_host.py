@@ -7,6 +7,8 @@ import subprocess
 import numpy as np
 import pytest
 
+from tests import helpers as H
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 SOURCE = r"""
@@ -49,6 +51,7 @@ def test_starts_are_spread_and_go_by_scale_differences(host):
         count = np.bincount(got, minlength=8)
         assert len(count) == 8 and count.min() > 4000 // 8 // 2 and count.max() < 4000 // 8 * 2, count
         assert [_start(host, w) for w in shifted[:200]] == got[:200].tolist()
+        assert [H.k_start_blocks(np.ascontiguousarray(w).tobytes()) for w in words[:500]] == (4 * got[:500]).tolist()
     for value in (0, 0x3f800000, 0x7f7f7f7f, 0xffffffff):
         assert _start(host, [value] * 4) == 0
 

@@ -151,3 +151,48 @@ def test_heavy_blocks_are_rectangles_of_one_expert_on_one_xcd(esmoe):
     for ts in blocks.values():
         n0s = sorted({t[4] for t in ts})
         assert n0s[-1] - n0s[0] == 256 * (len(n0s) - 1)
+
+
+@pytest.mark.parametrize("rows", [[3841, 0, 965, 70, 12, 64, 1], [5, 9, 0, 64], [200] * 12])
+def test_records_that_say_where_the_k_order_starts_decode_to_the_same_tiles(esmoe, rows):
+    """For K a multiple of 4096 the device writes the start of the expert's K order above its index (bits 16 and up)."""
+    from expert_specialization_moe_amd import _native
+
+    e, n = len(rows), 1280
+    ps = np.array([[m, n, 4096] for m in rows], dtype=np.int32)
+    plain = np.zeros(_native.lib.esmoe_gemm_workspace_bytes(e) // 4, dtype=np.int32)
+    ptr = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    assert _native.lib.esmoe_host_schedule(ptr(ps), e, n, 0, 0, ptr(plain)) == 0
+    device = plain.copy()
+    first = 64 + 32 * 8
+    for pos in range(e):
+        device[first + 4 * pos + 2] |= (1 + pos % 7) << 16
+
+    def tiles(ws):
+        out, got = np.zeros(5, dtype=np.int32), []
+        for xcd in range(8):
+            for ticket in range(32 * (int(ws[2]) // 8 + 1)):
+                rc = _native.lib.esmoe_host_decode_heavy(ptr(ps), ptr(ws), e, n, 0, 0, xcd, ticket, ptr(out))
+                got.append((rc, tuple(out) if rc == 0 else None))
+        for item in range(int(ws[1])):
+            rc = _native.lib.esmoe_host_decode_light(ptr(ps), ptr(ws), e, n, 0, 0, item, ptr(out))
+            got.append((rc, tuple(out) if rc == 0 else None))
+        return got
+
+    want = tiles(plain)
+    assert {t[0] for rc, t in want if rc == 0} == {i for i, m in enumerate(rows) if m}
+    assert tiles(device) == want
+
+
+def test_word_5_is_the_size_class_of_the_blocks(esmoe):
+    """The most tiles of a heavy expert's block, rounded up to a power of two (its logarithm)."""
+    from expert_specialization_moe_amd import _native
+
+    n = 1280                                                        # five column tiles
+    for rows, tiles in (([64, 3], 0), ([65, 1], 5), ([193, 400], 15), ([1500], 24), ([5000], 32), ([100, 193, 20], 10)):
+        e = len(rows)
+        ps = np.array([[m, n, 512] for m in rows], dtype=np.int32)
+        ws = np.full(_native.lib.esmoe_gemm_workspace_bytes(e) // 4, -1, dtype=np.int32)
+        assert _native.lib.esmoe_host_schedule(ps.ctypes.data_as(ctypes.c_void_p), e, n, 0, 0, ws.ctypes.data_as(ctypes.c_void_p)) == 0
+        assert ws[5] == (max(tiles - 1, 0)).bit_length(), (rows, ws[5])
+        assert ws[16] == 0
