@@ -1466,7 +1466,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   const int wg = (int)blockIdx.x, ticket = sched_first_ticket(wg, f);
   int half = -1;
   const bool first_light = sched_first_is_light(wg, f);
-  const int idx = first_light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(wg % kXcds, ticket);
+  const int idx = first_light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(sched_home_queue(wg), ticket);
   if ((first_light ? light : heavy) && idx >= before && idx < before + mine) *s_first = FirstRecord{before, word, m, row, scale_row};
   __syncthreads();
 }
@@ -1490,10 +1490,8 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     lsplit = ws[kWsLightSplit];
     first = first_tickets<FUSE>(args, hblocks, ws[kWsBlockLog], ltotal, ws[kWsLightShare]);
   }
-  // Workgroup i runs on XCD i % 8 (HW_REG_XCC_ID = 20, bits [3:0], says so directly).  Of every 32 workgroups
-  // of an XCD the last `light_share` start on the light items, the others on the heavy tickets; either kind
-  // moves on to the other when its own is exhausted.
-  const int xcd = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & (kXcds - 1);
+  // Of every 32 workgroups of an XCD the last `light_share` start on the light items, the others on the heavy tickets; either
+  // kind moves on to the other when its own is exhausted.
   const bool light_first = sched_first_is_light((int)blockIdx.x, first);
   int phase = 0, q = 0;
   // Queues known to be exhausted (bits 0-7: the XCDs' heavy queues, bit 8: the light items).  When a draw comes back
@@ -1504,7 +1502,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   int dead = undrawn;
   // Tickets in hand, [have, have_end): at first those that go by the workgroup's index (sched_first_tickets), then what a
   // draw gave (light ones: sched_light_draw).  `xq`: their queue.
-  int have = sched_first_ticket((int)blockIdx.x, first), xq = (int)blockIdx.x % kXcds;
+  int have = sched_first_ticket((int)blockIdx.x, first), xq = sched_home_queue((int)blockIdx.x);
   int have_end = have + (light_first ? first.light_draw : 1), seen = sched_first_seen((int)blockIdx.x, first);
   {
     const int total = light_first ? ltotal : sched_queue_tickets(xq, hblocks);
@@ -1526,7 +1524,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     if (have == have_end) {
       if (dead == kAllQueues) break;
       from_lds = false;
-      xq = (xcd + q) & (kXcds - 1);
+      xq = sched_drawn_queue((int)blockIdx.x, q);
       if ((dead >> (light ? 8 : xq)) & 1) {   // nothing (left) in this queue: the next XCD's, then the other kind
         if (light || ++q == kXcds) {
           q = 0;
@@ -1619,7 +1617,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       // one by one (a block of 6 x 4 tiles has eight of them, one of 1 x 5 twenty-seven, and each costs a draw and a look-up, 2 to
       // 3 us): 31 experts x 81 rows, 1280 x 768 24.1 -> 22.0 us, 45 experts, 3062 rows, 1024 x 2304 37.4 -> 35.3, MXFP8 MLP of 819
       // tokens, 64 experts 196.7 -> 187; 131072 rows, 3072 x 4096 1643 -> 1635.
-      const int next = (have + kBlkTiles - 1) / kBlkTiles * kBlkTiles - first.heavy_base;   // (`have` is one on)
+      const int next = sched_next_block(have - 1, first.heavy_base);   // (`have` is one on)
       if (past && next > 0 && threadIdx.x == 0) atomicMax(&ws[ws_xcd_counter(xq)], next);
       __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
       continue;

@@ -270,6 +270,18 @@ ESMOE_HD int sched_ticket_block(int xcd, int ticket) { return (ticket / kBlkTile
 // Tickets of XCD `xcd`'s queue when the launch has `hblocks` heavy blocks: queue x holds the blocks x, x + 8, ..., 32 tickets each.
 ESMOE_HD int sched_queue_tickets(int xcd, int hblocks) { return xcd < hblocks ? (hblocks - xcd + kXcds - 1) / kXcds * kBlkTiles : 0; }
 
+// Queue that a workgroup draws heavy tickets from when it has found `step` queues empty: first the one its first ticket is of, the
+// queue of its XCD (the hardware deals the workgroups of a launch out in turn, workgroup i to XCD i % 8), then the others in turn.
+// That the first draw is from the queue of the first ticket is more than locality: see sched_next_block.
+ESMOE_HD int sched_home_queue(int workgroup) { return workgroup % kXcds; }
+ESMOE_HD int sched_drawn_queue(int workgroup, int step) { return (sched_home_queue(workgroup) + step) % kXcds; }
+
+// What a queue's counter has to be at least when the tickets behind `ticket` in its block are no tiles (0 or less: nothing to do, the
+// rest of the block is not drawn from the counter).  Raising the counter is an atomic maximum that nobody waits for.  It must
+// have happened before the workgroup counts itself out, since the last one out zeroes the counters; it has, because the workgroup
+// goes on with a draw from the same queue, an add to the same address by the same thread, and waits for that.
+ESMOE_HD int sched_next_block(int ticket, int heavy_base) { return (ticket / kBlkTiles + 1) * kBlkTiles - heavy_base; }
+
 // First tickets: a workgroup's first ticket goes by its index, and the counters hand out what lies behind these.  Atomic adds to
 // one address are served one every 12 ns, so 256 workgroups that all begin with a draw wait 3 us for the last of them, and as
 // long again to count themselves out; a launch whose tickets are all first ones needs neither.

@@ -29,6 +29,9 @@ int first(int wgs, int hblocks, int block_tiles, int ltotal, int share, int draw
 int seen(int wgs, int hblocks, int block_tiles, int ltotal, int share, int draw, int wg) {
   return sched_first_seen(wg, sched_first_tickets(wgs, hblocks, sched_log2_ceil(block_tiles), ltotal, share, draw));
 }
+int home_queue(int wg) { return sched_home_queue(wg); }
+int drawn_queue(int wg, int step) { return sched_drawn_queue(wg, step); }
+int next_block(int ticket, int heavy_base) { return sched_next_block(ticket, heavy_base); }
 int light_draw(int total, int seen, int workgroups, int kblocks) { return sched_light_draw(total, seen, workgroups, kblocks, true); }
 }
 """
@@ -92,3 +95,30 @@ def test_a_heavy_first_ticket_says_nothing_about_the_light_queue(host):
             if not out[0].value:
                 assert host.light_draw(ltotal, seen, 256, 1) == min(max(ltotal >> 9, 1), 32)
         assert none == (64 if tiles == 16 else 0)
+
+
+def test_a_raised_counter_is_drawn_from_next(host):
+    """The counter of a heavy queue is raised past a block's empty tickets by an atomic that only the workgroup's next draw waits for.  So
+    that draw must be from the same queue, also behind a first ticket, and a queue that is never drawn from must never be raised."""
+    for wg in range(256):
+        assert host.drawn_queue(wg, 0) == host.home_queue(wg)
+        assert sorted(host.drawn_queue(wg, step) for step in range(8)) == list(range(8))
+    out = [ctypes.c_int() for _ in range(4)]
+    refs = [ctypes.byref(o) for o in out]
+    rng = random.Random(3)
+    raised = 0
+    for workgroups in (1, 8, 100, 256, 304, 512):
+        for hblocks in [1, 2, 7, 8, 9, 16, 17, 64, 65] + [rng.randrange(1, 200) for _ in range(20)]:
+            ltotal = rng.choice((0, 1, 300))
+            share, tiles = rng.randrange(33) if ltotal else 0, rng.choice((1, 2, 3, 5, 8, 9, 16, 17, 24, 31))
+            for wg in range(workgroups):
+                t = host.first(workgroups, hblocks, tiles, ltotal, share, 1, wg, *refs)
+                light, heavy_base, _, undrawn = (o.value for o in out)
+                queue = host.home_queue(wg)
+                if light or t >= host.queue_tickets(queue, hblocks):
+                    continue
+                raise_to = host.next_block(t, heavy_base)
+                assert raise_to + heavy_base == (t // 32 + 1) * 32
+                raised += raise_to > 0
+                assert raise_to <= 0 or not undrawn >> queue & 1, (workgroups, hblocks, tiles, ltotal, share, wg)
+    assert raised
