@@ -39,15 +39,18 @@ struct TileCoord {
   int n0;  // first column
 };
 
-// a / b for a >= 0, b > 0.  On the device an integer division by a variable is a chain of some forty instructions, and the
-// schedule of an expert with more than 64 rows takes four of them in front of the first tile, as does every heavy ticket.  The float
-// quotient of a number below 2^31 is off by less than 2^9, that of what it leaves by less than one, and the last remainder says which way.
-ESMOE_HD int sched_div(int a, int b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const float inverse = __builtin_amdgcn_rcpf((float)b);
+// a / b for 0 <= a <= 3 * 2^29 (more rows than the card has memory for), b > 0.  On the device an integer division by a
+// variable is a chain of some forty instructions, and the schedule of an expert with more than 64 rows takes three of them in
+// front of the first tile, every heavy ticket six.  The float quotient is off by less than 2^9, that of what it leaves by less
+// than one, and the last remainder says which way.  `inverse`: 1 / b, up to one unit in the last place off either way.
+ESMOE_HD int sched_div_by(int a, int b, float inverse) {
   const int q = (int)((float)a * inverse), left = (int)((uint32_t)a - (uint32_t)q * (uint32_t)b);
   const int more = (int)((float)left * inverse), r = left - more * b;
   return q + more + (r >= b ? 1 : 0) - (r < 0 ? 1 : 0);
+}
+ESMOE_HD int sched_div(int a, int b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return sched_div_by(a, b, __builtin_amdgcn_rcpf((float)b));
 #else
   return a / b;
 #endif
