@@ -344,9 +344,11 @@ ESMOE_HD int sched_undrawn_queues(int hblocks, int ltotal, const SchedFirst& f) 
 // tile goes through one L2 channel of sixteen, and tiles that all begin with block 0 stay in step and queue for one channel
 // after the other (128 experts x 8 rows: 768 x 4096 88.3 us in step, 68.6 apart; 4096 x 4096 337 and 325; the projection of a 64-token
 // expert MLP with hidden size 4096 19 us less).  So every expert begins at a place of its own, a multiple of four K blocks in the first
-// 32, and wraps; large launches, bound by the matrix cores, take as long either way.  The place goes by the expert's weight scales, so that its bytes depend on its rows and weights
-// alone, not on where or among which others it is listed: a hash of the differences between its first scales (four fp32 block
-// scales, or sixteen E8M0 bytes as four words), which a common power of two in all scales does not change.  Equal scales: block 0.
+// 32, and wraps; large launches, bound by the matrix cores, take as long either way.  The place goes by the expert's weight scales,
+// so that its bytes depend on its rows and weights alone, not on where or among which others it is listed: a hash of the differences
+// between its first scales (four fp32 block scales, or sixteen E8M0 bytes as four words), which a common power of two in all
+// scales does not change.  Equal scales: block 0.  One place for all columns, since a tile of 256 has one K loop: a call on a part of
+// the expert's weight rows takes the same order only if it begins with the same row.
 ESMOE_HD bool sched_spread_k(int k) { return (k & 4095) == 0; }
 constexpr int kStartUnit = 4;
 ESMOE_HD int sched_k_start(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3) {   // in units of kStartUnit K blocks

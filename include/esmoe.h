@@ -80,8 +80,11 @@ int esmoe_stream_workspace(void* stream, void** workspace, size_t* bytes);
  * Rows of `out` that belong to no expert (M_e == 0) are not written.
  *
  * An element's K blocks are summed in one order per expert, whatever else the call holds: 0, 1, 2, ... or, for K a multiple of
- * 4096, from a block that a hash of the first 16 bytes of the expert's weight scales gives, and round.  This holds for all grouped
- * GEMM entry points.
+ * 4096, from a block that a hash of the first 16 bytes of the expert's weight scales gives, and round.  So the same expert gives the
+ * same bytes in every call.  For K a multiple of 4096 a part of its weight rows does so only if it begins at the same row (`b` and
+ * `sb` of the first columns): gate and up rows in two calls, or a later slice of columns, differ from one call over all of
+ * them as another order of fp32 sums does.  For every other K any slice gives the same bytes.  This holds for all grouped GEMM entry
+ * points.
  */
 int esmoe_fp8_blockwise_grouped_mm(void* out, int out_dtype, const void* a, const void* b, const float* sa,
                                    const float* sb, const int32_t* problem_sizes, const int32_t* expert_offsets,

@@ -1,6 +1,7 @@
 """One K order for every tile and every place in the list, also where rows are a multiple of 4096 bytes apart.
 
-Every output element is accumulated K block by K block from the first to the last, whatever tile computes it and wherever its
+Every output element is accumulated K block by K block in one order that is the expert's own (from the first block to the last or,
+for K a multiple of 4096, from a place that the expert's first weight scales give, and round), whatever tile computes it and wherever its
 expert stands in the call: every forced tile height must give the bytes of the device schedule, the fused epilogues those of
 projection -> stand-alone quantiser, and an expert listed elsewhere, or in a call of its own, its own bytes again (another
 rank's share of the same experts is such a call).  FP8-blockwise is also checked against
@@ -96,3 +97,39 @@ def test_an_experts_bytes_do_not_depend_on_its_place_in_the_list(esmoe, kind, k)
         for e in order:
             sl = slice(int(offs[e]), int(offs[e]) + rows[e])
             assert torch.equal(got[sl].view(torch.int16), base[sl].view(torch.int16)), f"expert {e} of {order}"
+
+
+@pytest.mark.parametrize("k", [4096, 7168])
+@pytest.mark.parametrize("kind", ["fp8", "mx"])
+def test_columns_of_an_expert_by_themselves(esmoe, kind, k):
+    """The first columns give the bytes they have in the whole, whatever K; later ones too unless K is a multiple of 4096, where they are
+    the same sums in another order: both results lie within K roundings of fp32 sums (K * 2^-24 of the magnitudes' sum) and
+    one rounding to bfloat16 (2^-8) of the exact value."""
+    from expert_specialization_moe_amd import _native, workloads as W
+
+    n, rows = 768, [1, 200, 0, 33, 130, 64]
+    experts = len(rows)
+    prob = W.Problem("columns", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
+    make, mm = (W.make_mxfp8_operands, H.capi_mx_mm) if kind == "mx" else (W.make_fp8_blockwise_operands, H.capi_fp8_mm)
+    ops = make(prob, "cuda", seed=k + 1, out_dtype=torch.bfloat16, weight_std=0.05)
+    whole = mm(_native, ops, 0, out=torch.full_like(ops["output"], 3.0)).clone()
+    for lo, hi in ((0, 128), (0, 384), (256, 768), (384, 512)):
+        part = dict(ops, b_phys=ops["b_phys"][:, lo:hi].contiguous())
+        if kind == "mx":
+            part["sfb_phys"] = ops["sfb_phys"].view(experts, n, k // 32)[:, lo:hi].contiguous()
+        else:
+            part["scales_b_phys"] = ops["scales_b_phys"][:, lo // 128:hi // 128].contiguous()
+        part["problem_sizes"] = torch.tensor([[m, hi - lo, k] for m in rows], dtype=torch.int32, device="cuda")
+        want = whole[:, lo:hi].contiguous()
+        got = mm(_native, part, 0, out=torch.full_like(want, 3.0))
+        if lo == 0 or k % 4096:
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (lo, hi)
+        elif kind == "fp8":
+            a = ops["a"].double() * ops["scales_a"].double().repeat_interleave(128, dim=1)
+            off = 0
+            for e, m in enumerate(rows):
+                w = part["b_phys"][e].double() * part["scales_b_phys"][e].double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+                mag = a[off:off + m].abs() @ w.abs().t()
+                diff = (got[off:off + m].double() - want[off:off + m].double()).abs()
+                assert (diff <= 2 * (want[off:off + m].double().abs() * 2.0 ** -8 + mag * (k * 2.0 ** -24))).all(), (lo, hi, e)
+                off += m
