@@ -116,6 +116,33 @@ def k_start_blocks(scale_bytes):
     return 4 * (h >> 29)
 
 
+def integer_operands(kind, rows, n, k, seed, spare=0):
+    """Small-integer operands with unit scales for either kind, so that every sum is exact, and the product in fp64: (ops, product of the
+    rows that belong to an expert).  `spare`: rows behind the last expert's that belong to none."""
+    from expert_specialization_moe_amd import workloads as W
+
+    experts, total = len(rows), sum(rows)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    ints = lambda *shape: torch.randint(-2, 3, shape, generator=gen, device="cuda").float()
+    a, b = ints(total + spare, k), ints(experts, n, k)
+    bso, sf_rows = W.blockscale_offsets_of(rows)
+    ops = dict(a=a.to(torch.float8_e4m3fn), b_phys=b.to(torch.float8_e4m3fn),
+               problem_sizes=torch.tensor([[m, n, k] for m in rows], dtype=torch.int32, device="cuda"),
+               expert_offsets=torch.tensor(W.offsets_of(rows), dtype=torch.int32, device="cuda"),
+               blockscale_offsets=torch.tensor(bso, dtype=torch.int32, device="cuda"))
+    if kind == "mx":
+        ops["sfa"] = torch.full((max(int(sf_rows), 128), k // 32), 127, device="cuda", dtype=torch.uint8)
+        ops["sfb_phys"] = torch.full((experts * n, k // 32), 127, device="cuda", dtype=torch.uint8)
+    else:
+        ops["scales_a"] = torch.ones((total + spare, k // 128), device="cuda")
+        ops["scales_b_phys"] = torch.ones((experts, n // 128, k // 128), device="cuda")
+    product, off = torch.empty((total, n), dtype=torch.float64, device="cuda"), 0
+    for i, m in enumerate(rows):
+        product[off:off + m] = a[off:off + m].double() @ b[i].double().t()
+        off += m
+    return ops, product
+
+
 def hp_to_f32(t: torch.Tensor) -> np.ndarray:
     """bf16/fp16 tensor -> float32 numpy (exact)."""
     return t.detach().float().cpu().numpy()

@@ -23,28 +23,13 @@ CASES = {
 @pytest.mark.parametrize("kind", ["fp8", "mx"])
 @pytest.mark.parametrize("name", list(CASES))
 def test_every_tile_of_every_block_is_computed(esmoe, kind, name):
-    from expert_specialization_moe_amd import _native, workloads as W
+    from expert_specialization_moe_amd import _native
 
     rows, n = CASES[name]
     k, experts, total = 256, len(rows), sum(rows)
-    gen = torch.Generator(device="cuda").manual_seed(n + experts)
-    ints = lambda *shape: torch.randint(-2, 3, shape, generator=gen, device="cuda").float()
-    a, b = ints(total, k), ints(experts, n, k)
-    bso, sf_rows = W.blockscale_offsets_of(rows)
-    ops = dict(a=a.to(torch.float8_e4m3fn), b_phys=b.to(torch.float8_e4m3fn),
-               problem_sizes=torch.tensor([[m, n, k] for m in rows], dtype=torch.int32, device="cuda"),
-               expert_offsets=torch.tensor(W.offsets_of(rows), dtype=torch.int32, device="cuda"),
-               blockscale_offsets=torch.tensor(bso, dtype=torch.int32, device="cuda"))
-    if kind == "mx":   # unit scales
-        ops["sfa"] = torch.full((int(sf_rows), k // 32), 127, device="cuda", dtype=torch.uint8)
-        ops["sfb_phys"] = torch.full((experts * n, k // 32), 127, device="cuda", dtype=torch.uint8)
-    else:
-        ops["scales_a"] = torch.ones((total, k // 128), device="cuda")
-        ops["scales_b_phys"] = torch.ones((experts, n // 128, k // 128), device="cuda")
-    want, off = torch.full((total + 1, n), 3.0, dtype=torch.bfloat16, device="cuda"), 0
-    for i, m in enumerate(rows):
-        want[off:off + m] = (a[off:off + m].double() @ b[i].double().t()).float().to(torch.bfloat16)
-        off += m
+    ops, product = H.integer_operands(kind, rows, n, k, n + experts)
+    want = torch.full((total + 1, n), 3.0, dtype=torch.bfloat16, device="cuda")
+    want[:total] = product.float().to(torch.bfloat16)
     ws = torch.randint(0, 256, (_native.lib.esmoe_gemm_workspace_bytes(experts),), dtype=torch.uint8, device="cuda")
     for workspace in (None, None, ws):
         got = torch.full_like(want, 3.0)

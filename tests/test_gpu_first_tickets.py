@@ -36,29 +36,13 @@ CASES = {
 @pytest.mark.parametrize("kind", ["fp8", "mx"])
 @pytest.mark.parametrize("name", list(CASES))
 def test_calls_at_the_edges_of_the_first_tickets(esmoe, kind, name):
-    from expert_specialization_moe_amd import _native, workloads as W
+    from expert_specialization_moe_amd import _native
 
     rows, n, k = CASES[name]
     experts, total = len(rows), sum(rows)
-    gen = torch.Generator(device="cuda").manual_seed(experts + n)
-    ints = lambda *shape: torch.randint(-2, 3, shape, generator=gen, device="cuda").float()
-    a, b = ints(total + 1, k), ints(experts, n, k)   # (a spare row that belongs to no expert)
-    bso, sf_rows = W.blockscale_offsets_of(rows)
-    ops = dict(a=a.to(torch.float8_e4m3fn), b_phys=b.to(torch.float8_e4m3fn),
-               problem_sizes=torch.tensor([[m, n, k] for m in rows], dtype=torch.int32, device="cuda"),
-               expert_offsets=torch.tensor(W.offsets_of(rows), dtype=torch.int32, device="cuda"),
-               blockscale_offsets=torch.tensor(bso, dtype=torch.int32, device="cuda"))
-    if kind == "mx":   # unit scales
-        ops["sfa"] = torch.full((max(int(sf_rows), 128), k // 32), 127, device="cuda", dtype=torch.uint8)
-        ops["sfb_phys"] = torch.full((experts * n, k // 32), 127, device="cuda", dtype=torch.uint8)
-    else:
-        ops["scales_a"] = torch.ones((total + 1, k // 128), device="cuda")
-        ops["scales_b_phys"] = torch.ones((experts, n // 128, k // 128), device="cuda")
+    ops, product = H.integer_operands(kind, rows, n, k, experts + n, spare=1)   # (a spare row that belongs to no expert)
     want = torch.full((total + 2, n), 3.0, dtype=torch.bfloat16, device="cuda")
-    off = 0
-    for i, m in enumerate(rows):
-        want[off:off + m] = (a[off:off + m].double() @ b[i].double().t()).float().to(torch.bfloat16)
-        off += m
+    want[:total] = product.float().to(torch.bfloat16)
     for rep in range(2):
         got = torch.full_like(want, 3.0)
         _mm(_native, ops, kind, None, got[:total + 1])

@@ -2,8 +2,8 @@
 
 A row's bytes are the same however many other rows its expert has (short tiles, 128- and 192-row tiles, every K loop), with the
 schedule of the GEMM kernel and that of the schedule kernel (a caller's workspace; more experts than the kernel schedules
-itself).  The eight experts begin at different places, which the scales used here decide; each is also compared with the fp64
-product: one rounding to bfloat16 (2^-8 of the value) plus K roundings of fp32 sums (K * 2^-24 of the magnitudes' sum).
+itself).  The eight experts begin at four places at least, which is checked against the hash of their scales; each is also compared
+with the fp64 product: one rounding to bfloat16 (2^-8 of the value) plus K roundings of fp32 sums (K * 2^-24 of the magnitudes' sum).
 """
 import pytest
 import torch
@@ -23,6 +23,9 @@ def test_a_rows_bytes_do_not_depend_on_the_other_rows(esmoe, kind, k):
     prob = W.Problem("start", n, k, [rows] * experts, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
     make = W.make_mxfp8_operands if kind == "mx" else W.make_fp8_blockwise_operands
     ops = make(prob, "cuda", seed=k, out_dtype=torch.bfloat16, weight_std=0.05)
+    scales = ops["sfb_phys" if kind == "mx" else "scales_b_phys"].reshape(experts, -1).contiguous().view(torch.uint8).cpu().numpy()
+    starts = [H.k_start_blocks(scales[e].tobytes()) for e in range(experts)]
+    assert len(set(starts)) >= 4 and any(starts), starts
     fresh = lambda: torch.full_like(ops["output"], 3.0)
     base = _mm(_native, ops, kind, None, fresh()).clone()
     offs = [e * rows for e in range(experts)]

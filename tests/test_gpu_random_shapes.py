@@ -5,7 +5,8 @@ tile height (16 ... 192 rows) must give the bytes of the device schedule; FP8-bl
 against a torch fp32 product of the dequantised operands (tolerance of the path: 1e-2 of the expert's largest output),
 and where the shape allows it the fused SwiGLU + quantisation entry points against projection -> stand-alone
 quantiser, byte for byte.  Shapes are drawn from lists that mix empty, one-row, ragged and many-row experts, column
-counts that are no multiple of 256 and K from one block to 7168.
+counts that are no multiple of 256 and K from one block to 7168; one seed draws K from the multiples of 4096 only, where every expert's
+K order starts at a place of its own and the K loops wrap.
 """
 import random
 
@@ -20,13 +21,16 @@ ROW_POOLS = [[0, 1, 3, 7, 16, 17, 31], [0, 5, 33, 64, 65, 100, 128, 129], [0, 1,
              [2, 40, 70, 130, 200, 333, 577, 800], [0, 0, 0, 1, 2000, 1500, 191, 383], [96, 97, 95, 48, 49, 47, 0]]
 
 
-def _cases(seed, count):
+K_LIST, K_WRAPPED = [128, 256, 384, 512, 640, 896, 1024, 1536, 2048, 7168], [4096, 8192, 12288]
+
+
+def _cases(seed, count, ks):
     rng = random.Random(seed)
     for case in range(count):
         kind = rng.choice(["fp8", "mx"])
         e = rng.choice([1, 2, 3, 5, 8, 9, 17, 33, 40, 64])
         n = rng.choice([128, 256, 384, 512, 768, 1024, 1152, 2048])
-        k = rng.choice([128, 256, 384, 512, 640, 896, 1024, 1536, 2048, 7168])
+        k = rng.choice(ks)
         pool = rng.choice(ROW_POOLS)
         rows = [rng.choice(pool) for _ in range(e)]
         if sum(rows) == 0:
@@ -36,13 +40,13 @@ def _cases(seed, count):
         yield case, kind, n, k, rows, rng.choice([torch.bfloat16, torch.float16])
 
 
-@pytest.mark.parametrize("seed", [5, 6])
-def test_forced_heights_fused_forms_and_torch_agree(seed):
+@pytest.mark.parametrize("seed,ks", [(5, K_LIST), (6, K_LIST), (7, K_WRAPPED)], ids=["5", "6", "7-wrapped"])
+def test_forced_heights_fused_forms_and_torch_agree(seed, ks):
     import expert_specialization_moe_amd as es
     from expert_specialization_moe_amd import _native, workloads as W
 
     ran = 0
-    for case, kind, n, k, rows, dt in _cases(seed, 60):
+    for case, kind, n, k, rows, dt in _cases(seed, 60, ks):
         prob = W.Problem("rand", n, k, rows, kind="mxfp8" if kind == "mx" else "fp8_blockwise")
         tag = f"seed {seed} case {case}: {kind} n={n} k={k} {dt} rows={rows}"
         print(tag, flush=True)
