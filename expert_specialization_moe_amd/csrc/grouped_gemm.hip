@@ -1616,7 +1616,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       // The rest of the block's tickets are no tiles either: move the queue on to its next block, so that they are not drawn
       // one by one (a block of 6 x 4 tiles has eight of them, one of 1 x 5 twenty-seven, and each costs a draw and a look-up, 2 to
       // 3 us): 31 experts x 81 rows, 1280 x 768 24.1 -> 22.0 us, 45 experts, 3062 rows, 1024 x 2304 37.4 -> 35.3, MXFP8 MLP of 819
-      // tokens, 64 experts 196.7 -> 187; 131072 rows, 3072 x 4096 1643 -> 1635.
+      // tokens, 64 experts 196.7 -> 187.
       const int next = sched_next_block(have - 1, first.heavy_base);   // (`have` is one on)
       if (past && next > 0 && threadIdx.x == 0) atomicMax(&ws[ws_xcd_counter(xq)], next);
       __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first

@@ -48,7 +48,8 @@ extern "C" {
  *
  * Every GEMM entry point below also accepts workspace == NULL with workspace_bytes == 0: the library then uses a
  * workspace of its own, one per (device, stream), whose counters it knows to be zero between launches (zeroed when
- * allocated; the last workgroup of every launch zeroes them again).  Such a call is ONE kernel launch: every workgroup
+ * allocated; the last workgroup of a launch that draws from them zeroes them again, and a launch whose tickets all go by the
+ * workgroups' indices leaves them alone).  Such a call is ONE kernel launch: every workgroup
  * builds the schedule records itself (up to 512 experts; more fall back to the schedule kernel).  This replaces the
  * reference's pre-compute launch and its twelve per-call scratch tensors (es_fp8_blockwise_launcher.cuh:18-86,
  * es_fp8_blockwise.cu:58-75) by nothing.  The library's workspaces are allocated 16 at a time (hipMalloc + hipMemset):
