@@ -231,8 +231,8 @@ int launch_gemm(esmoe::GemmArgs& g, int mx, int force_bm, void* stream, bool own
   if ((g.policy.force_mt && !esmoe::sched_valid_mt(g.policy.force_mt)) || (g.policy.big_mt != 8 && g.policy.big_mt != 12))
     return fail(ESMOE_ERR_INVALID_ARGUMENT, "tile heights %d / %d rows are not compiled into the kernels",
                 g.policy.force_mt * 16, g.policy.big_mt * 16);
-  int grid = info.cus;   // one persistent workgroup per CU: its LDS ring takes the whole 160 KB
-  rc = esmoe_launch_grouped_gemm(&g, mx, grid, (hipStream_t)stream);
+  g.workgroups = info.cus;   // one persistent workgroup per CU: its LDS ring takes the whole 160 KB
+  rc = esmoe_launch_grouped_gemm(&g, mx, g.workgroups, (hipStream_t)stream);
   if (rc) return fail(rc, "grouped GEMM launch failed: %s", hipGetErrorString((hipError_t)rc));
   return 0;
 }

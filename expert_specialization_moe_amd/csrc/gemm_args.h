@@ -26,6 +26,7 @@ struct GemmArgs {
   int n;
   int k;
   int out_dtype;        // 0 bf16, 1 fp16
+  int workgroups;       // of the launch (gridDim.x stands in a part of the argument block that nothing else is read from)
   int self_schedule;    // 1: no schedule kernel ran; ws counters are zero and every workgroup builds the records itself
   SchedPolicy policy;
 };

@@ -1302,23 +1302,86 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
   if (num_experts < kXcds && e >= num_experts && e < kXcds) ws[ws_xcd_counter(e)] = 0;
 }
 
-template <bool FUSE>
-__device__ __forceinline__ SchedFirst first_tickets(const GemmArgs& g, int hblocks, int block_log, int ltotal, int lshare) {
-  return sched_first_tickets((int)gridDim.x, hblocks, block_log, ltotal, lshare, sched_light_draw(ltotal, 0, (int)gridDim.x, g.k >> 7, !FUSE));
-}
-
-// What a workgroup has to know of its first ticket (self_schedule).
-struct FirstRecord {
-  int first;   // first light item, or heavy block, of the expert
-  int expert, rows;   // (the expert's word: rec_expert, rec_first_kb)
-  int row, scale_row;   // expert_offsets[expert], blockscale_offsets[expert]
+// A tile, or a strip of `cols` neighbouring ones, of an expert of `rows` rows.
+struct Tile {
+  int mt, nt, cols;       // mt = 0: none
+  int m0, n0;
+  int expert, rows;       // (the expert's word: rec_expert, rec_first_kb)
+  int row, scale_row;     // expert_offsets[expert], blockscale_offsets[expert]
+  int taken;              // tickets that it is
 };
+
+// What a workgroup knows when the schedule is done: the queues, and the tickets in hand, [have, have_end).
+struct Hand {
+  int hblocks, ltotal, lsplit;   // heavy blocks, light tickets, the first of these that is a half item
+  int heavy_base, light_base;    // first tickets that come from the counters
+  int undrawn;                   // queues that hold nothing but first tickets (sched_undrawn_queues)
+  int light_first, have, have_end, seen;
+};
+template <bool FUSE>
+__device__ __forceinline__ Hand first_hand(const GemmArgs& g, int hblocks, int block_log, int ltotal, int lsplit, int lshare) {
+  const int wg = (int)blockIdx.x;
+  const SchedFirst f = sched_first_tickets(g.workgroups, hblocks, block_log, ltotal, lshare,
+                                           sched_light_draw(ltotal, 0, g.workgroups, g.k >> 7, !FUSE));
+  Hand h;
+  h.hblocks = hblocks;
+  h.ltotal = ltotal;
+  h.lsplit = lsplit;
+  h.heavy_base = f.heavy_base;
+  h.light_base = f.light_base;
+  h.undrawn = sched_undrawn_queues(hblocks, ltotal, f);
+  h.light_first = sched_first_is_light(wg, f);
+  h.have = sched_first_ticket(wg, f);
+  h.have_end = h.have + (h.light_first ? f.light_draw : 1);
+  h.seen = sched_first_seen(wg, f);
+  const int total = h.light_first ? ltotal : sched_queue_tickets(sched_home_queue(wg), hblocks);
+  if (h.have_end > total) h.have_end = total;
+  if (h.have > h.have_end) h.have = h.have_end;
+  return h;
+}
+// Light item or heavy block of a ticket (half: of a light one, sched_light_item_of_ticket).
+__device__ __forceinline__ int ticket_index(bool light, int queue, int ticket, int lsplit, int* half) {
+  *half = -1;
+  return light ? sched_light_item_of_ticket(ticket, lsplit, half) : sched_ticket_block(queue, ticket);
+}
+// Tile of ticket `have`, item or block `local` of its expert; moves `have` on by the tickets that it takes.  mt = 0: it is no tile
+// (`past`: nor are those behind it in its block).
+template <bool FUSE>
+__device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int& have, int have_end, int lsplit, int local, int half, int rows, bool* past) {
+  TileCoord t;
+  Tile d;
+  *past = false;
+  d.cols = 1;
+  d.rows = rows;
+  if (light) {
+    t = sched_decode_light(local, rows, g.policy, half);
+    if constexpr (!FUSE) {
+      const int tiles = sched_strip_tiles(have, have_end, lsplit, local, g.n, half);
+      if (tiles > 1) d.cols = tiles;
+      if (half == 0 && tiles > 0) {   // both halves: one whole tile
+        t.nt = 4;
+        half = -2;
+      }
+    }
+    have += half == -2 ? 2 * d.cols : d.cols;
+    if (t.n0 >= g.n) t.mt = 0;   // second half of a last column tile that is 128 columns wide
+  } else if (!sched_decode_heavy(local, have++ % kBlkTiles, rows, g.n, g.policy, &t, past)) {
+    t.mt = 0;
+  }
+  d.mt = t.mt;
+  d.nt = t.nt;
+  d.m0 = t.m0;
+  d.n0 = t.n0;
+  return d;
+}
+// Wave-uniform values that the compiler does not know to be.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // The schedule built by the GEMM kernel itself (one launch per call; schedule.h, kSelfScheduleMaxExperts): every
 // workgroup does what schedule_kernel does and writes the records into `ws`, where the hand-out loop finds them with
 // scalar loads.  All workgroups write the same values.  The launch constants are returned instead of stored.  `lds` is
-// the ring, free before the first tile.  The record of the workgroup's first ticket goes into `s_first` as well, so that
-// nothing in front of the first tile waits for the records' way to memory and back: the hand-out loop does before it reads one.
+// the ring, free before the first tile.  The workgroup's first tile goes into `first`, so that nothing in front of it waits for the
+// records' way to memory and back: the hand-out does before it reads one.
 //
 // This runs in front of every workgroup's first tile, so it is latency from end to end: trips to LDS, barriers and, at some five
 // clocks each, instructions.  Light experts (and empty ones) have at most 64 rows and the same number of items each, so a count
@@ -1329,9 +1392,107 @@ struct FirstRecord {
 // x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting
 // instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us; half as many divisions and a four-way search of the records:
 // 75.2 -> 74.7 (with both kinds of experts), an expert MLP of 1003 tokens in MXFP8 377.5 -> 376.1.
+// The workgroup's first tile, by the thread of the expert that the ticket belongs to (items or blocks [before, before + mine)).
+template <bool FUSE>
+__device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool light, bool heavy, int before, int mine, int rows, int word, int row,
+                                           int scale_row, Tile* first) {
+  if (h.have == h.have_end) return;
+  int half;
+  const int idx = ticket_index(h.light_first, sched_home_queue((int)blockIdx.x), h.have, h.lsplit, &half);
+  if ((h.light_first ? light : heavy) && idx >= before && idx < before + mine) {
+    bool past;
+    int have = h.have;
+    Tile d = take_tile<FUSE>(g, h.light_first, have, h.have_end, h.lsplit, idx - before, half, rows, &past);
+    d.expert = word;
+    d.row = row;
+    d.scale_row = scale_row;
+    d.taken = have - h.have;
+    if (d.mt) *first = d;
+  }
+}
+
+// The schedule of up to 64 experts, by the workgroup's first wavefront alone, a lane per expert: no barrier until everything is done (the
+// other wavefronts wait there), ranks from comparing every key with all others, prefix sums by DPP.  What bounds it is latency, three to
+// four clocks an instruction with what fetching cold code takes, so it is the count of instructions that matters.  With heavy experts
+// the first tile is known after 3000 clocks instead of 5600 (self_schedule passes five barriers), without after 2900 to 3200 as before,
+// but as a whole: the hand-out has 500 clocks less to do.  8 experts x 32 rows, 256 x 512 6.4 -> 6.0 us, x 100 rows 10.5 -> 9.1, 64 x 200
+// rows, 512 x 512 13.6 -> 12.8.
 template <bool MX, bool FUSE>
-__device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, FirstRecord* s_first, int& hblocks, int& ltotal, int& lsplit,
-                                              SchedFirst& f) {
+__device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, Tile* first) {
+  const int E = g.num_experts, lane = threadIdx.x;
+  const SchedPolicy policy = g.policy;
+  int* ws = g.ws;
+  int m = 0, row = 0, scale_row = 0, word = lane;
+  if (lane < E) {
+    m = g.problem_sizes[lane * 3];
+    row = g.expert_offsets[lane];
+    if constexpr (MX) scale_row = g.blockscale_offsets[lane];
+    word = rec_expert_word(lane, expert_k_start(g.sb, MX ? g.sfb : nullptr, lane, g.n, g.k));
+  }
+  if (lane == 0) first->mt = 0;
+  // (waited for here: a load that the compiler holds for outstanding puts a wait of its own into the K loops)
+  asm volatile("" : "+v"(row), "+v"(scale_row), "+v"(word));
+  if (m < 0) m = 0;
+  const bool heavy = lane < E && sched_is_heavy(m, policy), light = lane < E && !heavy;
+  const int num_heavy = __builtin_popcountll(__ballot(heavy)), num_light = __builtin_popcountll(__ballot(light && m > 0));
+  // heavy experts first, by sched_order_key (rows past 2^25 count as so many), then light ones, most rows first; ties by index
+  constexpr int kMostRows = (1 << 25) - 1;
+  const int capped = m < kMostRows ? m : kMostRows, by = light ? 64 - m : policy.order == 2 ? kMostRows - capped : capped;
+  const uint32_t key = lane < E ? (uint32_t)by << 6 | (uint32_t)lane | (light ? 1u << 31 : 0) : 0xffffffffu;
+  uint32_t* s_key = (uint32_t*)lds;
+  s_key[lane] = key;   // (a wavefront's LDS accesses stay in order)
+  int pos = 0;
+  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+  v4u a = *(const v4u*)s_key, b = *(const v4u*)(s_key + 4);
+#pragma unroll 1
+  for (int j = 8;; j += 8) {
+    const v4u next_a = *(const v4u*)(s_key + j), next_b = *(const v4u*)(s_key + j + 4);   // (what lies behind the keys is not looked at)
+    uint64_t less[8];   // (all compared first: as a chain of compare and add through one register a key took 18 clocks)
+#pragma unroll
+    for (int c = 0; c < 8; c++) less[c] = __ballot((c < 4 ? a[c] : b[c - 4]) < key);
+#pragma unroll
+    for (int c = 0; c < 8; c++) asm("v_addc_co_u32_e64 %0, vcc, 0, %0, %1" : "+v"(pos) : "s"(less[c]) : "vcc");
+    if (j >= E) break;
+    a = next_a;
+    b = next_b;
+  }
+  const int ntl = sched_ntiles(g.n, 4), items = num_light * ntl;
+  int before = 0, mine = 0, blocks = 0, block_log = 0, lshare = 0;
+  if (light) {
+    const int rank = pos - num_heavy;
+    before = (rank < num_light ? rank : num_light) * ntl;
+    mine = m > 0 ? ntl : 0;
+  }
+  if (num_heavy > 0) {
+    int tiles = 0;
+    if (heavy) {
+      mine = sched_heavy_blocks(m, g.n, policy);
+      tiles = sched_block_tiles(m, g.n, policy);
+    }
+    // blocks in the order of the schedule, their prefix sums, and back (a lane of no heavy expert sends nothing on to the sums)
+    const int placed = __builtin_amdgcn_ds_permute(pos * 4, heavy ? mine : 0);
+    const int sum = wave_inclusive_sum(lane < num_heavy ? placed : 0);
+    blocks = __builtin_amdgcn_readlane(sum, 63);
+    const int up_to = __builtin_amdgcn_ds_bpermute(pos * 4, sum);
+    if (heavy) before = up_to - mine;
+#pragma unroll
+    for (int i = 0; i < kBlkLog; i++) block_log += __ballot(tiles > 1 << i) != 0;
+    if (items > 0) {   // how many workgroups start on which kind, where a launch has both
+      const float hc = wave_sum_last(sched_heavy_cost(m, g.n, policy)), lc = wave_sum_last(light ? sched_light_cost(m, g.n, policy) : 0.f);
+      lshare = sched_light_share(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hc), 63)),
+                                 __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lc), 63)), policy);
+    }
+  }
+  if (lane < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
+  if (lane == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
+  const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
+  Hand h = first_hand<FUSE>(g, blocks, block_log, ltotal, lsplit, lshare);
+  first_tile<FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
+  if (lane == 0) *out = h;
+}
+
+template <bool MX, bool FUSE>
+__device__ __forceinline__ Hand self_schedule(const GemmArgs& g, uint8_t* lds, Tile* first) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
   constexpr int kLightRows = 64, kHistStride = kLightRows + 4;
   int* s_hist = (int*)lds;                              // [kWaves][kHistStride]: experts of a wavefront by rows (0 .. 64)
@@ -1353,6 +1514,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   s_hist[wave * kHistStride + lane] = 0;   // (a wavefront's LDS accesses stay in order)
   if (lane == 0) s_hist[wave * kHistStride + kLightRows] = 0;
   s_rank[t] = 0;
+  if (t == 0) first->mt = 0;
   // (waited for here: a load that the compiler holds for outstanding puts a wait of its own into the K loops)
   asm volatile("" : "+v"(row), "+v"(scale_row), "+v"(word));
   if (m < 0) m = 0;
@@ -1458,17 +1620,11 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, F
   if (t < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
   if (t == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
-  hblocks = blocks;
-  lsplit = sched_light_split(items, policy);
-  ltotal = lsplit + 2 * (items - lsplit);
-  // the thread of the expert that the first ticket belongs to says so
-  f = first_tickets<FUSE>(g, hblocks, block_log, ltotal, lshare);
-  const int wg = (int)blockIdx.x, ticket = sched_first_ticket(wg, f);
-  int half = -1;
-  const bool first_light = sched_first_is_light(wg, f);
-  const int idx = first_light ? sched_light_item_of_ticket(ticket, lsplit, &half) : sched_ticket_block(sched_home_queue(wg), ticket);
-  if ((first_light ? light : heavy) && idx >= before && idx < before + mine) *s_first = FirstRecord{before, word, m, row, scale_row};
+  const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
+  Hand h = first_hand<FUSE>(g, blocks, block_log, ltotal, lsplit, lshare);
+  first_tile<FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
   __syncthreads();
+  return h;
 }
 
 template <bool MX, bool FUSE>
@@ -1476,43 +1632,125 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   __shared__ int s_item;
   __shared__ int s_counters[kXcds + 1];
-  __shared__ FirstRecord s_first;
+  __shared__ Hand s_hand;
+  __shared__ Tile s_tile;
   int* ws = args.ws;
   // (the line of the arguments that holds the operands' addresses: asked for with the others, not in front of the first tile)
   asm volatile("" ::"s"(args.a));
-  int hblocks, ltotal, lsplit;
-  SchedFirst first;
-  if (args.self_schedule) {
-    self_schedule<MX, FUSE>(args, lds, &s_first, hblocks, ltotal, lsplit, first);
-  } else {
-    hblocks = ws[kWsHeavyBlocks];
-    ltotal = ws[kWsLightTotal];
-    lsplit = ws[kWsLightSplit];
-    first = first_tickets<FUSE>(args, hblocks, ws[kWsBlockLog], ltotal, ws[kWsLightShare]);
-  }
   // Of every 32 workgroups of an XCD the last `light_share` start on the light items, the others on the heavy tickets; either
   // kind moves on to the other when its own is exhausted.
-  const bool light_first = sched_first_is_light((int)blockIdx.x, first);
+  Hand hand;
+  Tile tile;
+  tile.mt = 0;
+  if (args.self_schedule) {
+    if (args.num_experts > 64) {
+      hand = self_schedule<MX, FUSE>(args, lds, &s_tile);
+    } else {
+      if (threadIdx.x < 64) wave_schedule<MX, FUSE>(args, lds, &s_hand, &s_tile);
+      __syncthreads();
+      const Hand h = s_hand;
+      hand = Hand{uniform(h.hblocks), uniform(h.ltotal), uniform(h.lsplit), uniform(h.heavy_base), uniform(h.light_base),
+                  uniform(h.undrawn), uniform(h.light_first), uniform(h.have), uniform(h.have_end), uniform(h.seen)};
+    }
+    tile = s_tile;
+    if (uniform(tile.mt)) hand.have += uniform(tile.taken);
+  } else {
+    hand = first_hand<FUSE>(args, ws[kWsHeavyBlocks], ws[kWsBlockLog], ws[kWsLightTotal], ws[kWsLightSplit], ws[kWsLightShare]);
+  }
   int phase = 0, q = 0;
   // Queues known to be exhausted (bits 0-7: the XCDs' heavy queues, bit 8: the light items).  When a draw comes back
   // past the end of its queue and the launch has heavy blocks on every XCD, one look at all nine counters marks every
   // queue that has run dry, so that a workgroup leaving its own queue does not spend an atomic round trip (about a
   // microsecond under load) on each empty one.
-  const int undrawn = sched_undrawn_queues(hblocks, ltotal, first);
-  int dead = undrawn;
+  int dead = hand.undrawn;
   // Tickets in hand, [have, have_end): at first those that go by the workgroup's index (sched_first_tickets), then what a
   // draw gave (light ones: sched_light_draw).  `xq`: their queue.
-  int have = sched_first_ticket((int)blockIdx.x, first), xq = sched_home_queue((int)blockIdx.x);
-  int have_end = have + (light_first ? first.light_draw : 1), seen = sched_first_seen((int)blockIdx.x, first);
-  {
-    const int total = light_first ? ltotal : sched_queue_tickets(xq, hblocks);
-    if (have_end > total) have_end = total;
-    if (have > have_end) have = have_end;
-  }
-  bool from_lds = args.self_schedule != 0;   // the next record is the first ticket's
-  bool records_pending = from_lds;           // this workgroup's records may still be on their way to memory
+  int have = hand.have, xq = sched_home_queue((int)blockIdx.x), have_end = hand.have_end, seen = hand.seen;
+  bool records_pending = args.self_schedule != 0;   // this workgroup's records may still be on their way to memory
   typedef const __attribute__((address_space(4))) GemmArgs* KernArgs;
   KernArgs kernargs = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  // The next tile of this workgroup; false: there is none.
+  auto next_tile = [&](const GemmArgs& g, Tile& d) -> bool {
+    for (;;) {
+      const bool light = (phase == 0) == (hand.light_first != 0);
+      if (have == have_end) {
+        if (dead == kAllQueues) return false;
+        xq = sched_drawn_queue((int)blockIdx.x, q);
+        if ((dead >> (light ? 8 : xq)) & 1) {   // nothing (left) in this queue: the next XCD's, then the other kind
+          if (light || ++q == kXcds) {
+            q = 0;
+            if (++phase == 2) return false;
+          }
+          continue;
+        }
+        const int draw = light ? sched_light_draw(hand.ltotal, seen, g.workgroups, g.k >> 7, !FUSE) : 1;
+        const int total = light ? hand.ltotal : sched_queue_tickets(xq, hand.hblocks);
+        if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
+        __syncthreads();
+        const int ticket = (light ? hand.light_base : hand.heavy_base) + uniform(s_item);
+        if (ticket >= total) {   // this queue is exhausted: see which others are
+          dead |= 1 << (light ? 8 : xq);
+          __syncthreads();                        // s_item and s_counters are rewritten next
+          // (worth its round trip only when every XCD has a queue to try: the look itself reads the hot counter line)
+          if (hand.hblocks <= kXcds) continue;
+          if (threadIdx.x < kXcds + 1)
+            s_counters[threadIdx.x] = __hip_atomic_load(threadIdx.x < kXcds ? &ws[ws_xcd_counter(threadIdx.x)] : &ws[kWsLightCounter],
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __syncthreads();
+#pragma unroll
+          for (int x = 0; x < kXcds; x++) {
+            if (hand.heavy_base + uniform(s_counters[x]) >= sched_queue_tickets(x, hand.hblocks)) dead |= 1 << x;
+          }
+          if (hand.light_base + uniform(s_counters[kXcds]) >= hand.ltotal) dead |= 256;
+          continue;
+        }
+        have = ticket;
+        have_end = ticket + draw < total ? ticket + draw : total;
+        if (light) seen = ticket;
+      }
+      if (records_pending) {   // every store of this workgroup has to be in L2 before a record is read
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        records_pending = false;
+      }
+      // schedule position of the ticket's item (a light one; the tickets past `lsplit` are halves of the narrow tail's items) or block:
+      // the last one whose first item or block is not behind it, found by halving the prefix sums twice a step, with scalar loads.
+      // The records are only read from here on, so they stay in the scalar cache, where a step costs a fraction of what a trip to L2
+      // costs while the chip streams weights, and three loads as much as one.
+      int half;
+      const int idx = ticket_index(light, xq, have, hand.lsplit, &half), kind = light ? kRecItem : kRecBlock;
+      int lo = 0, hi = g.num_experts;
+      while (hi - lo > 1) {
+        const int step = (hi - lo + 3) >> 2;
+        auto at = [&](int pos) { return (ws_rec(pos < g.num_experts ? pos : g.num_experts) + kind) * 4; };
+        int v0, v1, v2;
+        sload3(ws, at(lo + step), at(lo + 2 * step), at(lo + 3 * step), v0, v1, v2);   // (past `hi`: more than idx as well)
+        lo += ((v0 <= idx ? 1 : 0) + (v1 <= idx ? 1 : 0) + (v2 <= idx ? 1 : 0)) * step;
+        if (hi > lo + step) hi = lo + step;
+      }
+      // the whole record in one load, then the expert's first row (and first scale row) through the scalar cache as
+      // well: a vector load here waits its turn behind the weight streams of the whole chip
+      const v4i rec = sload4(ws, ws_rec(lo) * 4);
+      const int word = uniform(rec[kRecExpert]);
+      bool past;
+      d = take_tile<FUSE>(g, light, have, have_end, hand.lsplit, idx - uniform(light ? rec[kRecItem] : rec[kRecBlock]), half,
+                          uniform(rec[kRecRows]), &past);
+      d.expert = word;
+      if (d.mt) {
+        d.row = sload(g.expert_offsets, rec_expert(word) * 4);
+        d.scale_row = 0;
+        if constexpr (MX) d.scale_row = sload(g.blockscale_offsets, rec_expert(word) * 4);
+        return true;
+      }
+      // A heavy ticket (`have` is one on) that is no tile.  `past`: nor are the rest of its block's; then the queue moves on to its next
+      // block, so that they are not drawn one by one (a block of 6 x 4 tiles has eight of them, one of 1 x 5 twenty-seven, and each
+      // costs a draw and a look-up, 2 to 3 us): 31 experts x 81 rows, 1280 x 768 24.1 -> 22.0 us, 45 experts, 3062 rows, 1024 x 2304
+      // 37.4 -> 35.3, MXFP8 MLP of 819 tokens, 64 experts 196.7 -> 187.
+      const int next = sched_next_block(have - 1, hand.heavy_base);
+      if (past && next > 0 && threadIdx.x == 0) atomicMax(&ws[ws_xcd_counter(xq)], next);
+      __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
+    }
+  };
   for (;;) {
     // The arguments are read anew for every tile (scalar loads that hit): kept across tiles, what the many tile functions
     // need of them were up to 80 scalar registers spilled to lanes of vector registers, with reloads in front of every tile
@@ -1520,117 +1758,12 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     // 13.1 -> 12.1; 256 experts x 32 rows, 7168 x 256 fused 182 -> 167 us.
     asm volatile("" : "+s"(kernargs));
     const GemmArgs& g = *(const GemmArgs*)kernargs;
-    const bool light = (phase == 0) == light_first;
-    if (have == have_end) {
-      if (dead == kAllQueues) break;
-      from_lds = false;
-      xq = sched_drawn_queue((int)blockIdx.x, q);
-      if ((dead >> (light ? 8 : xq)) & 1) {   // nothing (left) in this queue: the next XCD's, then the other kind
-        if (light || ++q == kXcds) {
-          q = 0;
-          if (++phase == 2) break;
-        }
-        continue;
-      }
-      const int draw = light ? sched_light_draw(ltotal, seen, (int)gridDim.x, g.k >> 7, !FUSE) : 1;
-      const int total = light ? ltotal : sched_queue_tickets(xq, hblocks);
-      if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
-      __syncthreads();
-      const int ticket = (light ? first.light_base : first.heavy_base) + __builtin_amdgcn_readfirstlane(s_item);
-      if (ticket >= total) {   // this queue is exhausted: see which others are
-        dead |= 1 << (light ? 8 : xq);
-        __syncthreads();                        // s_item and s_counters are rewritten next
-        // (worth its round trip only when every XCD has a queue to try: the look itself reads the hot counter line)
-        if (hblocks <= kXcds) continue;
-        if (threadIdx.x < kXcds + 1)
-          s_counters[threadIdx.x] = __hip_atomic_load(threadIdx.x < kXcds ? &ws[ws_xcd_counter(threadIdx.x)] : &ws[kWsLightCounter],
-                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-#pragma unroll
-        for (int x = 0; x < kXcds; x++) {
-          if (first.heavy_base + __builtin_amdgcn_readfirstlane(s_counters[x]) >= sched_queue_tickets(x, hblocks)) dead |= 1 << x;
-        }
-        if (first.light_base + __builtin_amdgcn_readfirstlane(s_counters[kXcds]) >= ltotal) dead |= 256;
-        continue;
-      }
-      have = ticket;
-      have_end = ticket + draw < total ? ticket + draw : total;
-      if (light) seen = ticket;
-    }
-    const int kind = light ? kRecItem : kRecBlock;
-    // (a light ticket past `lsplit` is one half of an item of the narrow tail)
-    int half = -1;
-    const int idx = light ? sched_light_item_of_ticket(have, lsplit, &half) : sched_ticket_block(xq, have);
-    int rec_first, word, M, erow, ebso = 0;
-    if (from_lds) {
-      rec_first = __builtin_amdgcn_readfirstlane(s_first.first);
-      word = __builtin_amdgcn_readfirstlane(s_first.expert);
-      M = __builtin_amdgcn_readfirstlane(s_first.rows);
-      erow = __builtin_amdgcn_readfirstlane(s_first.row);
-      if constexpr (MX) ebso = __builtin_amdgcn_readfirstlane(s_first.scale_row);
-      from_lds = false;
-    } else {
-      if (records_pending) {   // every store of this workgroup has to be in L2 before a record is read
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        records_pending = false;
-      }
-      // schedule position of idx: the last one whose first block (item) is <= idx, found by halving the prefix sums twice a
-      // step, with scalar loads.  The records are only read from here on, so they stay in the scalar cache, where a step costs
-      // a fraction of what a trip to L2 costs while the chip streams weights, and three loads as much as one.
-      int lo = 0, hi = g.num_experts;
-      while (hi - lo > 1) {
-        const int d = (hi - lo + 3) >> 2;
-        auto at = [&](int pos) { return (ws_rec(pos < g.num_experts ? pos : g.num_experts) + kind) * 4; };
-        int v0, v1, v2;
-        sload3(ws, at(lo + d), at(lo + 2 * d), at(lo + 3 * d), v0, v1, v2);   // (past `hi`: more than idx as well)
-        lo += ((v0 <= idx ? 1 : 0) + (v1 <= idx ? 1 : 0) + (v2 <= idx ? 1 : 0)) * d;
-        if (hi > lo + d) hi = lo + d;
-      }
-      // the whole record in one load, then the expert's first row (and first scale row) through the scalar cache as
-      // well: a vector load here waits its turn behind the weight streams of the whole chip
-      const v4i rec = sload4(ws, ws_rec(lo) * 4);
-      rec_first = __builtin_amdgcn_readfirstlane(light ? rec[kRecItem] : rec[kRecBlock]);
-      word = __builtin_amdgcn_readfirstlane(rec[kRecExpert]);
-      M = __builtin_amdgcn_readfirstlane(rec[kRecRows]);
-      erow = sload(g.expert_offsets, rec_expert(word) * 4);
-      if constexpr (MX) ebso = sload(g.blockscale_offsets, rec_expert(word) * 4);
-    }
-    const int e = rec_expert(word), first_kb = rec_first_kb(word);
-    const int local = idx - rec_first;
-    TileCoord t;
-    bool past = false;
-    int cols = 1;
-    if (light) {
-      t = sched_decode_light(local, M, g.policy, half);
-      if constexpr (!FUSE) {
-        const int tiles = sched_strip_tiles(have, have_end, lsplit, local, g.n, half);
-        if (tiles > 1) cols = tiles;
-        if (half == 0 && tiles > 0) {   // both halves: one whole tile
-          t.nt = 4;
-          half = -2;
-        }
-      }
-      have += half == -2 ? 2 * cols : cols;
-    } else if (!sched_decode_heavy(local, have++ % kBlkTiles, M, g.n, g.policy, &t, &past)) {
-      // The rest of the block's tickets are no tiles either: move the queue on to its next block, so that they are not drawn
-      // one by one (a block of 6 x 4 tiles has eight of them, one of 1 x 5 twenty-seven, and each costs a draw and a look-up, 2 to
-      // 3 us): 31 experts x 81 rows, 1280 x 768 24.1 -> 22.0 us, 45 experts, 3062 rows, 1024 x 2304 37.4 -> 35.3, MXFP8 MLP of 819
-      // tokens, 64 experts 196.7 -> 187.
-      const int next = sched_next_block(have - 1, first.heavy_base);   // (`have` is one on)
-      if (past && next > 0 && threadIdx.x == 0) atomicMax(&ws[ws_xcd_counter(xq)], next);
-      __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
-      continue;
-    }
+    if (!uniform(tile.mt) && !next_tile(g, tile)) break;
     // (wave-uniform by construction; said again so that the copies' base pointers stay in scalar registers)
-    t.mt = __builtin_amdgcn_readfirstlane(t.mt);
-    t.nt = __builtin_amdgcn_readfirstlane(t.nt);
-    t.m0 = __builtin_amdgcn_readfirstlane(t.m0);
-    t.n0 = __builtin_amdgcn_readfirstlane(t.n0);
-    if (t.n0 >= g.n) {   // second half of a last column tile that is 128 columns wide
-      __syncthreads();
-      continue;
-    }
+    const Tile t = {uniform(tile.mt), uniform(tile.nt), uniform(tile.cols), uniform(tile.m0), uniform(tile.n0), 0, 0, 0, 0, 0};
+    const int e = rec_expert(uniform(tile.expert)), first_kb = rec_first_kb(uniform(tile.expert)), M = uniform(tile.rows);
+    const int erow = uniform(tile.row), ebso = MX ? uniform(tile.scale_row) : 0, cols = t.cols;
+    tile.mt = 0;
     // Tile heights (MT * 16 rows): 8 and 12 are the tall tiles with the hand-scheduled K block, 1, 2 and 4 the short
     // ones, also as 128-column halves.  The host refuses a policy that asks for any other height (launch_gemm), so
     // every ticket finds its tile function here.
@@ -1655,9 +1788,9 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   // The last workgroup to leave zeroes the hand-out counters (nobody draws any more: every workgroup counts itself
   // out after its last draw), so a workspace that held zero counters before the launch holds them again after it.  A launch
   // of first tickets only has drawn from none.
-  if (undrawn != kAllQueues && threadIdx.x == 0) {
+  if (hand.undrawn != kAllQueues && threadIdx.x == 0) {
     const int left = atomicAdd(&ws[kWsExitCounter], 1);
-    if (left == (int)gridDim.x - 1) {
+    if (left == args.workgroups - 1) {
 #pragma unroll
       for (int x = 0; x < kXcds; x++) __hip_atomic_store(&ws[ws_xcd_counter(x)], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&ws[kWsLightCounter], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
