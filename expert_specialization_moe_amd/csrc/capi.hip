@@ -116,7 +116,7 @@ const Knobs& knobs() {
 constexpr int kNarrowTail = 128;
 
 // Default schedule policy: the one the host mirrors describe.  kind: bit 0 mxfp8, bit 1 a fused SwiGLU epilogue.
-esmoe::SchedPolicy default_policy(int force_bm, int kind) {
+esmoe::SchedPolicy default_policy(int force_bm, int kind, int k) {
   const int mx = kind & 1;
   esmoe::SchedPolicy p;
   p.force_mt = force_bm / 16;
@@ -129,17 +129,19 @@ esmoe::SchedPolicy default_policy(int force_bm, int kind) {
   p.light_share = -1;
   // the fused epilogues quantise blocks that need a whole 256-row tile, and a forced height has no light items
   p.narrow_tail = (force_bm == 0 && !(kind & 2)) ? kNarrowTail : 0;
+  p.runs = force_bm == 0 && esmoe::sched_use_runs(k);
   return p;
 }
 
 // Policy of a launch: the default with the environment's overrides.
-esmoe::SchedPolicy launch_policy(int force_bm, int kind) {
-  esmoe::SchedPolicy p = default_policy(force_bm, kind);
-  const Knobs& k = knobs();
-  p.big_mt = (kind & 1) ? k.big_mt_mx : k.big_mt_fp8;
-  if (p.narrow_tail && k.narrow_tail >= 0) p.narrow_tail = k.narrow_tail;
-  p.order = k.order;
-  p.light_share = k.light_share;
+esmoe::SchedPolicy launch_policy(int force_bm, int kind, int k) {
+  esmoe::SchedPolicy p = default_policy(force_bm, kind, k);
+  const Knobs& v = knobs();
+  p.big_mt = (kind & 1) ? v.big_mt_mx : v.big_mt_fp8;
+  if (p.big_mt != 12) p.runs = 0;   // (which have 192-row tiles)
+  if (p.narrow_tail && v.narrow_tail >= 0) p.narrow_tail = v.narrow_tail;
+  p.order = v.order;
+  p.light_share = v.light_share;
   return p;
 }
 
@@ -225,7 +227,7 @@ int launch_gemm(esmoe::GemmArgs& g, int mx, int force_bm, void* stream, bool own
   }
   // One launch when the counters are known to be zero and a workgroup can rank the experts with a thread each.
   // (The kernel's own schedule knows the orders by rows, not the index order.)
-  g.policy = launch_policy(force_bm, (mx ? 1 : 0) | (g.q_out ? 2 : 0));
+  g.policy = launch_policy(force_bm, (mx ? 1 : 0) | (g.q_out ? 2 : 0), g.k);
   g.self_schedule = owned && knobs().self_schedule && g.num_experts <= esmoe::kSelfScheduleMaxExperts && g.policy.order != 1;
   // every height the schedule can hand out must be one the kernel has a tile function for (it has no other case)
   if ((g.policy.force_mt && !esmoe::sched_valid_mt(g.policy.force_mt)) || (g.policy.big_mt != 8 && g.policy.big_mt != 12))
@@ -543,7 +545,7 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
   g_err[0] = 0;
   if (!problem_sizes_host || !ws_host || num_experts < 1 || num_experts > ESMOE_MAX_EXPERTS || n <= 0 || n % 128)
     return fail(ESMOE_ERR_INVALID_ARGUMENT, "bad argument to esmoe_host_schedule");
-  const esmoe::SchedPolicy p = default_policy(force_bm, kind);
+  const esmoe::SchedPolicy p = default_policy(force_bm, kind, problem_sizes_host[2]);
   auto rows_of = [&](int e) { return problem_sizes_host[e * 3] < 0 ? 0 : problem_sizes_host[e * 3]; };
   // same ranking as the device schedule kernel: by sched_order_key, ties by expert index
   for (int e = 0; e < num_experts; e++) {
@@ -565,11 +567,12 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
     const int m = ws_host[esmoe::ws_rec(pos) + esmoe::kRecRows];
     ws_host[esmoe::ws_rec(pos) + esmoe::kRecBlock] = blocks;
     ws_host[esmoe::ws_rec(pos) + esmoe::kRecItem] = items;
-    blocks += esmoe::sched_heavy_blocks(m, n, p);
+    const bool heavy = esmoe::sched_is_heavy(m, p);
+    blocks += !heavy ? 0 : p.runs ? esmoe::sched_heavy_tiles(m, n) : esmoe::sched_heavy_blocks(m, n, p);
     items += esmoe::sched_light_items(m, n, p);
-    heavy_cost += esmoe::sched_heavy_cost(m, n, p);
+    heavy_cost += !heavy ? 0.f : p.runs ? esmoe::sched_run_cost(m, n) : esmoe::sched_heavy_cost(m, n, p);
     light_cost += esmoe::sched_light_cost(m, n, p);
-    const int log = esmoe::sched_is_heavy(m, p) ? esmoe::sched_log2_ceil(esmoe::sched_block_tiles(m, n, p)) : 0;
+    const int log = heavy ? esmoe::sched_log2_ceil(esmoe::sched_block_tiles(m, n, p)) : 0;
     if (log > block_log) block_log = log;
   }
   int32_t* last = ws_host + esmoe::ws_rec(num_experts);
@@ -577,9 +580,11 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
   last[esmoe::kRecItem] = items;
   last[esmoe::kRecExpert] = -1;
   last[esmoe::kRecRows] = 0;
-  ws_host[esmoe::kWsLightShare] = esmoe::sched_light_share(heavy_cost, light_cost, p);
-  ws_host[esmoe::kWsHeavyBlocks] = blocks;
-  ws_host[esmoe::kWsBlockLog] = block_log;
+  ws_host[esmoe::kWsLightShare] = esmoe::sched_light_share(heavy_cost, light_cost, p.runs ? blocks : 0, p);
+  const int run = p.runs ? esmoe::sched_run_tiles(blocks) : 0;
+  ws_host[esmoe::kWsRun] = run;
+  ws_host[esmoe::kWsHeavyBlocks] = run ? (blocks + esmoe::kBlkTiles - 1) / esmoe::kBlkTiles : blocks;
+  ws_host[esmoe::kWsBlockLog] = run ? esmoe::kBlkLog : block_log;
   const int split = esmoe::sched_light_split(items, p);
   ws_host[esmoe::kWsLightSplit] = split;
   ws_host[esmoe::kWsLightTotal] = split + 2 * (items - split);
@@ -606,15 +611,19 @@ int esmoe_host_decode_heavy(const int32_t* problem_sizes_host, const int32_t* ws
   g_err[0] = 0;
   if (!problem_sizes_host || !ws_host || !out5 || xcd < 0 || xcd >= esmoe::kXcds || ticket < 0)
     return fail(ESMOE_ERR_INVALID_ARGUMENT, "bad argument to esmoe_host_decode_heavy");
-  const esmoe::SchedPolicy p = default_policy(force_bm, kind);
-  const int blk = esmoe::sched_ticket_block(xcd, ticket);
-  if (blk >= ws_host[esmoe::kWsHeavyBlocks]) return 2;   // this XCD's queue is exhausted
-  const int pos = host_position(ws_host, num_experts, esmoe::kRecBlock, blk);
+  const esmoe::SchedPolicy p = default_policy(force_bm, kind, problem_sizes_host[2]);
+  const int run = ws_host[esmoe::kWsRun];
+  const int tickets = run ? esmoe::sched_run_tickets(xcd, ws_host[esmoe::ws_rec(num_experts) + esmoe::kRecBlock], run)
+                          : esmoe::sched_queue_tickets(xcd, ws_host[esmoe::kWsHeavyBlocks]);
+  if (ticket >= tickets) return 2;   // this XCD's queue is exhausted
+  const int unit = run ? esmoe::sched_run_tile(xcd, ticket, run) : esmoe::sched_ticket_block(xcd, ticket);
+  const int pos = host_position(ws_host, num_experts, esmoe::kRecBlock, unit);
   if (pos < 0) return fail(ESMOE_ERR_INVALID_ARGUMENT, "workspace does not hold a schedule");
   const int32_t* rec = ws_host + esmoe::ws_rec(pos);
   esmoe::TileCoord t;
   bool past = false;
-  if (!esmoe::sched_decode_heavy(blk - rec[esmoe::kRecBlock], ticket % esmoe::kBlkTiles, rec[esmoe::kRecRows], n, p, &t, &past))
+  if (run) t = esmoe::sched_decode_run(unit - rec[esmoe::kRecBlock], rec[esmoe::kRecRows], n);
+  else if (!esmoe::sched_decode_heavy(unit - rec[esmoe::kRecBlock], ticket % esmoe::kBlkTiles, rec[esmoe::kRecRows], n, p, &t, &past))
     return 1;   // ticket outside the expert's tile grid: skipped
   fill_out5(out5, esmoe::rec_expert(rec[esmoe::kRecExpert]), t);
   return 0;
@@ -624,7 +633,7 @@ int esmoe_host_decode_light(const int32_t* problem_sizes_host, const int32_t* ws
                             int force_bm, int kind, int item, int32_t* out5) {
   g_err[0] = 0;
   if (!problem_sizes_host || !ws_host || !out5) return fail(ESMOE_ERR_INVALID_ARGUMENT, "null pointer");
-  const esmoe::SchedPolicy p = default_policy(force_bm, kind);
+  const esmoe::SchedPolicy p = default_policy(force_bm, kind, problem_sizes_host[2]);
   if (item < 0 || item >= ws_host[esmoe::kWsLightTotal]) return fail(ESMOE_ERR_INVALID_ARGUMENT, "item out of range");
   int half = -1;
   const int idx = esmoe::sched_light_item_of_ticket(item, ws_host[esmoe::kWsLightSplit], &half);

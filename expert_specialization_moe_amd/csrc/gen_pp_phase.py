@@ -1,6 +1,7 @@
-"""Writes pp_phase.h: one K block of a tall fp8-blockwise tile as ONE inline-asm statement.
+"""Writes pp_phase.h and pp_phase_odd.h: one K block of a tall tile as ONE inline-asm statement.
 
-    python gen_pp_phase.py > pp_phase.h
+    python gen_pp_phase.py > pp_phase.h             # 128- and 192-row tiles: 4 and 6 row tiles of 16 a wavefront
+    python gen_pp_phase.py odd > pp_phase_odd.h     # 96- and 160-row tiles: 3 and 5
 
 The eight wavefronts of a tile form two groups of four (one wavefront of each group per SIMD); group 0 owns the upper
 half of the tile's token rows, group 1 the lower half, and every wavefront owns 64 of the 256 weight rows.  The groups
@@ -38,6 +39,7 @@ promotions follow the barrier; a fragment buffer is overwritten by a read that i
 the last one that used it, and LDS data returns much later than an MFMA reads its operands; s_nop 0 separates
 a write of m0 from the copy that uses it.
 """
+import sys
 
 NT = 4
 MATRIX_PRIO = 3   # wave priority during the matrix phase (the memory phase runs at 0): where both wavefronts of a SIMD
@@ -69,7 +71,8 @@ class Plan:
         self.sbu = self.sb + 1
         self.scu = (self.sa - mtw) // 2 * 2 if fuse else None    # fused form: products sa * sb_up of the up half
         self.lowest = self.scu if fuse else self.sa
-        self.ntc = mtw // 2                               # token copies per wavefront and K block
+        self.ntc = (mtw + 1) // 2                         # token copies per wavefront and K block (odd mtw: the last
+                                                          # wavefront of the group repeats some of its neighbour's)
 
     def clobbers(self):
         return [f'"v{i}"' for i in range(self.lowest, 256)] + ['"memory"', '"m0"', '"scc"', '"vcc"']
@@ -237,7 +240,7 @@ class MxPlan:
         self.sfw = 196                      # 4 weight-row scale registers
         self.sfa = 196 - mtw - (mtw % 2)    # mtw token-row scale registers
         self.lowest = self.sfa
-        self.ntc = mtw // 2
+        self.ntc = (mtw + 1) // 2
 
     def clobbers(self):
         return [f'"v{i}"' for i in range(self.lowest, 256)] + ['"memory"', '"m0"', '"scc"', '"vcc"']
@@ -333,9 +336,11 @@ def mx_matrix_phase(p):
             b = p.a[(mt + 2) % 3]
             L.append(f"ds_read_b128 {regs(b, 4)}, %[al] offset:{(mt + 2) * 2048}")
             L.append(f"ds_read_b128 {regs(b + 4, 4)}, %[ah] offset:{(mt + 2) * 2048}")
-        # one group of bookkeeping behind each of the first MFMAs; the token-slot group once al and ah are free
-        if j >= 1 and atoms:
-            L += atoms.pop(0)
+        # one group of bookkeeping behind each of the first MFMAs (two where there are few of these); the token-slot group
+        # once al and ah are free
+        for _ in range(1 if p.mtw > 3 else 2):
+            if j >= 1 and atoms:
+                L += atoms.pop(0)
         if j > last_roll and not atoms and late:
             L += late.pop(0)
     assert not atoms and not late, "more bookkeeping than MFMAs"
@@ -362,10 +367,10 @@ def emit_mx(name, mtw, fuse=False):
     print(f"#define {name}_LOWEST_FIXED_VGPR {p.lowest}")
 
 
-def main():
+def main(argv):
     print("// Generated by gen_pp_phase.py; do not edit.")
     print("#pragma once")
-    for mtw in (4, 6):
+    for mtw in (3, 5) if argv == ["odd"] else (4, 6):
         emit(f"ESMOE_PP{mtw * 2}", mtw, False)
         emit(f"ESMOE_PP{mtw * 2}F", mtw, True)
         emit_mx(f"ESMOE_PPX{mtw * 2}", mtw)
@@ -373,4 +378,4 @@ def main():
 
 
 if __name__ == "__main__":
-    main()
+    main(sys.argv[1:])

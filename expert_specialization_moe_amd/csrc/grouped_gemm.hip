@@ -3,7 +3,7 @@
 // One launch serves every expert.  Every workgroup (self_schedule), or a one-workgroup schedule kernel in front, turns
 // problem_sizes into a list of workgroup tiles (schedule.h); persistent workgroups of 8 wavefronts start on the tile that
 // their index gives and then pull tiles from atomic counters.  A tile is
-// (MT*16) token rows x 256 weight rows, MT in {1, 2, 4} (short tiles, gemm_tile) or {8, 12} (tall tiles,
+// (MT*16) token rows x 256 weight rows, MT in {1, 2, 4} (short tiles, gemm_tile) or {6, 8, 10, 12} (tall tiles,
 // gemm_tile_pp / gemm_tile_pp_mx); the short items that end a launch are handed out as two 128-column halves.
 //
 // Data movement.  Per 128-wide K block the workgroup copies the token rows, the weight rows and the block's scales
@@ -16,8 +16,8 @@
 //
 // Short tiles (up to 64 rows, bound by streaming their weight rows from HBM): a ring of up to 4 whole K-block
 // stages (148 KB), every wavefront owns all token rows and 32 weight rows, compiler-scheduled K loop.
-// Tall tiles (128 and 192 rows, bound by the matrix pipe and its feed): the K block is ONE hand-scheduled statement
-// (pp_phase.h, written by gen_pp_phase.py); two groups of four wavefronts, one of each per SIMD, run half a K block
+// Tall tiles (96 to 192 rows, bound by the matrix pipe and its feed): the K block is ONE hand-scheduled statement
+// (pp_phase.h, pp_phase_odd.h, written by gen_pp_phase.py); two groups of four wavefronts, one of each per SIMD, run half a K block
 // apart, so that one group's copies and fragment reads overlap the other group's MFMAs; the ring is split by
 // operand (three weight stages shared by both groups, two token stages per group).
 //
@@ -41,6 +41,7 @@
 #include "gemm_args.h"
 #include "mx_scale.h"
 #include "pp_phase.h"
+#include "pp_phase_odd.h"
 #include "schedule.h"
 #include "swiglu.h"
 #include "wave_scan.h"
@@ -287,7 +288,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, Acc& acc, int M
     return;
   }
   // epilogue: lane holds columns n0 + nw + nt*16 + 4*gq + [0,4) of token row m0 + mw + mt*16 + r
-  if constexpr (kWavesN == 4 && NTW == 4 && MTW >= 4) {
+  if constexpr (kWavesN == 4 && NTW == 4 && MTW >= 3) {
     // Tall tiles: a wavefront holds 64 columns of its rows, 128 bytes of output per row.  Stored straight from the MFMA
     // layout a store instruction writes 32-byte pieces of sixteen rows; passed through LDS (the ring is free, and each
     // wavefront reads back only what it wrote itself, so no barrier) it writes whole 128-byte lines of eight rows, in half
@@ -443,13 +444,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
   constexpr bool kStrip = !FUSE && BN == kBN;
   static_assert(kStripBlocks <= kMaxKB, "the weight block scales of a strip share the table of one tile");
   static_assert(!(FUSE && BN != kBN), "the fused epilogues need gate and up columns of a whole quantisation block in one tile");
-  static_assert(MT == 1 || MT == 2 || MT == 4, "short tiles; 128- and 192-row tiles are gemm_tile_pp / gemm_tile_pp_mx");
+  static_assert(MT == 1 || MT == 2 || MT == 4, "short tiles; 96- to 192-row tiles are gemm_tile_pp / gemm_tile_pp_mx");
   using G = TileGeom<MT, MX, BN>;
   constexpr int MTW = G::MTW, NTW = G::NTW, NBUF = G::kNBuf;
   int tid = threadIdx.x;
   // (hidden from the compiler, which otherwise forms this tile's addresses once in front of the hand-out loop and keeps them
-  // in vector registers that the tall tiles do not have: four were spilled to scratch.  The fused kernels have enough, and
-  // forming the addresses for every tile costs them 0.2 us a tile.)
+  // in vector registers that the tall tiles do not have: four were spilled to scratch.  The fused kernels have
+  // enough, and forming the addresses for every tile costs 0.2 us a tile: 128 experts, 16384 rows, 3072 x 4096 361.7 -> 359.0 us.)
   if constexpr (!FUSE) asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -826,7 +827,17 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
 }
 
 // ---------------------------------------------------------------------------------------------
-// Tall fp8-blockwise tiles (MT = 8 or 12, any K): the K block is one hand-scheduled statement
+// First 8-row block of a group's 2 * MTW blocks of token rows that wavefront wj of the group copies, (MTW + 1) / 2 blocks each: with an
+// odd MTW there are two blocks fewer than copies, and the last wavefront (the last two share, MTW = 3) copies blocks that its neighbour
+// copies as well, the same bytes to the same place.
+template <int MTW>
+__device__ __forceinline__ int first_token_block(int wj) {
+  constexpr int kCopies = (MTW + 1) / 2, kLast = 2 * MTW - kCopies;
+  return wj * kCopies < kLast ? wj * kCopies : kLast;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Tall fp8-blockwise tiles (MT = 6, 8, 10 or 12, any K): the K block is one hand-scheduled statement
 // (pp_phase.h, written by gen_pp_phase.py) and the ring is split by operand.
 //
 //   LDS   [0, 96 KB)            weight stages, 3 slots of 256 rows x 128 B, shared by the two groups
@@ -842,13 +853,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
 // kb is read in its memory and matrix phase of kb and refilled in its memory phase of kb + 1 with stage kb + 2.
 template <int MT, bool FUSE>
 __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first_kb, int erow, int M, int m0, int n0, uint8_t* lds) {
-  static_assert(MT == 8 || MT == 12, "hand-scheduled K block: 128- and 192-row tiles");
+  static_assert(MT == 6 || MT == 8 || MT == 10 || MT == 12, "hand-scheduled K block: 96- to 192-row tiles");
   constexpr int MTW = MT / 2, NTW = 4, BM = MT * 16, GR = MTW * 16;
-  constexpr int kTCopies = MTW / 2;                 // token copies per wavefront and K block (8 rows each)
+  constexpr int kTCopies = (MTW + 1) / 2;           // token copies per wavefront and K block (8 rows each)
   constexpr int kWSlot = kBN * 128, kTSlot = GR * 128, kSaBuf = 128 * 16;
   constexpr int kTBase = 3 * kWSlot, kSaBase = kTBase + 4 * kTSlot, kSbBase = kSaBase + 6 * kSaBuf;
   static_assert(kSbBase + 2 * kMaxKB * 4 <= kLdsBytes, "LDS map of the split ring");
-  const int tid = threadIdx.x;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (as in gemm_tile: nothing of it is kept across tiles)
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2, wj = wave & 3;
@@ -867,10 +879,11 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first
   constexpr int kBias = 3072;
   const int crow = lane >> 3, cslot = lane & 7;
   const int a_last = M - 1 - m0;
+  const int tblk = first_token_block<MTW>(wj);            // first 8-row block of the group's rows that this wavefront copies
   uint32_t va[kTCopies], vw[4], vs[4];
 #pragma unroll
   for (int i = 0; i < kTCopies; i++) {
-    const int lrow = (wj * kTCopies + i) * 8 + crow;      // row inside the group's token region
+    const int lrow = (tblk + i) * 8 + crow;               // row inside the group's token region
     const int trow = mw + lrow;
     const int grow = trow > a_last ? a_last : trow;
     va[i] = (uint32_t)grow * (uint32_t)K + (swz(lrow, cslot) << 4) + kBias - i * 1024;
@@ -900,7 +913,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first
   const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K + first_kb * 128 - kBias;
   const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K + first_kb * 128 - kBias;
   const uint8_t* sa_ptr = (const uint8_t*)(g.sa + (row_base + m0) * KB);
-  const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + wj * kTCopies * 1024;   // + slot * kTSlot
+  const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + tblk * 1024;            // + slot * kTSlot
   const uint32_t w_dst = lds0 + wave * 4096;                                        // + slot * kWSlot
   const uint32_t s_dst = lds0 + kSaBase + grp * 3 * kSaBuf + (wj & 1) * 64 * 16;    // + buffer * kSaBuf + q * 256
   auto issue_t = [&](int kb, int slot) { dma16xn<false>(t_dst + slot * kTSlot, a_ptr + (long)kb * 128, va); };
@@ -987,8 +1000,12 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first
   do {                                                                                                           \
     if constexpr (MT == 12 && FUSE) ESMOE_PP_STMT(ESMOE_PP12F);                                                  \
     else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PP12);                                                      \
-    else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PP8F);                                                          \
-    else ESMOE_PP_STMT(ESMOE_PP8);                                                                               \
+    else if constexpr (MT == 10 && FUSE) ESMOE_PP_STMT(ESMOE_PP10F);                                             \
+    else if constexpr (MT == 10) ESMOE_PP_STMT(ESMOE_PP10);                                                      \
+    else if constexpr (MT == 8 && FUSE) ESMOE_PP_STMT(ESMOE_PP8F);                                               \
+    else if constexpr (MT == 8) ESMOE_PP_STMT(ESMOE_PP8);                                                        \
+    else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PP6F);                                                          \
+    else ESMOE_PP_STMT(ESMOE_PP6);                                                                               \
   } while (0)
       ESMOE_PP_K_BLOCK();
       // the piece offsets rotate with q; the chunk buffer advances every fourth K block
@@ -1043,7 +1060,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first
 }
 
 // ---------------------------------------------------------------------------------------------
-// Tall mxfp8 tiles (MT = 8 or 12): the same two-group schedule and split ring as gemm_tile_pp with the scaled MFMA.
+// Tall mxfp8 tiles (MT = 6, 8, 10 or 12): the same two-group schedule and split ring as gemm_tile_pp with the scaled MFMA.
 //
 //   LDS   3 weight slots of 32 KB + 1 KB (the K block's two 512-byte scale tiles of the tile's 256 weight rows)
 //         4 token regions (group g, 2 slots) of GR rows x 128 B + 1 KB (the two scale tiles that hold the group's rows)
@@ -1052,13 +1069,14 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmArgs& g, int e, int first
 // its row from the row's position inside the two tiles that were fetched for its group.
 template <int MT, bool FUSE>
 __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int first_kb, int erow, int ebso, int M, int m0, int n0, uint8_t* lds) {
-  static_assert(MT == 8 || MT == 12, "hand-scheduled K block: 128- and 192-row tiles");
+  static_assert(MT == 6 || MT == 8 || MT == 10 || MT == 12, "hand-scheduled K block: 96- to 192-row tiles");
   constexpr int MTW = MT / 2, NTW = 4, BM = MT * 16, GR = MTW * 16;
-  constexpr int kTCopies = MTW / 2;
+  constexpr int kTCopies = (MTW + 1) / 2;
   constexpr int kWSlot = kBN * 128 + 1024, kTSlot = GR * 128 + 1024;
   constexpr int kTBase = 3 * kWSlot, kSpare = kTBase + 4 * kTSlot;
   static_assert(kSpare + 1024 <= kLdsBytes, "LDS map of the split ring");
-  const int tid = threadIdx.x;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (as in gemm_tile: nothing of it is kept across tiles)
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2, wj = wave & 3;
@@ -1073,10 +1091,11 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int fi
   constexpr int kBias = 3072;
   const int crow = lane >> 3, cslot = lane & 7;
   const int a_last = M - 1 - m0;
+  const int tblk = first_token_block<MTW>(wj);
   uint32_t va[kTCopies], vw[4];
 #pragma unroll
   for (int i = 0; i < kTCopies; i++) {
-    const int lrow = (wj * kTCopies + i) * 8 + crow;
+    const int lrow = (tblk + i) * 8 + crow;
     const int trow = mw + lrow;
     const int grow = trow > a_last ? a_last : trow;
     va[i] = (uint32_t)grow * (uint32_t)K + (swz(lrow, cslot) << 4) + kBias - i * 1024;
@@ -1097,7 +1116,7 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int fi
   // (position 0 of the expert's K order, see k_loop of gemm_tile_pp)
   const uint8_t* a_ptr = (const uint8_t*)g.a + (row_base + m0) * K + first_kb * 128 - kBias;
   const uint8_t* w_ptr = (const uint8_t*)g.b + ((long)e * N + (FUSE ? 0 : n0)) * K + first_kb * 128 - kBias;
-  const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + wj * kTCopies * 1024;   // + slot * kTSlot
+  const uint32_t t_dst = lds0 + kTBase + grp * 2 * kTSlot + tblk * 1024;            // + slot * kTSlot
   const uint32_t w_dst = lds0 + wave * 4096;                                        // + slot * kWSlot
   // scale copies, one per wavefront and K block: wavefront 0 the weight scale tiles (with the weight stage),
   // wavefronts 1 and 5 their group's token scale tiles (with the token stage), the others one line into the spare
@@ -1204,8 +1223,12 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int fi
       do {
       if constexpr (MT == 12 && FUSE) ESMOE_PP_STMT(ESMOE_PPX12F);
       else if constexpr (MT == 12) ESMOE_PP_STMT(ESMOE_PPX12);
-      else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PPX8F);
-      else ESMOE_PP_STMT(ESMOE_PPX8);
+      else if constexpr (MT == 10 && FUSE) ESMOE_PP_STMT(ESMOE_PPX10F);
+      else if constexpr (MT == 10) ESMOE_PP_STMT(ESMOE_PPX10);
+      else if constexpr (MT == 8 && FUSE) ESMOE_PP_STMT(ESMOE_PPX8F);
+      else if constexpr (MT == 8) ESMOE_PP_STMT(ESMOE_PPX8);
+      else if constexpr (FUSE) ESMOE_PP_STMT(ESMOE_PPX6F);
+      else ESMOE_PP_STMT(ESMOE_PPX6);
       } while (++kb < end);
     } while (kb < KB);
   };
@@ -1256,11 +1279,12 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
     }
     ws[ws_rec(pos) + kRecExpert] = rec_expert_word(e, expert_k_start(sb, sfb, e, n, k));
     ws[ws_rec(pos) + kRecRows] = m;
-    s_blocks[pos] = sched_heavy_blocks(m, n, policy);
+    const bool heavy = sched_is_heavy(m, policy);
+    s_blocks[pos] = !heavy ? 0 : policy.runs ? sched_heavy_tiles(m, n) : sched_heavy_blocks(m, n, policy);
     s_items[pos] = sched_light_items(m, n, policy);
-    s_cost[pos][0] = sched_heavy_cost(m, n, policy);
+    s_cost[pos][0] = !heavy ? 0.f : policy.runs ? sched_run_cost(m, n) : sched_heavy_cost(m, n, policy);
     s_cost[pos][1] = sched_light_cost(m, n, policy);
-    if (sched_is_heavy(m, policy)) tiles = sched_block_tiles(m, n, policy);
+    if (heavy && !policy.runs) tiles = sched_block_tiles(m, n, policy);
   }
   int block_log = 0;   // (over the wavefront)
 #pragma unroll
@@ -1283,7 +1307,9 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
       ws[ws_rec(num_experts) + kRecItem] = items;
       ws[ws_rec(num_experts) + kRecExpert] = -1;
       ws[ws_rec(num_experts) + kRecRows] = 0;
-      ws[kWsHeavyBlocks] = blocks;
+      const int run = policy.runs ? sched_run_tiles(blocks) : 0;
+      ws[kWsRun] = run;
+      ws[kWsHeavyBlocks] = run ? (blocks + kBlkTiles - 1) / kBlkTiles : blocks;
       const int split = sched_light_split(items, policy);
       ws[kWsLightSplit] = split;
       ws[kWsLightTotal] = split + 2 * (items - split);
@@ -1294,8 +1320,8 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
         heavy_cost += s_cost[j][0];
         light_cost += s_cost[j][1];
       }
-      ws[kWsLightShare] = sched_light_share(heavy_cost, light_cost, policy);
-      ws[kWsBlockLog] = s_block_log;
+      ws[kWsLightShare] = sched_light_share(heavy_cost, light_cost, run ? blocks : 0, policy);
+      ws[kWsBlockLog] = run ? kBlkLog : s_block_log;
     }
     if (pos < kXcds) ws[ws_xcd_counter(pos)] = 0;
   }
@@ -1312,42 +1338,53 @@ struct Tile {
 };
 
 // What a workgroup knows when the schedule is done: the queues, and the tickets in hand, [have, have_end).
+struct LightHand {
+  int total, split, base, unused;         // light tickets, the first that is a half item, the first that comes from the counter
+};
+struct HeavyHand {
+  int blocks, run, tiles, base;           // heavy blocks, tiles of a run (0: the queues hold blocks), heavy tiles where they hold runs,
+};                                        // the first ticket of a queue that comes from its counter
 struct Hand {
-  int hblocks, ltotal, lsplit;   // heavy blocks, light tickets, the first of these that is a half item
-  int heavy_base, light_base;    // first tickets that come from the counters
-  int undrawn;                   // queues that hold nothing but first tickets (sched_undrawn_queues)
+  LightHand light;
+  HeavyHand heavy;
+  int undrawn;                            // queues that hold nothing but first tickets (sched_undrawn_queues)
   int light_first, have, have_end, seen;
 };
+static_assert(sizeof(LightHand) == 16 && sizeof(HeavyHand) == 16, "one LDS read each");
+__device__ __forceinline__ int queue_tickets(const HeavyHand& h, int queue) {
+  return h.run ? sched_run_tickets(queue, h.tiles, h.run) : sched_queue_tickets(queue, h.blocks);
+}
+// `hunits`: heavy tiles where the queues hold runs, blocks otherwise.
 template <bool FUSE>
-__device__ __forceinline__ Hand first_hand(const GemmArgs& g, int hblocks, int block_log, int ltotal, int lsplit, int lshare) {
-  const int wg = (int)blockIdx.x;
+__device__ __forceinline__ Hand first_hand(const GemmArgs& g, int hunits, int run, int block_log, int ltotal, int lsplit, int lshare) {
+  const int wg = (int)blockIdx.x, htiles = run ? hunits : 0, hblocks = run ? (hunits + kBlkTiles - 1) / kBlkTiles : hunits;
   const SchedFirst f = sched_first_tickets(g.workgroups, hblocks, block_log, ltotal, lshare,
                                            sched_light_draw(ltotal, 0, g.workgroups, g.k >> 7, !FUSE));
   Hand h;
-  h.hblocks = hblocks;
-  h.ltotal = ltotal;
-  h.lsplit = lsplit;
-  h.heavy_base = f.heavy_base;
-  h.light_base = f.light_base;
+  h.light = LightHand{ltotal, lsplit, f.light_base, 0};
+  h.heavy = HeavyHand{hblocks, run, htiles, f.heavy_base};
   h.undrawn = sched_undrawn_queues(hblocks, ltotal, f);
+  if (run) {   // (a lane for every queue)
+    const int x = threadIdx.x & (kXcds - 1);
+    h.undrawn = (h.undrawn & 1 << kXcds) | (int)(__ballot(sched_run_tickets(x, htiles, run) <= f.heavy_base) & ((1 << kXcds) - 1));
+  }
   h.light_first = sched_first_is_light(wg, f);
   h.have = sched_first_ticket(wg, f);
   h.have_end = h.have + (h.light_first ? f.light_draw : 1);
   h.seen = sched_first_seen(wg, f);
-  const int total = h.light_first ? ltotal : sched_queue_tickets(sched_home_queue(wg), hblocks);
+  const int total = h.light_first ? ltotal : queue_tickets(h.heavy, sched_home_queue(wg));
   if (h.have_end > total) h.have_end = total;
   if (h.have > h.have_end) h.have = h.have_end;
   return h;
 }
-// Light item or heavy block of a ticket (half: of a light one, sched_light_item_of_ticket).
-__device__ __forceinline__ int ticket_index(bool light, int queue, int ticket, int lsplit, int* half) {
-  *half = -1;
-  return light ? sched_light_item_of_ticket(ticket, lsplit, half) : sched_ticket_block(queue, ticket);
+// Heavy tile or block of a ticket.
+__device__ __forceinline__ int heavy_index(int queue, int ticket, const HeavyHand& h) {
+  return h.run ? sched_run_tile(queue, ticket, h.run) : sched_ticket_block(queue, ticket);
 }
-// Tile of ticket `have`, item or block `local` of its expert; moves `have` on by the tickets that it takes.  mt = 0: it is no tile
+// Tile of ticket `have`, item, tile or block `local` of its expert; moves `have` on by the tickets that it takes.  mt = 0: it is no tile
 // (`past`: nor are those behind it in its block).
 template <bool FUSE>
-__device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int& have, int have_end, int lsplit, int local, int half, int rows, bool* past) {
+__device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int split, int run, int& have, int have_end, int local, int half, int rows, bool* past) {
   TileCoord t;
   Tile d;
   *past = false;
@@ -1356,7 +1393,7 @@ __device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int& ha
   if (light) {
     t = sched_decode_light(local, rows, g.policy, half);
     if constexpr (!FUSE) {
-      const int tiles = sched_strip_tiles(have, have_end, lsplit, local, g.n, half);
+      const int tiles = sched_strip_tiles(have, have_end, split, local, g.n, half);
       if (tiles > 1) d.cols = tiles;
       if (half == 0 && tiles > 0) {   // both halves: one whole tile
         t.nt = 4;
@@ -1365,6 +1402,9 @@ __device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int& ha
     }
     have += half == -2 ? 2 * d.cols : d.cols;
     if (t.n0 >= g.n) t.mt = 0;   // second half of a last column tile that is 128 columns wide
+  } else if (run) {
+    t = sched_decode_run(local, rows, g.n);
+    have++;
   } else if (!sched_decode_heavy(local, have++ % kBlkTiles, rows, g.n, g.policy, &t, past)) {
     t.mt = 0;
   }
@@ -1392,17 +1432,17 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting
 // instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us; half as many divisions and a four-way search of the records:
 // 75.2 -> 74.7 (with both kinds of experts), an expert MLP of 1003 tokens in MXFP8 377.5 -> 376.1.
-// The workgroup's first tile, by the thread of the expert that the ticket belongs to (items or blocks [before, before + mine)).
+// The workgroup's first tile, by the thread of the expert that the ticket belongs to (items, tiles or blocks [before, before + mine)).
 template <bool FUSE>
 __device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool light, bool heavy, int before, int mine, int rows, int word, int row,
                                            int scale_row, Tile* first) {
   if (h.have == h.have_end) return;
-  int half;
-  const int idx = ticket_index(h.light_first, sched_home_queue((int)blockIdx.x), h.have, h.lsplit, &half);
+  int half = -1;
+  const int idx = h.light_first ? sched_light_item_of_ticket(h.have, h.light.split, &half) : heavy_index(sched_home_queue((int)blockIdx.x), h.have, h.heavy);
   if ((h.light_first ? light : heavy) && idx >= before && idx < before + mine) {
     bool past;
     int have = h.have;
-    Tile d = take_tile<FUSE>(g, h.light_first, have, h.have_end, h.lsplit, idx - before, half, rows, &past);
+    Tile d = take_tile<FUSE>(g, h.light_first, h.light.split, h.heavy.run, have, h.have_end, idx - before, half, rows, &past);
     d.expert = word;
     d.row = row;
     d.scale_row = scale_row;
@@ -1457,7 +1497,7 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
     b = next_b;
   }
   const int ntl = sched_ntiles(g.n, 4), items = num_light * ntl;
-  int before = 0, mine = 0, blocks = 0, block_log = 0, lshare = 0;
+  int before = 0, mine = 0, blocks = 0, run = 0, block_log = 0, lshare = 0;   // (blocks: tiles where the queues hold runs)
   if (light) {
     const int rank = pos - num_heavy;
     before = (rank < num_light ? rank : num_light) * ntl;
@@ -1465,9 +1505,14 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
   }
   if (num_heavy > 0) {
     int tiles = 0;
-    if (heavy) {
+    float cost = 0.f;
+    if (heavy && policy.runs) {
+      mine = sched_heavy_tiles(m, g.n);
+      cost = sched_run_cost(m, g.n);
+    } else if (heavy) {
       mine = sched_heavy_blocks(m, g.n, policy);
       tiles = sched_block_tiles(m, g.n, policy);
+      cost = sched_heavy_cost(m, g.n, policy);
     }
     // blocks in the order of the schedule, their prefix sums, and back (a lane of no heavy expert sends nothing on to the sums)
     const int placed = __builtin_amdgcn_ds_permute(pos * 4, heavy ? mine : 0);
@@ -1475,24 +1520,29 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
     blocks = __builtin_amdgcn_readlane(sum, 63);
     const int up_to = __builtin_amdgcn_ds_bpermute(pos * 4, sum);
     if (heavy) before = up_to - mine;
+    if (policy.runs) {
+      run = sched_run_tiles(blocks);
+      block_log = kBlkLog;
+    } else {
 #pragma unroll
-    for (int i = 0; i < kBlkLog; i++) block_log += __ballot(tiles > 1 << i) != 0;
+      for (int i = 0; i < kBlkLog; i++) block_log += __ballot(tiles > 1 << i) != 0;
+    }
     if (items > 0) {   // how many workgroups start on which kind, where a launch has both
-      const float hc = wave_sum_last(sched_heavy_cost(m, g.n, policy)), lc = wave_sum_last(light ? sched_light_cost(m, g.n, policy) : 0.f);
+      const float hc = wave_sum_last(cost), lc = wave_sum_last(light ? sched_light_cost(m, g.n, policy) : 0.f);
       lshare = sched_light_share(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hc), 63)),
-                                 __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lc), 63)), policy);
+                                 __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lc), 63)), run ? blocks : 0, policy);
     }
   }
   if (lane < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
   if (lane == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
-  Hand h = first_hand<FUSE>(g, blocks, block_log, ltotal, lsplit, lshare);
+  Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
   first_tile<FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
   if (lane == 0) *out = h;
 }
 
 template <bool MX, bool FUSE>
-__device__ __forceinline__ Hand self_schedule(const GemmArgs& g, uint8_t* lds, Tile* first) {
+__device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, Tile* first) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
   constexpr int kLightRows = 64, kHistStride = kLightRows + 4;
   int* s_hist = (int*)lds;                              // [kWaves][kHistStride]: experts of a wavefront by rows (0 .. 64)
@@ -1559,7 +1609,10 @@ __device__ __forceinline__ Hand self_schedule(const GemmArgs& g, uint8_t* lds, T
     if (t >= num_heavy && t < ((num_heavy + 3) & ~3)) s_key[t] = 0x7fffffff;
     int hb = 0, tiles = 0;
     float heavy_cost = 0.f, light_cost = 0.f;
-    if (heavy) {
+    if (heavy && policy.runs) {
+      hb = sched_heavy_tiles(m, g.n);
+      heavy_cost = sched_run_cost(m, g.n);
+    } else if (heavy) {
       hb = sched_heavy_blocks(m, g.n, policy);
       tiles = sched_block_tiles(m, g.n, policy);
       heavy_cost = sched_heavy_cost(m, g.n, policy);
@@ -1614,17 +1667,21 @@ __device__ __forceinline__ Hand self_schedule(const GemmArgs& g, uint8_t* lds, T
     blocks = __builtin_amdgcn_readfirstlane(blocks);
     block_log = __builtin_amdgcn_readfirstlane(block_log);
     // how many workgroups start on which kind, where a launch has both
-    if (items > 0) lshare = __builtin_amdgcn_readfirstlane(sched_light_share(hc, lc, policy));
+    if (items > 0) lshare = __builtin_amdgcn_readfirstlane(sched_light_share(hc, lc, policy.runs ? blocks : 0, policy));
+  }
+  int run = 0;
+  if (policy.runs && blocks > 0) {
+    run = sched_run_tiles(blocks);
+    block_log = kBlkLog;
   }
   // the expert's record, at its schedule position; record E closes the prefix sums
   if (t < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
   if (t == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
   const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
-  Hand h = first_hand<FUSE>(g, blocks, block_log, ltotal, lsplit, lshare);
+  Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
   first_tile<FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
-  __syncthreads();
-  return h;
+  if (t == 0) *out = h;
 }
 
 template <bool MX, bool FUSE>
@@ -1639,40 +1696,42 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   asm volatile("" ::"s"(args.a));
   // Of every 32 workgroups of an XCD the last `light_share` start on the light items, the others on the heavy tickets; either
   // kind moves on to the other when its own is exhausted.
-  Hand hand;
+  // (What the hand-out needs of the heavy queues stays in LDS between two tiles: in scalar registers it made the fused kernels spill.)
   Tile tile;
   tile.mt = 0;
   if (args.self_schedule) {
-    if (args.num_experts > 64) {
-      hand = self_schedule<MX, FUSE>(args, lds, &s_tile);
-    } else {
-      if (threadIdx.x < 64) wave_schedule<MX, FUSE>(args, lds, &s_hand, &s_tile);
-      __syncthreads();
-      const Hand h = s_hand;
-      hand = Hand{uniform(h.hblocks), uniform(h.ltotal), uniform(h.lsplit), uniform(h.heavy_base), uniform(h.light_base),
-                  uniform(h.undrawn), uniform(h.light_first), uniform(h.have), uniform(h.have_end), uniform(h.seen)};
-    }
+    if (args.num_experts > 64) self_schedule<MX, FUSE>(args, lds, &s_hand, &s_tile);
+    else if (threadIdx.x < 64) wave_schedule<MX, FUSE>(args, lds, &s_hand, &s_tile);
+    __syncthreads();
     tile = s_tile;
-    if (uniform(tile.mt)) hand.have += uniform(tile.taken);
   } else {
-    hand = first_hand<FUSE>(args, ws[kWsHeavyBlocks], ws[kWsBlockLog], ws[kWsLightTotal], ws[kWsLightSplit], ws[kWsLightShare]);
+    const Hand h = first_hand<FUSE>(args, ws[ws_rec(args.num_experts) + kRecBlock], ws[kWsRun], ws[kWsBlockLog], ws[kWsLightTotal], ws[kWsLightSplit], ws[kWsLightShare]);
+    if (threadIdx.x == 0) s_hand = h;
+    __syncthreads();
   }
+  bool light = uniform(s_hand.light_first) != 0;
   int phase = 0, q = 0;
   // Queues known to be exhausted (bits 0-7: the XCDs' heavy queues, bit 8: the light items).  When a draw comes back
   // past the end of its queue and the launch has heavy blocks on every XCD, one look at all nine counters marks every
   // queue that has run dry, so that a workgroup leaving its own queue does not spend an atomic round trip (about a
   // microsecond under load) on each empty one.
-  int dead = hand.undrawn;
+  int dead = uniform(s_hand.undrawn);
   // Tickets in hand, [have, have_end): at first those that go by the workgroup's index (sched_first_tickets), then what a
   // draw gave (light ones: sched_light_draw).  `xq`: their queue.
-  int have = hand.have, xq = sched_home_queue((int)blockIdx.x), have_end = hand.have_end, seen = hand.seen;
+  int have = uniform(s_hand.have) + (uniform(tile.mt) ? uniform(tile.taken) : 0), have_end = uniform(s_hand.have_end), seen = uniform(s_hand.seen);
+  int xq = sched_home_queue((int)blockIdx.x);
+  const LightHand lights{uniform(s_hand.light.total), uniform(s_hand.light.split), uniform(s_hand.light.base), 0};
   bool records_pending = args.self_schedule != 0;   // this workgroup's records may still be on their way to memory
   typedef const __attribute__((address_space(4))) GemmArgs* KernArgs;
   KernArgs kernargs = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
   // The next tile of this workgroup; false: there is none.
   auto next_tile = [&](const GemmArgs& g, Tile& d) -> bool {
     for (;;) {
-      const bool light = (phase == 0) == (hand.light_first != 0);
+      HeavyHand heavies{0, 0, 0, 0};
+      if (!light) {
+        const HeavyHand h = s_hand.heavy;
+        heavies = HeavyHand{uniform(h.blocks), uniform(h.run), uniform(h.tiles), uniform(h.base)};
+      }
       if (have == have_end) {
         if (dead == kAllQueues) return false;
         xq = sched_drawn_queue((int)blockIdx.x, q);
@@ -1680,28 +1739,32 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
           if (light || ++q == kXcds) {
             q = 0;
             if (++phase == 2) return false;
+            light = !light;
           }
           continue;
         }
-        const int draw = light ? sched_light_draw(hand.ltotal, seen, g.workgroups, g.k >> 7, !FUSE) : 1;
-        const int total = light ? hand.ltotal : sched_queue_tickets(xq, hand.hblocks);
+        const int draw = light ? sched_light_draw(lights.total, seen, g.workgroups, g.k >> 7, !FUSE) : 1;
+        const int total = light ? lights.total : queue_tickets(heavies, xq);
         if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
         __syncthreads();
-        const int ticket = (light ? hand.light_base : hand.heavy_base) + uniform(s_item);
+        const int ticket = (light ? lights.base : heavies.base) + uniform(s_item);
         if (ticket >= total) {   // this queue is exhausted: see which others are
           dead |= 1 << (light ? 8 : xq);
+          if (dead == kAllQueues) return false;
           __syncthreads();                        // s_item and s_counters are rewritten next
-          // (worth its round trip only when every XCD has a queue to try: the look itself reads the hot counter line)
-          if (hand.hblocks <= kXcds) continue;
+          // (worth its round trip only when every XCD has a queue to try, as with runs: the look itself reads the hot counter line)
+          const HeavyHand h = s_hand.heavy;
+          heavies = HeavyHand{uniform(h.blocks), uniform(h.run), uniform(h.tiles), uniform(h.base)};
+          if (!heavies.run && heavies.blocks <= kXcds) continue;
           if (threadIdx.x < kXcds + 1)
             s_counters[threadIdx.x] = __hip_atomic_load(threadIdx.x < kXcds ? &ws[ws_xcd_counter(threadIdx.x)] : &ws[kWsLightCounter],
                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __syncthreads();
 #pragma unroll
           for (int x = 0; x < kXcds; x++) {
-            if (hand.heavy_base + uniform(s_counters[x]) >= sched_queue_tickets(x, hand.hblocks)) dead |= 1 << x;
+            if (heavies.base + uniform(s_counters[x]) >= queue_tickets(heavies, x)) dead |= 1 << x;
           }
-          if (hand.light_base + uniform(s_counters[kXcds]) >= hand.ltotal) dead |= 256;
+          if (lights.base + uniform(s_counters[kXcds]) >= lights.total) dead |= 256;
           continue;
         }
         have = ticket;
@@ -1717,8 +1780,8 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       // the last one whose first item or block is not behind it, found by halving the prefix sums twice a step, with scalar loads.
       // The records are only read from here on, so they stay in the scalar cache, where a step costs a fraction of what a trip to L2
       // costs while the chip streams weights, and three loads as much as one.
-      int half;
-      const int idx = ticket_index(light, xq, have, hand.lsplit, &half), kind = light ? kRecItem : kRecBlock;
+      int half = -1;
+      const int idx = light ? sched_light_item_of_ticket(have, lights.split, &half) : heavy_index(xq, have, heavies), kind = light ? kRecItem : kRecBlock;
       int lo = 0, hi = g.num_experts;
       while (hi - lo > 1) {
         const int step = (hi - lo + 3) >> 2;
@@ -1733,7 +1796,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       const v4i rec = sload4(ws, ws_rec(lo) * 4);
       const int word = uniform(rec[kRecExpert]);
       bool past;
-      d = take_tile<FUSE>(g, light, have, have_end, hand.lsplit, idx - uniform(light ? rec[kRecItem] : rec[kRecBlock]), half,
+      d = take_tile<FUSE>(g, light, lights.split, heavies.run, have, have_end, idx - uniform(light ? rec[kRecItem] : rec[kRecBlock]), half,
                           uniform(rec[kRecRows]), &past);
       d.expert = word;
       if (d.mt) {
@@ -1746,7 +1809,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       // block, so that they are not drawn one by one (a block of 6 x 4 tiles has eight of them, one of 1 x 5 twenty-seven, and each
       // costs a draw and a look-up, 2 to 3 us): 31 experts x 81 rows, 1280 x 768 24.1 -> 22.0 us, 45 experts, 3062 rows, 1024 x 2304
       // 37.4 -> 35.3, MXFP8 MLP of 819 tokens, 64 experts 196.7 -> 187.
-      const int next = sched_next_block(have - 1, hand.heavy_base);
+      const int next = sched_next_block(have - 1, heavies.base);
       if (past && next > 0 && threadIdx.x == 0) atomicMax(&ws[ws_xcd_counter(xq)], next);
       __syncthreads();   // s_item is rewritten next: every wavefront must have read this ticket first
     }
@@ -1764,15 +1827,21 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     const int e = rec_expert(uniform(tile.expert)), first_kb = rec_first_kb(uniform(tile.expert)), M = uniform(tile.rows);
     const int erow = uniform(tile.row), ebso = MX ? uniform(tile.scale_row) : 0, cols = t.cols;
     tile.mt = 0;
-    // Tile heights (MT * 16 rows): 8 and 12 are the tall tiles with the hand-scheduled K block, 1, 2 and 4 the short
+    // Tile heights (MT * 16 rows): 6 to 12 are the tall tiles with the hand-scheduled K block, 1, 2 and 4 the short
     // ones, also as 128-column halves.  The host refuses a policy that asks for any other height (launch_gemm), so
     // every ticket finds its tile function here.
     if (t.mt == 12) {
       if constexpr (MX) gemm_tile_pp_mx<12, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
       else gemm_tile_pp<12, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
+    } else if (t.mt == 10) {
+      if constexpr (MX) gemm_tile_pp_mx<10, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
+      else gemm_tile_pp<10, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
     } else if (t.mt == 8) {
       if constexpr (MX) gemm_tile_pp_mx<8, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
       else gemm_tile_pp<8, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
+    } else if (t.mt == 6) {
+      if constexpr (MX) gemm_tile_pp_mx<6, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
+      else gemm_tile_pp<6, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
     } else if (!FUSE && t.nt == 2) {
       if constexpr (!FUSE) {
         if (t.mt == 1) gemm_tile<1, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
@@ -1788,7 +1857,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   // The last workgroup to leave zeroes the hand-out counters (nobody draws any more: every workgroup counts itself
   // out after its last draw), so a workspace that held zero counters before the launch holds them again after it.  A launch
   // of first tickets only has drawn from none.
-  if (hand.undrawn != kAllQueues && threadIdx.x == 0) {
+  if (threadIdx.x == 0 && s_hand.undrawn != kAllQueues) {
     const int left = atomicAdd(&ws[kWsExitCounter], 1);
     if (left == args.workgroups - 1) {
 #pragma unroll

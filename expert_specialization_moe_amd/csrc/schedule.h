@@ -5,8 +5,8 @@
 // (expert_specialization/csrc/cuda/es_fp8_blockwise_functor.cuh:121-256): instead
 // of routing whole experts to one of three differently tiled kernels, every
 // expert is cut into full "big" row tiles plus one remainder tile whose height is
-// the smallest menu entry that covers the leftover rows, and all tiles of all
-// experts feed one persistent kernel.
+// the smallest menu entry that covers the leftover rows (sched_cover_mt,
+// sched_last_mt), and all tiles of all experts feed one persistent kernel.
 //
 // The same functions compile for the device (hipcc) and for the host (plain C++),
 // so the index math is unit-tested on the CPU.
@@ -30,6 +30,7 @@ struct SchedPolicy {
                   // 2: most rows first for both kinds
   int light_share;  // workgroups (of every 32) that start on the light items; -1 = from the cost estimate
   int narrow_tail;  // the last so many light items are handed out as two 128-column halves each (0: none)
+  int runs;         // 1: the queues hold runs of tiles instead of blocks, and last row tiles come in steps of 32 rows (sched_use_runs)
 };
 
 struct TileCoord {
@@ -56,7 +57,7 @@ ESMOE_HD int sched_div(int a, int b) {
 #endif
 }
 
-// The tile heights the kernels are compiled for.
+// The tile heights that can be forced (the kernels also have 6 and 10: sched_last_mt).
 ESMOE_HD bool sched_valid_mt(int mt) { return mt == 1 || mt == 2 || mt == 4 || mt == 8 || mt == 12; }
 
 // Smallest tile height of the menu {1, 2, 4, 8, 12} (x16 rows) that covers `rows`, at most max_mt.
@@ -69,6 +70,12 @@ ESMOE_HD int sched_cover_mt(int rows, int max_mt) {
   if (need > 8) mt = 12;
   return mt < max_mt ? mt : max_mt;
 }
+
+// Height / 16 of the last row tile of a heavy expert, `rows` (1 .. 192) rows of it, where the queues hold runs: tall tiles in steps of 32
+// rows.  What lies past the expert's rows is copied, read from LDS and multiplied like the rest: 8192 rows, 32 experts, 4096 x 7168
+// (MXFP8) had 11 % of such rows with 128 and 192 alone and has 6 %, 297.6 -> 292.6 us, of 6579 rows (FP8) 266.6 -> 262.7.  Up to 64 rows a
+// short tile costs less than a tall one (K = 1536: 64 rows 15.3 us, 96 or 128 rows 17 us).
+ESMOE_HD int sched_last_mt(int rows) { return rows > 64 ? (rows + 31) >> 5 << 1 : sched_cover_mt(rows, 4); }
 
 // Every compiled shape is 256 columns wide (NT = 4 units of 64).
 ESMOE_HD int sched_nt_for(int, const SchedPolicy&) { return 4; }
@@ -110,6 +117,26 @@ ESMOE_HD int sched_order_key(int m, const SchedPolicy& p) {
 ESMOE_HD int sched_mtiles(int m, const SchedPolicy& p) {
   const int rows = (p.force_mt ? p.force_mt : p.big_mt) * 16;
   return sched_div(m + rows - 1, rows);
+}
+
+// ---- Runs --------------------------------------------------------------------------------
+// From K = 640 on the queues hold runs instead of blocks: all heavy tiles of the launch stand in one line, expert after expert, each
+// down its columns (of at most eight tiles), and queue x has the x-th, (x + 8)-th, ... run of 32 of them.  Every ticket is a tile: blocks
+// leave holes where they have fewer than 32 tiles, and a hole costs a draw and a look-up, 2 to 3 us.  32 tiles that stand together
+// are 4 to 16 whole columns, so what an XCD works on at a time are a few weight panels and the token rows of mostly one expert, however many
+// of its workgroups are on heavy tiles; a block of 6 x 4 tiles leaves eight of them to the next one, of other rows.  Fetched into L2
+// (MB): 131072 rows, 128 experts, 3072 x 4096 5400 -> 3870, 6579 rows, 32 experts, 4096 x 7168 1470 -> 1250, 4012 rows (MXFP8) 1255 -> 1100.  us:
+// 1646 -> 1596, 257.4 -> 251.3, 204.0 -> 197.2; 44 experts, 11384 rows, 768 x 640 (MXFP8) 29.0 -> 16.4, 10 experts, 974 rows, 4096 x 1024
+// 26.2 -> 16.7; 110 drawn shapes of K = 640 to 7168 1.11 times as fast, one in twelve 2 to 5 % slower (an expert's tiles then stand
+// in two runs).  Row by row instead of down the columns: -2 % on the large launches; one run of an eighth of the launch per queue:
+// +0.4 % on these, -0.6 % on the drawn ones.  Up to K = 512 the queues hold blocks, which is what the host mirrors have described of
+// such calls so far (runs: 70 drawn shapes 1.15 times as fast, 0.87 to 1.95).
+ESMOE_HD bool sched_use_runs(int k) { return k > 512; }
+// Tiles of a run: 32, one per CU of an XCD.  In launches of at most 512 an eighth or a sixteenth of them, so that the queues hold one or
+// two runs each and about as many tiles.
+ESMOE_HD int sched_run_tiles(int tiles) {
+  constexpr int kAll = kXcds * kBlkTiles;
+  return tiles > 2 * kAll ? kBlkTiles : tiles > kAll ? (tiles + 2 * kXcds - 1) / (2 * kXcds) : (tiles + kXcds - 1) / kXcds;
 }
 
 // Block shape for an expert with mtl x ntl tiles: at most kBlkM tiles high and kBlkTiles tiles in all, with
@@ -163,11 +190,37 @@ ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolic
   if (ni >= ntl) return false;
   const int big = p.force_mt ? p.force_mt : p.big_mt;
   const int m0 = mi * big * 16;
-  t->mt = p.force_mt ? p.force_mt : (m - m0 >= big * 16 ? big : sched_cover_mt(m - m0, big));
+  t->mt = p.force_mt ? p.force_mt : m - m0 >= big * 16 ? big : sched_cover_mt(m - m0, big);
   t->nt = 4;
   t->m0 = m0;
   t->n0 = ni * 256;
   return true;
+}
+
+constexpr int kRunRows = 192;   // row tiles of a launch whose queues hold runs
+ESMOE_HD int sched_run_mtiles(int m) { return (m + kRunRows - 1) / kRunRows; }
+ESMOE_HD int sched_heavy_tiles(int m, int n) { return sched_run_mtiles(m) * sched_ntiles(n, 4); }
+ESMOE_HD float sched_run_cost(int m, int n) {
+  const int tiles = sched_run_mtiles(m), above = (tiles - 1) * kRunRows;
+  return (float)(above + sched_last_mt(m - above) * 16 + 16 * tiles) * (float)sched_ntiles(n, 4);
+}
+// Tile `local` of an expert of m rows.
+ESMOE_HD TileCoord sched_decode_run(int local, int m, int n) {
+  const int mtl = sched_run_mtiles(m), ntl = sched_ntiles(n, 4);
+  int rows = mtl, left = local, first = 0;   // of the row of blocks: tiles of a column, the tile's place, its first row tile
+  if (mtl > kBlkM) {
+    const int rbs = (mtl + kBlkM - 1) / kBlkM, bm = sched_div(mtl + rbs - 1, rbs), rb = sched_div(local, bm * ntl);
+    first = rb * bm;
+    left -= first * ntl;
+    rows = mtl - first < bm ? mtl - first : bm;
+  }
+  const int ni = sched_div(left, rows), mi = first + left - ni * rows;
+  TileCoord t;
+  t.mt = mi < mtl - 1 ? kRunRows / 16 : sched_last_mt(m - mi * kRunRows);
+  t.nt = 4;
+  t.m0 = mi * kRunRows;
+  t.n0 = ni * 256;
+  return t;
 }
 
 // Light items are handed out whole (256 columns) except the last `narrow_tail` of the launch, which go out as two
@@ -259,11 +312,22 @@ ESMOE_HD float sched_heavy_cost(int m, int n, const SchedPolicy& p) {
 ESMOE_HD float sched_light_cost(int m, int n, const SchedPolicy& p) {
   return (float)sched_light_items(m, n, p) * (float)(75 + m / 3);
 }
+// `run_tiles`: heavy tiles where the queues hold runs.  Up to 256 of them are all first tickets, and of a launch of about two rounds half: a
+// tall tile drawn when the other workgroups end theirs is the longest end a launch can have, and where nothing is drawn from the
+// heavy queues no workgroup has to look at all of them when the light items are used up.  106 experts, 6462 rows, 768 x 7168 (99 heavy
+// tiles) 148.4 -> 121.9 us, 64 experts, 4131 rows, 1536 x 1024 (132) 38.8 -> 29.6, 66 experts, 13232 rows, 1536 x 1536 (384) 71.9 -> 62.0, 32
+// experts, 256 rows, 7168 x 2048 (28) 77.2 -> 74.3.
 // Workgroups of every 32 that start on the light items.  (Floats: it is an estimate, and a 64-bit division and sum of both costs
 // stood 0.8 us in front of the first tile.)
-ESMOE_HD int sched_light_share(float heavy_cost, float light_cost, const SchedPolicy& p) {
+ESMOE_HD int sched_light_share(float heavy_cost, float light_cost, int run_tiles, const SchedPolicy& p) {
   if (p.light_share >= 0) return p.light_share > 32 ? 32 : p.light_share;
   if (heavy_cost <= 0 || light_cost <= 0) return 0;
+  if (run_tiles > 0) {
+    const int tiles = (run_tiles + kXcds - 1) / kXcds;
+    if (tiles <= kBlkTiles) return kBlkTiles - tiles;
+    const float rounds = (float)run_tiles * (heavy_cost + light_cost) / (heavy_cost * (kXcds * kBlkTiles));
+    if (rounds < 2.75f && tiles <= 2 * kBlkTiles) return kBlkTiles - (tiles + 1) / 2;
+  }
   return (int)(32 * light_cost / (heavy_cost + light_cost) + 0.5f);
 }
 
@@ -272,6 +336,18 @@ ESMOE_HD int sched_ticket_block(int xcd, int ticket) { return (ticket / kBlkTile
 
 // Tickets of XCD `xcd`'s queue when the launch has `hblocks` heavy blocks: queue x holds the blocks x, x + 8, ..., 32 tickets each.
 ESMOE_HD int sched_queue_tickets(int xcd, int hblocks) { return xcd < hblocks ? (hblocks - xcd + kXcds - 1) / kXcds * kBlkTiles : 0; }
+
+// Where the queues hold runs, queue x holds the runs x, x + 8, ... and every ticket is a tile: ticket -> tile of the launch, tickets of
+// a queue.  (Runs of less than 32 tiles: a queue has no more than two.)
+ESMOE_HD int sched_run_tile(int xcd, int ticket, int run) {
+  const int q = run == kBlkTiles ? ticket / kBlkTiles : ticket >= run ? 1 : 0;
+  return (q * kXcds + xcd) * run + ticket - q * run;
+}
+ESMOE_HD int sched_run_tickets(int xcd, int tiles, int run) {
+  const int round = kXcds * run, full = run == kBlkTiles ? tiles / (kXcds * kBlkTiles) : tiles >= round ? 1 : 0;   // rounds of all queues
+  const int left = tiles - full * round - xcd * run;
+  return full * run + (left < 0 ? 0 : left < run ? left : run);
+}
 
 // Queue that a workgroup draws heavy tickets from when it has found `step` queues empty: first the one its first ticket is of, the
 // queue of its XCD (the hardware deals the workgroups of a launch out in turn, workgroup i to XCD i % 8), then the others in turn.
@@ -362,15 +438,16 @@ ESMOE_HD int sched_k_start(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3) {
 // Workspace layout (int32 words).
 constexpr int kWsLightCounter = 32;  // next light ticket to hand out (every counter has a 128-byte line of its own)
 constexpr int kWsLightTotal = 1;     // number of light tickets: whole items, then two per item of the narrow tail
-constexpr int kWsHeavyBlocks = 2;    // number of heavy blocks
+constexpr int kWsHeavyBlocks = 2;    // number of heavy blocks (runs: of 32 tiles)
 constexpr int kWsLightShare = 3;     // workgroups of every 32 that start on the light items
 constexpr int kWsLightSplit = 4;     // first light ticket that is a half item (sched_light_split)
 constexpr int kWsBlockLog = 5;       // sched_log2_ceil of the most tiles of a heavy block (sched_block_tiles)
+constexpr int kWsRun = 6;            // tiles of a run (sched_run_tiles), 0: the queues hold blocks
 constexpr int kWsExitCounter = 16;   // workgroups of the launch that have left the hand-out loop: the last one zeroes every counter
 constexpr int kWsXcdCounter = 64;    // next heavy ticket of XCD x at word kWsXcdCounter + 32 * x (ws_xcd_counter)
 constexpr int kWsHeader = 64 + 32 * kXcds;   // then one record of kRecWords per schedule position, E + 1 of them
-// Record of schedule position p: first heavy block, first light item, expert index, rows (clamped at 0).
-// Record E closes the prefix sums: {heavy blocks, light items, -1, 0}.
+// Record of schedule position p: first heavy block (runs: first heavy tile), first light item, expert index, rows (clamped at 0).
+// Record E closes the prefix sums: {heavy blocks (tiles), light items, -1, 0}.
 constexpr int kRecWords = 4;
 constexpr int kRecBlock = 0, kRecItem = 1, kRecExpert = 2, kRecRows = 3;
 // The expert's word also holds where its K order starts (sched_k_start).

@@ -285,7 +285,9 @@ int esmoe_permute_rows(const void* in, const int32_t* dst_row, long num_pairs, i
  * Experts with more than 64 rows are "heavy": their tiles are handed out in blocks of 8 x 4 tiles, block b
  * to XCD b % 8, through one ticket counter per XCD; esmoe_host_decode_heavy maps ticket `ticket` of XCD `xcd`
  * to out5 = {expert, tile rows, tile cols, m0, n0} and returns 0, or 1 if the ticket falls outside the
- * expert's tile grid (the kernel skips it), or 2 if that XCD's queue is exhausted.
+ * expert's tile grid (the kernel skips it), or 2 if that XCD's queue is exhausted.  In a launch with K > 512 (the third
+ * value of problem_sizes_host) and no forced tile height they are handed out in runs instead (word 6 of the workspace: tiles of a run):
+ * all heavy tiles in one line, run r to XCD r % 8, every ticket a tile, last row tiles of 96 and 160 rows as well.
  * The other experts are "light": one short tile per 256 columns from a launch-wide counter, except that the last 128
  * light items of a launch go out as two 128-column halves each (word 4 of the workspace is the first ticket that is a
  * half, word 1 the number of light tickets); esmoe_host_decode_light maps ticket `item` (< word 1) to out5 and returns
