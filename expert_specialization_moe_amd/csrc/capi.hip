@@ -123,12 +123,11 @@ esmoe::SchedPolicy default_policy(int force_bm, int kind, int k) {
   // Full tiles are 192 rows for both kernels: the tallest tile whose ring (three weight stages, two token stages per
   // wavefront group) fits the 160 KB of LDS, which is what the hand-scheduled K block of the tall tiles needs.  (A
   // 256-row tile does more MFMA work per byte copied but only fits with two stages per operand and measured slower.)
-  (void)mx;
   p.big_mt = 12;
   p.order = 0;
   p.light_share = -1;
-  // the fused epilogues quantise blocks that need a whole 256-row tile, and a forced height has no light items
-  p.narrow_tail = (force_bm == 0 && !(kind & 2)) ? kNarrowTail : 0;
+  // the fused fp8-blockwise epilogue quantises blocks that need a whole 256-row tile, and a forced height has no light items
+  p.narrow_tail = force_bm == 0 && (!(kind & 2) || (mx && k > 512)) ? kNarrowTail : 0;
   p.runs = force_bm == 0 && esmoe::sched_use_runs(k);
   return p;
 }

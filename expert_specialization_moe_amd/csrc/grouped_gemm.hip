@@ -149,14 +149,15 @@ __device__ __forceinline__ void block_barrier() {
 }
 
 // Shape of a short tile (MT*16 <= 64 token rows) and the layout of one ring stage (token rows, weight rows, scales):
-// each of the 8 wavefronts has all token rows and 32 weight rows.  (Tall tiles: gemm_tile_pp, gemm_tile_pp_mx.)
-template <int MT, bool MX, int BN = kBN>
+// each of the 8 wavefronts has all token rows and 32 weight rows, 16 those of a half item; with WM = 2 two groups of four have half of the
+// rows each (all where there are 16).  (Tall tiles: gemm_tile_pp, gemm_tile_pp_mx.)
+template <int MT, bool MX, int BN = kBN, int WM = 1>
 struct TileGeom {
   static_assert(BN == 256 || BN == 128, "tile widths: 256 weight rows, or 128 for the narrow items that end a launch");
   static constexpr int BM = MT * 16;
-  static constexpr int kWavesM = 1;
+  static constexpr int kWavesM = WM;
   static constexpr int kWavesN = kWaves / kWavesM;
-  static constexpr int MTW = MT / kWavesM;          // row tiles per wavefront
+  static constexpr int MTW = MT > kWavesM ? MT / kWavesM : 1;   // row tiles per wavefront
   static constexpr int NTW = BN / 16 / kWavesN;     // weight-row tiles per wavefront
   static constexpr int kABytes = BM * 128;
   static constexpr int kWBytes = BN * 128;
@@ -178,13 +179,16 @@ struct TileGeom {
 // The fused epilogues gather a tile's quantised bytes in LDS, BM rows of 128 bytes `stride` apart, and the workgroup
 // writes them from there: eight lanes a row, a whole 128-byte line per row where the MFMA layout would give 16-byte
 // pieces.  `dst` is the tile's first byte of the expert's row 0 (row pitch `pitch`); rows at or past M are not written.
-template <int BM>
+template <int BM, int kBytes = 128>
 __device__ __forceinline__ void store_staged_rows(const uint8_t* stage, int stride, uint8_t* dst, int pitch, int M, int m0) {
-  const int tid = threadIdx.x;
+  constexpr int kLanes = kBytes / 16;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (nothing of it is kept across tiles: gemm_tile)
+  const int col = tid % kLanes * 16;
 #pragma unroll
-  for (int row = tid >> 3; row < BM; row += kThreads / 8) {
+  for (int row = tid / kLanes; row < BM; row += kThreads / kLanes) {
     const int m = m0 + row;
-    if (m < M) __builtin_nontemporal_store(*(const v4i*)(stage + row * stride + (tid & 7) * 16), (v4i_dwords*)(dst + (long)m * pitch + (tid & 7) * 16));
+    if (m < M) __builtin_nontemporal_store(*(const v4i*)(stage + row * stride + col), (v4i_dwords*)(dst + (long)m * pitch + col));
   }
 }
 
@@ -411,18 +415,21 @@ __device__ __forceinline__ void tile_epilogue_mxq(const GemmArgs& g, Acc& acc, i
     if (gq == 0 && (!kPair || (wn & 1) == 0)) lds[kCodeOff + row * 4 + (cblk & 3)] = (uint8_t)(m < M ? code : 0);
   }
   __syncthreads();
-  store_staged_rows<BM>(lds + kStageOff, kStageStride, (uint8_t*)g.q_out + row_base * (long)inter + (n0 >> 1), inter, M, m0);
-  for (int row = threadIdx.x; row < BM; row += kThreads) {
+  // (a half item has 64 h columns, two of the four scale columns of its dwords)
+  constexpr int kCols = kWavesN * kRW / 2;
+  typedef typename std::conditional<kCols == 128, uint32_t, uint16_t>::type Codes;
+  const int code0 = kCols == 128 ? 0 : (n0 >> 6) & 2;
+  store_staged_rows<BM, kCols>(lds + kStageOff, kStageStride, (uint8_t*)g.q_out + row_base * (long)inter + (n0 >> 1), inter, M, m0);
+  auto codes_of = [&](int m) { return (Codes*)(sf_e + ((long)(m >> 7) * (inter >> 7) + (n0 >> 8)) * 512 + (m & 31) * 16 + ((m & 127) >> 5) * 4 + code0); };
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  for (int row = tid; row < BM; row += kThreads) {
     const int m = m0 + row;
-    if (m < m_pad)
-      *(uint32_t*)(sf_e + ((long)(m >> 7) * (inter >> 7) + (n0 >> 8)) * 512 + (m & 31) * 16 + ((m & 127) >> 5) * 4) =
-          *(const uint32_t*)(lds + kCodeOff + row * 4);
+    if (m < m_pad) *codes_of(m) = *(const Codes*)(lds + kCodeOff + row * 4 + code0);
   }
-  // rows of the expert's last scale tile that lie below this tile: the tile's four scale columns are one dword
+  // rows of the expert's last scale tile that lie below this tile
   if (m0 + BM >= M) {
-    for (int m = m0 + BM + (int)threadIdx.x; m < m_pad; m += kThreads) {
-      *(uint32_t*)(sf_e + ((long)(m >> 7) * (inter >> 7) + (n0 >> 8)) * 512 + (m & 31) * 16 + ((m & 127) >> 5) * 4) = 0u;
-    }
+    for (int m = m0 + BM + tid; m < m_pad; m += kThreads) *codes_of(m) = 0;
   }
   __syncthreads();   // the stages (and s_amax) are ring memory: the next tile's copies must not land before they are read
 }
@@ -443,15 +450,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
                                           uint8_t* lds) {
   constexpr bool kStrip = !FUSE && BN == kBN;
   static_assert(kStripBlocks <= kMaxKB, "the weight block scales of a strip share the table of one tile");
-  static_assert(!(FUSE && BN != kBN), "the fused epilogues need gate and up columns of a whole quantisation block in one tile");
+  static_assert(!(FUSE && !MX && BN != kBN), "the fused epilogues need gate and up columns of a whole quantisation block in one tile");
   static_assert(MT == 1 || MT == 2 || MT == 4, "short tiles; 96- to 192-row tiles are gemm_tile_pp / gemm_tile_pp_mx");
-  using G = TileGeom<MT, MX, BN>;
+  using G = TileGeom<MT, MX, BN, FUSE && BN != kBN ? 2 : 1>;   // (half items: a wavefront needs gate and up of its columns)
   constexpr int MTW = G::MTW, NTW = G::NTW, NBUF = G::kNBuf;
   int tid = threadIdx.x;
   // (hidden from the compiler, which otherwise forms this tile's addresses once in front of the hand-out loop and keeps them
   // in vector registers that the tall tiles do not have: four were spilled to scratch.  The fused kernels have
   // enough, and forming the addresses for every tile costs 0.2 us a tile: 128 experts, 16384 rows, 3072 x 4096 361.7 -> 359.0 us.)
-  if constexpr (!FUSE) asm volatile("" : "+v"(tid));
+  if constexpr (!FUSE || BN != kBN) asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / G::kWavesN, wn = wave % G::kWavesN;
@@ -460,7 +467,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
   const int K = g.k, N = g.n, KB = K >> 7;
   const long row_base = erow;
   const int nw = wn * (NTW * 16);          // first weight row of this wavefront inside the tile
-  const int mw = wm * (MTW * 16);          // first token row of this wavefront inside the tile
+  const int mw = MT == 1 ? 0 : wm * (MTW * 16);   // first token row of this wavefront inside the tile
   const bool wave_active = n0 + nw < N;
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
   float* s_sb = (float*)(lds + kRingBytes);  // [2][kMaxKB] weight block scales of the tile's two 128-column blocks
@@ -582,7 +589,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
   const float* sb_tab = kStrip ? s_sb + (nw >> 7) * KB : s_sb + (FUSE ? 0 : (nw >> 7)) * kMaxKB;
   // mxfp8: per-lane bases of the scale dwords (weight rows nw + r, token rows mw + r of a tall tile)
   // (FUSE: n-tile 0 = gate rows n0/2 + wn*16 + r in the first tile, n-tile 1 the up rows at the same place in the second)
-  const int sfw_lane = FUSE ? kScaleOff + ((wn & 1) * 16 + r) * 16 + (wn >> 1) * 4
+  const int sfw_lane = FUSE ? kScaleOff + ((wn & 1) * 16 + r) * 16 + (wn >> 1) * 4 + (BN == kBN ? 0 : (n0 >> 4) & 8)
                             : kScaleOff + (nw >> 7) * 512 + ((nw & 127) >> 5) * 4 + ((nw & 31) + r) * 16;
   const int sfa_lane = kScaleOff + 1024 + (mw >> 7) * 512 + ((mw & 127) >> 5) * 4 + r * 16;
   const int sa_lane = kScaleOff + (mw + r) * 4;   // fp8-blockwise: float sa of token row mw + r
@@ -641,7 +648,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int e, int first_kb
 #pragma unroll
       for (int mt = 0; mt < MTW; mt++) {
         // token row inside its 128-row scale tile (a short tile starts on a multiple of 64 rows and never crosses one)
-        const int ml = (m0 & 127) + mt * 16 + r;
+        const int ml = (m0 & 127) + mw + mt * 16 + r;
         const uint32_t d = *(const uint32_t*)(lb + kScaleOff + 1024 + (ml & 31) * 16 + (ml >> 5) * 4);
         f.sfa[mt] = (int)(d >> (gq * 8));
       }
@@ -1878,11 +1885,11 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
     } else if (t.mt == 6) {
       if constexpr (MX) gemm_tile_pp_mx<6, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, lds);
       else gemm_tile_pp<6, FUSE>(g, e, first_kb, erow, M, t.m0, t.n0, lds);
-    } else if (!FUSE && t.nt == 2) {
-      if constexpr (!FUSE) {
-        if (t.mt == 1) gemm_tile<1, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
-        else if (t.mt == 2) gemm_tile<2, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
-        else gemm_tile<4, MX, false, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
+    } else if ((MX || !FUSE) && t.nt == 2) {
+      if constexpr (MX || !FUSE) {
+        if (t.mt == 1) gemm_tile<1, MX, FUSE, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
+        else if (t.mt == 2) gemm_tile<2, MX, FUSE, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
+        else gemm_tile<4, MX, FUSE, 128>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, 1, lds);
       }
     } else {
       if (t.mt == 1) gemm_tile<1, MX, FUSE>(g, e, first_kb, erow, ebso, M, t.m0, t.n0, cols, lds);

@@ -187,3 +187,19 @@ def test_fused_output_feeds_the_down_projection(esmoe):
     torch.cuda.synchronize()
     assert torch.equal(d1, d2)
     assert d1.float().abs().max().item() > 0
+
+
+@pytest.mark.parametrize("rows", [[1, 16, 17, 32, 33, 64, 0, 50], [5] * 130, [300, 64, 1, 129]])
+@pytest.mark.parametrize("inter", [128, 384, 1536])
+def test_half_items_of_a_fused_launch(esmoe, inter, rows):
+    """From K = 640 on the last 128 light items go out as halves of 64 h columns: all of a launch's or its last ones, at every short
+    height, next to whole items and tall tiles.  Bit-exact against the separate route, padding and untouched bytes included."""
+    from expert_specialization_moe_amd import _native
+    from expert_specialization_moe_amd import workloads as W
+
+    prob = W.Problem("gate_up", 2 * inter, 640, rows)
+    ops = W.make_mxfp8_operands(prob, "cuda", seed=11, out_dtype=torch.bfloat16, weight_std=0.05)
+    q, sf = _fused(_native, ops, rows, inter, torch.bfloat16)
+    q_ref, sf_ref = _separate(esmoe, _native, ops, rows, inter, torch.bfloat16, 0)
+    assert torch.equal(q, q_ref), f"{(q != q_ref).sum().item()} bytes differ"
+    assert torch.equal(sf, sf_ref), f"{(sf != sf_ref).sum().item()} scale bytes differ"
