@@ -621,7 +621,8 @@ int esmoe_host_decode_heavy(const int32_t* problem_sizes_host, const int32_t* ws
   const int32_t* rec = ws_host + esmoe::ws_rec(pos);
   esmoe::TileCoord t;
   bool past = false;
-  if (run) t = esmoe::sched_decode_run(unit - rec[esmoe::kRecBlock], rec[esmoe::kRecRows], n);
+  if (run) t = esmoe::sched_decode_run(unit - rec[esmoe::kRecBlock], rec[esmoe::kRecRows], n,
+                                      esmoe::sched_pair_rows(ws_host[esmoe::ws_rec(num_experts) + esmoe::kRecBlock], problem_sizes_host[2], kind & 1));
   else if (!esmoe::sched_decode_heavy(unit - rec[esmoe::kRecBlock], ticket % esmoe::kBlkTiles, rec[esmoe::kRecRows], n, p, &t, &past))
     return 1;   // ticket outside the expert's tile grid: skipped
   fill_out5(out5, esmoe::rec_expert(rec[esmoe::kRecExpert]), t);

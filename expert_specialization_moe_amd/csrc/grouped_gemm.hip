@@ -1409,10 +1409,10 @@ __device__ __forceinline__ Hand first_hand(const GemmArgs& g, int hunits, int ru
 __device__ __forceinline__ int heavy_index(int queue, int ticket, const HeavyHand& h) {
   return h.run ? sched_run_tile(queue, ticket, h.run) : sched_ticket_block(queue, ticket);
 }
-// Tile of ticket `have`, item, tile or block `local` of its expert; moves `have` on by the tickets that it takes.  mt = 0: it is no tile
+// Tile of ticket `have`, item, tile (`tiles`: of the launch) or block `local` of its expert; moves `have` on by the tickets that it takes.  mt = 0: it is no tile
 // (`past`: nor are those behind it in its block).
-template <bool FUSE>
-__device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int split, int run, int& have, int have_end, int local, int half, int rows, bool* past) {
+template <bool MX, bool FUSE>
+__device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int split, int tiles, int& have, int have_end, int local, int half, int rows, bool* past) {
   TileCoord t;
   Tile d;
   *past = false;
@@ -1430,8 +1430,8 @@ __device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int spl
     }
     have += half == -2 ? 2 * d.cols : d.cols;
     if (t.n0 >= g.n) t.mt = 0;   // second half of a last column tile that is 128 columns wide
-  } else if (run) {
-    t = sched_decode_run(local, rows, g.n);
+  } else if (tiles) {
+    t = sched_decode_run(local, rows, g.n, sched_pair_rows(tiles, g.k, MX));
     have++;
   } else if (!sched_decode_heavy(local, have++ % kBlkTiles, rows, g.n, g.policy, &t, past)) {
     t.mt = 0;
@@ -1461,7 +1461,7 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us; half as many divisions and a four-way search of the records:
 // 75.2 -> 74.7 (with both kinds of experts), an expert MLP of 1003 tokens in MXFP8 377.5 -> 376.1.
 // The workgroup's first tile, by the thread of the expert that the ticket belongs to (items, tiles or blocks [before, before + mine)).
-template <bool FUSE>
+template <bool MX, bool FUSE>
 __device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool light, bool heavy, int before, int mine, int rows, int word, int row,
                                            int scale_row, Tile* first) {
   if (h.have == h.have_end) return;
@@ -1470,7 +1470,7 @@ __device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool ligh
   if ((h.light_first ? light : heavy) && idx >= before && idx < before + mine) {
     bool past;
     int have = h.have;
-    Tile d = take_tile<FUSE>(g, h.light_first, h.light.split, h.heavy.run, have, h.have_end, idx - before, half, rows, &past);
+    Tile d = take_tile<MX, FUSE>(g, h.light_first, h.light.split, h.heavy.tiles, have, h.have_end, idx - before, half, rows, &past);
     d.expert = word;
     d.row = row;
     d.scale_row = scale_row;
@@ -1584,7 +1584,7 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
   if (lane == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
   Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
-  first_tile<FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
+  first_tile<MX, FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
   if (lane == 0) *out = h;
 }
 
@@ -1727,7 +1727,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, H
   static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
   const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
   Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
-  first_tile<FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
+  first_tile<MX, FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
   if (t == 0) *out = h;
 }
 
@@ -1839,7 +1839,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
       const v4i rec = sload4(ws, ws_rec(lo) * 4);
       const int word = uniform(rec[kRecExpert]);
       bool past;
-      d = take_tile<FUSE>(g, light, lights.split, heavies.run, have, have_end, idx - uniform(light ? rec[kRecItem] : rec[kRecBlock]), half,
+      d = take_tile<MX, FUSE>(g, light, lights.split, heavies.tiles, have, have_end, idx - uniform(light ? rec[kRecItem] : rec[kRecBlock]), half,
                           uniform(rec[kRecRows]), &past);
       d.expert = word;
       if (d.mt) {

@@ -200,12 +200,30 @@ ESMOE_HD bool sched_decode_heavy(int lb, int idx, int m, int n, const SchedPolic
 constexpr int kRunRows = 192;   // row tiles of a launch whose queues hold runs
 ESMOE_HD int sched_run_mtiles(int m) { return (m + kRunRows - 1) / kRunRows; }
 ESMOE_HD int sched_heavy_tiles(int m, int n) { return sched_run_mtiles(m) * sched_ntiles(n, 4); }
+// Most rows behind a first full tile that make two tall tiles of the expert's rows, of 128 and of 96 or 128, where 192 rows would leave a
+// short one to the rest.  For launches of up to 256 heavy tiles, all of one round: it lasts as long as its longest tile, and a short tile
+// beside a tall one, on the same panel, lasts longer than a tall one; for up to 512 from K = 4096 on.  `tiles`: of the launch.
+// us, 192 + rest against two tall tiles, 2048 columns.  14 experts x 208 rows MXFP8: K = 7168 66.1 / 43.8, K = 3200 35.5 / 26.3, K = 1024
+// 18.0 / 15.1; FP8: K = 7168 67.1 / 54.2, K = 3200 32.4 / 28.2, K = 2176 23.1 / 22.4, K = 2048 21.7 / 21.7.  14 x 256 rows MXFP8: K = 3200
+// 33.8 / 27.3, K = 1024 14.8 / 15.2; FP8: K = 4096 36.6 / 35.5, K = 3968 35.6 / 35.8.  Two rounds, 32 experts: x 208 rows MXFP8 K = 7168
+// 154.9 / 134.9, K = 4096 90.3 / 79.2, K = 3200 64.1 / 65.1, K = 2048 45.3 / 49.0; FP8 K = 4096 94.3 / 86.0; x 256 rows MXFP8 K = 4096
+// 89.8 / 86.2, K = 3200 60.4 / 69.6, FP8 K = 4096 92.9 / 91.8.  Past two rounds what counts is the sum of the work: 100 experts x 256
+// rows, 1024 x 4096 fused 165.5 / 179.3, 131072 rows, 128 experts, 3072 x 4096 1600 / 1610 (with experts of any size).
+ESMOE_HD int sched_pair_rows(int tiles, int k, bool mx) {
+  constexpr int kRound = kXcds * kBlkTiles;
+  if (k >= 4096) return tiles <= 2 * kRound ? 64 : 0;
+  return tiles > kRound ? 0 : mx && k > 3072 ? 64 : mx || k > 2048 ? 32 : 0;
+}
+// First row of an expert's last row tile.
+ESMOE_HD int sched_run_last_row(int m, int mtl, int pair_rows) {
+  return mtl == 2 && m - kRunRows <= pair_rows ? kRunRows - 64 : (mtl - 1) * kRunRows;
+}
 ESMOE_HD float sched_run_cost(int m, int n) {
   const int tiles = sched_run_mtiles(m), above = (tiles - 1) * kRunRows;
   return (float)(above + sched_last_mt(m - above) * 16 + 16 * tiles) * (float)sched_ntiles(n, 4);
 }
 // Tile `local` of an expert of m rows.
-ESMOE_HD TileCoord sched_decode_run(int local, int m, int n) {
+ESMOE_HD TileCoord sched_decode_run(int local, int m, int n, int pair_rows) {
   const int mtl = sched_run_mtiles(m), ntl = sched_ntiles(n, 4);
   int rows = mtl, left = local, first = 0;   // of the row of blocks: tiles of a column, the tile's place, its first row tile
   if (mtl > kBlkM) {
@@ -216,9 +234,10 @@ ESMOE_HD TileCoord sched_decode_run(int local, int m, int n) {
   }
   const int ni = sched_div(left, rows), mi = first + left - ni * rows;
   TileCoord t;
-  t.mt = mi < mtl - 1 ? kRunRows / 16 : sched_last_mt(m - mi * kRunRows);
+  const int last = sched_run_last_row(m, mtl, pair_rows);
+  t.m0 = mi < mtl - 1 ? mi * kRunRows : last;
+  t.mt = mi < mtl - 2 ? kRunRows / 16 : mi < mtl - 1 ? (last - t.m0) >> 4 : sched_last_mt(m - last);
   t.nt = 4;
-  t.m0 = mi * kRunRows;
   t.n0 = ni * 256;
   return t;
 }

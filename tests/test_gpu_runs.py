@@ -9,11 +9,11 @@ from tests.test_gpu_one_launch import _mm
 
 pytestmark = pytest.mark.gpu
 
-EDGES = [65, 80, 81, 96, 97, 128, 129, 144, 145, 160, 161, 192, 193, 208, 257, 288, 289, 300, 352, 353, 64, 33, 0, 1]
+EDGES = [65, 80, 81, 96, 97, 128, 129, 144, 145, 160, 161, 192, 193, 208, 224, 225, 256, 257, 288, 289, 300, 352, 353, 64, 33, 0, 1]
 
 
 @pytest.mark.parametrize("name,rows,n,k", [
-    ("edges", EDGES, 640, 640), ("edges from the middle of K", EDGES, 512, 4096), ("rows of blocks", [1700, 70, 3], 768, 768),
+    ("edges", EDGES, 640, 640), ("edges from the middle of K", EDGES, 512, 4096), ("edges", EDGES, 256, 2176), ("rows of blocks", [1700, 70, 3], 768, 768),
     ("255 tiles", [70] * 255, 256, 640), ("257 tiles", [100] * 257, 256, 640), ("513 tiles", [66] * 513, 256, 640)])
 @pytest.mark.parametrize("kind", ["fp8", "mx"])
 def test_same_bytes_as_a_forced_height(esmoe, kind, name, rows, n, k):

@@ -17,8 +17,8 @@ def _ptr(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
-def _schedule(lib, rows, n, kind):
-    ps = np.array([[m, n, 640] for m in rows], dtype=np.int32)
+def _schedule(lib, rows, n, kind, k=640):
+    ps = np.array([[m, n, k] for m in rows], dtype=np.int32)
     ws = np.zeros(lib.esmoe_gemm_workspace_bytes(len(rows)) // 4, dtype=np.int32)
     assert lib.esmoe_host_schedule(_ptr(ps), len(rows), n, 0, kind, _ptr(ws)) == 0
     return ps, ws
@@ -32,9 +32,10 @@ def test_every_ticket_is_a_tile_and_every_output_element_is_covered_once(esmoe, 
 
     lib, rng = _native.lib, random.Random(seed)
     for rows, n in (([65, 96, 97, 128, 129, 160, 161, 192, 193, 208, 209, 224, 256, 257, 288, 289, 352, 384, 0, 64, 1, 1700], 768),
-                    ([70] * (254 + seed), 256), ([70] * (510 + seed), 256), ([2000] * (3 + seed), 1280), ([5] * 9, 384),
+                    ([70] * (252 + seed) + [200, 256], 256), ([70] * (508 + seed) + [200, 256], 256), ([70] * (254 + seed), 256), ([70] * (510 + seed), 256), ([2000] * (3 + seed), 1280), ([5] * 9, 384),
                     ([rng.choice((0, rng.randrange(65), rng.randrange(65, 4000))) for _ in range(rng.randrange(1, 60))], 128 * rng.randrange(1, 30))):
-        ps, ws = _schedule(lib, rows, n, seed % 4)
+        k = (640, 640, 2048, 3072, 2176, 3200, 3968, 4096)[seed]
+        ps, ws = _schedule(lib, rows, n, seed % 4, k)
         tiles, out = int(ws[64 + 32 * 8 + 4 * len(rows)]), np.zeros(5, dtype=np.int32)
         cover = [np.zeros((m, n // 128), dtype=np.int32) for m in rows]
         queues = []
@@ -46,8 +47,11 @@ def test_every_ticket_is_a_tile_and_every_output_element_is_covered_once(esmoe, 
                     break
                 e, bm, bn, m0, n0 = (int(v) for v in out)
                 last = rows[e] - m0
-                assert rc == 0 and rows[e] > 64 and bn == 256 and m0 % 192 == 0
-                want = 192 if last > 160 else -(-last // 32) * 32 if last > 64 else 16 if last <= 16 else 32 if last <= 32 else 64
+                assert rc == 0 and rows[e] > 64 and bn == 256 and m0 % 64 == 0
+                # (from 193 rows to 224 or 256: two tall tiles, the first of 128 rows; odd seeds are MXFP8)
+                most = (64 if tiles <= 512 else 0) if k >= 4096 else 0 if tiles > 256 else 64 if k > 3072 and seed % 2 else 32 if k > 2048 or seed % 2 else 0
+                two = 192 < rows[e] <= 192 + most
+                want = 128 if two and m0 == 0 else 192 if last > 160 else -(-last // 32) * 32 if last > 64 else 16 if last <= 16 else 32 if last <= 32 else 64
                 assert bm == want, (rows[e], m0, bm)
                 cover[e][m0:m0 + bm, n0 // 128:(n0 + bn) // 128] += 1
                 ticket += 1
