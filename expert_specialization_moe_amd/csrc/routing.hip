@@ -79,13 +79,17 @@ __global__ void __launch_bounds__(kRouteThreads) route_count_kernel(const int* _
   if (tid < num_experts) chunk_counts[(long)blockIdx.x * num_experts + tid] = s_cnt[tid];
 }
 
-// One workgroup per chunk.  DIRECT: counts from the ids; otherwise from chunk_counts [gridDim.x, num_experts].
+// One workgroup per chunk.  Counts: kFromChunks from chunk_counts [gridDim.x, num_experts], kFromIds from the ids, kFromWaves from what the
+// workgroup's wavefronts find in their own pairs anyway, where it is the only one (up to 1024 pairs; launched with as few wavefronts as
+// hold the pairs and the experts).
 //
 // Latency from end to end (one workgroup per CU, a few thousand pairs): every id is read once per use with eight loads
 // in flight, a wavefront's 64 pairs are ranked by ballots once, and the prefix sums run on the vector ALU.  As one
 // workgroup that took up to 16384 pairs in dependent rounds, and as three launches past that, 128 experts took 10.5 us at
-// 512 pairs (now 3.5), 22.3 at 16384 (6.1), 20.2 at 32768 (6.3), 24.6 at 131072 (8.0).
-template <bool DIRECT>
+// 512 pairs (now 2.9), 22.3 at 16384 (6.1), 20.2 at 32768 (6.3), 24.6 at 131072 (8.0).  kFromWaves against a pass of LDS atomics by sixteen
+// wavefronts: 8 pairs of 8 experts 3.3 -> 2.6, 128 of 128 3.6 -> 2.9, 512 of 128 3.7 -> 3.05, 1024 of 1024 4.7 -> 4.4.
+enum Counts { kFromChunks, kFromIds, kFromWaves };
+template <Counts COUNTS>
 __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, long num_pairs, int first_expert,
                                                               int num_experts, long chunk, const int* __restrict__ chunk_counts,
                                                               int n, int k, int* __restrict__ problem_sizes,
@@ -99,12 +103,14 @@ __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, lo
   const int E = num_experts, me = blockIdx.x;
   const long base = (long)me * chunk;
   int raw = base + tid < num_pairs ? ids[base + tid] : 0;   // this thread's pair of the chunk's first 1024
-  s_before[tid] = 0;
-  s_rest[tid] = 0;
+  if constexpr (COUNTS != kFromWaves) {
+    s_before[tid] = 0;
+    s_rest[tid] = 0;
+  }
   for (int e = lane; e < E; e += 64) s_wave[w][e] = 0;
-  __syncthreads();
+  if constexpr (COUNTS != kFromWaves) __syncthreads();   // (the rows of s_wave are their wavefronts' own so far)
   constexpr int kBatch = 8;   // loads in flight
-  if constexpr (DIRECT) {
+  if constexpr (COUNTS == kFromIds) {
     for (long p0 = 0; p0 < num_pairs; p0 += kBatch * kRouteThreads) {
       int v[kBatch];
 #pragma unroll
@@ -120,7 +126,7 @@ __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, lo
         if (id >= 0) atomicAdd(first < base ? &s_before[id] : &s_rest[id], 1);   // (base is a multiple of 1024)
       }
     }
-  } else {
+  } else if constexpr (COUNTS == kFromChunks) {
     // the counts as one flat array: thread t takes the words t, t + 1024, ...
     const int words = (int)gridDim.x * E, mine = me * E;
     for (int i0 = 0; i0 < words; i0 += kBatch * kRouteThreads) {
@@ -138,6 +144,7 @@ __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, lo
     }
   }
   const int bits = id_bits(E);
+  const int waves = COUNTS == kFromWaves ? (int)blockDim.x >> 6 : kRouteWaves;
   int run = 0;   // thread e: next free row of expert e
   for (long off = 0;;) {
     const long p = base + off + tid;
@@ -147,9 +154,23 @@ __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, lo
     const int rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
     if (id >= 0 && rank == 0) s_wave[w][id] = __builtin_popcountll(same);
     __syncthreads();
+    int c[kRouteWaves];   // every wavefront's pairs of expert tid
+    auto counts = [&] {
+#pragma unroll
+      for (int i = 0; i < kRouteWaves; i++) c[i] = tid < E && i < waves ? s_wave[i][tid] : 0;
+    };
     if (off == 0) {
       // the offsets: prefix sums over the experts, thread = expert
-      const int before = s_before[tid], total = before + s_rest[tid], padded = (total + 127) & ~127;
+      int before = 0, total = 0;
+      if constexpr (COUNTS == kFromWaves) {
+        counts();
+#pragma unroll
+        for (int i = 0; i < kRouteWaves; i++) total += c[i];
+      } else {
+        before = s_before[tid];
+        total = before + s_rest[tid];
+      }
+      const int padded = (total + 127) & ~127;
       const int so = wave_inclusive_sum(total), sp = wave_inclusive_sum(padded);
       if (lane == 63) {
         s_sum[w][0] = so;
@@ -175,18 +196,17 @@ __global__ void __launch_bounds__(kRouteThreads) route_kernel(const int* ids, lo
         }
       }
     }
-    if (tid < E) {   // every wavefront's first row of expert tid
-      int c[kRouteWaves];
-#pragma unroll
-      for (int i = 0; i < kRouteWaves; i++) c[i] = s_wave[i][tid];
+    if (tid < E) {   // its first row of the expert
+      if constexpr (COUNTS != kFromWaves) counts();
 #pragma unroll
       for (int i = 0; i < kRouteWaves; i++) {
-        s_wave[i][tid] = run;
+        if (i < waves) s_wave[i][tid] = run;
         run += c[i];
       }
     }
     __syncthreads();
     if (p < num_pairs) dst_row[p] = id >= 0 ? s_wave[w][id] + rank : -1;
+    if constexpr (COUNTS == kFromWaves) break;
     off += kRouteThreads;
     if (off >= chunk || base + off >= num_pairs) break;   // the same for the whole workgroup
     raw = base + off + tid < num_pairs ? ids[base + off + tid] : 0;
@@ -288,15 +308,21 @@ extern "C" int esmoe_launch_route_metadata(const int* ids, long num_pairs, int f
   const long chunk = route_chunk_pairs(num_pairs);
   const int chunks = num_pairs > 0 ? (int)((num_pairs + chunk - 1) / chunk) : 1;
   // (ids that are overwritten by their rows, dst_row == ids: with several workgroups none may still count from the ids when
-  // another writes rows; route_kernel<false> reads a pair's id only in the thread that writes its row)
-  if (num_pairs <= kDirectPairs && (chunks == 1 || dst_row != ids)) {
-    hipLaunchKernelGGL(route_kernel<true>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
+  // another writes rows; route_kernel<kFromChunks> reads a pair's id only in the thread that writes its row)
+  if (num_pairs <= kRouteThreads) {
+    const int threads = ((int)num_pairs > num_experts ? (int)num_pairs + 63 : num_experts + 63) & ~63;
+    hipLaunchKernelGGL(route_kernel<kFromWaves>, dim3(1), dim3(threads), 0, stream, ids, num_pairs, first_expert, num_experts,
+                       chunk, (const int*)nullptr, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
+    return (int)hipGetLastError();
+  }
+  if (num_pairs <= kDirectPairs && dst_row != ids) {
+    hipLaunchKernelGGL(route_kernel<kFromIds>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
                        chunk, (const int*)nullptr, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(route_count_kernel, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
                      chunk, chunk_counts);
-  hipLaunchKernelGGL(route_kernel<false>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
+  hipLaunchKernelGGL(route_kernel<kFromChunks>, dim3(chunks), dim3(kRouteThreads), 0, stream, ids, num_pairs, first_expert, num_experts,
                      chunk, chunk_counts, n, k, problem_sizes, expert_offsets, blockscale_offsets, dst_row);
   return (int)hipGetLastError();
 }

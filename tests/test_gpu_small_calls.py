@@ -1,0 +1,13 @@
+"""The kernels around the GEMMs where a call is small: the edges of their small forms, against the same oracles as the large ones."""
+import pytest
+
+from tests import test_gpu_routing as R
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("pairs,experts,first,span", [(1, 1024, 0, 1024), (64, 65, 0, 65), (65, 64, 2, 70), (961, 7, 0, 9), (1024, 1024, 3, 1500),
+                                                      (1025, 40, 0, 40)])
+def test_route_metadata_of_one_workgroup(esmoe, pairs, experts, first, span):
+    """Up to 1024 pairs: as many wavefronts as hold the pairs or the experts, the counts from the wavefronts' own pairs."""
+    R.test_route_metadata_edges(esmoe, pairs, experts, first, span)
