@@ -26,9 +26,25 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
 constexpr int kActQuantThreads = 256;
-constexpr int kActQuantUnroll = 4;   // 16-byte loads in flight per lane
+// 16-byte loads in flight per lane: 4, or 1 where all wavefronts of the launch are resident at once (eight workgroups per CU): such a
+// launch is latency, and a good part of that is fetching its instructions, a quarter as many.  us, four loads through LDS lane swaps / as it
+// is: 8 x 4096 2.9 / 2.2, 64 x 7168 3.35 / 2.35, 256 x 4096 3.5 / 2.55, 1000 x 4096 3.9 / 3.15, 8192 x 512 4.1 / 3.0; four loads with the
+// maximum by DPP 1000 x 7168 4.4 / 4.25, 2048 x 4096 4.9 / 4.7, 8192 x 7168 28.05 / 27.8.
+constexpr long kActQuantSmall = 8L * 256 * kActQuantThreads;   // chunks
 
-template <bool FP16>
+// Maximum over the sixteen lanes of a row, through DPP (lane ^ 1, lane ^ 2, then the mirrors of eight and of sixteen lanes).  Every lane
+// has to be active.
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+  return __builtin_fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
+}
+__device__ __forceinline__ float row_max(float v) {
+  v = dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(v))));
+  asm volatile("" : "+v"(v));   // (keeps the exchanges in front of the stores' branch)
+  return v;
+}
+
+template <bool FP16, int kActQuantUnroll>
 __global__ void __launch_bounds__(kActQuantThreads) __attribute__((amdgpu_waves_per_eu(6, 8)))
 fp8_quant_act_kernel(const uint16_t* __restrict__ in, uint8_t* __restrict__ q, float* __restrict__ scales, long chunks) {
   // chunk c = 8 consecutive elements; 16 consecutive chunks form one 1x128 block
@@ -58,10 +74,7 @@ fp8_quant_act_kernel(const uint16_t* __restrict__ in, uint8_t* __restrict__ q, f
     float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; i++) amax = __builtin_fmaxf(amax, __builtin_fabsf(x[i]));
-    amax = __builtin_fmaxf(amax, __shfl_xor(amax, 1));
-    amax = __builtin_fmaxf(amax, __shfl_xor(amax, 2));
-    amax = __builtin_fmaxf(amax, __shfl_xor(amax, 4));
-    amax = __builtin_fmaxf(amax, __shfl_xor(amax, 8));
+    amax = row_max(amax);
     amax = __builtin_fmaxf(amax, 1e-4f);
     const float mult = (1.0f / amax) * 448.0f;   // two roundings, as torch does
     float y[8];
@@ -269,13 +282,16 @@ extern "C" int esmoe_launch_fp8_quant_act(const void* in, int in_dtype, void* q,
   using namespace esmoe;
   const long chunks = total_rows * (long)k / 8;
   if (chunks == 0) return 0;
-  const long per_wg = (long)kActQuantThreads * kActQuantUnroll;
-  const long grid = (chunks + per_wg - 1) / per_wg;
-  if (in_dtype == 1)
-    hipLaunchKernelGGL(fp8_quant_act_kernel<true>, dim3((unsigned)grid), dim3(kActQuantThreads), 0, stream,
-                       (const uint16_t*)in, (uint8_t*)q, scales, chunks);
-  else
-    hipLaunchKernelGGL(fp8_quant_act_kernel<false>, dim3((unsigned)grid), dim3(kActQuantThreads), 0, stream,
-                       (const uint16_t*)in, (uint8_t*)q, scales, chunks);
+  const int unroll = chunks <= kActQuantSmall ? 1 : 4;
+  const long per_wg = (long)kActQuantThreads * unroll;
+  const dim3 grid((unsigned)((chunks + per_wg - 1) / per_wg)), threads(kActQuantThreads);
+  const uint16_t* x = (const uint16_t*)in;
+  if (in_dtype == 1) {
+    if (unroll == 1) hipLaunchKernelGGL((fp8_quant_act_kernel<true, 1>), grid, threads, 0, stream, x, (uint8_t*)q, scales, chunks);
+    else hipLaunchKernelGGL((fp8_quant_act_kernel<true, 4>), grid, threads, 0, stream, x, (uint8_t*)q, scales, chunks);
+  } else {
+    if (unroll == 1) hipLaunchKernelGGL((fp8_quant_act_kernel<false, 1>), grid, threads, 0, stream, x, (uint8_t*)q, scales, chunks);
+    else hipLaunchKernelGGL((fp8_quant_act_kernel<false, 4>), grid, threads, 0, stream, x, (uint8_t*)q, scales, chunks);
+  }
   return (int)hipGetLastError();
 }

@@ -1,6 +1,8 @@
 """The kernels around the GEMMs where a call is small: the edges of their small forms, against the same oracles as the large ones."""
 import pytest
+import torch
 
+from tests import test_gpu_fp8_quant_act as A
 from tests import test_gpu_routing as R
 
 pytestmark = pytest.mark.gpu
@@ -11,3 +13,10 @@ pytestmark = pytest.mark.gpu
 def test_route_metadata_of_one_workgroup(esmoe, pairs, experts, first, span):
     """Up to 1024 pairs: as many wavefronts as hold the pairs or the experts, the counts from the wavefronts' own pairs."""
     R.test_route_metadata_edges(esmoe, pairs, experts, first, span)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 4096), (3, 640), (1024, 4096), (1025, 4096)])
+def test_quant_act_of_resident_launches(esmoe, dtype, shape):
+    """One 16-byte load per lane up to 1024 x 4096 values, four past that."""
+    A.test_quant_act_bit_exact(esmoe, dtype, shape)
