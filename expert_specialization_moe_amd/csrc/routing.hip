@@ -238,15 +238,17 @@ __global__ void __launch_bounds__(256) permute_rows_kernel(const uint8_t* __rest
   }
 }
 
-constexpr int kPermutePiece = 4096;           // four 16-byte loads in flight per lane
+// Pieces of 4096 bytes up to which they are cut in four: half a wavefront per SIMD, so that what counts is how long each takes.  us, as pieces
+// of 4096 / 1024 bytes: 1 token x 14 KB x top-8 2.9 / 2.4, 16 x 8 KB 3.5 / 2.6, 64 x 8 KB 3.75 / 3.1, 128 x 8 KB 4.0 / 3.4, 256 x 8 KB 4.5 / 4.4.
+constexpr long kPermuteSmall = 512;
 constexpr long kMaxPermutePieces = 1L << 22;     // of a launch (2^28 threads; a grid holds fewer than 2^32): larger inputs take several
 
-// The same packing for topk > 1 (at most 64): one wavefront per piece of 4096 bytes of a token's row reads it once and
+// The same packing for topk > 1 (at most 64): one wavefront per piece (4096 bytes, or 1024) of a token's row reads it once and
 // writes it to every local destination of the token's pairs, where one wavefront per pair would read it topk times.
 //
 // Bound by the output's bytes.  A wavefront per token walked the pieces one after the other: at 1003 tokens four wavefronts
-// per CU, each waiting for memory four times.  Pieces of 1024 bytes are slower (1003 tokens x 14336 bytes: 14.6 against
-// 12.7 us, 2048 x 8192: 27.4 / 24.7).
+// per CU, each waiting for memory four times.  Pieces of 1024 bytes are slower in calls of many (1003 tokens x 14336 bytes: 14.6
+// against 12.7 us, 2048 x 8192: 27.4 / 24.7).
 // Plain stores, where the launch moves more than 60 MB: the packed rows are what the caller quantises next, and what the
 // 256 MB cache keeps of them is not fetched from HBM.  Below that they are slower than the non-temporal ones: they leave the
 // rows dirty in the eight 4 MB L2s, and the launch's end waits until they are written back.  How many pairs have a local
@@ -256,6 +258,7 @@ constexpr long kMaxPermutePieces = 1L << 22;     // of a launch (2^28 threads; a
 //   700 x 14 KB x top-4, 38 MB:                   24.6 /  21.1 /  21.1      4096 x 4 KB x top-8, 1/8 local, 16 MB:  16.2 / 11.9 / 12.3
 //   1003 x 14 KB x top-8, 110 MB:                 48.5 /  53.8 /  48.5      4096 x 14 KB x top-8, 1/8 local, 56 MB: 36.0 / 37.3 / 36.1
 //   4096 x 8 KB x top-8, 256 MB:                 104.8 / 123.3 / 104.8      8192 x 14 KB x top-8, 1/64 local, 14 MB: 17.0 / 14.6 / 14.7
+template <int LOADS>   // 16-byte loads in flight per lane, of a piece of LOADS KB
 __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_t* __restrict__ in,
                                                                     const int* __restrict__ dst_row, uint32_t num_pieces,
                                                                     uint32_t pieces, int topk, long row_bytes, int plain_from,
@@ -267,11 +270,11 @@ __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_
   const uint32_t t = pieces == 1 ? piece : piece / pieces;
   const int mine = lane < topk ? dst_row[(long)t * topk + lane] : -1;   // lane j: destination of the token's pair j
   if (__ballot(mine >= 0) == 0) return;                               // no local pair: the row is not read
-  const long off = (long)(piece - t * pieces) * kPermutePiece + lane * 16;
+  const long off = (long)(piece - t * pieces) * LOADS * 1024 + lane * 16;
   const uint8_t* src = in + (long)t * row_bytes + off;
-  v4i v[4];
+  v4i v[LOADS];
 #pragma unroll
-  for (int u = 0; u < 4; u++)
+  for (int u = 0; u < LOADS; u++)
     if (off + u * 1024 < row_bytes) v[u] = __builtin_nontemporal_load((const v4i*)(src + u * 1024));
   // (behind the row's loads: the samples come from a cache and are there first)
   bool plain = false;
@@ -289,7 +292,7 @@ __global__ void __launch_bounds__(256) permute_rows_by_token_kernel(const uint8_
       if (dst < 0) continue;
       uint8_t* d = out + (long)dst * row_bytes + off;
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int u = 0; u < LOADS; u++)
         if (off + u * 1024 < row_bytes) {
           if constexpr (decltype(hint)::value) __builtin_nontemporal_store(v[u], (v4i*)(d + u * 1024));
           else *(v4i*)(d + u * 1024) = v[u];
@@ -332,12 +335,15 @@ extern "C" int esmoe_launch_permute_rows(const void* in, const int* dst_row, lon
   using namespace esmoe;
   if (num_pairs == 0) return 0;
   if (topk > 1 && topk <= 64 && num_pairs % topk == 0) {
-    const long tokens = num_pairs / topk, pieces = (row_bytes + kPermutePiece - 1) / kPermutePiece;
+    const long tokens = num_pairs / topk;
+    const int loads = tokens * ((row_bytes + 4095) / 4096) <= kPermuteSmall ? 1 : 4;
+    const long pieces = (row_bytes + loads * 1024 - 1) / (loads * 1024);
     const int plain_from = permute_plain_from(tokens, topk, row_bytes);
     const long step = pieces < kMaxPermutePieces ? kMaxPermutePieces / pieces : 1;   // tokens of a launch
     for (long t = 0; t < tokens; t += step) {
       const long n = tokens - t < step ? tokens - t : step;
-      hipLaunchKernelGGL(permute_rows_by_token_kernel, dim3((unsigned)((n * pieces + 3) / 4)), dim3(256), 0, stream,
+      auto kernel = loads == 1 ? permute_rows_by_token_kernel<1> : permute_rows_by_token_kernel<4>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((n * pieces + 3) / 4)), dim3(256), 0, stream,
                          (const uint8_t*)in + t * row_bytes, dst_row + t * topk, (uint32_t)(n * pieces), (uint32_t)pieces, topk, row_bytes,
                          n * topk >= kPermuteSamples ? plain_from : kPermuteSamples + 1, permute_sample_step(n * topk), (uint8_t*)out);
     }

@@ -20,3 +20,9 @@ def test_route_metadata_of_one_workgroup(esmoe, pairs, experts, first, span):
 def test_quant_act_of_resident_launches(esmoe, dtype, shape):
     """One 16-byte load per lane up to 1024 x 4096 values, four past that."""
     A.test_quant_act_bit_exact(esmoe, dtype, shape)
+
+
+@pytest.mark.parametrize("tokens,topk,row_elems", [(1, 2, 504), (3, 64, 520), (512, 2, 2040), (513, 2, 2040), (256, 2, 2056), (257, 3, 2056), (130, 2, 3 * 2048 + 520)])
+def test_permute_rows_on_both_sides_of_the_small_form(esmoe, tokens, topk, row_elems):
+    """Pieces of 1024 bytes up to 512 of 4096, of 4096 past that: rows that end inside a piece and inside a load."""
+    R.test_permute_rows_pieces(esmoe, tokens, topk, row_elems)
