@@ -21,7 +21,7 @@
 
 namespace esmoe {
 
-// Row-tile heights are MT * 16 rows with MT in {1, 2, 4, 8, 12} (sched_valid_mt); a workgroup tile
+// Row-tile heights are MT * 16 rows with MT in {1, 2, 4, 8, 12} (sched_valid_mt), with runs also 6 and 10; a workgroup tile
 // is (MT * 16) rows by 256 columns.
 struct SchedPolicy {
   int force_mt;   // 0 = choose per expert; else every tile uses this MT
