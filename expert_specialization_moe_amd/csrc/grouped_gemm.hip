@@ -1362,7 +1362,8 @@ struct Hand {
 static_assert(sizeof(Hand) == 64 && sizeof(Tile) == 64, "a word per lane (Words)");
 // A struct of sixteen words in one vector register, a word per lane: the hand-out's constants neither take scalar registers, which made
 // the fused kernels spill, nor are they read back from LDS, where the compiler first waits for everything that is outstanding, the last
-// tile's output stores among it (8 experts, 539 rows, 5760 x 256 18.7 -> 18.2 us).
+// tile's output stores among it (8 experts, 539 rows, 5760 x 256 18.7 -> 18.2 us).  Only for control flow that is the same in all lanes of
+// a wavefront: to the compiler `v` is a value of each lane, and where some are switched off a copy that it makes leaves their words behind.
 struct Words {
   int v;
   __device__ __forceinline__ explicit Words(const void* lds) : v(((const int*)lds)[threadIdx.x & 15]) {}
@@ -1900,7 +1901,8 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   // The last workgroup to leave zeroes the hand-out counters (nobody draws any more: every workgroup counts itself
   // out after its last draw), so a workspace that held zero counters before the launch holds them again after it.  A launch
   // of first tickets only has drawn from none.
-  if (threadIdx.x == 0 && hand[offsetof(Hand, undrawn)] != kAllQueues) {
+  const bool drawn = hand[offsetof(Hand, undrawn)] != kAllQueues;
+  if (drawn && threadIdx.x == 0) {
     const int left = atomicAdd(&ws[kWsExitCounter], 1);
     if (left == args.workgroups - 1) {
 #pragma unroll
