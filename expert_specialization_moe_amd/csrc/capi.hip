@@ -127,7 +127,9 @@ esmoe::SchedPolicy default_policy(int force_bm, int kind, int k) {
   p.order = 0;
   p.light_share = -1;
   // the fused fp8-blockwise epilogue quantises blocks that need a whole 256-row tile, and a forced height has no light items
-  p.narrow_tail = force_bm == 0 && (!(kind & 2) || (mx && k > 512)) ? kNarrowTail : 0;
+  const bool fused = kind & 2;
+  p.narrow_tail = force_bm == 0 && (!fused || (mx && k > 128)) ? kNarrowTail : 0;
+  p.narrow_fit = !fused ? 0 : k < 1024 ? 1 : 2;
   p.runs = force_bm == 0 && esmoe::sched_use_runs(k);
   return p;
 }
@@ -584,7 +586,7 @@ int esmoe_host_schedule(const int32_t* problem_sizes_host, int num_experts, int 
   ws_host[esmoe::kWsRun] = run;
   ws_host[esmoe::kWsHeavyBlocks] = run ? (blocks + esmoe::kBlkTiles - 1) / esmoe::kBlkTiles : blocks;
   ws_host[esmoe::kWsBlockLog] = run ? esmoe::kBlkLog : block_log;
-  const int split = esmoe::sched_light_split(items, p);
+  const int split = esmoe::sched_light_split(items, blocks, p.narrow_fit, p);
   ws_host[esmoe::kWsLightSplit] = split;
   ws_host[esmoe::kWsLightTotal] = split + 2 * (items - split);
   ws_host[esmoe::kWsLightCounter] = 0;

@@ -1317,7 +1317,7 @@ __global__ void __launch_bounds__(1024) schedule_kernel(const int* __restrict__ 
       const int run = policy.runs ? sched_run_tiles(blocks) : 0;
       ws[kWsRun] = run;
       ws[kWsHeavyBlocks] = run ? (blocks + kBlkTiles - 1) / kBlkTiles : blocks;
-      const int split = sched_light_split(items, policy);
+      const int split = sched_light_split(items, blocks, policy.narrow_fit, policy);
       ws[kWsLightSplit] = split;
       ws[kWsLightTotal] = split + 2 * (items - split);
       ws[kWsLightCounter] = 0;
@@ -1583,7 +1583,7 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
   }
   if (lane < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
   if (lane == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
-  const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
+  const int lsplit = FUSE && !MX ? items : sched_light_split(items, blocks, FUSE ? policy.narrow_fit : 0, policy), ltotal = lsplit + 2 * (items - lsplit);
   Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
   first_tile<MX, FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
   if (lane == 0) *out = h;
@@ -1726,7 +1726,7 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, H
   if (t < E) *(v4i*)(ws + ws_rec(pos)) = heavy ? v4i{before, 0, word, m} : v4i{blocks, before, word, m};
   if (t == 0) *(v4i*)(ws + ws_rec(E)) = v4i{blocks, items, -1, 0};
   static_assert(kRecBlock == 0 && kRecItem == 1 && kRecExpert == 2 && kRecRows == 3 && kRecWords == 4, "record layout");
-  const int lsplit = sched_light_split(items, policy), ltotal = lsplit + 2 * (items - lsplit);
+  const int lsplit = FUSE && !MX ? items : sched_light_split(items, blocks, FUSE ? policy.narrow_fit : 0, policy), ltotal = lsplit + 2 * (items - lsplit);
   Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
   first_tile<MX, FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
   if (t == 0) *out = h;

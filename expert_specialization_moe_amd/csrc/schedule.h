@@ -30,6 +30,7 @@ struct SchedPolicy {
                   // 2: most rows first for both kinds
   int light_share;  // workgroups (of every 32) that start on the light items; -1 = from the cost estimate
   int narrow_tail;  // the last so many light items are handed out as two 128-column halves each (0: none)
+  int narrow_fit;   // 1, 2: only where halves fill idle workgroups (sched_halves_fit; 1: of a launch of one round)
   int runs;         // 1: the queues hold runs of tiles instead of blocks, and last row tiles come in steps of 32 rows (sched_use_runs)
 };
 
@@ -250,8 +251,26 @@ ESMOE_HD TileCoord sched_decode_run(int local, int m, int n, int pair_rows) {
 // come out of one draw together and run as the whole tile again (sched_strip_tiles); only what a draw begins or ends with
 // stays a half.
 // Tickets [0, split) are the whole items 0 .. split-1, tickets split + 2j and split + 2j + 1 the halves of item split + j.
-ESMOE_HD int sched_light_split(int items, const SchedPolicy& p) {
-  const int narrow = p.narrow_tail < items ? p.narrow_tail : items;
+//
+// A fused launch's halves (MXFP8) are not much shorter than its whole items: both read all token rows, quantise and write.  They pay
+// only where they fill workgroups that would have nothing to do (`fit`, SchedPolicy::narrow_fit).  us, whole / halves:
+//   in a launch of one round of workgroups without heavy tiles where all halves are one round too: 52 items, K = 1536 14.5 / 11.1; 112,
+//     K = 1920 17.6 / 14.0; 100, K = 512 8.3 / 7.8; K = 128 5.8 / 5.9, not taken.  But 133 items, K = 1280 14.5 / 20.4, 189, K = 2944 29.5 /
+//     35.0; and beside heavy tiles, which last longer than any item, 18 + 126, K = 1280 22.1 / 25.7;
+//   in a longer one, from K = 1024 on, where up to half a round is left for the end: 264 items, K = 6784 108.0 / 90.7, 48 heavy tiles and
+//     222 items, K = 6016 96.4 / 86.2.  But 60 + 370 (174 left), K = 5632 106.8 / 112.8, 429 items (173), K = 4096 75.7 / 81.3; K = 768, 1290
+//     items 65.3 / 67.4;
+//   where a whole round of tall tiles runs before the items, whatever is left: 400 + 272, K = 7168 213.0 / 206.5, 1044 + 1152, K = 4096
+//     376.3 / 372.2.
+// 284 drawn fused launches of K = 128 to 7168 1.11 times as fast as with whole items (0.99 to 1.60); halves in every one 1.07 (0.68 to 1.60).
+ESMOE_HD bool sched_halves_fit(int items, int heavy, int fit) {   // `heavy`: heavy tiles
+  constexpr int kRound = kXcds * kBlkTiles;
+  if (items + heavy <= kRound) return heavy == 0 && 2 * items <= kRound;
+  const int last = (items + heavy) % kRound;
+  return fit > 1 && (heavy >= kRound || (last > 0 && 2 * last <= kRound));
+}
+ESMOE_HD int sched_light_split(int items, int heavy, int fit, const SchedPolicy& p) {
+  const int narrow = fit && !sched_halves_fit(items, heavy, fit) ? 0 : p.narrow_tail < items ? p.narrow_tail : items;
   return items - (narrow > 0 ? narrow : 0);
 }
 ESMOE_HD int sched_light_item_of_ticket(int ticket, int split, int* half) {

@@ -192,8 +192,8 @@ def test_fused_output_feeds_the_down_projection(esmoe):
 @pytest.mark.parametrize("rows", [[1, 16, 17, 32, 33, 64, 0, 50], [5] * 130, [300, 64, 1, 129]])
 @pytest.mark.parametrize("inter", [128, 384, 1536])
 def test_half_items_of_a_fused_launch(esmoe, inter, rows):
-    """From K = 640 on the last 128 light items go out as halves of 64 h columns: all of a launch's or its last ones, at every short
-    height, next to whole items and tall tiles.  Bit-exact against the separate route, padding and untouched bytes included."""
+    """Launches of up to 128 light items and nothing else go out as halves of 64 h columns, at every short height; the others here as
+    whole items, next to tall tiles too.  Bit-exact against the separate route, padding and untouched bytes included."""
     from expert_specialization_moe_amd import _native
     from expert_specialization_moe_amd import workloads as W
 
