@@ -1082,8 +1082,7 @@ __device__ __forceinline__ void gemm_tile_pp_mx(const GemmArgs& g, int e, int fi
   constexpr int kWSlot = kBN * 128 + 1024, kTSlot = GR * 128 + 1024;
   constexpr int kTBase = 3 * kWSlot, kSpare = kTBase + 4 * kTSlot;
   static_assert(kSpare + 1024 <= kLdsBytes, "LDS map of the split ring");
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));   // (as in gemm_tile: nothing of it is kept across tiles)
+  const int tid = threadIdx.x;   // (not hidden: the MXFP8 kernels have the registers to keep what is formed of it)
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2, wj = wave & 3;
@@ -1406,6 +1405,15 @@ __device__ __forceinline__ Hand first_hand(const GemmArgs& g, int hunits, int ru
   if (h.have > h.have_end) h.have = h.have_end;
   return h;
 }
+// The hand, and, in a launch with heavy experts, how many tickets every queue has (the light items last), counted once, a lane for a queue.
+// Counted anew for every draw, and for all queues in a row where a workgroup looks at all of them, it was the longest part of what a ticket
+// that is no tile costs.  us: 11 experts, 2234 rows, 2688 x 256 (MXFP8) 19.6 -> 17.9, 14 experts, 4553 rows, 4736 x 256 29.9 -> 29.1, 9
+// experts, 19591 rows, 4480 x 256 74.9 -> 72.4; launches of K > 512 of up to four rounds, which have no such tickets, 0.8 % on average.
+__device__ __forceinline__ void write_hand(const Hand& h, Hand* out, int* tickets) {
+  const int t = threadIdx.x;
+  if (h.heavy.blocks > 0 && t <= kXcds) tickets[t] = t < kXcds ? queue_tickets(h.heavy, t) : h.light.total;
+  if (t == 0) *out = h;
+}
 // Heavy tile or block of a ticket.
 __device__ __forceinline__ int heavy_index(int queue, int ticket, const HeavyHand& h) {
   return h.run ? sched_run_tile(queue, ticket, h.run) : sched_ticket_block(queue, ticket);
@@ -1487,7 +1495,7 @@ __device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool ligh
 // but as a whole: the hand-out has 500 clocks less to do.  8 experts x 32 rows, 256 x 512 6.4 -> 6.0 us, x 100 rows 10.5 -> 9.1, 64 x 200
 // rows, 512 x 512 13.6 -> 12.8.
 template <bool MX, bool FUSE>
-__device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, Tile* first) {
+__device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, int* tickets, Tile* first) {
   const int E = g.num_experts, lane = threadIdx.x;
   const SchedPolicy policy = g.policy;
   int* ws = g.ws;
@@ -1586,11 +1594,11 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
   const int lsplit = FUSE && !MX ? items : sched_light_split(items, blocks, FUSE ? policy.narrow_fit : 0, policy), ltotal = lsplit + 2 * (items - lsplit);
   Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
   first_tile<MX, FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
-  if (lane == 0) *out = h;
+  write_hand(h, out, tickets);
 }
 
 template <bool MX, bool FUSE>
-__device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, Tile* first) {
+__device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, int* tickets, Tile* first) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
   constexpr int kLightRows = 64, kHistStride = kLightRows + 4;
   int* s_hist = (int*)lds;                              // [kWaves][kHistStride]: experts of a wavefront by rows (0 .. 64)
@@ -1729,14 +1737,14 @@ __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, H
   const int lsplit = FUSE && !MX ? items : sched_light_split(items, blocks, FUSE ? policy.narrow_fit : 0, policy), ltotal = lsplit + 2 * (items - lsplit);
   Hand h = first_hand<FUSE>(g, blocks, run, block_log, ltotal, lsplit, lshare);
   first_tile<MX, FUSE>(g, h, light, heavy, before, mine, m, word, row, scale_row, first);
-  if (t == 0) *out = h;
+  write_hand(h, out, tickets);
 }
 
 template <bool MX, bool FUSE>
 __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   __shared__ int s_item;
-  __shared__ int s_counters[kXcds + 1];
+  __shared__ int s_counters[kXcds + 1], s_tickets[kXcds + 1];
   __shared__ Hand s_hand;
   __shared__ Tile s_tile;
   int* ws = args.ws;
@@ -1747,15 +1755,15 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   Tile tile;
   tile.mt = 0;
   if (args.self_schedule) {
-    if (args.num_experts > 64) self_schedule<MX, FUSE>(args, lds, &s_hand, &s_tile);
-    else if (threadIdx.x < 64) wave_schedule<MX, FUSE>(args, lds, &s_hand, &s_tile);
+    if (args.num_experts > 64) self_schedule<MX, FUSE>(args, lds, &s_hand, s_tickets, &s_tile);
+    else if (threadIdx.x < 64) wave_schedule<MX, FUSE>(args, lds, &s_hand, s_tickets, &s_tile);
     __syncthreads();
     const Words w(&s_tile);
     tile = {w[offsetof(Tile, mt)], w[offsetof(Tile, nt)], w[offsetof(Tile, cols)], w[offsetof(Tile, m0)], w[offsetof(Tile, n0)], w[offsetof(Tile, expert)],
             w[offsetof(Tile, rows)], w[offsetof(Tile, row)], w[offsetof(Tile, scale_row)], w[offsetof(Tile, taken)], {}};
   } else {
     const Hand h = first_hand<FUSE>(args, ws[ws_rec(args.num_experts) + kRecBlock], ws[kWsRun], ws[kWsBlockLog], ws[kWsLightTotal], ws[kWsLightSplit], ws[kWsLightShare]);
-    if (threadIdx.x == 0) s_hand = h;
+    write_hand(h, &s_hand, s_tickets);
     __syncthreads();
   }
   const Words hand(&s_hand);
@@ -1790,10 +1798,9 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
           continue;
         }
         const int draw = light ? sched_light_draw(lights.total, seen, g.workgroups, g.k >> 7, !FUSE) : 1;
-        const int total = light ? lights.total : queue_tickets(heavies, xq);
         if (threadIdx.x == 0) s_item = atomicAdd(light ? &ws[kWsLightCounter] : &ws[ws_xcd_counter(xq)], draw);
         __syncthreads();
-        const int ticket = (light ? lights.base : heavies.base) + uniform(s_item);
+        const int ticket = (light ? lights.base : heavies.base) + uniform(s_item), total = light ? lights.total : uniform(s_tickets[xq]);
         if (ticket >= total) {   // this queue is exhausted: see which others are
           dead |= 1 << (light ? 8 : xq);
           if (dead == kAllQueues) return false;
@@ -1804,11 +1811,8 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
             s_counters[threadIdx.x] = __hip_atomic_load(threadIdx.x < kXcds ? &ws[ws_xcd_counter(threadIdx.x)] : &ws[kWsLightCounter],
                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __syncthreads();
-#pragma unroll
-          for (int x = 0; x < kXcds; x++) {
-            if (heavies.base + uniform(s_counters[x]) >= queue_tickets(heavies, x)) dead |= 1 << x;
-          }
-          if (lights.base + uniform(s_counters[kXcds]) >= lights.total) dead |= 256;
+          const int x = threadIdx.x & 63, at = x <= kXcds ? x : kXcds;   // (a lane for a queue)
+          dead |= (int)__ballot((x < kXcds ? heavies.base : lights.base) + s_counters[at] >= s_tickets[at]) & kAllQueues;
           continue;
         }
         have = ticket;
