@@ -1454,21 +1454,6 @@ __device__ __forceinline__ Tile take_tile(const GemmArgs& g, bool light, int spl
 // Wave-uniform values that the compiler does not know to be.
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// The schedule built by the GEMM kernel itself (one launch per call; schedule.h, kSelfScheduleMaxExperts): every
-// workgroup does what schedule_kernel does and writes the records into `ws`, where the hand-out loop finds them with
-// scalar loads.  All workgroups write the same values.  The launch constants are returned instead of stored.  `lds` is
-// the ring, free before the first tile.  The workgroup's first tile goes into `first`, so that nothing in front of it waits for the
-// records' way to memory and back: the hand-out does before it reads one.
-//
-// This runs in front of every workgroup's first tile, so it is latency from end to end: trips to LDS, barriers and, at some five
-// clocks each, instructions.  Light experts (and empty ones) have at most 64 rows and the same number of items each, so a count
-// per row number puts them in order, and an expert's first item is its rank times that number.  Experts of one wavefront find
-// those of their row number with a ballot per bit.  Only heavy experts are compared with each other, packed into a list (all 512 threads
-// share the comparisons), and only they need a prefix sum.  Comparing all experts took 0.5 / 1.1 / 3.7 us at 8 / 32 / 256 experts and
-// the cost totals of a launch with both kinds 0.8 us.  Whole calls, first tickets without a draw (schedule.h, sched_first_tickets): 8 experts
-// x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting
-// instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us; half as many divisions and a four-way search of the records:
-// 75.2 -> 74.7 (with both kinds of experts), an expert MLP of 1003 tokens in MXFP8 377.5 -> 376.1.
 // The workgroup's first tile, by the thread of the expert that the ticket belongs to (items, tiles or blocks [before, before + mine)).
 template <bool MX, bool FUSE>
 __device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool light, bool heavy, int before, int mine, int rows, int word, int row,
@@ -1496,6 +1481,7 @@ __device__ __forceinline__ void first_tile(const GemmArgs& g, Hand& h, bool ligh
 // rows, 512 x 512 13.6 -> 12.8.
 template <bool MX, bool FUSE>
 __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, int* tickets, Tile* first) {
+  static_assert(kWaveScheduleMaxExperts <= 64, "a lane per expert, and its index in six bits of the sort key");
   const int E = g.num_experts, lane = threadIdx.x;
   const SchedPolicy policy = g.policy;
   int* ws = g.ws;
@@ -1597,6 +1583,21 @@ __device__ __forceinline__ void wave_schedule(const GemmArgs& g, uint8_t* lds, H
   write_hand(h, out, tickets);
 }
 
+// The schedule built by the GEMM kernel itself (one launch per call; schedule.h, kSelfScheduleMaxExperts): every
+// workgroup does what schedule_kernel does and writes the records into `ws`, where the hand-out loop finds them with
+// scalar loads.  All workgroups write the same values.  The launch constants go into `out` and `tickets`.  `lds` is
+// the ring, free before the first tile.  The workgroup's first tile goes into `first`, so that nothing in front of it waits for the
+// records' way to memory and back: the hand-out does before it reads one.
+//
+// This runs in front of every workgroup's first tile, so it is latency from end to end: trips to LDS, barriers and, at some five
+// clocks each, instructions.  Light experts (and empty ones) have at most 64 rows and the same number of items each, so a count
+// per row number puts them in order, and an expert's first item is its rank times that number.  Experts of one wavefront find
+// those of their row number with a ballot per bit.  Only heavy experts are compared with each other, packed into a list (all 512 threads
+// share the comparisons), and only they need a prefix sum.  Comparing all experts took 0.5 / 1.1 / 3.7 us at 8 / 32 / 256 experts and
+// the cost totals of a launch with both kinds 0.8 us.  Whole calls, first tickets without a draw (schedule.h, sched_first_tickets): 8 experts
+// x 32 rows, 256 x 512 9.2 -> 6.9 us, 32 x 8 x 7168 x 2048 77.0 -> 75.6 us, 256 x 32 x 7168 x 256 129.0 -> 125.8 us; counting
+// instead of comparing: 6.9 -> 6.4, 75.6 -> 75.3, 125.8 -> 121.9 us; half as many divisions and a four-way search of the records:
+// 75.2 -> 74.7 (with both kinds of experts), an expert MLP of 1003 tokens in MXFP8 377.5 -> 376.1.
 template <bool MX, bool FUSE>
 __device__ __forceinline__ void self_schedule(const GemmArgs& g, uint8_t* lds, Hand* out, int* tickets, Tile* first) {
   static_assert(kSelfScheduleMaxExperts <= kThreads, "one thread per expert");
@@ -1755,7 +1756,7 @@ __global__ void __launch_bounds__(kThreads) grouped_gemm_kernel(GemmArgs args) {
   Tile tile;
   tile.mt = 0;
   if (args.self_schedule) {
-    if (args.num_experts > 64) self_schedule<MX, FUSE>(args, lds, &s_hand, s_tickets, &s_tile);
+    if (args.num_experts > kWaveScheduleMaxExperts) self_schedule<MX, FUSE>(args, lds, &s_hand, s_tickets, &s_tile);
     else if (threadIdx.x < 64) wave_schedule<MX, FUSE>(args, lds, &s_hand, s_tickets, &s_tile);
     __syncthreads();
     const Words w(&s_tile);

@@ -106,9 +106,10 @@ ESMOE_HD bool sched_is_heavy(int m, const SchedPolicy& p) { return p.force_mt ? 
 // Sort key of the hand-out order (smallest first, ties by expert index).  The heavy experts and the light ones are
 // handed out from separate queues, so only the order inside each kind matters.  Light items: most rows first, the
 // longest items first.  Heavy experts: fewest rows first (order 0): the launch then ends on the tiles of the experts with
-// the most rows, whose many blocks spread over all eight XCD queues and whose operand panels are shared behind an L2,
-// where an expert of one block ends on a single queue and streams its own weights (measured against most rows first,
-// order 2: C4 -2.5 %, C3 at 2048 tokens -1.8 %, C1 and C3 at 8192 tokens -0.3 to -0.8 %).
+// the most rows, many of which share an operand panel behind an L2, where an expert of few rows streams its own weights.  Measured
+// against most rows first (order 2): where the queues hold runs, 36 drawn launches of more than a round of heavy tiles -2.8 % (-13 to
+// +0.2), 153 of experts of about the same size -0.4 % (-9 to +13); as blocks, where an expert of one block also ended on a single
+// queue, C4 -2.5 %, C3 at 2048 tokens -1.8 %, C1 and C3 at 8192 tokens -0.3 to -0.8 %.
 ESMOE_HD int sched_order_key(int m, const SchedPolicy& p) {
   if (p.order == 2 || !sched_is_heavy(m, p)) return (1 << 30) - m;
   return m;
@@ -124,14 +125,24 @@ ESMOE_HD int sched_mtiles(int m, const SchedPolicy& p) {
 // From K = 640 on the queues hold runs instead of blocks: all heavy tiles of the launch stand in one line, expert after expert, each
 // down its columns (of at most eight tiles), and queue x has the x-th, (x + 8)-th, ... run of 32 of them.  Every ticket is a tile: blocks
 // leave holes where they have fewer than 32 tiles, and a hole costs a draw and a look-up, 2 to 3 us.  32 tiles that stand together
-// are 4 to 16 whole columns, so what an XCD works on at a time are a few weight panels and the token rows of mostly one expert, however many
-// of its workgroups are on heavy tiles; a block of 6 x 4 tiles leaves eight of them to the next one, of other rows.  Fetched into L2
+// are 4 columns of eight tiles to 32 of one, so what an XCD works on at a time are a few weight panels and the token rows of mostly one
+// expert, however many of its workgroups are on heavy tiles; a block of 6 x 4 tiles leaves eight of them to the next one, of other rows.
+// (Nothing holds a column's tiles together: a run ends inside one where 32 is no multiple of its height, 191 of 286 times with 131072
+// rows, 128 experts, 3072 x 4096, and the column's panel then goes through two L2s, 0.2 GB in all.)  Fetched into L2
 // (MB): 131072 rows, 128 experts, 3072 x 4096 5400 -> 3870, 6579 rows, 32 experts, 4096 x 7168 1470 -> 1250, 4012 rows (MXFP8) 1255 -> 1100.  us:
 // 1646 -> 1596, 257.4 -> 251.3, 204.0 -> 197.2; 44 experts, 11384 rows, 768 x 640 (MXFP8) 29.0 -> 16.4, 10 experts, 974 rows, 4096 x 1024
-// 26.2 -> 16.7; 110 drawn shapes of K = 640 to 7168 1.11 times as fast, one in twelve 2 to 5 % slower (an expert's tiles then stand
-// in two runs).  Row by row instead of down the columns: -2 % on the large launches; one run of an eighth of the launch per queue:
-// +0.4 % on these, -0.6 % on the drawn ones.  Up to K = 512 the queues hold blocks, which is what the host mirrors have described of
-// such calls so far (runs: 70 drawn shapes 1.15 times as fast, 0.87 to 1.95).
+// 26.2 -> 16.7; 110 drawn shapes of K = 640 to 7168 1.11 times as fast.  Row by row instead of down the columns: -2 % on the large
+// launches; one run of an eighth of the launch per queue: +0.4 % on these, -0.6 % on the drawn ones.
+// Slower than blocks are launches of one to four rounds of heavy experts of about the same size, two row tiles each: tall and short tiles
+// alternate in a column, and where a few tiles are left for another round half of them are tall ones, while a block, laid row by row,
+// ends on the short row.  us, blocks / runs: 12 experts x 367 rows, 2816 x 3712 (MXFP8) 62.9 / 72.8, 24 x 194 rows, 2304 x 768 (MXFP8,
+// fused) 28.8 / 33.1, 22 x 256 rows, 3072 x 7040 199 / 204; but 28 x 232 rows, 2304 x 768 35.3 / 27.7, 100 x 201 rows, 512 x 1152 36.5 /
+// 32.6.  420 drawn launches of that kind 1.02 times as fast as with blocks (0.86 to 1.27), one in five more than 2 % slower.  Tried on
+// these: row by row -0.3 %, runs of equal length +0.2 %, most rows first -0.4 %, all last row tiles behind the others -6 % (a column's
+// panel is then read twice).
+// Up to K = 512 the queues hold blocks.  That line is not one of speed: the host mirrors and their tests hold such schedules.  53 drawn
+// launches of K = 128 to 512 with heavy experts are 1.10 times as fast with runs (0.92 to 1.86): those of few tiles gain most (11 experts,
+// 2234 rows, 2688 x 256 MXFP8 19.9 / 10.7 us), FP8 ones of many rounds lose (62552 rows, 175 experts, 4480 x 512 327 / 353).
 ESMOE_HD bool sched_use_runs(int k) { return k > 512; }
 // Tiles of a run: 32, one per CU of an XCD.  In launches of at most 512 an eighth or a sixteenth of them, so that the queues hold one or
 // two runs each and about as many tiles.
@@ -203,7 +214,9 @@ ESMOE_HD int sched_run_mtiles(int m) { return (m + kRunRows - 1) / kRunRows; }
 ESMOE_HD int sched_heavy_tiles(int m, int n) { return sched_run_mtiles(m) * sched_ntiles(n, 4); }
 // Most rows behind a first full tile that make two tall tiles of the expert's rows, of 128 and of 96 or 128, where 192 rows would leave a
 // short one to the rest.  For launches of up to 256 heavy tiles, all of one round: it lasts as long as its longest tile, and a short tile
-// beside a tall one, on the same panel, lasts longer than a tall one; for up to 512 from K = 4096 on.  `tiles`: of the launch.
+// beside a tall one, on the same panel, lasts longer than a tall one; for up to 512 from K = 4096 on (84 FP8 launches of 216 to 256 rows an
+// expert, 512 to 2560 columns, K = 4096 to 7168 1.08 times as fast, 0.975 to 1.22: 3 % slower 24 experts x 248 rows, 2560 x 5120, 1 to 1.5 %
+// 40 x 240 to 256 rows, 1024 x 7168).  `tiles`: of the launch.
 // us, 192 + rest against two tall tiles, 2048 columns.  14 experts x 208 rows MXFP8: K = 7168 66.1 / 43.8, K = 3200 35.5 / 26.3, K = 1024
 // 18.0 / 15.1; FP8: K = 7168 67.1 / 54.2, K = 3200 32.4 / 28.2, K = 2176 23.1 / 22.4, K = 2048 21.7 / 21.7.  14 x 256 rows MXFP8: K = 3200
 // 33.8 / 27.3, K = 1024 14.8 / 15.2; FP8: K = 4096 36.6 / 35.5, K = 3968 35.6 / 35.8.  Two rounds, 32 experts: x 208 rows MXFP8 K = 7168
@@ -498,8 +511,10 @@ ESMOE_HD int ws_words(int num_experts) { return kWsHeader + (num_experts + 1) * 
 
 // One launch per call: when the counters of a workspace are known to be zero (a workspace the library owns: it is
 // zeroed when it is allocated, and the last workgroup to leave a launch zeroes the counters again), the GEMM kernel
-// needs no schedule kernel in front of it: every workgroup ranks the experts with all of its 512 threads (so no more experts
-// than that), builds the records itself and writes them (the same values from every workgroup) for its own scalar loads.
+// needs no schedule kernel in front of it: every workgroup ranks the experts, builds the records itself and writes them (the same
+// values from every workgroup) for its own scalar loads.  Up to 64 experts its first wavefront does so alone, a lane for an expert,
+// while the others wait (wave_schedule), past that all of its 512 threads (self_schedule), so no more experts than that.
+constexpr int kWaveScheduleMaxExperts = 64;
 constexpr int kSelfScheduleMaxExperts = 512;
 
 }  // namespace esmoe

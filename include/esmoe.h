@@ -285,16 +285,21 @@ int esmoe_permute_rows(const void* in, const int32_t* dst_row, long num_pairs, i
  * Experts with more than 64 rows are "heavy": their tiles are handed out in blocks of 8 x 4 tiles, block b
  * to XCD b % 8, through one ticket counter per XCD; esmoe_host_decode_heavy maps ticket `ticket` of XCD `xcd`
  * to out5 = {expert, tile rows, tile cols, m0, n0} and returns 0, or 1 if the ticket falls outside the
- * expert's tile grid (the kernel skips it), or 2 if that XCD's queue is exhausted.  In a launch with K > 512 (the third
- * value of problem_sizes_host) and no forced tile height they are handed out in runs instead (word 6 of the workspace: tiles of a run):
- * all heavy tiles in one line, run r to XCD r % 8, every ticket a tile, last row tiles of 96 and 160 rows as well.
+ * expert's tile grid (the kernel skips it), or 2 if that XCD's queue is exhausted.  In a launch with K > 512
+ * and no forced tile height they are handed out in runs instead (word 6 of the workspace: tiles of a run):
+ * all heavy tiles in one line, run r to XCD r % 8, every ticket a tile, last row tiles of 96 and 160 rows as well.  The row tiles are then
+ * of 192 rows but for the last one; in launches of up to 512 heavy tiles an expert of 193 to 256 rows is a tile of 128 rows and one of 96
+ * or 128 instead, where that is faster for the launch's K (schedule.h, sched_pair_rows).
+ * K is the third value of problem_sizes_host's first expert.  A launch takes it from its tensors: a program whose device metadata serve
+ * both projections of an MLP writes each projection's own K there before it asks the mirrors.
  * The other experts are "light": one short tile per 256 columns from a launch-wide counter, except that the last 128
  * light items of a launch go out as two 128-column halves each (word 4 of the workspace is the first ticket that is a
  * half, word 1 the number of light tickets); esmoe_host_decode_light maps ticket `item` (< word 1) to out5 and returns
  * 0, or 1 for the second half of a last column tile that is only 128 columns wide (the kernel skips it).
  * kind: bit 0 clear describes the FP8-blockwise launch, set the MXFP8 launch (both cut experts into full tiles of 192
- * rows today); bit 1 set describes a launch with a fused SwiGLU epilogue, whose items all stay 256 columns wide, as do
- * those of a launch with a forced tile height.
+ * rows today); bit 1 set describes a launch with a fused SwiGLU epilogue.  FP8-blockwise its items all stay 256 columns wide, as do
+ * those of a launch with a forced tile height; MXFP8 the last 128 go out as halves only where these fill idle workgroups (schedule.h,
+ * sched_halves_fit: K > 128, from the number of items and of heavy tiles).
  * The mirrors describe the default policy; the ESMOE_* environment variables, which a launch reads once per process, do not
  * reach them.
  */
