@@ -127,6 +127,7 @@ esmoe::SchedPolicy default_policy(int force_bm, int kind, int k) {
   p.order = 0;
   p.light_share = -1;
   // the fused fp8-blockwise epilogue quantises blocks that need a whole 256-row tile, and a forced height has no light items
+  // (which of a fused MXFP8 launch's items, and why from these K on: sched_halves_fit)
   const bool fused = kind & 2;
   p.narrow_tail = force_bm == 0 && (!fused || (mx && k > 128)) ? kNarrowTail : 0;
   p.narrow_fit = !fused ? 0 : k < 1024 ? 1 : 2;
